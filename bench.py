@@ -266,7 +266,7 @@ def phase_kernel(phase, word, broadphase, threads=0, largest=0):
     fits a wavefront's slice, else it and k_sweep_colours)."""
     if phase == "sweeps":
         if word == 8:
-            return "k_solve_flow"
+            return "k_solve_ordered"
         if threads != 64:
             return "k_sweep_colours"
         return ("k_sweep_waves" if largest <= SWEEP_WAVE_MAX_BODIES

@@ -136,8 +136,7 @@ typedef struct shp_step_stats {
   int64_t misses;       /* contacts absent from last frame's cache */
   int32_t max_levels;   /* most colours of a world (coloured solver) */
   int32_t flags;        /* bit 0 pair overflow, 1 contact overflow,
-                           2 non-finite, 3 coloured schedule overflow,
-                           4 ordered solver stopped waiting (defect) */
+                           2 non-finite, 3 coloured schedule overflow */
   /* Solve quality after the last sweep (FP64 state), maxima over contacts
    * of: penetration depth, |min(lambda_n, Jn.v + b)| and
    * |lambda_t - clamp(lambda_t - Jt.v / mt, +-mu*lambda_n)|; for the last
@@ -357,7 +356,7 @@ shp_status shp_mlp_train(shp_mlp* m, const int32_t* indices, int32_t steps,
  * 5 contact scan, 6 world ranges, 7 contacts (constraintGen + warm-start
  * join), 8 learned inference, 9 solve set-up (the coloured solver: the wait
  * for the colouring and the manifold packing), 10 sweeps (k_sweep_colours or
- * k_solve_flow), 11 solve write-back (coloured: k_colour_unpack), 12 advance
+ * k_solve_ordered), 11 solve write-back (coloured: k_colour_unpack), 12 advance
  * + moveShapes + AABBs + solve quality (k_finish), 13 cache store; and 14
  * the coloured solver's colouring (k_colour), timed on the second stream,
  * where it overlaps phases 5-9. */
@@ -370,8 +369,7 @@ shp_status shp_batch_set_timing(shp_batch* b, int32_t enable);
 shp_status shp_batch_read_timing(shp_batch* b, double* ms_per_phase,
                                  int32_t* steps);
 /* Average microseconds per timed step of the solve's sub-phases in world 0:
- * ordered: 0 per-body ranks, 1 counter clearing and velocity staging,
- * 2 levels + level sort (level-synchronous worlds) + record packing, 3
+ * ordered: 0 the schedule's links, 1 velocity and lagrangian staging, 2 -, 3
  * warm-start pass and sweeps, 4 write-back; coloured: 0 colouring, 1 bucketing + packing +
  * velocity staging, 2 warm-start pass, 3 sweeps, 4 write-back. */
 shp_status shp_batch_read_solve_profile(shp_batch* b, double* us5);

@@ -20,18 +20,18 @@
 // stay 512 B below it for the kernels' own static LDS
 #define LDS_BYTES_PER_CU (160 * 1024)
 #define LDS_MAX_BYTES (LDS_BYTES_PER_CU - 512)
-// coloured solver: colour offsets per world; ordered solver: level bins
+// coloured solver: colour offsets per world
 #define COLOR_CAP 256
 // one wavefront per world in the coloured sweeps (solver_threads 64) for
 // worlds of up to this many bodies, SWEEP_WAVES wavefronts per workgroup
 #define SWEEP_WAVE_MAX_BODIES 1024
 #define SWEEP_WAVES 4
-#define LEVEL_CAP 4095
 // the coloured solver keeps a world's FP32 velocities (12 B per body) in
 // LDS up to this many bodies; beyond, in global memory
 #define VEL_LDS_MAX_BODIES ((LDS_MAX_BYTES - (2 * (COLOR_CAP + 3) + 2) * 4) / 12)
-// the ordered solver's compact FP64 record (doubles per contact)
-#define FLOW_RECORD_DOUBLES 21
+// the ordered solver's FP64 records (16-byte words per contact slot,
+// shp_records.h) and its global schedule scratch (words per contact slot)
+enum { FLOW_WORDS = 8, SCH_GLOB = 7 };
 // an LDS array's footprint: the compiler places each on a 16-byte boundary
 constexpr size_t lds16(size_t bytes) { return (bytes + 15) & ~(size_t)15; }
 // coloured solver records: 112 B per manifold and 64 B for its second
@@ -75,8 +75,7 @@ enum {
   SHP_FLAG_PAIR_OVERFLOW = 1,
   SHP_FLAG_CONTACT_OVERFLOW = 2,
   SHP_FLAG_NONFINITE = 4,
-  SHP_FLAG_SCHEDULE_OVERFLOW = 8,
-  SHP_FLAG_SOLVER_STALL = 16
+  SHP_FLAG_SCHEDULE_OVERFLOW = 8
 };
 
 struct Ctx {
@@ -125,21 +124,19 @@ struct Ctx {
   // coloured schedule: per pair its colour and its manifold slot
   int32_t* sched_level;   // pair_cap
   int32_t* sched_order;   // pair_cap
-  // ordered (dataflow) schedule: every (contact, dynamic side) listed in
-  // its body's segment, per contact {rank a, degree a, rank b, degree b},
-  // per-body offsets/cursors/counters for worlds too large for LDS
-  int32_t* flow_list;  // 2 x contact_cap
-  int4* flow_rk;       // contact_cap
-  int32_t *flow_off, *flow_cur;  // NB
-  // level of every contact and the contacts in level order
-  // (level-synchronous worlds), contact_cap each
-  int32_t *flow_lvl, *flow_order;
-  // contact constants packed for the solver (compact FP64 records in
-  // contact order for the ordered solver, FP32 records + FP64 lambdas in
-  // colour order for the coloured one)
+  // ordered solver: per contact its local bodies for the schedule
+  // (contact_cap); links, tokens and levels of worlds too large for LDS
+  // (SCH_GLOB x contact_cap, and per body); their velocities (NB) and
+  // lagrangians (contact_cap)
+  int2* sch_ab;
+  uint32_t* sch_glob;
+  int32_t *sch_off, *sch_first;
+  double4* gvel;
+  double2* glam;
+  // contact constants packed for the solver (FP64 records at the contacts'
+  // own slots for the ordered solver, FP32 records + FP64 lambdas in colour
+  // order for the coloured one)
   double* pk;
-  int32_t* pk_g;  // bodies a, b: 2 x contact_cap (ordered solver)
-  uint8_t* pk_f;  // flags per contact (ordered solver)
   ulonglong2* col_bu;  // per body: round priority, colours taken (large worlds)
   uint2* col_list;     // 2 x pair_cap: uncoloured manifolds, pair index and body word
   uint32_t* pair_ab;             // per pair: world-local bodies for the colouring (k_sat)
@@ -207,10 +204,9 @@ struct StepPlan {
   int ppb = 8;
   bool use_grid = false, grid_wide = false;  // grid broadphase; 16 lanes per body
   int solver = 0, warm = 0;
-  // ordered solver: lanes per world, dynamic LDS, velocities / counters in LDS
+  // ordered solver: lanes per world, dynamic LDS
   int solve_threads = 256;
   size_t solve_lds = 0;
-  bool solve_vlds = false, solve_clds = false;
   // coloured solver: lanes per world, dynamic LDS of the colouring, LDS pool
   int color_threads = 256;
   size_t color_lds = 0, color_pool = 0;

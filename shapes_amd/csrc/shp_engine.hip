@@ -18,7 +18,7 @@
 //                    coloured solver, after its k_colour (on a second
 //                    stream), also each manifold's record in colour order
 //   solve            warm-start application + Gauss-Seidel sweeps
-//                    (k_solve_flow, or k_sweep_colours + k_colour_unpack)
+//                    (k_solve_ordered, or k_sweep_colours + k_colour_unpack)
 //   k_finish         advance + moveShapes + AABBs (k_integrate's tiles) and
 //                    the solve quality maxima, in one launch
 //   k_cache_store    this frame's (key, lambda) become next frame's cache,
@@ -524,6 +524,15 @@ __device__ void contacts_of_pair(const Ctx& c, int p, int n, int& hits) {
     c.mcn[dst] = mcn;
     c.mct[dst] = mct;
     if (M >= 0) write_record_rows(P, M, k, im[2], im[5], jn[2], jn[5], jt[2], jt[5], bn, mcn, mct);
+    if (c.solver == SHP_SOLVER_ORDERED_F64) {
+      if (k == 0) {
+        const bool two = n > 1 && dst + 1 < c.contact_cap;
+        write_flow_head(c, dst, ga, gb, b0, flip ? neg(nn) : nn, im, two);
+      } else {
+        c.sch_ab[dst] = make_int2(-1, -1);
+      }
+      write_flow_con(c, dst, jn[2], jn[5], jt[2], jt[5], bn, mcn, mct);
+    }
     // warm start lookup in the descending cache segment [cache_lo,
     // cache_hi): the first entry <= key, then equality.  This frame's
     // contacts come in the same order and mostly persist, so the search
@@ -1131,7 +1140,7 @@ static void batch_buffers(const StepPlan& P, Ctx& c, int32_t** scan_part, std::v
   add(&c.jx, CC * 32);
   for (double** q : {&c.bn, &c.rax, &c.ray, &c.rbx, &c.rby, &c.mcn, &c.mct, &c.ln, &c.lt})
     add(q, CC * 8);
-  add(&c.warm, CC);
+  add(&c.warm, CC + 1);  // the ordered solver reads two at a time
   add(&c.cache_key, CC * 8);
   add(&c.cache_ln, CC * 8);
   add(&c.cache_lt, CC * 8);
@@ -1160,15 +1169,13 @@ static void batch_buffers(const StepPlan& P, Ctx& c, int32_t** scan_part, std::v
     add(&c.large_ids, std::max<size_t>(P.n_large, 1) * 4);
   }
   if (P.solver == SHP_SOLVER_ORDERED_F64) {
-    add(&c.pk, FLOW_RECORD_DOUBLES * CC * 8);
-    add(&c.pk_g, 2 * CC * 4);
-    add(&c.pk_f, CC);
-    add(&c.flow_list, 2 * CC * 4);
-    add(&c.flow_rk, CC * 16);
-    add(&c.flow_off, NB * 4);
-    add(&c.flow_cur, NB * 4);
-    add(&c.flow_lvl, CC * 4);
-    add(&c.flow_order, CC * 4);
+    add(&c.pk, FLOW_WORDS * (CC + 1) * 16);  // a manifold's loads take the next slot too
+    add(&c.sch_ab, CC * 8);
+    add(&c.sch_glob, SCH_GLOB * CC * 4);
+    add(&c.sch_off, NB * 4);
+    add(&c.sch_first, NB * 4);
+    add(&c.gvel, NB * 32);
+    add(&c.glam, CC * 16);
   } else {
     add(&c.pk, COLOR_PACK_FLOATS(PC) * 4);
     add(&c.sched_level, PC * 4);
@@ -1447,8 +1454,7 @@ void plan_launches(const StepPlan& P, bool infer, bool logging, std::vector<Laun
           (size_t)SWEEP_WAVES * P.sweep_slice * 4, 0);
     add("k_colour_unpack", P.g_unpack, 256, 0, 0);
   } else {
-    add("k_solve_flow", P.W, P.solve_threads, std::max<size_t>(P.solve_lds, 16),
-        ordered_static_lds(P.solve_threads));
+    add("k_solve_ordered", P.W, P.solve_threads, P.solve_lds, ordered_static_lds(P.solve_threads));
   }
   if (logging) add("k_mlp_log", P.g_log, 256, 0, 0);
   add("k_finish", P.g_finish_ni + P.g_finish_nq, INTEGRATE_THREADS, 0, FINISH_STATIC_LDS);

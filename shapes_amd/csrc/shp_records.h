@@ -1,6 +1,6 @@
-// shp_records.h - the coloured solver's manifold records: their layout,
-// and how one is written from a pair's contacts (by the contact kernel,
-// which has every value in registers) and patched by the learned warm start.
+// shp_records.h - the solvers' records: their layout, and how one is written
+// from a pair's contacts (by the contact kernel, which has every value in
+// registers); the coloured solver's are patched by the learned warm start.
 #pragma once
 
 #pragma clang fp contract(off)
@@ -117,6 +117,49 @@ __device__ __forceinline__ void write_null_record(const PackF& P, int M, int ga,
 __device__ __forceinline__ void patch_record_warm(const PackF& P, int M, int j, double ln, double lt) {
   write_record_lambda(P, M, j, ln, lt);
   atomicOr((int*)(rec_of(P.rec, M) + 2 * RB) + 2, j ? MFL_WARM1 : MFL_WARM0);
+}
+
+// The ordered solver's FP64 records, 8 words of 16 bytes per contact slot:
+// a manifold's head at its first contact,
+//   0 ux, uy (row normal, flip applied)  1 iml_a, imr_a  2 iml_b, imr_b
+//   3 mu, local bodies a | b << 32 with flags
+// and every contact's rows, for the lane of body a and the lane of body b
+//   4 jn2, jt2  5 jn5, jt5  6 0, mct  7 bn, mcn
+// The contact kernel writes them (it has every value in registers), so that
+// the solve, one workgroup per world, need not gather them: on one
+// 8192-polygon world that took 0.3 ms of one CU, here it adds 3 us.
+enum { FLOW_BODY = 0x1FFFFFFF, FLOW_BOUNCE = 0x20000000, FLOW_TWO = 0x40000000,
+       FLOW_STATIC = (int)0x80000000 };
+
+__device__ __forceinline__ double2* flow_rec(const Ctx& c, int k) {
+  return (double2*)c.pk + (long)k * FLOW_WORDS;
+}
+
+__device__ __forceinline__ void write_flow_head(const Ctx& c, int k, int ga, int gb, int b0, d2 u,
+                                                const double* im, bool two) {
+  double2* h = flow_rec(c, k);
+  const int la = (ga - b0) | (c.is_static[ga] ? FLOW_STATIC : 0);
+  const int lb = (gb - b0) | (c.is_static[gb] ? FLOW_STATIC : 0);
+  const int fl = (two ? FLOW_TWO : 0) | (hs_min(c.e[ga], c.e[gb]) != 0.0 ? FLOW_BOUNCE : 0);
+  h[0] = make_double2(u.x, u.y);
+  h[1] = make_double2(im[0], im[2]);
+  h[2] = make_double2(im[3], im[5]);
+  // pairMu (Friction.hs:46-48)
+  h[3] = make_double2((c.mu[ga] + c.mu[gb]) / 2.0,
+                      __longlong_as_double((long long)(uint32_t)(la | fl) |
+                                           ((long long)(lb | fl) << 32)));
+  c.sch_ab[k] = make_int2(la, lb);
+}
+
+// bn + 0: the bias with a bounce term of 0 (turns -0 into 0)
+__device__ __forceinline__ void write_flow_con(const Ctx& c, int k, double jn2, double jn5,
+                                               double jt2, double jt5, double bn, double mcn,
+                                               double mct) {
+  double2* w = flow_rec(c, k) + 4;
+  w[0] = make_double2(jn2, jt2);
+  w[1] = make_double2(jn5, jt5);
+  w[2] = make_double2(0.0, mct);
+  w[3] = make_double2(bn + 0.0, mcn);
 }
 
 }  // namespace shp

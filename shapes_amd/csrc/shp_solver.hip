@@ -1,701 +1,730 @@
-// shp_solver.hip - ordered FP64 (drop-in) solve: dataflow over per-body
-// counters.
+// shp_solver.hip - ordered FP64 (drop-in) solve: the sequential sweep run
+// as a schedule of independent items.
 //
 // The reference applies the cached lagrangians in descending key order
 // (applyCachedSlns, shapes/src/Physics/Solvers/Contact.hs:74-121) and then
 // sweeps the contacts `iterations` times in the same order (improveWorld,
-// :146-157).  Written as one sequence, item (p, k) is pass p of contact k
-// (pass 0 is the warm start) and the items run in (p, k) order.  An item
-// reads and writes the velocities of its two bodies and the lagrangians of
-// its own contact only, so it depends on nothing but the latest earlier
-// items touching one of its dynamic bodies.  For a dynamic body a touched
-// by d(a) contacts, with contact k at rank r_a(k) among them in key order,
-// the items on a are numbered p * d(a) + r_a(k) in sequence order.  A
-// per-body counter holds how many items on the body have completed: item
-// (p, k) runs when counter[a] == p * d(a) + r_a(k) and the same holds for
-// b, and on completion it raises both counters by one (a release store
-// after its velocity stores; the waiting side loads with acquire).  Every
-// read therefore sees exactly the values of the sequential sweep and the
-// result is the sequential result bit for bit, whatever the timing.  Static
-// bodies (both inverse masses 0) are read-only and carry no counter.
+// :146-157).  A pair's one or two contacts (a manifold) are adjacent in that
+// order, so the sequence is a sequence of items (p, m): pass p of manifold m
+// (pass 0 is the warm start), both contacts one after the other.  An item
+// reads and writes the velocities of its two bodies and its own lagrangians
+// only, so it depends on nothing but the latest earlier item on each of its
+// dynamic bodies.  Running every item as early as that allows - level by
+// level, an item one level after the later of its two predecessors, whatever
+// their passes - performs exactly the sequential floating-point operations
+// on the same inputs: the result is the sequential one bit for bit.  Static
+// bodies (both inverse masses 0) are read-only and order nothing.
 //
-// Lane t of the workgroup owns contacts t, t + T, t + 2T, ... and runs its
-// items in sequence order.  The earliest unfinished item of the world is
-// always ready (every earlier item is done) and it is its lane's current
-// item, and lanes wait on nothing but counters inside the loop, so the loop
-// always progresses.  As a bound that holds even if this argument were
-// broken by a defect, a lane that sees no item of the workgroup complete
-// for WAIT_LIMIT consecutive polls stops and raises SHP_FLAG_SOLVER_STALL.
-//
-// Which lane runs which item only changes the speed.  Sequence order per
-// lane (lane t: contacts t, t + T, ...) is ideal while a world has no more
-// contacts than lanes; beyond that a lane's second contact holds up its
-// next pass.  That still pays while velocities sit in LDS.  A world whose
-// velocities live in global memory and that has more contacts than lanes
-// runs level-synchronously instead: the dataflow computes, integer work
-// only, every contact's level in one pass (1 + the largest level of the
-// earlier contacts on its dynamic bodies; contacts of one level share no
-// dynamic body), the contacts are sorted by level, and each pass runs
-// level by level with a barrier between levels, the next level's records
-// loaded before the barrier.  Both give the sequential result bit for bit.
+// What bounds it is the chain of levels, so the levels run across the
+// passes (an 8192-polygon pile of 11.5-14.6 k manifolds and 9 passes has
+// about 200 of them where pass after pass has 1060, a column scene of 900
+// boxes 166 instead of 444), and a level costs the instructions of one
+// wavefront, 4.4 cycles each, hardly any latency beside them: so two lanes
+// share an item, and one wavefront in four makes the schedule beside the
+// others, which run it.
 //
 // One workgroup per world:
-//   1. degrees d(a) by atomics, prefix sum -> per-body segments; every
-//      (contact, side) is listed in its body's segment; rank r_a(k) = number
-//      of entries of the segment that precede it in key order
-//   2. counters are cleared, velocities staged in LDS when they fit
-//   3. level-synchronous worlds: levels, counting sort by level
-//   4. each contact's constants are packed into a compact record (the
-//      jacobian rows are rebuilt from the normal and the two cross terms,
-//      exactly: every other component is a sign change of the normal), in
-//      contact order or in level order
-//   5. dataflow loop over all items, or the passes level by level
-//   6. lagrangians and velocities are written back
+//   1. links: per body the manifolds on it in sequence order; a manifold's
+//      link on a body is the next manifold there, after the last one the
+//      first (of the next pass)
+//   2. the schedule (integer work only): a manifold holds a token count; an
+//      item that runs passes a token to the next manifold on each of its
+//      dynamic bodies, and a manifold with the tokens of all its dynamic
+//      sides is an item of the next level.  Three levels ahead of
+//   3. the items, level by level, a barrier after each: entry and record of
+//      the next level are loaded while the current one runs; velocities and
+//      lagrangians are in LDS when they fit
+//   4. velocities and lagrangians are written back
+// The links and tokens are 16-bit LDS arrays when they fit (6 bytes a
+// contact), else 32-bit arrays in global memory: the same code.
+//
+// Measured (this kernel; before, items waited on per-body counters or ran
+// pass after pass): 55-box pyramid 72 us (159), 900 boxes 61 us (741), 512
+// worlds of 8-1024 bodies 183 us (752), 8192 polygons 1.48 ms (3.45; there
+// the state is in global memory and its line accesses bound a level).
 #pragma clang fp contract(off)
 
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "shp_engine.h"
 #include "shp_geom.h"
+#include "shp_records.h"
 #include "shp_solve_common.h"
 
 using namespace shp;
 
-#define WAIT_LIMIT (1u << 20)
+// levels in flight: level l runs while level l + 3 is made from level l + 2
+#define RING 4
+// LDS of the levels' items (more go to global memory): 1016 (2040 with more
+// lanes) 16-bit items a level
+constexpr int front_bytes(int threads) { return RING * (threads > 256 ? 4096 : 2048); }
 
-// compact record fields (doubles), stride contact_cap
-enum {
-  FL_UX = 0,  // jn[3], jn[4]; jn[0..1] = -u, jt[3..4] = clockwise(u), jt[0..1] = -jt[3..4]
-  FL_UY,
-  FL_JN2,
-  FL_JN5,
-  FL_JT2,
-  FL_JT5,
-  FL_BN,
-  FL_RAX,
-  FL_RAY,
-  FL_RBX,
-  FL_RBY,
-  FL_MCN,
-  FL_MCT,
-  FL_MU,
-  FL_E,
-  FL_IMLA,
-  FL_IMRA,
-  FL_IMLB,
-  FL_IMRB,
-  FL_LN,
-  FL_LT,
-  FL_FIELDS
+// ---- items ------------------------------------------------------------------
+// Two lanes per item: the even lane has body a and the friction row's
+// lagrangian, the odd lane body b and the normal row's.
+
+__device__ __forceinline__ double dpp_pair(double x, bool from_odd) {
+  const int lo = __double2loint(x), hi = __double2hiint(x);
+  return from_odd ? __hiloint2double(__builtin_amdgcn_mov_dpp(hi, 0xF5, 0xf, 0xf, true),
+                                     __builtin_amdgcn_mov_dpp(lo, 0xF5, 0xf, 0xf, true))
+                  : __hiloint2double(__builtin_amdgcn_mov_dpp(hi, 0xA0, 0xf, 0xf, true),
+                                     __builtin_amdgcn_mov_dpp(lo, 0xA0, 0xf, 0xf, true));
+}
+// the value of the pair's odd / even lane, in both
+__device__ __forceinline__ double from_b(double x) { return dpp_pair(x, true); }
+__device__ __forceinline__ double from_a(double x) { return dpp_pair(x, false); }
+
+// An item: its manifold's first contact (world-local), top bit: pass 0.
+#define ITEM_WARM 0x80000000u
+
+// One lane's half of an item's record (shp_records.h), as loaded: nothing is
+// computed from it before the item runs, so that no instruction waits for
+// the loads of the next item.
+struct ORec {
+  uint32_t item;
+  uint16_t warm;     // the contacts' warm flags, a byte each
+  double2 u, m, q;   // row normal; this side's inverse masses; mu, ids
+  double2 a[2];      // per contact: this side's angular entries of the rows
+  double2 f[2];      // per contact: bias and effective mass of this lane's row
 };
 
-struct FRec {
-  double ux, uy, jn2, jn5, jt2, jt5, bn, rax, ray, rbx, rby, mcn, mct, mu, e;
-  double ima, ira, imb, irb, ln, lt;
-  int ga, gb, flags;  // flags: 1 a static, 2 b static, 4 warm
-};
-
-__device__ __forceinline__ void load_frec(const Ctx& c, int k, FRec& r) {
-  const double* P = c.pk;
-  const long CC = c.contact_cap;
-  r.ux = P[FL_UX * CC + k];
-  r.uy = P[FL_UY * CC + k];
-  r.jn2 = P[FL_JN2 * CC + k];
-  r.jn5 = P[FL_JN5 * CC + k];
-  r.jt2 = P[FL_JT2 * CC + k];
-  r.jt5 = P[FL_JT5 * CC + k];
-  r.bn = P[FL_BN * CC + k];
-  r.rax = P[FL_RAX * CC + k];
-  r.ray = P[FL_RAY * CC + k];
-  r.rbx = P[FL_RBX * CC + k];
-  r.rby = P[FL_RBY * CC + k];
-  r.mcn = P[FL_MCN * CC + k];
-  r.mct = P[FL_MCT * CC + k];
-  r.mu = P[FL_MU * CC + k];
-  r.e = P[FL_E * CC + k];
-  r.ima = P[FL_IMLA * CC + k];
-  r.ira = P[FL_IMRA * CC + k];
-  r.imb = P[FL_IMLB * CC + k];
-  r.irb = P[FL_IMRB * CC + k];
-  r.ln = P[FL_LN * CC + k];
-  r.lt = P[FL_LT * CC + k];
-  r.ga = c.pk_g[k];
-  r.gb = c.pk_g[CC + k];
-  r.flags = c.pk_f[k];
+__device__ __forceinline__ void load_orec(const Ctx& c, int c0, uint32_t item, int side, ORec& r) {
+  const int k = c0 + (int)(item & ~ITEM_WARM);
+  const double2* h = flow_rec(c, k);
+  const double2* hs = h + side;
+  r.item = item;
+  r.u = h[0];
+  r.q = h[3];
+  r.m = hs[1];
+  r.a[0] = hs[4];
+  r.f[0] = hs[6];
+  r.a[1] = hs[FLOW_WORDS + 4];  // the next slot, also when there is one contact
+  r.f[1] = hs[FLOW_WORDS + 6];
+  __builtin_memcpy(&r.warm, c.warm + k, 2);
 }
 
-// The full rows of contact k: non-flipped, jn = (-n, xa_n, n, xb_n) and
-// jt = (-cw(n), xa_t, cw(n), xb_t); flipped, the halves are swapped back
-// (shp_engine.hip, constraint generation), which gives the same shape with
-// u = -n.  So jn[3..4] = u, jn[0..1] = -u, jt[3..4] = clockwise(u) and
-// jt[0..1] = -jt[3..4] in both cases, and negation is exact.
-__device__ __forceinline__ void pack_flow(const Ctx& c, int k, int dst) {
-  const long CC = c.contact_cap;
-  const int ga = c.ga[k], gb = c.gb[k];
-  // every value is loaded before the first store, so the loads are not
-  // serialised behind stores the compiler cannot prove disjoint
-  double f[FL_FIELDS];
-  const d2 u = row_normal(c, k);
-  const double4 x = c.jx[k];
-  f[FL_UX] = u.x;
-  f[FL_UY] = u.y;
-  f[FL_JN2] = x.x;
-  f[FL_JN5] = x.y;
-  f[FL_JT2] = x.z;
-  f[FL_JT5] = x.w;
-  f[FL_BN] = c.bn[k];
-  f[FL_RAX] = c.rax[k];
-  f[FL_RAY] = c.ray[k];
-  f[FL_RBX] = c.rbx[k];
-  f[FL_RBY] = c.rby[k];
-  f[FL_MCN] = c.mcn[k];
-  f[FL_MCT] = c.mct[k];
-  f[FL_MU] = (c.mu[ga] + c.mu[gb]) / 2.0;  // pairMu (Friction.hs:46-48)
-  f[FL_E] = hs_min(c.e[ga], c.e[gb]);       // min bounciness
-  f[FL_IMLA] = c.iml[ga];
-  f[FL_IMRA] = c.imr[ga];
-  f[FL_IMLB] = c.iml[gb];
-  f[FL_IMRB] = c.imr[gb];
-  f[FL_LN] = c.ln[k];
-  f[FL_LT] = c.lt[k];
-  const uint8_t fl = (uint8_t)((c.is_static[ga] ? 1 : 0) | (c.is_static[gb] ? 2 : 0) | (c.warm[k] ? 4 : 0));
-  double* P = c.pk;
-#pragma unroll
-  for (int q = 0; q < FL_FIELDS; ++q) P[q * CC + dst] = f[q];
-  c.pk_g[dst] = ga;
-  c.pk_g[CC + dst] = gb;
-  c.pk_f[dst] = fl;
+__device__ __forceinline__ int orec_id(const ORec& r, int side) {
+  const long long ids = __double_as_longlong(r.q.y);
+  return (int)(side ? ids >> 32 : ids);
 }
 
-__device__ __forceinline__ void rows(const FRec& r, double* jn, double* jt, double* im) {
-  d2 t = clockwise(mk(r.ux, r.uy));
-  jn[0] = -r.ux;
-  jn[1] = -r.uy;
-  jn[2] = r.jn2;
-  jn[3] = r.ux;
-  jn[4] = r.uy;
-  jn[5] = r.jn5;
-  jt[0] = -t.x;
-  jt[1] = -t.y;
-  jt[2] = r.jt2;
-  jt[3] = t.x;
-  jt[4] = t.y;
-  jt[5] = r.jt5;
-  im[0] = r.ima;
-  im[1] = r.ima;
-  im[2] = r.ira;
-  im[3] = r.imb;
-  im[4] = r.imb;
-  im[5] = r.irb;
+__device__ __forceinline__ double flip_sign(double x, int mask) {
+  return __hiloint2double(__double2hiint(x) ^ mask, __double2loint(x));
 }
 
-// Velocity access: LDS (3 doubles per local body) or the global arrays.
-template <bool VLDS>
-struct Vel {
-  double* lds;
+// Velocities (3 doubles per local body in LDS, or gvel) and lagrangians (two
+// doubles per contact, normal first, in LDS or glam).  In global memory a
+// compute unit's loads and stores cost a cycle per line each instruction
+// touches, so there the pair's lanes share every access: lane 0 takes the
+// first 16 bytes of a body's word, lane 1 the rest, first body a's, then b's.
+template <bool VLDS, bool LLDS>
+struct OState {
+  double* vel;
+  double* lam;
   const Ctx* c;
-  int b0;
-  __device__ __forceinline__ void load(int g, double* v) const {
+  int b0, c0;
+  // la, lb: the item's bodies; v: this lane's own
+  __device__ __forceinline__ void load(int la, int lb, int side, double* v) const {
     if (VLDS) {
-      const double* p = lds + 3 * (g - b0);
+      const double* p = vel + 3 * (side ? lb : la);
       v[0] = p[0];
       v[1] = p[1];
       v[2] = p[2];
     } else {
-      v[0] = c->vx[g];
-      v[1] = c->vy[g];
-      v[2] = c->w[g];
+      const double2 a = ((const double2*)(c->gvel + b0 + la))[side];
+      const double2 b = ((const double2*)(c->gvel + b0 + lb))[side];
+      const double bx = from_a(b.x), by = from_a(b.y), aw = from_b(a.x);
+      v[0] = side ? bx : a.x;
+      v[1] = side ? by : a.y;
+      v[2] = side ? b.x : aw;
     }
   }
-  __device__ __forceinline__ void store(int g, const double* v) const {
+  __device__ __forceinline__ void store(int la, int lb, int side, bool fixed, const double* v) const {
     if (VLDS) {
-      double* p = lds + 3 * (g - b0);
+      double* p = vel + 3 * (side ? lb : la);
+      if (fixed) return;
       p[0] = v[0];
       p[1] = v[1];
       p[2] = v[2];
     } else {
-      c->vx[g] = v[0];
-      c->vy[g] = v[1];
-      c->w[g] = v[2];
+      // a static body's word gets its own velocity (no other item changes it)
+      const double bx = from_b(v[0]), by = from_b(v[1]), aw = from_a(v[2]);
+      ((double2*)(c->gvel + b0 + la))[side] = side ? make_double2(aw, 0.0) : make_double2(v[0], v[1]);
+      ((double2*)(c->gvel + b0 + lb))[side] = side ? make_double2(v[2], 0.0) : make_double2(bx, by);
     }
+  }
+  // this lane's lagrangian of contact k: the normal one in lane 1
+  __device__ __forceinline__ double load_lam(int k, int side) const {
+    if (LLDS) return lam[2 * k + 1 - side];
+    const double2 l = c->glam[c0 + k];
+    return side ? l.x : l.y;
+  }
+  __device__ __forceinline__ void store_lam(int k, int side, double l) const {
+    if (LLDS)
+      lam[2 * k + 1 - side] = l;
+    else
+      ((double*)(c->glam + c0 + k))[1 - side] = l;
   }
 };
 
-// useCache (Solvers/Contact.hs:100-114): applySln with the cached lambdas
-template <bool VLDS>
-__device__ __forceinline__ void warm_frec(const FRec& r, const Vel<VLDS>& V) {
-  double v[6], jn[6], jt[6], im[6];
-  rows(r, jn, jt, im);
-  V.load(r.ga, v);
-  V.load(r.gb, v + 3);
-  apply_lag(r.ln, jn, im, v);
-  apply_lag(r.lt, jt, im, v);
-  if (!(r.flags & 1)) V.store(r.ga, v);
-  if (!(r.flags & 2)) V.store(r.gb, v + 3);
+// One item.  Pass 0: useCache (Solvers/Contact.hs:
+// 100-114), applySln with the cached lambdas.  Later passes:
+// improveContactSln (:124-143), i.e. contactLagrangian with bounceB
+// (Constraints/Contact.hs:74-95, Restitution.hs:34-47), solutionProcessor =
+// positive / clampAbs (Constraints/Contact.hs:101-110,
+// SolutionProcessors.hs:33-53), applySln.  The contacts' rows are jn =
+// (-u, jn2, u, jn5) and jt = (-cw(u), jt2, cw(u), jt5): (sx, sy, jn) and
+// (sy, -sx, jt) on one side.  The rows' products are folded from index 0
+// on: the even lane folds body a's three, the odd lane goes on with body
+// b's.  Without restitution the bounce term is min 0 (0 * x) = 0.
+// GENERAL: some lane of the wavefront is in pass 0 or has restitution.
+template <bool GENERAL, bool VLDS, bool LLDS>
+__device__ __forceinline__ void run_item(const ORec& r, int side, const OState<VLDS, LLDS>& S) {
+  double v[3], lam[2];
+  const int k = (int)(r.item & ~ITEM_WARM);
+  const bool warm = GENERAL && (r.item & ITEM_WARM);
+  const int id = orec_id(r, side), la = orec_id(r, 0) & FLOW_BODY, lb = orec_id(r, 1) & FLOW_BODY;
+  const bool fixed = id < 0, two = (id & FLOW_TWO) != 0;  // FLOW_STATIC is the sign bit
+  S.load(la, lb, side, v);
+  lam[0] = S.load_lam(k, side);
+  lam[1] = two ? S.load_lam(k + 1, side) : 0.0;
+  const int neg_a = side ? 0 : (int)0x80000000;
+  const double sx = flip_sign(r.u.x, neg_a), sy = flip_sign(r.u.y, neg_a);
+  const double iml = r.m.x, imr = r.m.y;
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    if (j && !two) break;
+    const double l = lam[j];
+    const double n0 = sx, n1 = sy, n2 = r.a[j].x, t0 = sy, t1 = -sx, t2 = r.a[j].y;
+    const double pn0 = n0 * v[0], pn1 = n1 * v[1], pn2 = n2 * v[2];
+    const double pt0 = t0 * v[0], pt1 = t1 * v[1], pt2 = t2 * v[2];
+    const double an = from_a((pn0 + pn1) + pn2), at = from_a((pt0 + pt1) + pt2);
+    const double dn = ((an + pn0) + pn1) + pn2;  // odd lane
+    const double dt = from_b(((at + pt0) + pt1) + pt2);
+    double bias = r.f[j].x;
+    if (GENERAL && (id & FLOW_BOUNCE)) {
+      // closing = ((-va + zcross(-wa, ra)) + vb) + zcross(wb, rb)
+      const Ctx& c = *S.c;
+      const int kg = S.c0 + k + j;
+      const double es = c.e[S.b0 + (side ? lb : la)], e = hs_min(from_a(es), from_b(es));
+      const double rx = (side ? c.rbx : c.rax)[kg], ry = (side ? c.rby : c.ray)[kg];
+      const double w = side ? v[2] : -v[2];
+      const double zx = -(w * ry), zy = w * rx;
+      const double ax = from_a(-v[0] + zx), ay = from_a(-v[1] + zy);
+      const double cx = (ax + v[0]) + zx, cy = (ay + v[1]) + zy;  // odd lane
+      const double bb = hs_min(0.0, e * (cx * sx + cy * sy));
+      if (side) bias = bias + bb;
+    }
+    const double q = (-((side ? dn : dt) + bias)) / r.f[j].y;
+    const double m = hs_max(q, -l);
+    const double z = side ? m : q;
+    const double tot = l + z;
+    const double thr = from_b(tot * r.q.x);
+    double acc = tot;
+    if (!side) acc = tot > thr ? thr : (tot < -thr ? -thr : tot);
+    double app = side ? z : acc - l;
+    bool apply = !fixed;
+    if (warm) {  // the lagrangians as they are
+      acc = l;
+      app = l;
+      apply = apply && ((r.warm >> (8 * j)) & 0xFF) != 0;
+    }
+    S.store_lam(k + j, side, acc);
+    const double gn = from_b(app), gt = from_a(app);
+    // applyLagrangian (Constraint.hs:182-221), normal first; a static side
+    // keeps its velocity (the reference adds +-0 to it)
+    if (apply) {
+      v[0] = (v[0] + ((n0 * gn) * iml)) + ((t0 * gt) * iml);
+      v[1] = (v[1] + ((n1 * gn) * iml)) + ((t1 * gt) * iml);
+      v[2] = (v[2] + ((n2 * gn) * imr)) + ((t2 * gt) * imr);
+    }
+  }
+  S.store(la, lb, side, fixed, v);
 }
 
-// improveContactSln (Solvers/Contact.hs:124-143): contactLagrangian with
-// bounceB (Constraints/Contact.hs:74-95, Restitution.hs:34-47), then
-// solutionProcessor = positive / clampAbs (Constraints/Contact.hs:101-110,
-// SolutionProcessors.hs:33-53), then applySln, on a compact record.  The
-// new lagrangians go to the record and to the packed array.
-template <bool VLDS>
-__device__ __forceinline__ void improve_frec(const Ctx& c, int k, FRec& r, const Vel<VLDS>& V) {
-  double v[6], jn[6], jt[6], im[6];
-  rows(r, jn, jt, im);
-  V.load(r.ga, v);
-  V.load(r.gb, v + 3);
-  d2 ra = mk(r.rax, r.ray), rb = mk(r.rbx, r.rby), nr = mk(r.ux, r.uy);
-  d2 closing = add(add(add(neg(mk(v[0], v[1])), zcross(-v[2], ra)), mk(v[3], v[4])), zcross(v[5], rb));
-  double bb = hs_min(0.0, r.e * dot(closing, nr));
-  double bn = r.bn + bb;
-  double new_n = (-(dot6(jn, v) + bn)) / r.mcn;
-  double new_t = (-(dot6(jt, v) + 0.0)) / r.mct;
-  double app_n = hs_max(new_n, -r.ln);
-  double acc_n = r.ln + app_n;
-  double thr = acc_n * r.mu;
-  double acc_t = r.lt + new_t;
-  double accp = acc_t > thr ? thr : (acc_t < -thr ? -thr : acc_t);
-  double app_t = accp - r.lt;
-  apply_lag(app_n, jn, im, v);
-  apply_lag(app_t, jt, im, v);
-  if (!(r.flags & 1)) V.store(r.ga, v);
-  if (!(r.flags & 2)) V.store(r.gb, v + 3);
-  const long CC = c.contact_cap;
-  r.ln = acc_n;
-  r.lt = accp;
-  c.pk[FL_LN * CC + k] = acc_n;
-  c.pk[FL_LT * CC + k] = accp;
-}
+// ---- schedule ---------------------------------------------------------------
 
-__device__ __forceinline__ int ld_acquire(int* p) {
-  return __hip_atomic_load(p, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP);
-}
-__device__ __forceinline__ void st_release(int* p, int v) {
-  __hip_atomic_store(p, v, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
-}
-
-// Exclusive prefix sum of a[0, n) in place by the T threads of the
-// workgroup; wsum holds T / 64 ints of LDS.
+// Exclusive prefix sum over the T threads of one value each.  wsum holds T / 64 ints of LDS.
 template <int T>
-__device__ void block_scan_exclusive(int* a, int n, int* wsum) {
+__device__ __forceinline__ int block_exclusive(int s, int* wsum) {
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
-  const int chunk = (n + T - 1) / T;
-  const int lo = min(n, tid * chunk), hi = min(n, lo + chunk);
-  int s = 0;
-  for (int i = lo; i < hi; ++i) s += a[i];
   int x = s;
   for (int o = 1; o < 64; o <<= 1) {
-    int y = __shfl_up(x, o);
+    const int y = __shfl_up(x, o);
     if (lane >= o) x += y;
   }
+  __syncthreads();  // wsum may still be read from an earlier call
   if (lane == 63) wsum[wid] = x;
   __syncthreads();
-  if (tid == 0) {
-    int acc = 0;
-    for (int q = 0; q < T / 64; ++q) {
-      int t = wsum[q];
-      wsum[q] = acc;
-      acc += t;
-    }
-  }
-  __syncthreads();
-  int run = wsum[wid] + x - s;
-  for (int i = lo; i < hi; ++i) {
-    int t = a[i];
-    a[i] = run;
-    run += t;
-  }
-  __syncthreads();
-}
-
-// Ranks of every (contact, dynamic side) of world contacts [c0, c0 + n):
-// flow_rk[k] = {r_a, d(a), r_b, d(b)}, with r = -1 for a static side.
-// off and cur hold nb ints each (LDS or global, local body index).
-template <int T>
-__device__ void compute_ranks(const Ctx& c, int c0, int n, int b0, int nb, int* off, int* cur,
-                              int* wsum) {
-  const int tid = threadIdx.x;
-  int* list = c.flow_list + 2L * c0;
-  for (int i = tid; i < nb; i += T) off[i] = 0;
-  __syncthreads();
-  for (int i = tid; i < n; i += T) {
-    int ga = c.ga[c0 + i], gb = c.gb[c0 + i];
-    if (!c.is_static[ga]) atomicAdd(&off[ga - b0], 1);
-    if (!c.is_static[gb]) atomicAdd(&off[gb - b0], 1);
-  }
-  __syncthreads();
-  block_scan_exclusive<T>(off, nb, wsum);
-  for (int i = tid; i < nb; i += T) cur[i] = off[i];
-  __syncthreads();
-  for (int i = tid; i < n; i += T) {
-    int ga = c.ga[c0 + i], gb = c.gb[c0 + i];
-    if (!c.is_static[ga]) list[atomicAdd(&cur[ga - b0], 1)] = 2 * i;
-    if (!c.is_static[gb]) list[atomicAdd(&cur[gb - b0], 1)] = 2 * i + 1;
-  }
-  __syncthreads();
-  // segment of body x: [off[x], cur[x]); entries are 2 * contact + side,
-  // so ascending entries are ascending key order
-  for (int i = tid; i < n; i += T) {
-    int4 rk = make_int4(-1, 0, -1, 0);
-    int g[2] = {c.ga[c0 + i], c.gb[c0 + i]};
+  int before = 0;
 #pragma unroll
-    for (int s = 0; s < 2; ++s) {
-      if (c.is_static[g[s]]) continue;
-      int x = g[s] - b0, lo = off[x], hi = cur[x], me = 2 * i + s, r = 0;
-      for (int j = lo; j < hi; ++j) r += list[j] < me;
-      if (s == 0) {
-        rk.x = r;
-        rk.y = hi - lo;
-      } else {
-        rk.z = r;
-        rk.w = hi - lo;
-      }
-    }
-    c.flow_rk[c0 + i] = rk;
-  }
-  __syncthreads();
+  for (int q = 0; q < T / 64; ++q) before += q < wid ? wsum[q] : 0;
+  return before + x - s;
 }
 
-// Bounded waiting shared by the dataflow loops: every wave iteration in
-// which some lane completed an item adds to the workgroup's progress count;
-// a lane that sees the count unchanged for WAIT_LIMIT consecutive polls
-// stops (SHP_FLAG_SOLVER_STALL).  Returns false when the lane must stop.
-struct Waiter {
-  unsigned spins = 0;
-  int seen = -1;
-  __device__ __forceinline__ bool after_poll(const Ctx& c, bool ready, int* progress) {
-    const unsigned long long m = __ballot(ready);
-    if (m) {
-      if ((int)(threadIdx.x & 63) == __ffsll((long long)m) - 1) atomicAdd(progress, __popcll(m));
+// All LDS accesses of the workgroup before this point precede all after it;
+// global loads and stores stay in flight.
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// Schedule state of one world.  A manifold is named by its first contact
+// (world-local index).  L: 16-bit entries in LDS, else 32-bit ones in global
+// memory.  A link is a manifold, with its top bit set when that manifold has
+// one dynamic side only; NONE ends a static side.
+template <bool L>
+struct Sched {
+  using E = std::conditional_t<L, uint16_t, uint32_t>;
+  static constexpr uint32_t NONE = L ? 0xFFFFu : 0xFFFFFFFFu;
+  static constexpr uint32_t ONE = L ? 0x8000u : 0x80000000u;
+  E* next;   // 2 per contact slot: the next manifold on body a, on body b
+  E* cnt;    // tokens received, a one-sided manifold's counting twice; the
+             // per-body lists while the links are built
+  E* off;    // per body (build): end of its list of manifolds it is body b of
+  E* first;  // per body (build): the first manifold it is body a of
+  // adds v to p[i], returns the old value
+  __device__ __forceinline__ static uint32_t add(E* p, uint32_t i, uint32_t v) {
+    if constexpr (L) {  // half of an LDS word (no half ever overflows)
+      const uint32_t sh = 16u * (i & 1u);
+      const uint32_t o = __hip_atomic_fetch_add((uint32_t*)p + (i >> 1), v << sh, __ATOMIC_RELAXED,
+                                                __HIP_MEMORY_SCOPE_WORKGROUP);
+      return (o >> sh) & 0xFFFFu;
     } else {
-      __builtin_amdgcn_s_sleep(1);
+      return __hip_atomic_fetch_add(p + i, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     }
-    if (ready) {
-      spins = 0;
-      return true;
+  }
+  __device__ __forceinline__ uint32_t count(uint32_t m) const {
+    const uint32_t* p = L ? (const uint32_t*)cnt + (m >> 1) : (const uint32_t*)cnt + m;
+    const uint32_t x = __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    return L ? (x >> (16u * (m & 1u))) & 0xFFFFu : x;
+  }
+  // the manifolds body x is body b of: cnt[lo, hi), unordered
+  __device__ __forceinline__ uint32_t lo(int x) const { return x ? off[x - 1] : 0u; }
+  __device__ __forceinline__ uint32_t list_min(int x, int above) const {
+    uint32_t best = NONE;
+    for (uint32_t q = lo(x), hi = off[x]; q < hi; ++q) {
+      const uint32_t t = cnt[q];
+      if ((int)(t & ~ONE) > above && (t & ~ONE) < (best & ~ONE)) best = t;
     }
-    int pr = __hip_atomic_load(progress, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    if (pr != seen) {
-      seen = pr;
-      spins = 0;
-    } else if (++spins > WAIT_LIMIT) {
-      atomicOr(&c.counters[CNT_FLAGS], SHP_FLAG_SOLVER_STALL);
-      return false;
-    }
-    return true;
+    return best;
+  }
+  // the first manifold on body x: the pairs of larger bodies come first
+  __device__ __forceinline__ uint32_t first_of(int x) const {
+    const uint32_t t = list_min(x, -1);
+    return t != NONE ? t : (uint32_t)first[x];
   }
 };
 
-// Whether item (p, contact with ranks rk) may run: both counters at its
-// rank for pass p.  la/lb: local body indices.
-__device__ __forceinline__ bool item_ready(int* cnt, int la, int lb, int4 rk, int p) {
-  bool ready = true;
-  if (rk.x >= 0) ready = ld_acquire(cnt + la) == p * rk.y + rk.x;
-  if (ready && rk.z >= 0) ready = ld_acquire(cnt + lb) == p * rk.w + rk.z;
-  return ready;
-}
-
-__device__ __forceinline__ void item_done(int* cnt, int la, int lb, int4 rk, int p) {
-  if (rk.x >= 0) st_release(cnt + la, p * rk.y + rk.x + 1);
-  if (rk.z >= 0) st_release(cnt + lb, p * rk.w + rk.z + 1);
-}
-
-// Lane order "cyclic": lane t runs (p, t), (p, t + T), ... for p = 0, 1,
-// ..., which is sequence order.  With at most one contact per lane this is
-// the best order (a lane's items are then one contact's passes, which
-// depend on each other anyway).  cnt: per-body counters, cleared.
-template <bool VLDS, int T>
-__device__ void run_flow(const Ctx& c, int c0, int n, int b0, int* cnt, const Vel<VLDS>& V,
-                         int* progress) {
+// Links of the world's manifolds and the tokens of pass 0.  ab: per contact
+// its local bodies (FLOW_STATIC set for a static one), -1 for the second
+// contact of a manifold.
+template <int T, bool L>
+__device__ __forceinline__ void build_links(const Sched<L>& S, const int2* ab, int n, int nb,
+                                            int* wsum) {
+  using E = typename Sched<L>::E;
+  constexpr uint32_t NONE = Sched<L>::NONE, ONE = Sched<L>::ONE;
   const int tid = threadIdx.x;
-  const int P = c.iterations;
-  int i = tid, p = 0;
-  bool live = i < n;
-  FRec r;
-  int4 rk = make_int4(-1, 0, -1, 0);
-  if (live) {
-    load_frec(c, c0 + i, r);
-    rk = c.flow_rk[c0 + i];
-  }
-  Waiter wt;
-  while (live) {
-    const int la = r.ga - b0, lb = r.gb - b0;
-    const bool ready = item_ready(cnt, la, lb, rk, p);
-    if (ready) {
-      if (p == 0) {
-        if (r.flags & 4) warm_frec<VLDS>(r, V);
-      } else {
-        improve_frec<VLDS>(c, c0 + i, r, V);
-      }
-      item_done(cnt, la, lb, rk, p);
-      int ni = i + T, np = p;
-      if (ni >= n) {
-        ni = tid;
-        ++np;
-      }
-      if (np > P) {
-        live = false;
-      } else {
-        if (ni != i) {
-          load_frec(c, c0 + ni, r);
-          rk = c.flow_rk[c0 + ni];
-        }
-        i = ni;
-        p = np;
-      }
-    }
-    if (!wt.after_poll(c, ready, progress)) live = false;
-  }
-}
-
-// Level of every contact in one pass (the same counters, integer work
-// only, cyclic lane order): lvl[k] = 1 + max(level of the previous contact
-// on a, on b), with last[] holding per body the level of its latest
-// contact (cleared).  Returns the lane's largest level.
-template <int T>
-__device__ int run_levels(const Ctx& c, int c0, int n, int b0, int* cnt, int* last, int* lvl,
-                          int* progress) {
-  const int tid = threadIdx.x;
-  const int P = 0;
-  int i = tid, p = 0, maxl = 0;
-  bool live = i < n;
-  int la = 0, lb = 0;
-  int4 rk = make_int4(-1, 0, -1, 0);
-  if (live) {
-    la = c.ga[c0 + i] - b0;
-    lb = c.gb[c0 + i] - b0;
-    rk = c.flow_rk[c0 + i];
-  }
-  Waiter wt;
-  while (live) {
-    const bool ready = item_ready(cnt, la, lb, rk, p);
-    if (ready) {
-      int l = 0;
-      if (rk.x >= 0) l = last[la];
-      if (rk.z >= 0) l = max(l, last[lb]);
-      ++l;
-      if (rk.x >= 0) last[la] = l;
-      if (rk.z >= 0) last[lb] = l;
-      lvl[i] = l;
-      maxl = max(maxl, l);
-      item_done(cnt, la, lb, rk, p);
-      int ni = i + T, np = p;
-      if (ni >= n) {
-        ni = tid;
-        ++np;
-      }
-      if (np > P) {
-        live = false;
-      } else {
-        if (ni != i) {
-          la = c.ga[c0 + ni] - b0;
-          lb = c.gb[c0 + ni] - b0;
-          rk = c.flow_rk[c0 + ni];
-        }
-        i = ni;
-        p = np;
-      }
-    }
-    if (!wt.after_poll(c, ready, progress)) live = false;
-  }
-  return maxl;
-}
-
-// Counting sort of the n contacts by level (levels 1..maxl): order[s]
-// gets the contact of slot s, and bins[l] (LDS, maxl + 1 ints) ends as the
-// end of level l's slots (level l = [bins[l - 1], bins[l]), bins[0] = 0).
-template <int T>
-__device__ void sort_by_level(const int* lvl, int n, int maxl, int* bins, int* order, int* wsum) {
-  const int tid = threadIdx.x;
-  for (int l = tid; l <= maxl; l += T) bins[l] = 0;
-  __syncthreads();
-  for (int q = tid; q < n; q += T) atomicAdd(&bins[lvl[q]], 1);
-  __syncthreads();
-  block_scan_exclusive<T>(bins, maxl + 1, wsum);
-  for (int q = tid; q < n; q += T) order[atomicAdd(&bins[lvl[q]], 1)] = q;
-  __syncthreads();
-}
-
-// Pass p over slot-ordered records, level by level.  Thread t takes slots
-// start(l) + t, + T, ... of every level, so a slot keeps its thread in
-// every pass and the lagrangians it wrote last pass are its own; the
-// record of its first slot of the next level (lagrangians included) is
-// loaded before the barrier, the velocities after it.
-template <bool VLDS, int T>
-__device__ void run_pass_levels(const Ctx& c, int c0, int p, int maxl, const int* bins,
-                                const Vel<VLDS>& V) {
-  const int tid = threadIdx.x;
-  FRec r, rn;
-  int s = tid;  // level 1 starts at slot 0
-  bool has = maxl >= 1 && s < bins[1];
-  if (has) load_frec(c, c0 + s, r);
-  for (int l = 1; l <= maxl; ++l) {
-    const int end = bins[l];
-    const int sn = end + tid;
-    const bool hasn = l < maxl && sn < bins[l + 1];
-    if (hasn) load_frec(c, c0 + sn, rn);
-    if (has) {
-      if (p == 0) {
-        if (r.flags & 4) warm_frec<VLDS>(r, V);
-      } else {
-        improve_frec<VLDS>(c, c0 + s, r, V);
-      }
-    }
-    for (int s2 = s + T; s2 < end; s2 += T) {
-      FRec r2;
-      load_frec(c, c0 + s2, r2);
-      if (p == 0) {
-        if (r2.flags & 4) warm_frec<VLDS>(r2, V);
-      } else {
-        improve_frec<VLDS>(c, c0 + s2, r2, V);
-      }
-    }
-    __syncthreads();
-    r = rn;
-    has = hasn;
-    s = sn;
-  }
-}
-
-// CLDS: per-body offsets/counters in LDS (else in flow_off/flow_cur);
-// VLDS: velocities in LDS.
-template <bool CLDS, bool VLDS, int T>
-__global__ __launch_bounds__(T) void k_solve_flow(Ctx c) {
-  extern __shared__ double lds_d[];
-  __shared__ int wsum[T / 64];
-  __shared__ int progress;
-  __shared__ int s_maxl;
-  const int w = c.world_order[blockIdx.x];
-  const int tid = threadIdx.x;
-  const int c0 = c.wcont_off[w], c1 = c.wcont_off[w + 1];
-  if (c1 <= c0) return;
-  const int n = c1 - c0;
-  const int b0 = c.body_off[w], nb = c.body_off[w + 1] - b0;
-  double* vel = lds_d;
-  int* ip = (int*)(lds_d + (VLDS ? 3 * nb : 0));
-  int* bins = ip;  // LEVEL_CAP + 1
-  int* off = CLDS ? ip + (LEVEL_CAP + 1) : c.flow_off + b0;
-  int* cur = CLDS ? off + nb : c.flow_cur + b0;
-  tmark(c, 0);
-  compute_ranks<T>(c, c0, n, b0, nb, off, cur, wsum);
-  tmark(c, 1);
-  int* cnt = off;
-  int* last = cur;
-  const bool levels = !VLDS && n > T;
   for (int i = tid; i < nb; i += T) {
-    cnt[i] = 0;
-    if (levels) last[i] = 0;
+    S.first[i] = (E)NONE;
+    if constexpr (!L) S.off[i] = 0;
   }
-  if (tid == 0) {
-    progress = 0;
-    s_maxl = 0;
+  if constexpr (L)
+    for (int i = tid; i < (nb + 1) / 2; i += T) ((uint32_t*)S.off)[i] = 0u;
+  __syncthreads();
+  // per body: how many manifolds it is body b of, the first it is body a of
+  // (a body's pairs as a are adjacent)
+  for (int k = tid; k < n; k += T) {
+    const int2 g = ab[k];
+    if (g.x == -1) continue;
+    const int2 p = k > 0 ? ab[k - 1] : make_int2(-2, -2);
+    const int pa = p.x == -1 ? ab[k - 2].x : p.x;  // a second contact has a first
+    if (g.y >= 0) (void)S.add(S.off, (uint32_t)g.y, 1u);
+    if (g.x >= 0 && pa != g.x) S.first[g.x] = (E)((uint32_t)k | (g.y < 0 ? ONE : 0u));
   }
-  Vel<VLDS> V;
-  V.lds = vel;
-  V.c = &c;
-  V.b0 = b0;
-  if (VLDS) {
-    for (int i = tid; i < nb; i += T) {
-      vel[3 * i] = c.vx[b0 + i];
-      vel[3 * i + 1] = c.vy[b0 + i];
-      vel[3 * i + 2] = c.w[b0 + i];
+  __syncthreads();
+  {  // counts -> starts
+    const int chunk = (nb + T - 1) / T;
+    const int x0 = min(nb, tid * chunk), x1 = min(nb, x0 + chunk);
+    int s = 0;
+    for (int x = x0; x < x1; ++x) s += (int)S.off[x];
+    int run = block_exclusive<T>(s, wsum);
+    for (int x = x0; x < x1; ++x) {
+      const int t = (int)S.off[x];
+      S.off[x] = (E)run;
+      run += t;
+    }
+  }
+  __syncthreads();
+  for (int k = tid; k < n; k += T) {  // the lists; off becomes their ends
+    const int2 g = ab[k];
+    if (g.x == -1 || g.y < 0) continue;
+    S.cnt[S.add(S.off, (uint32_t)g.y, 1u)] = (E)((uint32_t)k | (g.x < 0 ? ONE : 0u));
+  }
+  __syncthreads();
+  for (int k = tid; k < n; k += T) {
+    const int2 g = ab[k];
+    if (g.x == -1) continue;
+    uint32_t na = NONE, nx = NONE;
+    if (g.x >= 0) {
+      // the next pair of the same body a, or its first manifold (next pass)
+      int k1 = k + 1;
+      int2 f = k1 < n ? ab[k1] : make_int2(-2, -2);
+      if (f.x == -1) {
+        ++k1;
+        f = k1 < n ? ab[k1] : make_int2(-2, -2);
+      }
+      na = f.x == g.x ? (uint32_t)k1 | (f.y < 0 ? ONE : 0u) : S.first_of(g.x);
+    }
+    if (g.y >= 0) {
+      // the next manifold that has it as body b, the first that has it as
+      // body a, or its first one (next pass)
+      nx = S.list_min(g.y, k);
+      if (nx == NONE) nx = S.first[g.y];
+      if (nx == NONE) nx = S.first_of(g.y);
+    }
+    S.next[2 * k] = (E)na;
+    S.next[2 * k + 1] = (E)nx;
+  }
+  __syncthreads();
+  for (int x = tid; x < nb; x += T) S.first[x] = (E)S.first_of(x);
+  __syncthreads();
+  if constexpr (L) {
+    for (int i = tid; i < (n + 1) / 2; i += T) ((uint32_t*)S.cnt)[i] = 0u;
+  } else {
+    for (int i = tid; i < n; i += T) S.cnt[i] = 0u;
+  }
+  __syncthreads();
+}
+
+// The items of the last levels (a ring): CAP of each in LDS (16-bit entries
+// when the schedule is in LDS, its manifolds then being below 2^15), the rest
+// in global memory; one spare slot a level.  Slots beyond a level's width
+// hold older items or 0.  width: the levels' widths, a ring of twice the size.
+template <int T, bool L>
+struct Front {
+  using E = std::conditional_t<L, uint16_t, uint32_t>;
+  static constexpr int STRIDE = front_bytes(T) / RING / (int)sizeof(E), CAP = STRIDE - 8;
+  static constexpr uint32_t TOP = L ? 0x8000u : 0x80000000u;
+  E* lds;
+  uint32_t* spill;  // RING x cap
+  int* width;       // 2 * RING
+  int cap;
+  __device__ __forceinline__ static uint32_t item(uint32_t m) {
+    return L ? ((m & TOP) << 16) | (m & ~TOP) : m;
+  }
+  __device__ __forceinline__ E* row(int l) const { return lds + (l & (RING - 1)) * STRIDE; }
+  __device__ __forceinline__ uint32_t* far(int l, int i) const {
+    return spill + (long)(l & (RING - 1)) * cap + i;
+  }
+  __device__ __forceinline__ uint32_t near(int l, int i) const { return item(row(l)[i]); }
+  // item i of level l, any i below its width
+  __device__ __forceinline__ uint32_t get(int l, int i) const {
+    uint32_t m = near(l, min(i, CAP - 1));
+    // (an atomic load, so that the two do not become one flat load of a
+    // selected address, which would wait for every load in flight)
+    if (i >= CAP)
+      m = __hip_atomic_load(far(l, i), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    return m;
+  }
+  __device__ __forceinline__ void put(int l, int i, uint32_t k, bool warm) const {
+    if (i < CAP)
+      row(l)[i] = (E)(k | (warm ? TOP : 0u));
+    else
+      *far(l, i) = k | (warm ? ITEM_WARM : 0u);
+  }
+  __device__ __forceinline__ int n(int l) const {
+    return __builtin_amdgcn_readfirstlane(width[l & (2 * RING - 1)]);
+  }
+};
+
+// Makes level l + 1 from level l with NS wavefronts (sw: this one's number
+// among them): every item passes its tokens on.  passes: the last pass.  A
+// lane without a token to pass adds 0 to its own item's count, and one
+// without an item to list writes the spare slot, so that the common case
+// has no branches (a taken one costs as much as six instructions).
+template <int NS, int T, bool L>
+__device__ __forceinline__ void make_level(const Sched<L>& S, const Front<T, L>& fr, int l, int sw,
+                                           int passes) {
+  using F = Front<T, L>;
+  constexpr uint32_t NONE = Sched<L>::NONE, ONE = Sched<L>::ONE;
+  const int lane = threadIdx.x & 63;
+  const unsigned long long below = (1ull << lane) - 1ull;
+  const int width = fr.n(l);
+  int* out = fr.width + ((l + 1) & (2 * RING - 1));
+  auto* row = fr.row(l + 1);
+  int made = 0;  // NS == 1
+  for (int i0 = sw * 64; i0 < width; i0 += NS * 64) {
+    const int i = i0 + lane;
+    const bool act = i < width;
+    uint32_t k = width <= F::CAP ? fr.near(l, min(i, F::CAP - 1)) : fr.get(l, act ? i : 0);
+    k &= ~ITEM_WARM;
+    uint32_t t0, t1;
+    if constexpr (L) {
+      const uint32_t x = ((const uint32_t*)S.next)[k];
+      t0 = x & 0xFFFFu;
+      t1 = x >> 16;
+    } else {
+      t0 = S.next[2 * k];
+      t1 = S.next[2 * k + 1];
+    }
+    // a link that does not lead forward leads to the next pass
+    const bool last = (int)(S.count(k) >> 1) - 1 >= passes;
+    const bool go0 = act && t0 != NONE && !(last && (t0 & ~ONE) <= k);
+    const bool go1 = act && t1 != NONE && !(last && (t1 & ~ONE) <= k);
+    const uint32_t v0 = go0 ? ((t0 & ONE) ? 2u : 1u) : 0u, v1 = go1 ? ((t1 & ONE) ? 2u : 1u) : 0u;
+    const uint32_t n0 = S.add(S.cnt, go0 ? t0 & ~ONE : k, v0) + v0;
+    const uint32_t n1 = S.add(S.cnt, go1 ? t1 & ~ONE : k, v1) + v1;
+    // an even count: all tokens of a pass, 2 those of pass 0
+    const bool r0 = go0 && (n0 & 1u) == 0u, r1 = go1 && (n1 & 1u) == 0u;
+    const unsigned long long b0 = __ballot(r0), b1 = __ballot(r1);
+    const int c0 = (int)__popcll(b0), all = c0 + (int)__popcll(b1);
+    int base = made;
+    if constexpr (NS > 1) {
+      if (all) {
+        if (lane == 0) base = atomicAdd(out, all);
+        base = __builtin_amdgcn_readfirstlane(base);
+      }
+    }
+    const int p0 = base + (int)__popcll(b0 & below), p1 = base + c0 + (int)__popcll(b1 & below);
+    if (base + all <= F::CAP) {
+      row[r0 ? p0 : F::CAP] = (typename F::E)((t0 & ~ONE) | (n0 == 2u ? F::TOP : 0u));
+      row[r1 ? p1 : F::CAP] = (typename F::E)((t1 & ~ONE) | (n1 == 2u ? F::TOP : 0u));
+    } else {
+      if (r0) fr.put(l + 1, p0, t0 & ~ONE, n0 == 2u);
+      if (r1) fr.put(l + 1, p1, t1 & ~ONE, n1 == 2u);
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    }
+    made += all;
+  }
+  if constexpr (NS == 1) {
+    if (lane == 0) *out = made;
+  } else {
+    // the ring's entry after next, free by now
+    if (sw == 0 && lane == 0) fr.width[(l + 2) & (2 * RING - 1)] = 0;
+  }
+}
+
+// All levels: the last NS wavefronts make the schedule, the others run it,
+// STEP items of a level at a time.
+template <int T, bool L, bool VLDS, bool LLDS>
+__device__ __forceinline__ void run_levels(const Ctx& c, const Sched<L>& Q,
+                                           const OState<VLDS, LLDS>& S, const Front<T, L>& fr) {
+  constexpr int NS = T / 256, NE = T / 64 - NS, STEP = NE * 32;
+  static_assert(STEP <= Front<T, L>::CAP, "a level's first step reads its LDS slots");
+  const int wave = threadIdx.x >> 6;
+  auto sync = [] {
+    if (VLDS && LLDS)
+      lds_barrier();
+    else
+      __syncthreads();
+  };
+  // Both loops end at the first empty level: a manifold sends tokens into
+  // its next pass only before the last one, and else only forward.
+  const int passes = c.iterations;
+  for (int l = 0; l < RING - 2; ++l) {  // levels 1 and 2
+    if (wave >= NE) make_level<NS, T, L>(Q, fr, l, wave - NE, passes);
+    __syncthreads();
+  }
+  if (wave >= NE) {
+    for (int l = 0; fr.n(l) != 0; ++l) {
+      make_level<NS, T, L>(Q, fr, l + RING - 2, wave - NE, passes);
+      sync();
+    }
+    return;
+  }
+  const int side = threadIdx.x & 1, e = (int)threadIdx.x >> 1;
+  int l = 0, base = 0, width = fr.n(0);
+  ORec x, y;
+  load_orec(c, S.c0, fr.near(0, e), side, x);
+  auto step = [&](const ORec& now, ORec& nxt) {
+    // the next step's item: of this level, or of the next level (a lane
+    // beyond the width loads some item's record and does not run it)
+    const bool more = base + STEP < width;
+    const uint32_t item = more ? fr.get(l, min(base + STEP + e, width - 1))
+                               : fr.near(l + 1, e);
+    load_orec(c, S.c0, item, side, nxt);
+    const bool act = base + e < width;
+    if (__ballot(act && ((now.item & ITEM_WARM) || (orec_id(now, side) & FLOW_BOUNCE)))) {
+      if (act) run_item<true>(now, side, S);
+    } else {
+      if (act) run_item<false>(now, side, S);
+    }
+    base += STEP;
+    if (!more) {
+      const int w = fr.width[(l + 1) & (2 * RING - 1)];
+      sync();
+      ++l;
+      base = 0;
+      width = __builtin_amdgcn_readfirstlane(w);
+    }
+  };
+  while (width > 0) {
+    step(x, y);
+    if (width == 0) break;
+    step(y, x);
+  }
+}
+
+template <int T, bool L>
+__device__ __forceinline__ void solve_world(const Ctx& c, const Sched<L>& Q, unsigned char* pool,
+                                            long pool_bytes, int c0, int n, int b0, int nb,
+                                            const Front<T, L>& fr, int* wsum) {
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int2* ab = c.sch_ab + c0;
+  build_links<T, L>(Q, ab, n, nb, wsum);
+  // a token to the first manifold of every body; the ready ones are level 0
+  for (int x0 = 0; x0 < nb; x0 += T) {
+    const int x = x0 + tid;
+    const uint32_t t = x < nb ? (uint32_t)Q.first[x] : Sched<L>::NONE;
+    bool ready = false;
+    if (t != Sched<L>::NONE) {
+      const uint32_t v = (t & Sched<L>::ONE) ? 2u : 1u;
+      ready = ((Q.add(Q.cnt, t & ~Sched<L>::ONE, v) + v) & 1u) == 0u;
+    }
+    const unsigned long long bal = __ballot(ready);
+    int base = 0;
+    if (bal) {
+      if (lane == 0) base = atomicAdd(&fr.width[0], (int)__popcll(bal));
+      base = __builtin_amdgcn_readfirstlane(base);
+    }
+    if (ready)
+      fr.put(0, base + (int)__popcll(bal & ((1ull << lane) - 1ull)), t & ~Sched<L>::ONE, true);
+  }
+  __syncthreads();
+  tmark(c, 1);
+  // velocities, then lagrangians, in the rest of the LDS pool (over the
+  // build's per-body arrays)
+  const bool vlds = 24L * nb <= pool_bytes;
+  const long vbytes = vlds ? 24L * nb : 0;
+  const bool llds = vlds && vbytes + 16L * n <= pool_bytes;
+  double* vel = (double*)pool;
+  double* lam = vel + 3L * nb;
+  for (int i = tid; i < nb; i += T) {
+    const double x = c.vx[b0 + i], y = c.vy[b0 + i], w = c.w[b0 + i];
+    if (vlds) {
+      vel[3 * i] = x;
+      vel[3 * i + 1] = y;
+      vel[3 * i + 2] = w;
+    } else {
+      c.gvel[b0 + i] = make_double4(x, y, w, 0.0);
+    }
+  }
+  for (int k = tid; k < n; k += T) {
+    const double2 l = make_double2(c.ln[c0 + k], c.lt[c0 + k]);
+    if (llds) {
+      lam[2 * k] = l.x;
+      lam[2 * k + 1] = l.y;
+    } else {
+      c.glam[c0 + k] = l;
     }
   }
   __syncthreads();
   tmark(c, 2);
-  int maxl = 0;
-  int* order = c.flow_order + c0;
-  if (levels) {
-    int m = run_levels<T>(c, c0, n, b0, cnt, last, c.flow_lvl + c0, &progress);
-    for (int o = 32; o > 0; o >>= 1) m = max(m, __shfl_xor(m, o));
-    if ((tid & 63) == 0) atomicMax(&s_maxl, m);
-    __syncthreads();
-    maxl = s_maxl;
-    if (maxl <= LEVEL_CAP) {
-      sort_by_level<T>(c.flow_lvl + c0, n, maxl, bins, order, wsum);  // ends with a barrier
-      for (int s = tid; s < n; s += T) pack_flow(c, c0 + order[s], c0 + s);
-    } else {  // too deep for the bins: the dataflow with its counters
-      for (int i = tid; i < nb; i += T) cnt[i] = 0;
-      if (tid == 0) progress = 0;
-      for (int k = c0 + tid; k < c1; k += T) pack_flow(c, k, k);
-    }
-  } else {
-    for (int k = c0 + tid; k < c1; k += T) pack_flow(c, k, k);
-  }
-  __syncthreads();
   tmark(c, 3);
-  const bool sync = levels && maxl <= LEVEL_CAP;
-  if (sync) {
-    for (int p = 0; p <= c.iterations; ++p) run_pass_levels<VLDS, T>(c, c0, p, maxl, bins, V);
-  } else {
-    run_flow<VLDS, T>(c, c0, n, b0, cnt, V, &progress);
-  }
+  if (llds)
+    run_levels<T, L>(c, Q, OState<true, true>{vel, lam, &c, b0, c0}, fr);
+  else if (vlds)
+    run_levels<T, L>(c, Q, OState<true, false>{vel, lam, &c, b0, c0}, fr);
+  else
+    run_levels<T, L>(c, Q, OState<false, false>{vel, lam, &c, b0, c0}, fr);
   __syncthreads();
   tmark(c, 4);
-  const long CC = c.contact_cap;
-  for (int s = tid; s < n; s += T) {
-    const int k = sync ? c0 + order[s] : c0 + s;
-    c.ln[k] = c.pk[FL_LN * CC + c0 + s];
-    c.lt[k] = c.pk[FL_LT * CC + c0 + s];
+  for (int k = tid; k < n; k += T) {
+    double2 l;
+    if (llds)
+      l = make_double2(lam[2 * k], lam[2 * k + 1]);
+    else
+      l = c.glam[c0 + k];
+    c.ln[c0 + k] = l.x;
+    c.lt[c0 + k] = l.y;
   }
-  if (VLDS) {
-    for (int i = tid; i < nb; i += T) {
-      if (c.is_static[b0 + i]) continue;
-      c.vx[b0 + i] = vel[3 * i];
-      c.vy[b0 + i] = vel[3 * i + 1];
-      c.w[b0 + i] = vel[3 * i + 2];
+  for (int i = tid; i < nb; i += T) {
+    const int g = b0 + i;
+    if (c.is_static[g]) continue;
+    if (vlds) {
+      c.vx[g] = vel[3 * i];
+      c.vy[g] = vel[3 * i + 1];
+      c.w[g] = vel[3 * i + 2];
+    } else {
+      const double4 v = c.gvel[g];
+      c.vx[g] = v.x;
+      c.vy[g] = v.y;
+      c.w[g] = v.z;
     }
   }
   __syncthreads();
   tmark(c, 5);
 }
 
-template <bool CLDS, bool VLDS>
-static const void* flow_kernel(int threads) {
-  return threads == 512 ? (const void*)k_solve_flow<CLDS, VLDS, 512>
-                        : (const void*)k_solve_flow<CLDS, VLDS, 256>;
-}
-
-static_assert(FL_FIELDS <= FLOW_RECORD_DOUBLES, "compact record exceeds the packed buffer");
-
-// LDS per world: level bins, then velocities (24 B/body) and offsets +
-// cursors (8 B/body) when they fit; offsets + cursors alone; else both in
-// global memory.  4 waves per world; a large world gets 8 (a
-// level-synchronous pass keeps two records per lane, so 8 waves leave it
-// 256 registers per lane).
-void plan_ordered_solver(StepPlan* P, int solver_threads) {
-  const size_t bins = 4UL * (LEVEL_CAP + 1);
-  const size_t both = bins + 32UL * P->max_nb, cnt_only = bins + 8UL * P->max_nb;
-  if (both <= LDS_MAX_BYTES) {
-    P->solve_clds = true;
-    P->solve_vlds = true;
-    P->solve_lds = both;
-  } else if (cnt_only <= LDS_MAX_BYTES) {
-    P->solve_clds = true;
-    P->solve_vlds = false;
-    P->solve_lds = cnt_only;
+template <int T>
+__global__ __launch_bounds__(T) void k_solve_ordered(Ctx c, int pool_bytes) {
+  extern __shared__ __align__(16) unsigned char pool[];
+  __shared__ int wsum[T / 64];
+  __shared__ int s_front[front_bytes(T) / 4];
+  __shared__ int s_width[2 * RING];
+  const int w = c.world_order[blockIdx.x];
+  const int tid = threadIdx.x;
+  const int c0 = c.wcont_off[w], c1 = c.wcont_off[w + 1];
+  if (c1 <= c0) return;
+  const int n = c1 - c0;
+  const int b0 = c.body_off[w], nb = c.body_off[w + 1] - b0;
+  tmark(c, 0);
+  if (tid < 2 * RING) s_width[tid] = 0;
+  for (int i = tid; i < front_bytes(T) / 4; i += T) s_front[i] = 0;
+  uint32_t* glob = c.sch_glob + (3L + RING) * c0;
+  // LDS: links 4 B and tokens 2 B a contact, then 4 B a body while they are
+  // built (then the velocities)
+  const long hot = (4L * n + 2L * ((n + 1) & ~1) + 15) & ~15L;
+  const long body2 = 2L * ((nb + 1) & ~1);
+  if (n < 0x7FFF && c.iterations < 0x7FF0 && nb < 0x7FFF && hot + 2 * body2 <= pool_bytes) {
+    Sched<true> Q;
+    Q.next = (uint16_t*)pool;
+    Q.cnt = Q.next + 2 * n;
+    Q.off = (uint16_t*)(pool + hot);
+    Q.first = (uint16_t*)(pool + hot + body2);
+    solve_world<T, true>(c, Q, pool + hot, pool_bytes - hot, c0, n, b0, nb,
+                         Front<T, true>{(uint16_t*)s_front, glob + 3L * n, s_width, n}, wsum);
   } else {
-    P->solve_clds = false;
-    P->solve_vlds = false;
-    P->solve_lds = bins;
+    Sched<false> Q;
+    Q.next = glob;
+    Q.cnt = glob + 2L * n;
+    Q.off = (uint32_t*)c.sch_off + b0;
+    Q.first = (uint32_t*)c.sch_first + b0;
+    solve_world<T, false>(c, Q, pool, pool_bytes, c0, n, b0, nb,
+                          Front<T, false>{(uint32_t*)s_front, glob + 3L * n, s_width, n}, wsum);
   }
-  P->solve_threads = solver_threads ? solver_threads : (P->max_nb > 2048 ? 512 : 256);
 }
 
-// wsum[T / 64], progress, s_maxl
-size_t ordered_static_lds(int threads) { return lds16((size_t)(threads / 64) * 4) + 2 * lds16(4); }
+// static LDS: wsum, s_front, s_width
+size_t ordered_static_lds(int threads) {
+  return lds16((size_t)(threads / 64) * 4) + lds16(front_bytes(threads)) + lds16(2 * RING * 4);
+}
+
+// LDS per world: velocities 24 B a body, about 2.2 contacts of 22 B a body,
+// as far as it goes.  4 waves per world; a world of more than
+// 512 bodies gets 8 (with 16, at 128 registers a lane, an 8192-polygon pile
+// took 1.93 ms instead of 1.64).
+void plan_ordered_solver(StepPlan* P, int solver_threads) {
+  P->solve_threads = solver_threads ? solver_threads : (P->max_nb > 512 ? 512 : 256);
+  const size_t room = LDS_BYTES_PER_CU - ordered_static_lds(P->solve_threads) - 256;
+  P->solve_lds = std::min<size_t>(room, 72UL * P->max_nb + 1024);
+}
+
+static const void* ordered_kernel(int threads) {
+  return threads == 512 ? (const void*)k_solve_ordered<512> : (const void*)k_solve_ordered<256>;
+}
 
 shp_status solver_alloc(shp_batch* b) {
   const StepPlan& P = b->plan;
   if (P.solver != SHP_SOLVER_ORDERED_F64) return colored_alloc(b);
-  const void* fn = P.solve_clds ? (P.solve_vlds ? flow_kernel<true, true>(P.solve_threads)
-                                                : flow_kernel<true, false>(P.solve_threads))
-                                : flow_kernel<false, false>(P.solve_threads);
-  if (hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize,
-                          (int)std::max<size_t>(P.solve_lds, 16)) != hipSuccess) {
+  const void* fn = ordered_kernel(P.solve_threads);
+  if (hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)P.solve_lds) !=
+      hipSuccess) {
     shp_set_error("hipFuncSetAttribute (ordered solver LDS) failed");
     return SHP_E_HIP;
   }
@@ -708,21 +737,11 @@ shp_status solver_alloc(shp_batch* b) {
   return SHP_OK;
 }
 
-template <int T>
-static void launch_flow(shp_batch* b) {
-  const StepPlan& P = b->plan;
-  const size_t lds = std::max<size_t>(P.solve_lds, 16);
-  if (P.solve_clds && P.solve_vlds)
-    k_solve_flow<true, true, T><<<b->ctx.W, T, lds, b->stream>>>(b->ctx);
-  else if (P.solve_clds)
-    k_solve_flow<true, false, T><<<b->ctx.W, T, lds, b->stream>>>(b->ctx);
-  else
-    k_solve_flow<false, false, T><<<b->ctx.W, T, lds, b->stream>>>(b->ctx);
-}
-
 void launch_ordered_solver(shp_batch* b) {
-  if (b->plan.solve_threads == 512)
-    launch_flow<512>(b);
+  const StepPlan& P = b->plan;
+  const Ctx& c = b->ctx;
+  if (P.solve_threads == 512)
+    k_solve_ordered<512><<<c.W, 512, P.solve_lds, b->stream>>>(c, (int)P.solve_lds);
   else
-    launch_flow<256>(b);
+    k_solve_ordered<256><<<c.W, 256, P.solve_lds, b->stream>>>(c, (int)P.solve_lds);
 }
