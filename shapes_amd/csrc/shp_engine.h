@@ -47,6 +47,8 @@ constexpr size_t lds16(size_t bytes) { return (bytes + 15) & ~(size_t)15; }
 // stream, is phase SHP_MAIN_PHASES of the timing ABI)
 #define SHP_MAIN_PHASES (SHP_NUM_PHASES - 1)
 
+// bytes before the rows in a batch's pinned readback memory
+enum { STAGE_FLAGS = 64 };
 enum { CNT_FLAGS = 0, CNT_WARM = 1, CNT_LEARNED = 2, CNT_LEVELS = 3, CNT_MISS = 4, CNT_MANIFOLDS = 5 };
 // grid broadphase: partners per body kept by the count pass for the emit
 // pass (bodies with more are visited again)
@@ -181,6 +183,7 @@ struct Ctx {
   int32_t* grid_slots;
   int32_t *large_off, *large_ids;
   int32_t* counters;  // 8 ints: flags, warm hits, learned starts, levels
+  int32_t* host_flags;  // pinned host memory: the last step's flags
   unsigned long long* quality;  // Q_ENTRIES entries, see Q_*
 };
 
@@ -283,6 +286,13 @@ struct shp_batch {
   bool graph_ready = false;  // ... and it matches the current kernel arguments
   int32_t last_flags = 0;
   std::vector<void*> allocs;
+  // pinned host memory the readback kernels write: the last step's flags
+  // (STAGE_FLAGS bytes), then stage_bytes for one call's rows
+  unsigned char* stage = nullptr;
+  size_t stage_bytes = 0;
+  // the device's flags are newer than the pinned copy (a placement or a probe
+  // since the last step)
+  bool flags_on_device = false;
   // per-phase event timing (shp_batch_set_timing)
   bool timing = false;
   bool events_made = false;

@@ -145,7 +145,7 @@ def load_library(path: str = LIB_PATH):
     L.shp_batch_step_async.argtypes = [C.c_void_p, C.c_int32, C.c_int32]
     L.shp_batch_sync.argtypes = [C.c_void_p]
     L.shp_batch_num_bodies.argtypes = [C.c_void_p, C.c_int32, _ip]
-    L.shp_batch_read_bodies.argtypes = [C.c_void_p, C.c_int32] + [_dp] * 6
+    L.shp_batch_read_bodies.argtypes = [C.c_void_p, C.c_int32] + [C.c_void_p] * 6
     L.shp_batch_read_pairs.argtypes = [C.c_void_p, C.c_int32, _ip, _ip]
     L.shp_batch_read_contacts.argtypes = [C.c_void_p, C.c_int32, _ip, _ip, _ip,
                                           _dp, _dp, _ip]
@@ -307,10 +307,11 @@ class Batch:
     def bodies(self, world: int = 0) -> np.ndarray:
         """(n, 6) array of px, py, theta, vx, vy, omega."""
         n = self.sizes[world]
-        cols = [np.empty(n, dtype=np.float64) for _ in range(6)]
-        _check(self._L.shp_batch_read_bodies(self._h, world,
-                                             *[_dptr(c) for c in cols]))
-        return np.stack(cols, axis=1)
+        cols = np.empty((6, n), dtype=np.float64)
+        p = cols.ctypes.data
+        _check(self._L.shp_batch_read_bodies(self._h, world, p, p + 8 * n, p + 16 * n, p + 24 * n,
+                                             p + 32 * n, p + 40 * n))
+        return np.ascontiguousarray(cols.T)
 
     def pairs(self, world: int = 0) -> np.ndarray:
         cnt = C.c_int32()
