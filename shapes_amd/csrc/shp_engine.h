@@ -150,10 +150,10 @@ struct Ctx {
   // coloured solver state: FP32 velocities (vx, vy, w, unused) per body,
   // one 16-byte word so that a body's gather reads one cache line
   float4* fv;
-  // learned warm start: padded FP32 master / BF16 weights, the step's
+  // learned warm start: padded FP32 master weights (the biases) and BF16 fragments, the step's
   // cache misses (contact index + 14 features) and the training-data log
   const float* mlp_w;
-  const uint16_t* mlp_wbf;
+  const uint16_t* mlp_wfr;
   int mlp_ready;
   int collect_misses;
   int features_in_contacts;  // the misses' features from k_contacts (the log needs them)

@@ -1448,7 +1448,7 @@ shp_status plan_staged(const shp_config& cfg, HostBatch* hb) {
   P.g_ranges = blocks(n_worlds + 1, 256);
   P.g_contacts = gs_blocks(PC);
   P.g_pack = gs_blocks(PC);
-  P.g_infer = std::min<long>(std::max<long>(1, blocks(P.miss_cap, 64)), 256);
+  P.g_infer = std::min<long>(std::max<long>(1, blocks(P.miss_cap, MLP_INFER_ROWS)), 512);
   P.g_unpack = std::max(1L, std::min(blocks(std::max(PC, NB), 256), 4096L));
   P.g_log = std::max<long>(1, blocks(P.miss_cap, 256));
   P.g_finish_ni = blocks(NB, INTEGRATE_THREADS);
@@ -1488,7 +1488,7 @@ void plan_launches(const StepPlan& P, bool infer, bool logging, std::vector<Laun
   scan_launches(P.scan_pairs, "scan_pairs", out);
   add("k_world_ranges", P.g_ranges, 256, 0, 0);
   add("k_contacts", P.g_contacts, 256, 0, lds16(4));
-  if (infer) add("k_mlp_infer", P.g_infer, 256, 0, mlp_infer_static_lds());
+  if (infer) add("k_mlp_infer", P.g_infer, MLP_INFER_THREADS, 0, mlp_infer_static_lds());
   if (col) {
     if (!P.records_in_contacts) add("k_pack_manifolds", P.g_pack, 256, 0, 0);
     if (P.sweep_big > 0)
@@ -2057,7 +2057,7 @@ shp_status shp_batch_set_mlp(shp_batch* b, const float* params) {
   if (!b->mlp.w) TRY(mlp_params_alloc(&b->mlp));
   TRY(mlp_params_upload(&b->mlp, params, b->stream));
   b->ctx.mlp_w = b->mlp.w;
-  b->ctx.mlp_wbf = b->mlp.wbf;
+  b->ctx.mlp_wfr = b->mlp.wfr;
   b->ctx.mlp_ready = 1;
   b->ctx.collect_misses = (b->cfg.warm_start == SHP_WARM_LEARNED) || b->logging;
   b->ctx.features_in_contacts = b->logging;
@@ -2320,7 +2320,7 @@ static shp_status rebuild_with(shp_batch* b, long g, const StagedBody& s) {
   c.tstamp_store = keep.tstamp_store;
   c.tstamp = keep.tstamp;
   c.mlp_w = keep.mlp_w;
-  c.mlp_wbf = keep.mlp_wbf;
+  c.mlp_wfr = keep.mlp_wfr;
   c.mlp_ready = keep.mlp_ready;
   c.collect_misses = keep.collect_misses;
   c.features_in_contacts = keep.features_in_contacts;

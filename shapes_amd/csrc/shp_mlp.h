@@ -23,9 +23,27 @@
 #define MLP_OFF_B4 (MLP_OFF_W4 + 128 * 16)
 #define MLP_NPARAM_PAD (MLP_OFF_B4 + 16)
 
+// BF16 weights in matrix-core operand order: a fragment is one 16x16 block of
+// a weight matrix as the 64 lanes of a wavefront hold it (4 values, 8 bytes a
+// lane), so a wavefront loads it with one contiguous 512-byte access.
+// Forward fragments hold W^T blocks: lane l has W[16 kb + 4 (l / 16) + 0..3]
+// [16 ct + l % 16] of block (output columns ct, input rows kb), layer after
+// layer, kb inside ct.
+#define MLP_FRAG 256
+#define MLP_F1 0                       // 8 ct
+#define MLP_F2 (MLP_F1 + 8 * MLP_FRAG)   // 8 ct x 8 kb
+#define MLP_F3 (MLP_F2 + 64 * MLP_FRAG)  // 8 ct x 8 kb
+#define MLP_F4 (MLP_F3 + 64 * MLP_FRAG)  // 8 kb
+#define MLP_NFRAG (MLP_F4 + 8 * MLP_FRAG)
+
+// the in-step inference: misses per workgroup at a time, and its lanes
+#define MLP_INFER_ROWS 64
+#define MLP_INFER_THREADS 256
+
 struct MlpParams {
   float* w = nullptr;       // FP32 master copy, padded layout
-  uint16_t* wbf = nullptr;  // BF16 copy used by the matrix cores
+  uint16_t* wbf = nullptr;  // BF16 copy, padded layout (training)
+  uint16_t* wfr = nullptr;  // BF16 copy in fragments
 };
 
 // The 14 input features of a contact that missed the cache, computed from

@@ -7,18 +7,26 @@
 // rounded to BF16 only where they feed the next product.
 //
 // Kernels:
-//   k_mlp_forward   fused forward of tiles of 64 rows (one workgroup of 4
-//                   waves per tile, activations in LDS); optionally stores
-//                   pre-activations and BF16 activations for training
+//   k_mlp_eval      forward of feature rows, 16 at a time (4 waves)
+//   k_mlp_infer     the same on a step's cache misses, features and output
+//                   head included
+//   k_mlp_forward   forward of tiles of 64 rows storing what training needs
 //   k_mlp_backward  fused backward over tiles; weight gradients accumulate
 //                   in MFMA accumulators across a workgroup's tiles and are
 //                   written as one partial per workgroup (no atomics)
 //   k_mlp_reduce    sums the partials in a fixed order (deterministic)
-//   k_mlp_adam      Adam update of the FP32 master weights + BF16 copy
+//   k_mlp_adam      Adam update of the FP32 master weights + BF16 copies
+//
+// The inference kernels keep the weights in registers: wave w computes output
+// columns [32 w, 32 w + 32) of every layer, so it needs 2 x (1 + 8 + 8 + 8)
+// fragments (shp_mlp.h), loaded once per workgroup, and a layer reads only
+// activations from LDS.  They compute the transposed products W^T h^T: a lane
+// then holds four consecutive columns of one row and stores them with one
+// 8-byte LDS write, where the next layer's operand is one 8-byte read.  The
+// sums over k are those of h W, in the same order.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
-#include <mutex>
 #include <string>
 #include <vector>
 
@@ -113,15 +121,6 @@ struct TrainBufs {
 
 // One 64-row tile: X (64 x 16 BF16) in LDS -> Y (64 x 16 FP32).
 // Wave w owns rows 16w..16w+15.
-// The inference kernel's LDS copies of the weights: transposed ([out][in])
-// with rows of WT1 (first layer) or WT2 entries, padded so that its
-// transposing stores spread over the LDS banks while a fragment stays one
-// aligned 8-byte read.
-constexpr int WT1 = 20, WT2 = 132;
-
-// WT: the weights of m transposed and padded as above instead of
-// row-major [in][out].
-template <bool WT>
 __device__ void forward_tile(const MlpDev& m, uint16_t* sx, uint16_t* s1, uint16_t* s2,
                              float* yout /* 64 x 16 */, const TrainBufs* tb, int row0) {
   int wv = threadIdx.x >> 6, l = threadIdx.x & 63;
@@ -130,7 +129,7 @@ __device__ void forward_tile(const MlpDev& m, uint16_t* sx, uint16_t* s1, uint16
   for (int ct = 0; ct < 8; ++ct) {
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
     acc = mfma16(frag_a(sx, 16, r0, 0),
-                 WT ? frag_bt(m.w1, WT1, 0, 16 * ct) : frag_b(m.w1, 128, 0, 16 * ct), acc);
+                 frag_b(m.w1, 128, 0, 16 * ct), acc);
     int col = 16 * ct + (l & 15);
     for (int i = 0; i < 4; ++i) {
       int row = r0 + 4 * (l >> 4) + i;
@@ -157,7 +156,7 @@ __device__ void forward_tile(const MlpDev& m, uint16_t* sx, uint16_t* s1, uint16
     for (int k0 = 0; k0 < 128; k0 += 16) {
       bf16x4 a = frag_a(in, 128, r0, k0);
       for (int ct = 0; ct < 8; ++ct)
-        acc[ct] = mfma16(a, WT ? frag_bt(W, WT2, k0, 16 * ct) : frag_b(W, 128, k0, 16 * ct), acc[ct]);
+        acc[ct] = mfma16(a, frag_b(W, 128, k0, 16 * ct), acc[ct]);
     }
     __syncthreads();  // every wave has read `in` before `out` (== in of layer 1) is overwritten
     for (int ct = 0; ct < 8; ++ct) {
@@ -178,7 +177,7 @@ __device__ void forward_tile(const MlpDev& m, uint16_t* sx, uint16_t* s1, uint16
   // layer 4: 128 -> 16 (2 used), input in s1
   f32x4 acc = {0.f, 0.f, 0.f, 0.f};
   for (int k0 = 0; k0 < 128; k0 += 16)
-    acc = mfma16(frag_a(s1, 128, r0, k0), WT ? frag_bt(m.w4, WT2, k0, 0) : frag_b(m.w4, 16, k0, 0), acc);
+    acc = mfma16(frag_a(s1, 128, r0, k0), frag_b(m.w4, 16, k0, 0), acc);
   int col = l & 15;
   for (int i = 0; i < 4; ++i) {
     int row = r0 + 4 * (l >> 4) + i;
@@ -189,7 +188,7 @@ __device__ void forward_tile(const MlpDev& m, uint16_t* sx, uint16_t* s1, uint16
 
 __global__ __launch_bounds__(256) void k_mlp_forward(MlpDev m, const uint16_t* X /* rows x 16 */,
                                                      int rows, float* Y /* rows x 16 */,
-                                                     TrainBufs tb, int store) {
+                                                     TrainBufs tb) {
   __shared__ uint16_t sx[TILE * 16];
   __shared__ uint16_t s1[TILE * 128];
   __shared__ uint16_t s2[TILE * 128];
@@ -198,7 +197,7 @@ __global__ __launch_bounds__(256) void k_mlp_forward(MlpDev m, const uint16_t* X
     int row0 = t * TILE;
     for (int i = threadIdx.x; i < TILE * 16; i += 256) sx[i] = X[(size_t)row0 * 16 + i];
     __syncthreads();
-    forward_tile<false>(m, sx, s1, s2, sy, store ? &tb : nullptr, row0);
+    forward_tile(m, sx, s1, s2, sy, &tb, row0);
     for (int i = threadIdx.x; i < TILE * 16; i += 256) Y[(size_t)row0 * 16 + i] = sy[i];
     __syncthreads();
   }
@@ -340,9 +339,39 @@ __global__ void k_mlp_reduce(const float* partial, int parts, float* grad) {
   grad[i] = s;
 }
 
+// Master weight i (padded layout) into its BF16 places.
+__device__ __forceinline__ void store_weight(int i, float x, uint16_t* wbf, uint16_t* wfr) {
+  const uint16_t v = f2bf(x);
+  wbf[i] = v;
+  int f = -1, k = 0, o = 0, nkb = 1;  // fragments of its layer, row, column
+  if (i < MLP_OFF_B1) {
+    f = MLP_F1;
+    k = i >> 7;
+    o = i & 127;
+  } else if (i >= MLP_OFF_W2 && i < MLP_OFF_B2) {
+    f = MLP_F2;
+    k = (i - MLP_OFF_W2) >> 7;
+    o = (i - MLP_OFF_W2) & 127;
+    nkb = 8;
+  } else if (i >= MLP_OFF_W3 && i < MLP_OFF_B3) {
+    f = MLP_F3;
+    k = (i - MLP_OFF_W3) >> 7;
+    o = (i - MLP_OFF_W3) & 127;
+    nkb = 8;
+  } else if (i >= MLP_OFF_W4 && i < MLP_OFF_B4) {
+    f = MLP_F4;
+    k = (i - MLP_OFF_W4) >> 4;
+    o = (i - MLP_OFF_W4) & 15;
+    nkb = 8;
+  }
+  if (f < 0) return;  // a bias
+  const int lane = (o & 15) + 16 * ((k & 15) >> 2);
+  wfr[f + ((o >> 4) * nkb + (k >> 4)) * MLP_FRAG + 4 * lane + (k & 3)] = v;
+}
+
 // Adam on the padded FP32 master weights; padding entries stay zero.
 __global__ void k_mlp_adam(float* w, float* mom, float* vel, const float* grad, const uint8_t* mask,
-                           uint16_t* wbf, float lr, float b1c, float b2c) {
+                           uint16_t* wbf, uint16_t* wfr, float lr, float b1c, float b2c) {
   int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= MLP_NPARAM_PAD) return;
   if (!mask[i]) return;
@@ -353,12 +382,13 @@ __global__ void k_mlp_adam(float* w, float* mom, float* vel, const float* grad, 
   vel[i] = v;
   float x = w[i] - lr * (m / b1c) / (sqrtf(v / b2c) + 1e-8f);
   w[i] = x;
-  wbf[i] = f2bf(x);
+  store_weight(i, x, wbf, wfr);
 }
 
-__global__ void k_f32_to_bf16(const float* in, uint16_t* out, long n) {
-  long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) out[i] = f2bf(in[i]);
+// The BF16 copies of every master weight.
+__global__ void k_mlp_pack(const float* w, uint16_t* wbf, uint16_t* wfr) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < MLP_NPARAM_PAD) store_weight(i, w[i], wbf, wfr);
 }
 
 // features (n x 14 FP32) -> padded BF16 rows (rows x 16), zero rows beyond n
@@ -368,6 +398,128 @@ __global__ void k_pack_features(const float* f, long n, long rows, uint16_t* X) 
   long r = i >> 4;
   int cc = (int)(i & 15);
   X[i] = (r < n && cc < MLP_IN) ? f2bf(f[r * MLP_IN + cc]) : (uint16_t)0;
+}
+
+// ---- inference ----------------------------------------------------------------
+
+// Row strides in LDS (BF16 entries): a fragment read takes 8 bytes of each of
+// 16 rows, which then start 8 bytes further round the banks each.
+constexpr int HS = 132, XS = 20;
+
+// Wave w's fragments of every layer.
+struct WaveWeights {
+  bf16x4 w1[2], w2[2][8], w3[2][8], w4[8];
+};
+
+__device__ __forceinline__ void load_weights(const uint16_t* wfr, WaveWeights& W) {
+  const bf16x4* f = (const bf16x4*)wfr + (threadIdx.x & 63);
+  const int c0 = 2 * (threadIdx.x >> 6);
+#pragma unroll
+  for (int c = 0; c < 2; ++c) {
+    W.w1[c] = f[(MLP_F1 / MLP_FRAG + c0 + c) * 64];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      W.w2[c][k] = f[(MLP_F2 / MLP_FRAG + (c0 + c) * 8 + k) * 64];
+      W.w3[c][k] = f[(MLP_F3 / MLP_FRAG + (c0 + c) * 8 + k) * 64];
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < 8; ++k) W.w4[k] = f[(MLP_F4 / MLP_FRAG + k) * 64];
+}
+
+__device__ __forceinline__ bf16x4 act_frag(const uint16_t* h, int stride, int kb) {
+  const int l = threadIdx.x & 63;
+  return *(const bf16x4*)(h + (l & 15) * stride + 16 * kb + 4 * (l >> 4));
+}
+
+// silu(acc + bias) of this lane's four columns from `col`, to row `row`
+__device__ __forceinline__ void put_acts(uint16_t* h, int row, int col, f32x4 acc, const float* bias) {
+  const float4 b = *(const float4*)(bias + col);
+  uint32_t lo = f2bf(silu(acc[0] + b.x)) | (uint32_t)f2bf(silu(acc[1] + b.y)) << 16;
+  uint32_t hi = f2bf(silu(acc[2] + b.z)) | (uint32_t)f2bf(silu(acc[3] + b.w)) << 16;
+  *(uint2*)(h + row * HS + col) = make_uint2(lo, hi);
+}
+
+// The layers of 16 rows (BF16 features x in LDS, stride XS) by 4 waves; ha
+// and hb hold 16 rows of HS.  sb: b1, b2, b3, b4.  Calls out(row, y0, y1) from
+// one lane per row.  Begins and ends with a barrier.
+template <class Out>
+__device__ __forceinline__ void mlp_layers(const WaveWeights& W, const float* sb, const uint16_t* x,
+                                           uint16_t* ha, uint16_t* hb, Out out) {
+  const int l = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int c0 = 32 * wv + 4 * (l >> 4), r = l & 15;
+  __syncthreads();
+  {
+    const bf16x4 v = act_frag(x, XS, 0);
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+      put_acts(ha, r, c0 + 16 * c, mfma16(W.w1[c], v, f32x4{0.f, 0.f, 0.f, 0.f}), sb);
+  }
+  __syncthreads();
+#pragma unroll
+  for (int layer = 0; layer < 2; ++layer) {
+    const uint16_t* in = layer ? hb : ha;
+    f32x4 acc[2];
+    acc[0] = acc[1] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const bf16x4 v = act_frag(in, HS, k);
+#pragma unroll
+      for (int c = 0; c < 2; ++c) acc[c] = mfma16(layer ? W.w3[c][k] : W.w2[c][k], v, acc[c]);
+    }
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+      put_acts(layer ? ha : hb, r, c0 + 16 * c, acc[c], sb + 128 * (layer + 1));
+    __syncthreads();
+  }
+  if (wv == 0) {
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int k = 0; k < 8; ++k) acc = mfma16(W.w4[k], act_frag(ha, HS, k), acc);
+    if (l < 16) out(l, acc[0] + sb[384], acc[1] + sb[385]);
+  }
+  __syncthreads();
+}
+
+__device__ __forceinline__ void load_biases(const float* w, float* sb) {
+  for (int i = threadIdx.x; i < 3 * 128 + 16; i += blockDim.x)
+    sb[i] = i < 128   ? w[MLP_OFF_B1 + i]
+            : i < 256 ? w[MLP_OFF_B2 + i - 128]
+            : i < 384 ? w[MLP_OFF_B3 + i - 256]
+                      : w[MLP_OFF_B4 + i - 384];
+}
+
+// out[2 r + k] = output k of row r (n x 14 FP32 features), tiles of 16 rows
+// (tiles of 32 and 64 took as long or longer from 4 k to 65 k rows).  Bound by
+// the chain of layers while every workgroup has one tile, by the
+// activations' exponentials and divisions beyond.  One launch and 2 floats
+// written a row (before: features packed, 16 floats a row, outputs taken):
+// 4099 rows 27 -> 6.8 us, 65536 rows 26.6 us.
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_mlp_eval(const uint16_t* __restrict__ wfr,
+                                                  const float* __restrict__ w,
+                                                  const float* __restrict__ feats, int n,
+                                                  float* __restrict__ out) {
+  __shared__ __align__(16) uint16_t x[16 * XS], ha[16 * HS], hb[16 * HS];
+  __shared__ __align__(16) float sb[3 * 128 + 16];
+  WaveWeights W;
+  load_weights(wfr, W);
+  load_biases(w, sb);
+  for (int t = blockIdx.x; t * 16 < n; t += gridDim.x) {
+    const int row0 = t * 16, r = threadIdx.x >> 4, q = threadIdx.x & 15;
+    const float f = row0 + r < n && q < MLP_IN ? feats[(size_t)(row0 + r) * MLP_IN + q] : 0.0f;
+    x[r * XS + q] = f2bf(f);
+    mlp_layers(W, sb, x, ha, hb, [&](int i, float y0, float y1) {
+      if (row0 + i >= n) return;
+      out[2 * (size_t)(row0 + i)] = y0;
+      out[2 * (size_t)(row0 + i) + 1] = y1;
+    });
+  }
+}
+
+// 4 workgroups on each of 256 CUs
+void launch_eval(const MlpParams& p, const float* feats, int n, float* out, hipStream_t s) {
+  const int tiles = (n + 15) / 16;
+  k_mlp_eval<<<tiles < 1024 ? tiles : 1024, 256, 0, s>>>(p.wfr, p.w, feats, n, out);
 }
 
 }  // namespace
@@ -409,98 +561,80 @@ int mlp_padded_index(int k) {
 shp_status mlp_params_alloc(MlpParams* p) {
   if (hipMalloc(&p->w, MLP_NPARAM_PAD * sizeof(float)) != hipSuccess) return SHP_E_OOM;
   if (hipMalloc(&p->wbf, MLP_NPARAM_PAD * sizeof(uint16_t)) != hipSuccess) return SHP_E_OOM;
+  if (hipMalloc(&p->wfr, MLP_NFRAG * sizeof(uint16_t)) != hipSuccess) return SHP_E_OOM;
   return SHP_OK;
 }
 
 void mlp_params_free(MlpParams* p) {
   if (p->w) (void)hipFree(p->w);
   if (p->wbf) (void)hipFree(p->wbf);
+  if (p->wfr) (void)hipFree(p->wfr);
   p->w = nullptr;
   p->wbf = nullptr;
+  p->wfr = nullptr;
 }
 
 shp_status mlp_params_upload(MlpParams* p, const float* params, hipStream_t s) {
   std::vector<float> pad(MLP_NPARAM_PAD, 0.0f);
   for (int k = 0; k < MLP_NPARAM; ++k) pad[mlp_padded_index(k)] = params[k];
   if (hipMemcpyAsync(p->w, pad.data(), pad.size() * 4, hipMemcpyHostToDevice, s) != hipSuccess) return SHP_E_HIP;
-  k_f32_to_bf16<<<(MLP_NPARAM_PAD + 255) / 256, 256, 0, s>>>(p->w, p->wbf, MLP_NPARAM_PAD);
+  k_mlp_pack<<<(MLP_NPARAM_PAD + 255) / 256, 256, 0, s>>>(p->w, p->wbf, p->wfr);
   if (hipStreamSynchronize(s) != hipSuccess) return SHP_E_HIP;
   return SHP_OK;
 }
 
-void mlp_launch_forward(const MlpParams& p, const uint16_t* X, int rows, float* Y, hipStream_t s) {
-  TrainBufs tb{};
-  int tiles = (rows + TILE - 1) / TILE;
-  int grid = tiles < 1024 ? (tiles > 0 ? tiles : 1) : 1024;
-  k_mlp_forward<<<grid, 256, 0, s>>>(mlp_view(p), X, rows, Y, tb, 0);
-}
-
 // ---- engine hooks ------------------------------------------------------------
 
-// Learned warm start of the step's cache misses: tiles of 64 misses, the
-// features rounded to BF16, the forward pass on the matrix cores, then the
-// output head lambda_n = max(y0, 0) / mn, lambda_t = y1 / mt projected onto
-// |lambda_t| <= mu * lambda_n.  The contact is marked warm (2) so the
-// solver applies the predicted impulses like a cached solution (the
-// coloured solver's manifold record, already written, gets them too); a
-// non-finite prediction keeps the zero start.
-__global__ __launch_bounds__(256) void k_mlp_infer(Ctx c, MlpDev m) {
-  __shared__ uint16_t sx[TILE * 16];
-  __shared__ uint16_t s1[TILE * 128];
-  __shared__ uint16_t s2[TILE * 128];
-  __shared__ float sy[TILE * 16];
-  // the weights, transposed, and biases, once per workgroup for all its
-  // tiles: a B fragment is then one 8-byte LDS read
-  __shared__ __align__(16) uint16_t s_w1[128 * WT1], s_w2[128 * WT2], s_w3[128 * WT2], s_w4[16 * WT2];
-  __shared__ float s_b[3 * 128 + 16];
+// Learned warm start of the step's cache misses: the features rounded to
+// BF16, the forward pass on the matrix cores, then the output head lambda_n =
+// max(y0, 0) / mn, lambda_t = y1 / mt projected onto |lambda_t| <= mu *
+// lambda_n.  The contact is marked warm (2) so the solver applies the
+// predicted impulses like a cached solution (the coloured solver's manifold
+// record, already written, gets them too); a non-finite prediction keeps the
+// zero start.  A miss's contact and bodies lie on about 27 cache lines of
+// their own, whose gathers bound the kernel, so a workgroup gathers for 64
+// misses at once (256 piles, 43 k misses: 75 us; with 32 misses a
+// workgroup of 8 waves 95 us; with the weights in LDS, which left one
+// workgroup to a CU, 160 us).
+constexpr int INFER_ROWS = MLP_INFER_ROWS, INFER_THREADS = MLP_INFER_THREADS;
+
+__global__ __launch_bounds__(INFER_THREADS) __attribute__((amdgpu_waves_per_eu(3))) void k_mlp_infer(Ctx c) {
+  __shared__ __align__(16) uint16_t sx[INFER_ROWS * XS], ha[16 * HS], hb[16 * HS];
+  __shared__ __align__(16) float sb[3 * 128 + 16];
+  __shared__ float2 sy[INFER_ROWS];
   int n = c.counters[CNT_MISS];
   if (n > c.miss_cap) n = c.miss_cap;
-  if ((int)blockIdx.x * TILE >= n) return;  // no tile: skip the staging (no barrier follows)
-  for (int i = threadIdx.x; i < 128 * 128; i += 256) {
-    const int k = i >> 7, o = i & 127;  // read row-major [k][o], coalesced
-    s_w2[o * WT2 + k] = m.w2[i];
-    s_w3[o * WT2 + k] = m.w3[i];
-    if (k < 16) s_w1[o * WT1 + k] = m.w1[i];
-    if (o < 16) s_w4[o * WT2 + k] = m.w4[k * 16 + o];
-  }
-  for (int i = threadIdx.x; i < 3 * 128 + 16; i += 256)
-    s_b[i] = i < 128 ? m.b1[i] : i < 256 ? m.b2[i - 128] : i < 384 ? m.b3[i - 256] : m.b4[i - 384];
-  __syncthreads();
-  MlpDev ml;
-  ml.w1 = s_w1;
-  ml.w2 = s_w2;
-  ml.w3 = s_w3;
-  ml.w4 = s_w4;
-  ml.b1 = s_b;
-  ml.b2 = s_b + 128;
-  ml.b3 = s_b + 256;
-  ml.b4 = s_b + 384;
-  for (int t = blockIdx.x; t * TILE < n; t += gridDim.x) {
-    int row0 = t * TILE;
-    // the output head's inputs of this lane's row (first wavefront), loaded
-    // with the features so that the head waits on no load after the layers
-    static_assert(TILE == 64, "one row per lane of the first wavefront");
-    const bool row_ok = threadIdx.x < TILE && row0 + (int)threadIdx.x < n;
+  if ((int)blockIdx.x * INFER_ROWS >= n) return;  // nothing to do (no barrier follows)
+  WaveWeights W;
+  load_weights(c.mlp_wfr, W);
+  load_biases(c.mlp_w, sb);
+  static_assert(INFER_ROWS == 64 && INFER_THREADS == 256, "a row per lane of the first wavefront");
+  const int r = threadIdx.x;
+  const bool row_lane = r < INFER_ROWS;
+  for (int t = blockIdx.x; t * INFER_ROWS < n; t += gridDim.x) {
+    const int row0 = t * INFER_ROWS;
+    // the output head's inputs of this lane's row, loaded with the features so
+    // that the head waits on no load after the layers
+    const bool row_ok = row_lane && row0 + r < n;
     int hk = 0, hmr = -1;
     double hmcn = 1.0, hmct = 1.0, hmu = 0.0;
     if (row_ok) {
-      hk = c.miss_idx[row0 + threadIdx.x];
-      hmr = c.solver == SHP_SOLVER_COLORED_F32 ? c.miss_rec[row0 + threadIdx.x] : -1;
+      hk = c.miss_idx[row0 + r];
+      hmr = c.solver == SHP_SOLVER_COLORED_F32 ? c.miss_rec[row0 + r] : -1;
       hmcn = c.mcn[hk];
       hmct = c.mct[hk];
       hmu = (c.mu[c.ga[hk]] + c.mu[c.gb[hk]]) / 2.0;
     }
     if (c.features_in_contacts) {
-      for (int i = threadIdx.x; i < TILE * 16; i += 256) {
-        int r = i >> 4, q = i & 15;
-        float f = (row0 + r < n && q < MLP_IN) ? c.miss_feat[(size_t)(row0 + r) * MLP_IN + q] : 0.0f;
-        sx[i] = f2bf(f);
+      for (int i = threadIdx.x; i < INFER_ROWS * 16; i += INFER_THREADS) {
+        const int i_r = i >> 4, q = i & 15;
+        float f = (row0 + i_r < n && q < MLP_IN) ? c.miss_feat[(size_t)(row0 + i_r) * MLP_IN + q] : 0.0f;
+        sx[i_r * XS + q] = f2bf(f);
       }
-    } else if (threadIdx.x < TILE) {
-      // one row per lane of the first wavefront: the features of the
-      // stored contact, as the contact kernel would compute them (the
-      // velocities are those it saw: nothing has changed them since)
-      const int r = threadIdx.x;
+    } else if (row_lane) {
+      // the features of the stored contact, as the contact kernel would
+      // compute them (the velocities are those it saw: nothing has changed
+      // them since)
       float f[MLP_IN];
       for (int q = 0; q < MLP_IN; ++q) f[q] = 0.0f;
       if (row_ok) {
@@ -512,33 +646,30 @@ __global__ __launch_bounds__(256) void k_mlp_infer(Ctx c, MlpDev m) {
                      c.rby[k], c.iml[ga], c.iml[gb], c.imr[ga], c.imr[gb],
                      (c.mu[ga] + c.mu[gb]) / 2.0, f);
       }
-      for (int q = 0; q < 16; ++q) sx[r * 16 + q] = f2bf(q < MLP_IN ? f[q] : 0.0f);
+      for (int q = 0; q < 16; ++q) sx[r * XS + q] = f2bf(q < MLP_IN ? f[q] : 0.0f);
     }
-    __syncthreads();
-    forward_tile<true>(ml, sx, s1, s2, sy, nullptr, row0);
-    if (threadIdx.x < TILE) {  // the first wavefront: one row per lane
-      bool set = false;
-      if (row_ok) {
-        int r = threadIdx.x;
-        int k = hk;
-        double ln = (double)sy[r * 16];
-        ln = ln > 0.0 ? ln / hmcn : 0.0;
-        double lt = (double)sy[r * 16 + 1] / hmct;
-        double mu = hmu;
-        double thr = ln * mu;
-        lt = lt > thr ? thr : (lt < -thr ? -thr : lt);
-        if (ln - ln == 0.0 && lt - lt == 0.0) {
-          c.ln[k] = ln;
-          c.lt[k] = lt;
-          c.warm[k] = 2;
-          set = true;
-          if (hmr >= 0) shp::patch_record_warm(shp::packf(c), hmr >> 1, hmr & 1, ln, lt);
-        }
+    for (int o = 0; o < INFER_ROWS; o += 16)
+      mlp_layers(W, sb, sx + o * XS, ha, hb,
+                 [&](int i, float y0, float y1) { sy[o + i] = make_float2(y0, y1); });
+    bool set = false;
+    if (row_ok) {
+      const int k = hk;
+      double ln = (double)sy[r].x;
+      ln = ln > 0.0 ? ln / hmcn : 0.0;
+      double lt = (double)sy[r].y / hmct;
+      const double thr = ln * hmu;
+      lt = lt > thr ? thr : (lt < -thr ? -thr : lt);
+      if (ln - ln == 0.0 && lt - lt == 0.0) {
+        c.ln[k] = ln;
+        c.lt[k] = lt;
+        c.warm[k] = 2;
+        set = true;
+        if (hmr >= 0) shp::patch_record_warm(shp::packf(c), hmr >> 1, hmr & 1, ln, lt);
       }
-      const unsigned long long setm = __ballot(set);  // one atomic per tile
-      if (threadIdx.x == 0 && setm) atomicAdd(&c.counters[CNT_LEARNED], (int)__popcll(setm));
     }
-    __syncthreads();
+    const unsigned long long setm = __ballot(set);  // one atomic per tile
+    if (threadIdx.x == 0 && setm) atomicAdd(&c.counters[CNT_LEARNED], (int)__popcll(setm));
+    // (the next rows' features and outputs are written behind barriers)
   }
 }
 
@@ -558,23 +689,13 @@ __global__ void k_mlp_log(Ctx c) {
 }
 
 void mlp_launch_infer(shp_batch* b) {
-  MlpDev m;
-  m.w1 = b->ctx.mlp_wbf + MLP_OFF_W1;
-  m.w2 = b->ctx.mlp_wbf + MLP_OFF_W2;
-  m.w3 = b->ctx.mlp_wbf + MLP_OFF_W3;
-  m.w4 = b->ctx.mlp_wbf + MLP_OFF_W4;
-  m.b1 = b->ctx.mlp_w + MLP_OFF_B1;
-  m.b2 = b->ctx.mlp_w + MLP_OFF_B2;
-  m.b3 = b->ctx.mlp_w + MLP_OFF_B3;
-  m.b4 = b->ctx.mlp_w + MLP_OFF_B4;
-  k_mlp_infer<<<b->plan.g_infer, 256, 0, b->stream>>>(b->ctx, m);
+  k_mlp_infer<<<b->plan.g_infer, INFER_THREADS, 0, b->stream>>>(b->ctx);
 }
 
-// sx, s1, s2 (BF16) and sy (FP32) of k_mlp_infer
+// sx, ha, hb (BF16), sb and sy (FP32) of k_mlp_infer
 size_t mlp_infer_static_lds() {
-  return lds16(TILE * 16 * 2) + 2 * lds16(TILE * 128 * 2) + lds16(TILE * 16 * 4) +
-         lds16(128 * WT1 * 2) + 2 * lds16(128 * WT2 * 2) + lds16(16 * WT2 * 2) +
-         lds16((3 * 128 + 16) * 4);
+  return lds16(INFER_ROWS * XS * 2) + 2 * lds16(16 * HS * 2) + lds16((3 * 128 + 16) * 4) +
+         lds16(INFER_ROWS * 8);
 }
 
 void mlp_launch_log(shp_batch* b) {
@@ -593,7 +714,9 @@ struct shp_mlp {
   int cap_rows = 0;
   uint16_t* X = nullptr;   // cap_rows x 16
   float* T = nullptr;      // cap_rows x 2
-  float* Fin = nullptr;    // cap_rows x 14 staging
+  int cap_fwd = 0;
+  float* Fin = nullptr;    // cap_fwd x 14 staging
+  float* out = nullptr;    // cap_fwd x 2 outputs
   TrainBufs tb{};
   long adam_t = 0;
   // training set on device
@@ -608,49 +731,37 @@ static shp_status mlp_fail(shp_status s, const char* m) {
   return s;
 }
 
-// ---- forward pass that allocates nothing (shp_mlp_forward_noalloc) --------
-// Its staging - the padded BF16 input rows and the FP32 output rows of up
-// to MLP_NOALLOC_MAX_ROWS rows (96 B a row, 6 MiB) - lives in this
-// file-scope device array instead of the handle's buffers.  Each GPU holds
-// its own copy until the process ends; every call on a GPU shares it.
+// rows of one shp_mlp_forward_noalloc call
 #define MLP_NOALLOC_MAX_ROWS 65536
-static __device__ __align__(256) unsigned char scratch[(size_t)MLP_NOALLOC_MAX_ROWS * 16 * (2 + 4)];
-#define MLP_MAX_DEVICES 64
-static void* g_scratch_ptr[MLP_MAX_DEVICES];  // device address of `scratch` per GPU
-static std::mutex g_scratch_mu;
-
-// The device address of `scratch` on the current GPU, taken once per GPU
-// (its host-side name is not a device address).
-static shp_status scratch_setup(int dev) {
-  if (dev < 0 || dev >= MLP_MAX_DEVICES) return mlp_fail(SHP_E_UNSUPPORTED, "device index");
-  std::lock_guard<std::mutex> lock(g_scratch_mu);
-  if (g_scratch_ptr[dev]) return SHP_OK;
-  void* ptr = nullptr;
-  if (hipGetSymbolAddress(&ptr, HIP_SYMBOL(scratch)) != hipSuccess || !ptr)
-    return mlp_fail(SHP_E_HIP, "hipGetSymbolAddress(scratch) failed");
-  g_scratch_ptr[dev] = ptr;
-  return SHP_OK;
-}
-
-// out[2 r + k] = y[16 r + k], k < 2, r < n
-__global__ void k_take_outputs(const float* y, int n, float* out) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < 2 * n) out[i] = y[(size_t)(i >> 1) * 16 + (i & 1)];
-}
 
 #define MCHK(x) \
   do { if ((x) != hipSuccess) return mlp_fail(SHP_E_HIP, #x); } while (0)
 
+// feature rows and outputs of calls on host memory
+static shp_status mlp_reserve_forward(shp_mlp* h, int rows) {
+  if (rows <= h->cap_fwd) return SHP_OK;
+  for (void* q : {(void*)h->Fin, (void*)h->out})
+    if (q) (void)hipFree(q);
+  h->Fin = h->out = nullptr;
+  h->cap_fwd = 0;
+  rows = ((rows + TILE - 1) / TILE) * TILE;
+  MCHK(hipMalloc(&h->Fin, (size_t)rows * MLP_IN * 4));
+  MCHK(hipMalloc(&h->out, (size_t)rows * 2 * 4));
+  h->cap_fwd = rows;
+  return SHP_OK;
+}
+
 static shp_status mlp_reserve(shp_mlp* h, int rows) {
+  shp_status st = mlp_reserve_forward(h, rows);
+  if (st != SHP_OK) return st;
   if (rows <= h->cap_rows) return SHP_OK;
   rows = ((rows + TILE - 1) / TILE) * TILE;
-  void* ptrs[] = {h->X, h->T, h->Fin, h->tb.z1, h->tb.z2, h->tb.z3, h->tb.h1, h->tb.h2, h->tb.h3, h->tb.y};
+  void* ptrs[] = {h->X, h->T, h->tb.z1, h->tb.z2, h->tb.z3, h->tb.h1, h->tb.h2, h->tb.h3, h->tb.y};
   for (void* q : ptrs)
     if (q) (void)hipFree(q);
   size_t R = rows;
   MCHK(hipMalloc(&h->X, R * 16 * 2));
   MCHK(hipMalloc(&h->T, R * 2 * 4));
-  MCHK(hipMalloc(&h->Fin, R * MLP_IN * 4));
   MCHK(hipMalloc(&h->tb.z1, R * 128 * 4));
   MCHK(hipMalloc(&h->tb.z2, R * 128 * 4));
   MCHK(hipMalloc(&h->tb.z3, R * 128 * 4));
@@ -683,7 +794,7 @@ static shp_status mlp_grad_rows(shp_mlp* h, int n) {
   int tiles = rows / TILE;
   int fg = tiles < 1024 ? tiles : 1024;
   MlpDev m = mlp_view(h->p);
-  k_mlp_forward<<<fg, 256, 0, h->stream>>>(m, h->X, rows, h->tb.y, h->tb, 1);
+  k_mlp_forward<<<fg, 256, 0, h->stream>>>(m, h->X, rows, h->tb.y, h->tb);
   int parts = tiles < h->parts ? tiles : h->parts;
   k_mlp_backward<<<parts, 256, 0, h->stream>>>(m, h->X, h->T, rows, n, h->tb, h->partial, h->huber);
   k_mlp_reduce<<<(MLP_NPARAM_PAD + 255) / 256, 256, 0, h->stream>>>(h->partial, parts, h->grad);
@@ -701,10 +812,6 @@ shp_status shp_mlp_create(const float* params, shp_mlp** out) {
   if (hipGetDevice(&h->device) != hipSuccess) {
     delete h;
     return mlp_fail(SHP_E_HIP, "no HIP device");
-  }
-  if (scratch_setup(h->device) != SHP_OK) {
-    delete h;
-    return SHP_E_HIP;
   }
   if (hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking) != hipSuccess) {
     delete h;
@@ -740,7 +847,7 @@ shp_status shp_mlp_destroy(shp_mlp* h) {
   if (!h) return SHP_OK;
   if (h->stream) (void)hipStreamSynchronize(h->stream);
   mlp_params_free(&h->p);
-  void* ptrs[] = {h->mom, h->vel, h->grad, h->partial, h->mask, h->X, h->T, h->Fin, h->tb.z1,
+  void* ptrs[] = {h->mom, h->vel, h->grad, h->partial, h->mask, h->X, h->T, h->Fin, h->out, h->tb.z1,
                   h->tb.z2, h->tb.z3, h->tb.h1, h->tb.h2, h->tb.h3, h->tb.y, h->dX, h->dT};
   for (void* q : ptrs)
     if (q) (void)hipFree(q);
@@ -761,19 +868,13 @@ shp_status shp_mlp_get_params(shp_mlp* h, float* params) {
 shp_status shp_mlp_forward(shp_mlp* h, const float* feats, int32_t n, float* out) {
   if (!h || n < 0 || (n > 0 && (!feats || !out))) return mlp_fail(SHP_E_INVAL, "bad argument");
   if (n == 0) return SHP_OK;
-  shp_status st = mlp_reserve(h, n);
+  shp_status st = mlp_reserve_forward(h, n);
   if (st != SHP_OK) return st;
-  int rows = ((n + TILE - 1) / TILE) * TILE;
   MCHK(hipMemcpyAsync(h->Fin, feats, (size_t)n * MLP_IN * 4, hipMemcpyHostToDevice, h->stream));
-  k_pack_features<<<(rows * 16 + 255) / 256, 256, 0, h->stream>>>(h->Fin, n, rows, h->X);
-  mlp_launch_forward(h->p, h->X, rows, h->tb.y, h->stream);
-  std::vector<float> y((size_t)rows * 16);
-  MCHK(hipMemcpyAsync(y.data(), h->tb.y, y.size() * 4, hipMemcpyDeviceToHost, h->stream));
+  launch_eval(h->p, h->Fin, n, h->out, h->stream);
+  MCHK(hipGetLastError());
+  MCHK(hipMemcpyAsync(out, h->out, (size_t)n * 2 * 4, hipMemcpyDeviceToHost, h->stream));
   MCHK(hipStreamSynchronize(h->stream));
-  for (int r = 0; r < n; ++r) {
-    out[2 * r] = y[(size_t)r * 16];
-    out[2 * r + 1] = y[(size_t)r * 16 + 1];
-  }
   return SHP_OK;
 }
 
@@ -781,21 +882,12 @@ shp_status shp_mlp_forward_noalloc(shp_mlp* h, const float* d_feats, int32_t n, 
                                    void* stream) {
   if (!h || n < 0 || (n > 0 && (!d_feats || !d_out))) return mlp_fail(SHP_E_INVAL, "bad argument");
   if (n > MLP_NOALLOC_MAX_ROWS)
-    return mlp_fail(SHP_E_INVAL, "n exceeds the 65536 rows of the static scratch");
+    return mlp_fail(SHP_E_INVAL, "n exceeds 65536 rows");
   if (n == 0) return SHP_OK;
   int dev = -1;
   MCHK(hipGetDevice(&dev));
   if (dev != h->device) return mlp_fail(SHP_E_INVAL, "the current device is not the handle's");
-  void* base = g_scratch_ptr[dev];
-  if (!base) return mlp_fail(SHP_E_HIP, "scratch not set up on this device");
-  uint16_t* X = (uint16_t*)base;                                                    // rows x 16 BF16
-  float* Y = (float*)((unsigned char*)base + (size_t)MLP_NOALLOC_MAX_ROWS * 16 * 2);  // rows x 16
-  hipStream_t s = stream ? (hipStream_t)stream : h->stream;
-  const int rows = ((n + TILE - 1) / TILE) * TILE;
-  // the rows n..rows-1 are packed as zeros, so nothing needs clearing
-  k_pack_features<<<(rows * 16 + 255) / 256, 256, 0, s>>>(d_feats, n, rows, X);
-  mlp_launch_forward(h->p, X, rows, Y, s);
-  k_take_outputs<<<(2 * n + 255) / 256, 256, 0, s>>>(Y, n, d_out);
+  launch_eval(h->p, d_feats, n, d_out, stream ? (hipStream_t)stream : h->stream);
   MCHK(hipGetLastError());
   return SHP_OK;
 }
@@ -884,7 +976,7 @@ shp_status shp_mlp_train(shp_mlp* h, const int32_t* indices, int32_t steps, int3
     float b1c = 1.0f - powf(0.9f, (float)h->adam_t);
     float b2c = 1.0f - powf(0.999f, (float)h->adam_t);
     k_mlp_adam<<<(MLP_NPARAM_PAD + 255) / 256, 256, 0, h->stream>>>(h->p.w, h->mom, h->vel, h->grad, h->mask,
-                                                                    h->p.wbf, lr, b1c, b2c);
+                                                                    h->p.wbf, h->p.wfr, lr, b1c, b2c);
     if (loss_out) {
       MCHK(hipMemcpyAsync(y.data(), h->tb.y, y.size() * 4, hipMemcpyDeviceToHost, h->stream));
       MCHK(hipMemcpyAsync(t.data(), h->T, t.size() * 4, hipMemcpyDeviceToHost, h->stream));
