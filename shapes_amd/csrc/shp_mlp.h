@@ -34,7 +34,12 @@
 #define MLP_F2 (MLP_F1 + 8 * MLP_FRAG)   // 8 ct x 8 kb
 #define MLP_F3 (MLP_F2 + 64 * MLP_FRAG)  // 8 ct x 8 kb
 #define MLP_F4 (MLP_F3 + 64 * MLP_FRAG)  // 8 kb
-#define MLP_NFRAG (MLP_F4 + 8 * MLP_FRAG)
+// Backward fragments hold W blocks: lane l has W[16 it + l % 16][16 kb +
+// 4 (l / 16) + 0..3] of block (input rows it, output columns kb), kb inside it.
+#define MLP_G4 (MLP_F4 + 8 * MLP_FRAG)   // 8 it
+#define MLP_G3 (MLP_G4 + 8 * MLP_FRAG)   // 8 it x 8 kb
+#define MLP_G2 (MLP_G3 + 64 * MLP_FRAG)  // 8 it x 8 kb
+#define MLP_NFRAG (MLP_G2 + 64 * MLP_FRAG)
 
 // the in-step inference: misses per workgroup at a time, and its lanes
 #define MLP_INFER_ROWS 64
@@ -42,8 +47,7 @@
 
 struct MlpParams {
   float* w = nullptr;       // FP32 master copy, padded layout
-  uint16_t* wbf = nullptr;  // BF16 copy, padded layout (training)
-  uint16_t* wfr = nullptr;  // BF16 copy in fragments
+  uint16_t* wfr = nullptr;  // BF16 copy used by the matrix cores, in fragments
 };
 
 // The 14 input features of a contact that missed the cache, computed from
@@ -84,7 +88,6 @@ __device__ __forceinline__ void mlp_features(double nrx, double nry, double dept
   }
 }
 
-int mlp_padded_index(int k);
 shp_status mlp_params_alloc(MlpParams* p);
 void mlp_params_free(MlpParams* p);
 shp_status mlp_params_upload(MlpParams* p, const float* params, hipStream_t s);

@@ -10,12 +10,11 @@
 //   k_mlp_eval      forward of feature rows, 16 at a time (4 waves)
 //   k_mlp_infer     the same on a step's cache misses, features and output
 //                   head included
-//   k_mlp_forward   forward of tiles of 64 rows storing what training needs
-//   k_mlp_backward  fused backward over tiles; weight gradients accumulate
-//                   in MFMA accumulators across a workgroup's tiles and are
-//                   written as one partial per workgroup (no atomics)
-//   k_mlp_reduce    sums the partials in a fixed order (deterministic)
-//   k_mlp_adam      Adam update of the FP32 master weights + BF16 copies
+//   k_mlp_rows      training: forward and backward of 16 rows at a time; the
+//                   activations and their gradients in fragments
+//   k_mlp_weights   training: the weight gradients from those, summed in a
+//                   fixed order (deterministic), then Adam on the FP32
+//                   master weights and their BF16 fragments
 //
 // The inference kernels keep the weights in registers: wave w computes output
 // columns [32 w, 32 w + 32) of every layer, so it needs 2 x (1 + 8 + 8 + 8)
@@ -26,6 +25,7 @@
 // sums over k are those of h W, in the same order.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <string.h>
 
 #include <string>
 #include <vector>
@@ -61,305 +61,34 @@ __device__ __forceinline__ f32x4 mfma16(bf16x4 a, bf16x4 b, f32x4 c) {
 // Operand fragments of v_mfma_f32_16x16x16_bf16: lane l holds
 //   A[row = l%16][k = 4*(l/16) + 0..3]   B[k = 4*(l/16) + 0..3][col = l%16]
 // and receives D[row = 4*(l/16) + i][col = l%16], i = 0..3.
-__device__ __forceinline__ bf16x4 frag_a(const uint16_t* A, int lda, int r0, int k0) {
-  int l = threadIdx.x & 63;
-  const uint16_t* p = A + (r0 + (l & 15)) * lda + k0 + 4 * (l >> 4);
-  bf16x4 v;
-  v[0] = (short)p[0];
-  v[1] = (short)p[1];
-  v[2] = (short)p[2];
-  v[3] = (short)p[3];
-  return v;
-}
-// A stored transposed: element (r, k) at A[k * lda + r]
-__device__ __forceinline__ bf16x4 frag_at(const uint16_t* A, int lda, int r0, int k0) {
-  int l = threadIdx.x & 63;
-  int r = r0 + (l & 15), k = k0 + 4 * (l >> 4);
-  bf16x4 v;
-  v[0] = (short)A[(k + 0) * lda + r];
-  v[1] = (short)A[(k + 1) * lda + r];
-  v[2] = (short)A[(k + 2) * lda + r];
-  v[3] = (short)A[(k + 3) * lda + r];
-  return v;
-}
-// B row-major K x N: element (k, n) at B[k * ldb + n]
-__device__ __forceinline__ bf16x4 frag_b(const uint16_t* B, int ldb, int k0, int c0) {
-  int l = threadIdx.x & 63;
-  int n = c0 + (l & 15), k = k0 + 4 * (l >> 4);
-  bf16x4 v;
-  v[0] = (short)B[(k + 0) * ldb + n];
-  v[1] = (short)B[(k + 1) * ldb + n];
-  v[2] = (short)B[(k + 2) * ldb + n];
-  v[3] = (short)B[(k + 3) * ldb + n];
-  return v;
-}
-// B given as its transpose: element (k, n) at B[n * ldb + k]
-__device__ __forceinline__ bf16x4 frag_bt(const uint16_t* B, int ldb, int k0, int c0) {
-  int l = threadIdx.x & 63;
-  const uint16_t* p = B + (c0 + (l & 15)) * ldb + k0 + 4 * (l >> 4);
-  bf16x4 v;
-  v[0] = (short)p[0];
-  v[1] = (short)p[1];
-  v[2] = (short)p[2];
-  v[3] = (short)p[3];
-  return v;
-}
+#define TILE 64  // rows of a training tile: weight gradients are summed over a tile, then over tiles
+#define MLP_PARTS 64  // ... in this many sums, tile t in sum t % MLP_PARTS, which are added in order
 
-struct MlpDev {
-  // BF16 weights, row-major [in][out] with padded shapes
-  const uint16_t *w1, *w2, *w3, *w4;  // 16x128, 128x128, 128x128, 128x16
-  const float *b1, *b2, *b3, *b4;     // 128, 128, 128, 16
-};
-
-struct TrainBufs {
-  float *z1, *z2, *z3;        // pre-activations, rows x 128
-  uint16_t *h1, *h2, *h3;     // BF16 activations, rows x 128
-  float* y;                   // outputs, rows x 16 (cols 0,1 used)
-};
-
-#define TILE 64
-
-// One 64-row tile: X (64 x 16 BF16) in LDS -> Y (64 x 16 FP32).
-// Wave w owns rows 16w..16w+15.
-__device__ void forward_tile(const MlpDev& m, uint16_t* sx, uint16_t* s1, uint16_t* s2,
-                             float* yout /* 64 x 16 */, const TrainBufs* tb, int row0) {
-  int wv = threadIdx.x >> 6, l = threadIdx.x & 63;
-  int r0 = 16 * wv;
-  // layer 1: K = 16
-  for (int ct = 0; ct < 8; ++ct) {
-    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-    acc = mfma16(frag_a(sx, 16, r0, 0),
-                 frag_b(m.w1, 128, 0, 16 * ct), acc);
-    int col = 16 * ct + (l & 15);
-    for (int i = 0; i < 4; ++i) {
-      int row = r0 + 4 * (l >> 4) + i;
-      float z = acc[i] + m.b1[col];
-      uint16_t h = f2bf(silu(z));
-      s1[row * 128 + col] = h;
-      if (tb) {
-        tb->z1[(size_t)(row0 + row) * 128 + col] = z;
-        tb->h1[(size_t)(row0 + row) * 128 + col] = h;
-      }
-    }
-  }
-  __syncthreads();
-  // layers 2 and 3: K = 128
-  for (int layer = 0; layer < 2; ++layer) {
-    const uint16_t* in = layer == 0 ? s1 : s2;
-    uint16_t* out = layer == 0 ? s2 : s1;
-    const uint16_t* W = layer == 0 ? m.w2 : m.w3;
-    const float* bias = layer == 0 ? m.b2 : m.b3;
-    float* zs = tb ? (layer == 0 ? tb->z2 : tb->z3) : nullptr;
-    uint16_t* hs = tb ? (layer == 0 ? tb->h2 : tb->h3) : nullptr;
-    f32x4 acc[8];
-    for (int ct = 0; ct < 8; ++ct) acc[ct] = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (int k0 = 0; k0 < 128; k0 += 16) {
-      bf16x4 a = frag_a(in, 128, r0, k0);
-      for (int ct = 0; ct < 8; ++ct)
-        acc[ct] = mfma16(a, frag_b(W, 128, k0, 16 * ct), acc[ct]);
-    }
-    __syncthreads();  // every wave has read `in` before `out` (== in of layer 1) is overwritten
-    for (int ct = 0; ct < 8; ++ct) {
-      int col = 16 * ct + (l & 15);
-      for (int i = 0; i < 4; ++i) {
-        int row = r0 + 4 * (l >> 4) + i;
-        float z = acc[ct][i] + bias[col];
-        uint16_t h = f2bf(silu(z));
-        out[row * 128 + col] = h;
-        if (tb) {
-          zs[(size_t)(row0 + row) * 128 + col] = z;
-          hs[(size_t)(row0 + row) * 128 + col] = h;
-        }
-      }
-    }
-    __syncthreads();
-  }
-  // layer 4: 128 -> 16 (2 used), input in s1
-  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-  for (int k0 = 0; k0 < 128; k0 += 16)
-    acc = mfma16(frag_a(s1, 128, r0, k0), frag_b(m.w4, 16, k0, 0), acc);
-  int col = l & 15;
-  for (int i = 0; i < 4; ++i) {
-    int row = r0 + 4 * (l >> 4) + i;
-    yout[row * 16 + col] = acc[i] + m.b4[col];
-  }
-  __syncthreads();
-}
-
-__global__ __launch_bounds__(256) void k_mlp_forward(MlpDev m, const uint16_t* X /* rows x 16 */,
-                                                     int rows, float* Y /* rows x 16 */,
-                                                     TrainBufs tb) {
-  __shared__ uint16_t sx[TILE * 16];
-  __shared__ uint16_t s1[TILE * 128];
-  __shared__ uint16_t s2[TILE * 128];
-  __shared__ float sy[TILE * 16];
-  for (int t = blockIdx.x; t * TILE < rows; t += gridDim.x) {
-    int row0 = t * TILE;
-    for (int i = threadIdx.x; i < TILE * 16; i += 256) sx[i] = X[(size_t)row0 * 16 + i];
-    __syncthreads();
-    forward_tile(m, sx, s1, s2, sy, &tb, row0);
-    for (int i = threadIdx.x; i < TILE * 16; i += 256) Y[(size_t)row0 * 16 + i] = sy[i];
-    __syncthreads();
-  }
-}
-
-// Backward of the mean loss over `rows` rows (rows % 64 == 0) given the
-// forward buffers: squared error (huber = 0), dY = 2 (Y - T) / n_real, or
-// twice the Huber loss with threshold `huber`, dY = 2 clamp(Y - T, +-huber)
-// / n_real (the same gradient where |Y - T| <= huber).
-// Workgroup g accumulates the weight gradients of its tiles in MFMA
-// accumulators and writes partial g (MLP_NPARAM_PAD floats).
-__global__ __launch_bounds__(256) void k_mlp_backward(MlpDev m, const uint16_t* X, const float* T,
-                                                      int rows, int n_real, TrainBufs tb,
-                                                      float* partial, float huber) {
-  __shared__ uint16_t s_dy[TILE * 16];
-  __shared__ uint16_t s_da[TILE * 128];
-  __shared__ uint16_t s_db[TILE * 128];
-  __shared__ float s_bias[3 * 128 + 16];
-  int wv = threadIdx.x >> 6, l = threadIdx.x & 63;
-  // this wave's output tiles of each weight gradient
-  //   dW4 128x16: 8 row tiles -> wave w owns row tiles {2w, 2w+1}
-  //   dW3, dW2 128x128: 64 tiles -> wave w owns row tiles {2w, 2w+1} x 8 cols
-  //   dW1 16x128: 8 col tiles -> wave w owns col tiles {2w, 2w+1}
-  f32x4 g4[2], g3[16], g2[16], g1[2];
-  for (int i = 0; i < 2; ++i) g4[i] = g1[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-  for (int i = 0; i < 16; ++i) g3[i] = g2[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-  for (int i = threadIdx.x; i < 3 * 128 + 16; i += 256) s_bias[i] = 0.f;
-  float inv_n = 2.0f / (float)n_real;
-  for (int t = blockIdx.x; t * TILE < rows; t += gridDim.x) {
-    int row0 = t * TILE;
-    __syncthreads();
-    for (int i = threadIdx.x; i < TILE * 16; i += 256) {
-      int r = i >> 4, cc = i & 15;
-      float d = 0.f;
-      if (cc < 2 && row0 + r < n_real) {
-        float e = tb.y[(size_t)(row0 + r) * 16 + cc] - T[(size_t)(row0 + r) * 2 + cc];
-        if (huber > 0.f) e = fminf(fmaxf(e, -huber), huber);
-        d = e * inv_n;
-      }
-      s_dy[i] = f2bf(d);
-      if (cc < 2) atomicAdd(&s_bias[3 * 128 + cc], d);
-    }
-    __syncthreads();
-    // dW4 += H3^T dY   (H3 rows x 128 global, transposed read)
-    for (int i = 0; i < 2; ++i) {
-      int rt = 2 * wv + i;
-      for (int k0 = 0; k0 < TILE; k0 += 16)
-        g4[i] = mfma16(frag_at(tb.h3 + (size_t)row0 * 128, 128, 16 * rt, k0), frag_b(s_dy, 16, k0, 0), g4[i]);
-    }
-    // dZ3 = (dY W4^T) * silu'(Z3)   (64 x 128): wave w rows 16w.., 8 col tiles, K = 16
-    const uint16_t* Ws[3] = {m.w3, m.w2, nullptr};
-    uint16_t* dz_cur = s_da;
-    {
-      int r0 = 16 * wv;
-      for (int ct = 0; ct < 8; ++ct) {
-        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-        acc = mfma16(frag_a(s_dy, 16, r0, 0), frag_bt(m.w4, 16, 0, 16 * ct), acc);
-        int col = 16 * ct + (l & 15);
-        float bsum = 0.f;
-        for (int i = 0; i < 4; ++i) {
-          int row = r0 + 4 * (l >> 4) + i;
-          float d = acc[i] * dsilu(tb.z3[(size_t)(row0 + row) * 128 + col]);
-          dz_cur[row * 128 + col] = f2bf(d);
-          bsum += d;
-        }
-        atomicAdd(&s_bias[2 * 128 + col], bsum);
-      }
-    }
-    __syncthreads();
-    // layers 3 and 2: dW_L += H_{L-1}^T dZ_L ; dZ_{L-1} = (dZ_L W_L^T) * silu'(Z_{L-1})
-    for (int layer = 0; layer < 2; ++layer) {
-      const uint16_t* hprev = layer == 0 ? tb.h2 : tb.h1;
-      const float* zprev = layer == 0 ? tb.z2 : tb.z1;
-      f32x4* g = layer == 0 ? g3 : g2;
-      uint16_t* dz_next = dz_cur == s_da ? s_db : s_da;
-      for (int i = 0; i < 2; ++i) {
-        int rt = 2 * wv + i;
-        for (int k0 = 0; k0 < TILE; k0 += 16) {
-          bf16x4 a = frag_at(hprev + (size_t)row0 * 128, 128, 16 * rt, k0);
-          for (int ct = 0; ct < 8; ++ct) g[8 * i + ct] = mfma16(a, frag_b(dz_cur, 128, k0, 16 * ct), g[8 * i + ct]);
-        }
-      }
-      int r0 = 16 * wv;
-      f32x4 acc[8];
-      for (int ct = 0; ct < 8; ++ct) acc[ct] = f32x4{0.f, 0.f, 0.f, 0.f};
-      for (int k0 = 0; k0 < 128; k0 += 16) {
-        bf16x4 a = frag_a(dz_cur, 128, r0, k0);
-        for (int ct = 0; ct < 8; ++ct) acc[ct] = mfma16(a, frag_bt(Ws[layer], 128, k0, 16 * ct), acc[ct]);
-      }
-      for (int ct = 0; ct < 8; ++ct) {
-        int col = 16 * ct + (l & 15);
-        float bsum = 0.f;
-        for (int i = 0; i < 4; ++i) {
-          int row = r0 + 4 * (l >> 4) + i;
-          float d = acc[ct][i] * dsilu(zprev[(size_t)(row0 + row) * 128 + col]);
-          dz_next[row * 128 + col] = f2bf(d);
-          bsum += d;
-        }
-        atomicAdd(&s_bias[(1 - layer) * 128 + col], bsum);
-      }
-      __syncthreads();
-      dz_cur = dz_next;
-    }
-    // dW1 += X^T dZ1   (16 x 128): wave w col tiles {2w, 2w+1}
-    for (int i = 0; i < 2; ++i) {
-      int ct = 2 * wv + i;
-      for (int k0 = 0; k0 < TILE; k0 += 16)
-        g1[i] = mfma16(frag_at(X + (size_t)row0 * 16, 16, 0, k0), frag_b(dz_cur, 128, k0, 16 * ct), g1[i]);
-    }
-  }
-  __syncthreads();
-  float* P = partial + (size_t)blockIdx.x * MLP_NPARAM_PAD;
-  int col = l & 15;
-  for (int i = 0; i < 2; ++i) {
-    int rt = 2 * wv + i;
-    for (int q = 0; q < 4; ++q) {
-      int row = 4 * (l >> 4) + q;
-      P[MLP_OFF_W4 + (16 * rt + row) * 16 + col] = g4[i][q];
-      P[MLP_OFF_W1 + row * 128 + 16 * (2 * wv + i) + col] = g1[i][q];
-      for (int ct = 0; ct < 8; ++ct) {
-        P[MLP_OFF_W3 + (16 * rt + row) * 128 + 16 * ct + col] = g3[8 * i + ct][q];
-        P[MLP_OFF_W2 + (16 * rt + row) * 128 + 16 * ct + col] = g2[8 * i + ct][q];
-      }
-    }
-  }
-  for (int i = threadIdx.x; i < 128; i += 256) {
-    P[MLP_OFF_B1 + i] = s_bias[i];
-    P[MLP_OFF_B2 + i] = s_bias[128 + i];
-    P[MLP_OFF_B3 + i] = s_bias[256 + i];
-  }
-  if (threadIdx.x < 16) P[MLP_OFF_B4 + threadIdx.x] = threadIdx.x < 2 ? s_bias[384 + threadIdx.x] : 0.f;
-}
-
-__global__ void k_mlp_reduce(const float* partial, int parts, float* grad) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= MLP_NPARAM_PAD) return;
-  float s = 0.f;
-  for (int p = 0; p < parts; ++p) s += partial[(size_t)p * MLP_NPARAM_PAD + i];
-  grad[i] = s;
-}
-
-// Master weight i (padded layout) into its BF16 places.
-__device__ __forceinline__ void store_weight(int i, float x, uint16_t* wbf, uint16_t* wfr) {
+// Master weight i (padded layout) into its BF16 fragments.
+__device__ __forceinline__ void store_weight(int i, float x, uint16_t* wfr) {
   const uint16_t v = f2bf(x);
-  wbf[i] = v;
-  int f = -1, k = 0, o = 0, nkb = 1;  // fragments of its layer, row, column
+  int f = -1, g = -1, k = 0, o = 0, nkb = 1, gkb = 1;  // fragments of its layer, row, column
   if (i < MLP_OFF_B1) {
     f = MLP_F1;
     k = i >> 7;
     o = i & 127;
   } else if (i >= MLP_OFF_W2 && i < MLP_OFF_B2) {
     f = MLP_F2;
+    g = MLP_G2;
+    gkb = 8;
     k = (i - MLP_OFF_W2) >> 7;
     o = (i - MLP_OFF_W2) & 127;
     nkb = 8;
   } else if (i >= MLP_OFF_W3 && i < MLP_OFF_B3) {
     f = MLP_F3;
+    g = MLP_G3;
+    gkb = 8;
     k = (i - MLP_OFF_W3) >> 7;
     o = (i - MLP_OFF_W3) & 127;
     nkb = 8;
   } else if (i >= MLP_OFF_W4 && i < MLP_OFF_B4) {
     f = MLP_F4;
+    g = MLP_G4;
     k = (i - MLP_OFF_W4) >> 4;
     o = (i - MLP_OFF_W4) & 15;
     nkb = 8;
@@ -367,28 +96,40 @@ __device__ __forceinline__ void store_weight(int i, float x, uint16_t* wbf, uint
   if (f < 0) return;  // a bias
   const int lane = (o & 15) + 16 * ((k & 15) >> 2);
   wfr[f + ((o >> 4) * nkb + (k >> 4)) * MLP_FRAG + 4 * lane + (k & 3)] = v;
+  if (g < 0) return;  // the first layer has no backward product
+  const int glane = (k & 15) + 16 * ((o & 15) >> 2);
+  wfr[g + ((k >> 4) * gkb + (o >> 4)) * MLP_FRAG + 4 * glane + (o & 3)] = v;
 }
 
-// Adam on the padded FP32 master weights; padding entries stay zero.
-__global__ void k_mlp_adam(float* w, float* mom, float* vel, const float* grad, const uint8_t* mask,
-                           uint16_t* wbf, uint16_t* wfr, float lr, float b1c, float b2c) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= MLP_NPARAM_PAD) return;
-  if (!mask[i]) return;
-  float g = grad[i];
-  float m = 0.9f * mom[i] + 0.1f * g;
-  float v = 0.999f * vel[i] + 0.001f * g * g;
-  mom[i] = m;
-  vel[i] = v;
-  float x = w[i] - lr * (m / b1c) / (sqrtf(v / b2c) + 1e-8f);
-  w[i] = x;
-  store_weight(i, x, wbf, wfr);
+// What a training call does with gradient entry i (padded layout): writes it
+// (grad), or takes an Adam step on the FP32 master weights (padding entries
+// stay zero).
+struct MlpStep {
+  float* grad;  // null: Adam
+  float *w, *mom, *vel;
+  uint16_t* wfr;
+  float lr, b1c, b2c;
+};
+
+__device__ __forceinline__ void apply_gradient(const MlpStep& s, int i, float g, bool real) {
+  if (s.grad) {
+    s.grad[i] = g;
+    return;
+  }
+  if (!real) return;
+  float m = 0.9f * s.mom[i] + 0.1f * g;
+  float v = 0.999f * s.vel[i] + 0.001f * g * g;
+  s.mom[i] = m;
+  s.vel[i] = v;
+  float x = s.w[i] - s.lr * (m / s.b1c) / (sqrtf(v / s.b2c) + 1e-8f);
+  s.w[i] = x;
+  store_weight(i, x, s.wfr);
 }
 
 // The BF16 copies of every master weight.
-__global__ void k_mlp_pack(const float* w, uint16_t* wbf, uint16_t* wfr) {
+__global__ void k_mlp_pack(const float* w, uint16_t* wfr) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < MLP_NPARAM_PAD) store_weight(i, w[i], wbf, wfr);
+  if (i < MLP_NPARAM_PAD) store_weight(i, w[i], wfr);
 }
 
 // features (n x 14 FP32) -> padded BF16 rows (rows x 16), zero rows beyond n
@@ -516,6 +257,316 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
   }
 }
 
+// ---- training -----------------------------------------------------------------
+
+// Where a training call's rows come from: row r is row idx[r] of the BF16 set
+// dX / dT, or (idx null) row r of FP32 features and targets.
+struct TrainRows {
+  const uint16_t* dX;
+  const float* dT;
+  const int32_t* idx;
+  const float* feats;
+  const float* targets;
+};
+
+__device__ __forceinline__ bf16x4 wfrag(const uint16_t* wfr, int f) {
+  return ((const bf16x4*)wfr)[f / MLP_FRAG * 64 + (threadIdx.x & 63)];
+}
+
+// What the backward pass leaves for the weight gradients, per 16 rows: the
+// rows' features, h1, h2, h3, the gradients of the three pre-activations and
+// of the outputs as fragments (lane l: column 16 ct + l % 16, rows 4 (l / 16) +
+// 0..3), 1.6 KB a row, and the columns' FP32 gradient sums over each lane's
+// four rows.
+#define MLP_RX 0
+#define MLP_RH (MLP_RX + MLP_FRAG)          // 3 x 8
+#define MLP_RD (MLP_RH + 24 * MLP_FRAG)     // 3 x 8
+#define MLP_RY (MLP_RD + 24 * MLP_FRAG)
+#define MLP_RSUB (MLP_RY + MLP_FRAG)        // entries per 16 rows
+#define MLP_BSUB 400                        // of 4 rows: b1, b2, b3, b4
+
+// A barrier for LDS alone: global loads and stores stay in flight across it.
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// Forward and backward of the mean loss over n rows: squared error (huber =
+// 0), dY = 2 (Y - T) / n, or twice the Huber loss with threshold `huber`, dY =
+// 2 clamp(Y - T, +-huber) / n (the same gradient where |Y - T| <= huber), for
+// the rows of whole tiles (those beyond n with dY = 0).  frags and bsum: see
+// above; y and t (rows x 2, may be null) receive outputs and targets.
+//
+// 4 waves take 16 rows: wave w owns columns [32 w, 32 w + 32) of every layer,
+// whose pre-activations stay in its registers from the forward to the
+// backward pass; the rows move between layers through LDS.  A lane holds four
+// rows of one column, which is a fragment of the weight gradients' products
+// as it is.  A batch of 4096 rows is one workgroup to a CU, bound by the chain
+// of 7 layers: 16.4 us; separate forward and backward kernels on 64-row
+// tiles, which stored the FP32 pre-activations, took 94, one kernel on such
+// tiles with the weight gradients in it 35 (64 CUs, bound by the
+// activations' exponentials and divisions).
+__global__ __launch_bounds__(256) void k_mlp_rows(const uint16_t* __restrict__ wfr,
+                                                  const float* __restrict__ w, TrainRows rows, int n,
+                                                  uint16_t* __restrict__ frags,
+                                                  float* __restrict__ bsum, float huber, float* y,
+                                                  float* t) {
+  __shared__ __align__(16) uint16_t x[16 * XS], dy[16 * XS], hbuf[2][16 * HS];
+  __shared__ __align__(16) float sb[3 * 128 + 16];
+  __shared__ f32x4 z[3 * 2][256];  // each lane's own pre-activations
+  const int l = threadIdx.x & 63, wv = threadIdx.x >> 6, c = l & 15, r4 = 4 * (l >> 4);
+  load_biases(w, sb);
+  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+  const float inv_n = 2.0f / (float)n;
+  const int subs = (n + TILE - 1) / TILE * (TILE / 16);
+  bf16x4 a[2][8];  // a layer's fragments, fetched a layer ahead
+  auto fetch = [&](int f) {
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+#pragma unroll
+      for (int k = 0; k < 8; ++k) a[q][k] = wfrag(wfr, f + (8 * (2 * wv + q) + k) * MLP_FRAG);
+  };
+  auto product = [&](const uint16_t* in, f32x4* acc) {
+    acc[0] = acc[1] = zero;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const bf16x4 v = act_frag(in, HS, k);
+#pragma unroll
+      for (int q = 0; q < 2; ++q) acc[q] = mfma16(v, a[q][k], acc[q]);
+    }
+  };
+  // this lane's four rows of column 32 wv + 16 q + c: to LDS and to fragment f
+  auto put = [&](uint16_t* rowbuf, uint16_t* f, int q, const uint16_t* h) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) rowbuf[(r4 + i) * HS + 32 * wv + 16 * q + c] = h[i];
+    *(uint2*)(f + (2 * wv + q) * MLP_FRAG + 4 * l) =
+        make_uint2(h[0] | (uint32_t)h[1] << 16, h[2] | (uint32_t)h[3] << 16);
+  };
+#pragma unroll 1
+  for (int sub = blockIdx.x; sub < subs; sub += gridDim.x) {
+    const int row0 = 16 * sub;
+    uint16_t* out = frags + (size_t)sub * MLP_RSUB;
+    float* bout = bsum + (size_t)(4 * sub + (l >> 4)) * MLP_BSUB;
+    // the targets of the lanes that hold outputs (columns 0 and 1 in wave 0)
+    const bool has_out = wv == 0 && c < 2;
+    float target[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int row = row0 + r4 + i;
+      target[i] = 0.f;
+      if (has_out && row < n)
+        target[i] = rows.idx ? rows.dT[2L * rows.idx[row] + c] : rows.targets[2L * row + c];
+    }
+    {
+      const int r = threadIdx.x >> 4, q = threadIdx.x & 15, row = row0 + r;
+      uint16_t v = 0;
+      if (row < n) {
+        if (rows.idx)
+          v = rows.dX[(long)rows.idx[row] * 16 + q];
+        else if (q < MLP_IN)
+          v = f2bf(rows.feats[(size_t)row * MLP_IN + q]);
+      }
+      x[r * XS + q] = v;
+    }
+    bf16x4 a1[2], a4[2];
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      a1[q] = wfrag(wfr, MLP_F1 + (2 * wv + q) * MLP_FRAG);
+      a4[q] = wfrag(wfr, MLP_G4 + (2 * wv + q) * MLP_FRAG);
+    }
+    fetch(MLP_F2);
+    lds_barrier();
+    if (wv == 0) {
+      bf16x4 v;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] = (short)x[(r4 + i) * XS + c];
+      *(bf16x4*)(out + MLP_RX + 4 * l) = v;
+    }
+    f32x4 acc[2];
+#pragma unroll 1
+    for (int L = 0; L < 3; ++L) {
+      if (L == 0) {
+#pragma unroll
+        for (int q = 0; q < 2; ++q) acc[q] = mfma16(act_frag(x, XS, 0), a1[q], zero);
+      } else {
+        product(hbuf[(L - 1) & 1], acc);
+        fetch(L == 1 ? MLP_F3 : MLP_G3);
+      }
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        const float b = sb[128 * L + 32 * wv + 16 * q + c];
+        uint16_t h[4];
+        f32x4 zz;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          zz[i] = acc[q][i] + b;
+          h[i] = f2bf(silu(zz[i]));
+        }
+        z[2 * L + q][threadIdx.x] = zz;
+        put(hbuf[L & 1], out + MLP_RH + L * 8 * MLP_FRAG, q, h);
+      }
+      lds_barrier();
+    }
+    if (wv == 0) {  // outputs and their gradient
+      f32x4 o = zero;
+#pragma unroll
+      for (int k = 0; k < 8; ++k)
+        o = mfma16(act_frag(hbuf[0], HS, k), wfrag(wfr, MLP_F4 + k * MLP_FRAG), o);
+      const float b = sb[384 + c];
+      float sum = 0.f;
+      uint16_t h[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int row = row0 + r4 + i;
+        float d = 0.f;
+        if (has_out && row < n) {
+          const float yy = o[i] + b;
+          float e = yy - target[i];
+          if (y) y[2L * row + c] = yy;
+          if (t) t[2L * row + c] = target[i];
+          if (huber > 0.f) e = fminf(fmaxf(e, -huber), huber);
+          d = e * inv_n;
+        }
+        h[i] = f2bf(d);
+        sum += d;
+        dy[(r4 + i) * XS + c] = h[i];
+      }
+      *(uint2*)(out + MLP_RY + 4 * l) =
+          make_uint2(h[0] | (uint32_t)h[1] << 16, h[2] | (uint32_t)h[3] << 16);
+      bout[384 + c] = sum;
+    }
+    lds_barrier();
+#pragma unroll 1
+    for (int L = 2; L >= 0; --L) {
+      if (L == 2) {
+#pragma unroll
+        for (int q = 0; q < 2; ++q) acc[q] = mfma16(act_frag(dy, XS, 0), a4[q], zero);
+      } else {
+        product(hbuf[L & 1], acc);
+        if (L == 1) fetch(MLP_G2);
+      }
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        const f32x4 zz = z[2 * L + q][threadIdx.x];
+        uint16_t h[4];
+        float sum = 0.f;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float d = acc[q][i] * dsilu(zz[i]);
+          h[i] = f2bf(d);
+          sum += d;
+        }
+        put(hbuf[(L + 1) & 1], out + MLP_RD + L * 8 * MLP_FRAG, q, h);
+        bout[128 * L + 32 * wv + 16 * q + c] = sum;
+      }
+      lds_barrier();
+    }
+  }
+}
+
+// Weight gradients and what follows from them (apply_gradient).  Workgroups
+// [0, 144): one 16x16 block of a weight matrix each: the products of every
+// tile are summed in MFMA accumulators, tile t into sum t % MLP_PARTS (each
+// wave has an eighth of the sums), and the sums are added in order; the rest:
+// 64 bias entries each, likewise.  What the row kernel wrote is read from L2
+// (12 MB a 4096-row batch over the blocks): 10.6 us, Adam included (one partial of
+// 149 KB a tile, then summing those, took 20).
+constexpr int W_BLOCKS = 8 + 64 + 64 + 8, B_BLOCKS = (386 + 63) / 64;
+
+__global__ __launch_bounds__(512) void k_mlp_weights(const uint16_t* __restrict__ frags,
+                                                     const float* __restrict__ bsum, int tiles,
+                                                     MlpStep step) {
+  __shared__ float s_sum[MLP_PARTS][256];
+  constexpr int PER = MLP_PARTS / 8, SUBS = TILE / 16;
+  const int l = threadIdx.x & 63, wv = threadIdx.x >> 6, blk = blockIdx.x;
+  const int parts = tiles < MLP_PARTS ? tiles : MLP_PARTS;
+  if (blk < W_BLOCKS) {
+    // matrix W(L + 1), block (it, jt): fragments of its inputs and of the
+    // gradients of its outputs
+    int in, dz, off, ld, it, jt;
+    if (blk < 8) {
+      it = 0;
+      jt = blk;
+      in = MLP_RX;
+      dz = MLP_RD + jt * MLP_FRAG;
+      off = MLP_OFF_W1;
+      ld = 128;
+    } else if (blk < 136) {
+      const int L = (blk - 8) >> 6;
+      it = ((blk - 8) >> 3) & 7;
+      jt = blk & 7;
+      in = MLP_RH + (8 * L + it) * MLP_FRAG;
+      dz = MLP_RD + (8 * (L + 1) + jt) * MLP_FRAG;
+      off = L ? MLP_OFF_W3 : MLP_OFF_W2;
+      ld = 128;
+    } else {
+      it = blk - 136;
+      jt = 0;
+      in = MLP_RH + (16 + it) * MLP_FRAG;
+      dz = MLP_RY;
+      off = MLP_OFF_W4;
+      ld = 16;
+    }
+    f32x4 acc[PER];
+#pragma unroll
+    for (int q = 0; q < PER; ++q) acc[q] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int t0 = wv * PER; t0 < tiles; t0 += MLP_PARTS) {
+      bf16x4 u[PER][SUBS], v[PER][SUBS];  // in flight together
+#pragma unroll
+      for (int q = 0; q < PER; ++q) {
+        const int tile = t0 + q < tiles ? t0 + q : t0;
+        const uint16_t* f = frags + (size_t)tile * SUBS * MLP_RSUB + 4 * l;
+#pragma unroll
+        for (int k = 0; k < SUBS; ++k) {
+          u[q][k] = *(const bf16x4*)(f + k * MLP_RSUB + in);
+          v[q][k] = *(const bf16x4*)(f + k * MLP_RSUB + dz);
+        }
+      }
+#pragma unroll
+      for (int q = 0; q < PER; ++q)
+        if (t0 + q < tiles)
+#pragma unroll
+          for (int k = 0; k < SUBS; ++k) acc[q] = mfma16(u[q][k], v[q][k], acc[q]);
+    }
+#pragma unroll
+    for (int q = 0; q < PER; ++q)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) s_sum[wv * PER + q][(4 * (l >> 4) + i) * 16 + (l & 15)] = acc[q][i];
+    __syncthreads();
+    if (threadIdx.x >= 256) return;
+    const int r = threadIdx.x >> 4, c = threadIdx.x & 15;
+    float g = 0.f;
+#pragma unroll 16
+    for (int p = 0; p < parts; ++p) g += s_sum[p][threadIdx.x];
+    const bool real = off == MLP_OFF_W1 ? r < MLP_IN : off == MLP_OFF_W4 ? c < 2 : true;
+    apply_gradient(step, off + (16 * it + r) * ld + 16 * jt + c, g, real);
+    return;
+  }
+  const int e = 64 * (blk - W_BLOCKS) + l;  // bias entry
+  for (int q = 0; q < PER; ++q) {
+    float sum = 0.f;
+    for (int tile = wv * PER + q; tile < tiles; tile += MLP_PARTS) {
+      const float* b = bsum + (size_t)tile * TILE / 4 * MLP_BSUB + (e < 386 ? e : 0);
+      float part[TILE / 4];
+#pragma unroll
+      for (int k = 0; k < TILE / 4; ++k) part[k] = b[k * MLP_BSUB];
+#pragma unroll
+      for (int k = 0; k < TILE / 4; ++k) sum += part[k];
+    }
+    s_sum[wv * PER + q][l] = sum;
+  }
+  __syncthreads();
+  if (wv != 0) return;
+  float g = 0.f;
+  for (int p = 0; p < parts; ++p) g += s_sum[p][l];
+  const int i = e < 128   ? MLP_OFF_B1 + e
+                : e < 256 ? MLP_OFF_B2 + e - 128
+                : e < 384 ? MLP_OFF_B3 + e - 256
+                          : MLP_OFF_B4 + e - 384;
+  if (e < 386) apply_gradient(step, i, g, true);
+}
+
 // 4 workgroups on each of 256 CUs
 void launch_eval(const MlpParams& p, const float* feats, int n, float* out, hipStream_t s) {
   const int tiles = (n + 15) / 16;
@@ -526,59 +577,45 @@ void launch_eval(const MlpParams& p, const float* feats, int n, float* out, hipS
 
 // ------------------------------------------------------------------ host
 
-MlpDev mlp_view(const MlpParams& p) {
-  MlpDev m;
-  m.w1 = p.wbf + MLP_OFF_W1;
-  m.w2 = p.wbf + MLP_OFF_W2;
-  m.w3 = p.wbf + MLP_OFF_W3;
-  m.w4 = p.wbf + MLP_OFF_W4;
-  m.b1 = p.w + MLP_OFF_B1;
-  m.b2 = p.w + MLP_OFF_B2;
-  m.b3 = p.w + MLP_OFF_B3;
-  m.b4 = p.w + MLP_OFF_B4;
-  return m;
+// The published blob and the padded layout: W1 has 14 of 16 rows, W4 2 of 16
+// columns, b4 2 of 16 entries; b1 to b3 are the same range of both.
+constexpr int BLOB_B1 = MLP_IN * 128, BLOB_W4 = BLOB_B1 + (MLP_OFF_W4 - MLP_OFF_B1);
+
+template <class T>
+static void mlp_pad(const T* blob, T* pad) {
+  memcpy(pad + MLP_OFF_W1, blob, BLOB_B1 * sizeof(T));
+  memcpy(pad + MLP_OFF_B1, blob + BLOB_B1, (BLOB_W4 - BLOB_B1) * sizeof(T));
+  for (int k = 0; k < 128; ++k)
+    for (int q = 0; q < 2; ++q) pad[MLP_OFF_W4 + 16 * k + q] = blob[BLOB_W4 + 2 * k + q];
+  for (int q = 0; q < 2; ++q) pad[MLP_OFF_B4 + q] = blob[BLOB_W4 + 256 + q];
 }
 
-// padded index of logical parameter k of the published blob layout
-int mlp_padded_index(int k) {
-  if (k < MLP_IN * 128) return MLP_OFF_W1 + k;  // W1 rows 0..13 of 16
-  k -= MLP_IN * 128;
-  if (k < 128) return MLP_OFF_B1 + k;
-  k -= 128;
-  if (k < 128 * 128) return MLP_OFF_W2 + k;
-  k -= 128 * 128;
-  if (k < 128) return MLP_OFF_B2 + k;
-  k -= 128;
-  if (k < 128 * 128) return MLP_OFF_W3 + k;
-  k -= 128 * 128;
-  if (k < 128) return MLP_OFF_B3 + k;
-  k -= 128;
-  if (k < 128 * 2) return MLP_OFF_W4 + (k / 2) * 16 + (k % 2);
-  k -= 128 * 2;
-  return MLP_OFF_B4 + k;
+static void mlp_unpad(const float* pad, float* blob) {
+  memcpy(blob, pad + MLP_OFF_W1, BLOB_B1 * sizeof(float));
+  memcpy(blob + BLOB_B1, pad + MLP_OFF_B1, (BLOB_W4 - BLOB_B1) * sizeof(float));
+  for (int k = 0; k < 128; ++k)
+    for (int q = 0; q < 2; ++q) blob[BLOB_W4 + 2 * k + q] = pad[MLP_OFF_W4 + 16 * k + q];
+  for (int q = 0; q < 2; ++q) blob[BLOB_W4 + 256 + q] = pad[MLP_OFF_B4 + q];
 }
 
 shp_status mlp_params_alloc(MlpParams* p) {
   if (hipMalloc(&p->w, MLP_NPARAM_PAD * sizeof(float)) != hipSuccess) return SHP_E_OOM;
-  if (hipMalloc(&p->wbf, MLP_NPARAM_PAD * sizeof(uint16_t)) != hipSuccess) return SHP_E_OOM;
   if (hipMalloc(&p->wfr, MLP_NFRAG * sizeof(uint16_t)) != hipSuccess) return SHP_E_OOM;
   return SHP_OK;
 }
 
 void mlp_params_free(MlpParams* p) {
   if (p->w) (void)hipFree(p->w);
-  if (p->wbf) (void)hipFree(p->wbf);
   if (p->wfr) (void)hipFree(p->wfr);
   p->w = nullptr;
-  p->wbf = nullptr;
   p->wfr = nullptr;
 }
 
 shp_status mlp_params_upload(MlpParams* p, const float* params, hipStream_t s) {
   std::vector<float> pad(MLP_NPARAM_PAD, 0.0f);
-  for (int k = 0; k < MLP_NPARAM; ++k) pad[mlp_padded_index(k)] = params[k];
+  mlp_pad(params, pad.data());
   if (hipMemcpyAsync(p->w, pad.data(), pad.size() * 4, hipMemcpyHostToDevice, s) != hipSuccess) return SHP_E_HIP;
-  k_mlp_pack<<<(MLP_NPARAM_PAD + 255) / 256, 256, 0, s>>>(p->w, p->wbf, p->wfr);
+  k_mlp_pack<<<(MLP_NPARAM_PAD + 255) / 256, 256, 0, s>>>(p->w, p->wfr);
   if (hipStreamSynchronize(s) != hipSuccess) return SHP_E_HIP;
   return SHP_OK;
 }
@@ -708,16 +745,17 @@ struct shp_mlp {
   int device = 0;  // the GPU the handle's weights live on
   hipStream_t stream = nullptr;
   MlpParams p{};
-  float *mom = nullptr, *vel = nullptr, *grad = nullptr, *partial = nullptr;
-  uint8_t* mask = nullptr;
-  int parts = 64;
-  int cap_rows = 0;
-  uint16_t* X = nullptr;   // cap_rows x 16
-  float* T = nullptr;      // cap_rows x 2
+  float *mom = nullptr, *vel = nullptr, *grad = nullptr;
+  // of cap_tiles training tiles: fragments and bias sums (k_mlp_rows)
+  int cap_tiles = 0;
+  uint16_t* frags = nullptr;
+  float* bsum = nullptr;
   int cap_fwd = 0;
   float* Fin = nullptr;    // cap_fwd x 14 staging
   float* out = nullptr;    // cap_fwd x 2 outputs
-  TrainBufs tb{};
+  float* T = nullptr;      // cap_fwd x 2 targets
+  int32_t* didx = nullptr;  // cap_idx row indices of a training call
+  long cap_idx = 0;
   long adam_t = 0;
   // training set on device
   uint16_t* dX = nullptr;
@@ -737,69 +775,43 @@ static shp_status mlp_fail(shp_status s, const char* m) {
 #define MCHK(x) \
   do { if ((x) != hipSuccess) return mlp_fail(SHP_E_HIP, #x); } while (0)
 
-// feature rows and outputs of calls on host memory
-static shp_status mlp_reserve_forward(shp_mlp* h, int rows) {
+// feature rows, outputs and targets of calls on host memory
+static shp_status mlp_reserve(shp_mlp* h, int rows) {
   if (rows <= h->cap_fwd) return SHP_OK;
-  for (void* q : {(void*)h->Fin, (void*)h->out})
+  for (void* q : {(void*)h->Fin, (void*)h->out, (void*)h->T})
     if (q) (void)hipFree(q);
-  h->Fin = h->out = nullptr;
+  h->Fin = h->out = h->T = nullptr;
   h->cap_fwd = 0;
-  rows = ((rows + TILE - 1) / TILE) * TILE;
+  rows = ((rows + 63) / 64) * 64;
   MCHK(hipMalloc(&h->Fin, (size_t)rows * MLP_IN * 4));
   MCHK(hipMalloc(&h->out, (size_t)rows * 2 * 4));
+  MCHK(hipMalloc(&h->T, (size_t)rows * 2 * 4));
   h->cap_fwd = rows;
   return SHP_OK;
 }
 
-static shp_status mlp_reserve(shp_mlp* h, int rows) {
-  shp_status st = mlp_reserve_forward(h, rows);
-  if (st != SHP_OK) return st;
-  if (rows <= h->cap_rows) return SHP_OK;
-  rows = ((rows + TILE - 1) / TILE) * TILE;
-  void* ptrs[] = {h->X, h->T, h->tb.z1, h->tb.z2, h->tb.z3, h->tb.h1, h->tb.h2, h->tb.h3, h->tb.y};
-  for (void* q : ptrs)
+static shp_status mlp_reserve_tiles(shp_mlp* h, int n) {
+  const int tiles = (n + TILE - 1) / TILE;
+  if (tiles <= h->cap_tiles) return SHP_OK;
+  for (void* q : {(void*)h->frags, (void*)h->bsum})
     if (q) (void)hipFree(q);
-  size_t R = rows;
-  MCHK(hipMalloc(&h->X, R * 16 * 2));
-  MCHK(hipMalloc(&h->T, R * 2 * 4));
-  MCHK(hipMalloc(&h->tb.z1, R * 128 * 4));
-  MCHK(hipMalloc(&h->tb.z2, R * 128 * 4));
-  MCHK(hipMalloc(&h->tb.z3, R * 128 * 4));
-  MCHK(hipMalloc(&h->tb.h1, R * 128 * 2));
-  MCHK(hipMalloc(&h->tb.h2, R * 128 * 2));
-  MCHK(hipMalloc(&h->tb.h3, R * 128 * 2));
-  MCHK(hipMalloc(&h->tb.y, R * 16 * 4));
-  h->cap_rows = rows;
+  h->frags = nullptr;
+  h->bsum = nullptr;
+  h->cap_tiles = 0;
+  const size_t subs = (size_t)tiles * (TILE / 16);
+  MCHK(hipMalloc(&h->frags, subs * MLP_RSUB * sizeof(uint16_t)));
+  MCHK(hipMalloc(&h->bsum, 4 * subs * MLP_BSUB * sizeof(float)));
+  h->cap_tiles = tiles;
   return SHP_OK;
 }
 
-// rows of X/T are taken from the device training set by index
-__global__ void k_gather_rows(const uint16_t* dX, const float* dT, const int32_t* idx, int n, int rows,
-                              uint16_t* X, float* T) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= rows * 16) return;
-  int r = i >> 4, cc = i & 15;
-  if (r < n) {
-    long src = idx[r];
-    X[i] = dX[src * 16 + cc];
-    if (cc < 2) T[r * 2 + cc] = dT[src * 2 + cc];
-  } else {
-    X[i] = 0;
-    if (cc < 2) T[r * 2 + cc] = 0.f;
-  }
-}
-
-static shp_status mlp_grad_rows(shp_mlp* h, int n) {
-  int rows = ((n + TILE - 1) / TILE) * TILE;
-  int tiles = rows / TILE;
-  int fg = tiles < 1024 ? tiles : 1024;
-  MlpDev m = mlp_view(h->p);
-  k_mlp_forward<<<fg, 256, 0, h->stream>>>(m, h->X, rows, h->tb.y, h->tb);
-  int parts = tiles < h->parts ? tiles : h->parts;
-  k_mlp_backward<<<parts, 256, 0, h->stream>>>(m, h->X, h->T, rows, n, h->tb, h->partial, h->huber);
-  k_mlp_reduce<<<(MLP_NPARAM_PAD + 255) / 256, 256, 0, h->stream>>>(h->partial, parts, h->grad);
-  MCHK(hipGetLastError());
-  return SHP_OK;
+// The gradient over n rows (at most the reserved tiles), then `step`.
+static void launch_train(shp_mlp* h, const TrainRows& rows, int n, float* y, float* t,
+                         const MlpStep& step) {
+  const int tiles = (n + TILE - 1) / TILE, subs = tiles * (TILE / 16);
+  k_mlp_rows<<<subs < 1024 ? subs : 1024, 256, 0, h->stream>>>(h->p.wfr, h->p.w, rows, n, h->frags,
+                                                              h->bsum, h->huber, y, t);
+  k_mlp_weights<<<W_BLOCKS + B_BLOCKS, 512, 0, h->stream>>>(h->frags, h->bsum, tiles, step);
 }
 
 extern "C" {
@@ -821,17 +833,13 @@ shp_status shp_mlp_create(const float* params, shp_mlp** out) {
   if (st == SHP_OK) st = mlp_params_upload(&h->p, params, h->stream);
   if (st == SHP_OK) {
     if (hipMalloc(&h->mom, MLP_NPARAM_PAD * 4) != hipSuccess || hipMalloc(&h->vel, MLP_NPARAM_PAD * 4) != hipSuccess ||
-        hipMalloc(&h->grad, MLP_NPARAM_PAD * 4) != hipSuccess ||
-        hipMalloc(&h->partial, (size_t)h->parts * MLP_NPARAM_PAD * 4) != hipSuccess ||
-        hipMalloc(&h->mask, MLP_NPARAM_PAD) != hipSuccess)
+        hipMalloc(&h->grad, MLP_NPARAM_PAD * 4) != hipSuccess)
       st = SHP_E_OOM;
   }
   if (st == SHP_OK) {
-    std::vector<uint8_t> mask(MLP_NPARAM_PAD, 0);
-    for (int k = 0; k < MLP_NPARAM; ++k) mask[mlp_padded_index(k)] = 1;
     std::vector<float> zero(MLP_NPARAM_PAD, 0.f);
-    if (hipMemcpy(h->mask, mask.data(), MLP_NPARAM_PAD, hipMemcpyHostToDevice) != hipSuccess ||
-        hipMemcpy(h->mom, zero.data(), MLP_NPARAM_PAD * 4, hipMemcpyHostToDevice) != hipSuccess ||
+    if (hipMemcpy(h->mom, zero.data(), MLP_NPARAM_PAD * 4, hipMemcpyHostToDevice) != hipSuccess ||
+        hipMemcpy(h->grad, zero.data(), MLP_NPARAM_PAD * 4, hipMemcpyHostToDevice) != hipSuccess ||
         hipMemcpy(h->vel, zero.data(), MLP_NPARAM_PAD * 4, hipMemcpyHostToDevice) != hipSuccess)
       st = SHP_E_HIP;
   }
@@ -847,8 +855,8 @@ shp_status shp_mlp_destroy(shp_mlp* h) {
   if (!h) return SHP_OK;
   if (h->stream) (void)hipStreamSynchronize(h->stream);
   mlp_params_free(&h->p);
-  void* ptrs[] = {h->mom, h->vel, h->grad, h->partial, h->mask, h->X, h->T, h->Fin, h->out, h->tb.z1,
-                  h->tb.z2, h->tb.z3, h->tb.h1, h->tb.h2, h->tb.h3, h->tb.y, h->dX, h->dT};
+  void* ptrs[] = {h->mom, h->vel, h->grad, h->frags, h->bsum, h->T, h->Fin,
+                  h->out, h->didx, h->dX, h->dT};
   for (void* q : ptrs)
     if (q) (void)hipFree(q);
   if (h->stream) (void)hipStreamDestroy(h->stream);
@@ -861,14 +869,14 @@ shp_status shp_mlp_get_params(shp_mlp* h, float* params) {
   std::vector<float> pad(MLP_NPARAM_PAD);
   MCHK(hipStreamSynchronize(h->stream));
   MCHK(hipMemcpy(pad.data(), h->p.w, MLP_NPARAM_PAD * 4, hipMemcpyDeviceToHost));
-  for (int k = 0; k < MLP_NPARAM; ++k) params[k] = pad[mlp_padded_index(k)];
+  mlp_unpad(pad.data(), params);
   return SHP_OK;
 }
 
 shp_status shp_mlp_forward(shp_mlp* h, const float* feats, int32_t n, float* out) {
   if (!h || n < 0 || (n > 0 && (!feats || !out))) return mlp_fail(SHP_E_INVAL, "bad argument");
   if (n == 0) return SHP_OK;
-  shp_status st = mlp_reserve_forward(h, n);
+  shp_status st = mlp_reserve(h, n);
   if (st != SHP_OK) return st;
   MCHK(hipMemcpyAsync(h->Fin, feats, (size_t)n * MLP_IN * 4, hipMemcpyHostToDevice, h->stream));
   launch_eval(h->p, h->Fin, n, h->out, h->stream);
@@ -896,27 +904,25 @@ shp_status shp_mlp_gradient(shp_mlp* h, const float* feats, const float* targets
                             float* grad_out, float* loss_out) {
   if (!h || n <= 0 || !feats || !targets || !grad_out) return mlp_fail(SHP_E_INVAL, "bad argument");
   shp_status st = mlp_reserve(h, n);
+  if (st == SHP_OK) st = mlp_reserve_tiles(h, n);
   if (st != SHP_OK) return st;
-  int rows = ((n + TILE - 1) / TILE) * TILE;
   MCHK(hipMemcpyAsync(h->Fin, feats, (size_t)n * MLP_IN * 4, hipMemcpyHostToDevice, h->stream));
-  std::vector<float> t((size_t)rows * 2, 0.f);
-  for (int i = 0; i < 2 * n; ++i) t[i] = targets[i];
-  MCHK(hipMemcpyAsync(h->T, t.data(), t.size() * 4, hipMemcpyHostToDevice, h->stream));
-  k_pack_features<<<(rows * 16 + 255) / 256, 256, 0, h->stream>>>(h->Fin, n, rows, h->X);
-  st = mlp_grad_rows(h, n);
-  if (st != SHP_OK) return st;
-  std::vector<float> g(MLP_NPARAM_PAD), y((size_t)rows * 16);
+  MCHK(hipMemcpyAsync(h->T, targets, (size_t)n * 2 * 4, hipMemcpyHostToDevice, h->stream));
+  MlpStep step{};
+  step.grad = h->grad;
+  launch_train(h, TrainRows{nullptr, nullptr, nullptr, h->Fin, h->T}, n, h->out, nullptr, step);
+  MCHK(hipGetLastError());
+  std::vector<float> g(MLP_NPARAM_PAD), y((size_t)n * 2);
   MCHK(hipMemcpyAsync(g.data(), h->grad, g.size() * 4, hipMemcpyDeviceToHost, h->stream));
-  MCHK(hipMemcpyAsync(y.data(), h->tb.y, y.size() * 4, hipMemcpyDeviceToHost, h->stream));
+  if (loss_out) MCHK(hipMemcpyAsync(y.data(), h->out, y.size() * 4, hipMemcpyDeviceToHost, h->stream));
   MCHK(hipStreamSynchronize(h->stream));
-  for (int k = 0; k < MLP_NPARAM; ++k) grad_out[k] = g[mlp_padded_index(k)];
+  mlp_unpad(g.data(), grad_out);
   if (loss_out) {
     double l = 0.0;
-    for (int r = 0; r < n; ++r)
-      for (int q = 0; q < 2; ++q) {
-        double d = (double)y[(size_t)r * 16 + q] - targets[2 * r + q];
-        l += d * d;
-      }
+    for (size_t i = 0; i < y.size(); ++i) {
+      const double d = (double)y[i] - targets[i];
+      l += d * d;
+    }
     *loss_out = (float)(l / n);
   }
   return SHP_OK;
@@ -959,40 +965,47 @@ shp_status shp_mlp_train(shp_mlp* h, const int32_t* indices, int32_t steps, int3
                          float* loss_out) {
   if (!h || !indices || steps <= 0 || batch <= 0 || batch % TILE) return mlp_fail(SHP_E_INVAL, "bad argument");
   if (!h->dX) return mlp_fail(SHP_E_INVAL, "no training data");
-  for (long i = 0; i < (long)steps * batch; ++i)
-    if (indices[i] < 0 || indices[i] >= h->n_data) return mlp_fail(SHP_E_INVAL, "training index out of range");
-  shp_status st = mlp_reserve(h, batch);
+  const long total = (long)steps * batch;
+  int32_t lo = 0, hi = 0;
+  for (long i = 0; i < total; ++i) {
+    lo = indices[i] < lo ? indices[i] : lo;
+    hi = indices[i] > hi ? indices[i] : hi;
+  }
+  if (lo < 0 || hi >= h->n_data) return mlp_fail(SHP_E_INVAL, "training index out of range");
+  shp_status st = mlp_reserve_tiles(h, batch);
+  if (st == SHP_OK && loss_out) st = mlp_reserve(h, batch);
   if (st != SHP_OK) return st;
-  int32_t* didx = nullptr;
-  MCHK(hipMalloc(&didx, (size_t)steps * batch * 4));
-  MCHK(hipMemcpy(didx, indices, (size_t)steps * batch * 4, hipMemcpyHostToDevice));
-  std::vector<float> y((size_t)batch * 16), t((size_t)batch * 2);
+  if (total > h->cap_idx) {
+    if (h->didx) (void)hipFree(h->didx);
+    h->didx = nullptr;
+    h->cap_idx = 0;
+    MCHK(hipMalloc(&h->didx, (size_t)total * 4));
+    h->cap_idx = total;
+  }
+  MCHK(hipMemcpy(h->didx, indices, (size_t)total * 4, hipMemcpyHostToDevice));
+  std::vector<float> y((size_t)batch * 2), t((size_t)batch * 2);
   for (int s = 0; s < steps; ++s) {
-    k_gather_rows<<<(batch * 16 + 255) / 256, 256, 0, h->stream>>>(h->dX, h->dT, didx + (size_t)s * batch,
-                                                                  batch, batch, h->X, h->T);
-    st = mlp_grad_rows(h, batch);
-    if (st != SHP_OK) break;
+    const TrainRows rows{h->dX, h->dT, h->didx + (size_t)s * batch, nullptr, nullptr};
     ++h->adam_t;
     float b1c = 1.0f - powf(0.9f, (float)h->adam_t);
     float b2c = 1.0f - powf(0.999f, (float)h->adam_t);
-    k_mlp_adam<<<(MLP_NPARAM_PAD + 255) / 256, 256, 0, h->stream>>>(h->p.w, h->mom, h->vel, h->grad, h->mask,
-                                                                    h->p.wbf, h->p.wfr, lr, b1c, b2c);
+    launch_train(h, rows, batch, loss_out ? h->out : nullptr, loss_out ? h->T : nullptr,
+                 MlpStep{nullptr, h->p.w, h->mom, h->vel, h->p.wfr, lr, b1c, b2c});
+    MCHK(hipGetLastError());
     if (loss_out) {
-      MCHK(hipMemcpyAsync(y.data(), h->tb.y, y.size() * 4, hipMemcpyDeviceToHost, h->stream));
+      MCHK(hipMemcpyAsync(y.data(), h->out, y.size() * 4, hipMemcpyDeviceToHost, h->stream));
       MCHK(hipMemcpyAsync(t.data(), h->T, t.size() * 4, hipMemcpyDeviceToHost, h->stream));
       MCHK(hipStreamSynchronize(h->stream));
       double l = 0.0;
-      for (int r = 0; r < batch; ++r)
-        for (int q = 0; q < 2; ++q) {
-          double d = (double)y[(size_t)r * 16 + q] - t[(size_t)r * 2 + q];
-          l += d * d;
-        }
+      for (size_t i = 0; i < y.size(); ++i) {
+        const double d = (double)y[i] - t[i];
+        l += d * d;
+      }
       loss_out[s] = (float)(l / batch);
     }
   }
   (void)hipStreamSynchronize(h->stream);
-  (void)hipFree(didx);
-  return st;
+  return SHP_OK;
 }
 
 }  // extern "C"
