@@ -32,6 +32,11 @@
 // FP32).  A lane keeps its slot of a colour in every pass, so the record
 // of its manifold of the next colour (lagrangians included) is loaded
 // before the barrier that ends the current colour.
+//
+// A large world with CUs to spare is coloured and swept by many workgroups
+// instead, whose manifolds wait for the bodies they need, not for each other
+// (colour_flow, sweep_flow): the same colours and the same updates of each
+// body in the same order, so the same results.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -75,7 +80,7 @@ struct ConF {
 
 struct ManF {
   float ux, uy, mu, e, ax, ay, bx, by;
-  int ga, gb, flags;
+  int ga, gb, flags, turns;
   ConF k[2];
 };
 
@@ -94,10 +99,10 @@ __device__ __forceinline__ RecW recw(const Ctx& c, const PackF& P, int p0) {
   return r;
 }
 
-// Words 3-6 of a record: one contact.
-__device__ __forceinline__ void load_contact(const float4* w, ConF& k) {
-  const float4 a = w[0], b = w[RB], d = w[2 * RB];
-  const double2 l = *(const double2*)(w + 3 * RB);
+// Words 3-6 of a record, `step` apart: one contact.
+__device__ __forceinline__ void load_contact(const float4* w, int step, ConF& k) {
+  const float4 a = w[0], b = w[step], d = w[2 * step];
+  const double2 l = *(const double2*)(w + 3 * step);
   k.jn2 = a.x;
   k.jn5 = a.y;
   k.jt2 = a.z;
@@ -113,12 +118,10 @@ __device__ __forceinline__ void load_contact(const float4* w, ConF& k) {
   k.lt = l.y;
 }
 
-// Manifold m of the world (local index) and its contacts; the second
-// contact's record loads only when the manifold has one.
-__device__ __forceinline__ void load_man(const RecW& R, int m_loc, ManF& m) {
-  const float4* r = rec_of(R.rec, R.p0 + m_loc);
-  const float4 a = r[0], b = r[RB];
-  const int4 g = *(const int4*)(r + 2 * RB);
+// Words 0-2: the manifold.
+__device__ __forceinline__ void load_head(const float4* r, int step, ManF& m) {
+  const float4 a = r[0], b = r[step];
+  const int4 g = *(const int4*)(r + 2 * step);
   m.ux = a.x;
   m.uy = a.y;
   m.mu = a.z;
@@ -130,8 +133,21 @@ __device__ __forceinline__ void load_man(const RecW& R, int m_loc, ManF& m) {
   m.ga = g.x;
   m.gb = g.y;
   m.flags = g.z;
-  load_contact(r + 3 * RB, m.k[0]);
-  if (m.flags & MFL_TWO) load_contact(rec2_of(R.rec2, R.p0 + m_loc), m.k[1]);
+  m.turns = g.w;
+}
+
+// Manifold m of the world (local index) and its contacts; the second
+// contact's record loads only when the manifold has one.
+__device__ __forceinline__ void load_man(const RecW& R, int m_loc, ManF& m) {
+  const float4* r = rec_of(R.rec, R.p0 + m_loc);
+  load_head(r, RB, m);
+  load_contact(r + 3 * RB, RB, m.k[0]);
+  if (m.flags & MFL_TWO) load_contact(rec2_of(R.rec2, R.p0 + m_loc), RB, m.k[1]);
+}
+
+// Where contact j's lagrangians of manifold m_loc are.
+__device__ __forceinline__ double2* lambda_of(const RecW& R, int m_loc, int j) {
+  return (double2*)(j ? rec2_of(R.rec2, R.p0 + m_loc) + 3 * RB : rec_of(R.rec, R.p0 + m_loc) + 6 * RB);
 }
 
 // v += l * w, fused per entry (w: a row times the inverse masses)
@@ -146,6 +162,16 @@ struct VelF {
   float* lds;
   const Ctx* c;
   int b0;
+  // the velocities of a manifold's bodies, and back
+  __device__ __forceinline__ void load(const ManF& m, float* v) const {
+    load(m.ga, v);
+    load(m.gb, v + 3);
+  }
+  __device__ __forceinline__ void store(const ManF& m, const float* v, bool changed) const {
+    if (!changed) return;
+    if (!(m.flags & MFL_A_STATIC)) store(m.ga, v);
+    if (!(m.flags & MFL_B_STATIC)) store(m.gb, v + 3);
+  }
   __device__ __forceinline__ void load(int g, float* v) const {
     if (VLDS) {
       const float* p = lds + 3 * (g - b0);
@@ -171,19 +197,122 @@ struct VelF {
   }
 };
 
+// Agent-scope accesses of a single word, which other workgroups' wavefronts
+// read and write while this one runs.
+template <class X>
+__device__ __forceinline__ X peek(const X* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <class X>
+__device__ __forceinline__ void poke(X* p, X v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Polls before a wait on another workgroup gives up and flags the step.  The
+// waits end by themselves: what one waits for is held by a wavefront that has
+// joined the world, so that it runs, and comes earlier in the schedule.
+constexpr int FLOW_POLLS = 1 << 20;
+
+// Velocities of a world swept by several workgroups: two words per body in
+// global memory, vx | omega's low half << 32 | turn << 48 and vy | omega's
+// high half << 32 | turn << 48, where `turn` counts the manifolds that have
+// had the body.  A manifold takes its bodies when the count is its own turn,
+// pass * (the body's manifolds) + its place among them by colour, and hands
+// them on by writing the words with the count raised: the data carry their
+// own flag, so that no barrier, fence or acknowledged store lies between two
+// colours, only one store and the load that sees it (0.54 us between CUs of
+// an XCD, 0.68 across XCDs; a barrier of 256 workgroups alone takes 3.5).
+// (No word can be a whole 2^16 turns behind: the manifold itself has had the
+// body in the last pass.)  Both words move in one 16-byte access, each with
+// its own count, past the L1 cache (sc1, as agent-scope atomics compile to;
+// there is none of 16 bytes): as two accesses of 8 bytes a hand-over takes
+// 0.70 and 0.86 us.  A body has a line of 128 bytes to itself: accesses to one
+// line from many CUs wait for each other (8192 polygons 114 us with 8 bodies to
+// a line, 96 with one; with the 16-byte accesses 88).
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+struct VelFlow {
+  const Ctx* c;
+  int* abort;
+  mutable bool dead;
+  mutable unsigned long long w[4];  // the words as loaded
+
+  static __device__ __forceinline__ void unpack(unsigned long long x, unsigned long long y, float* v) {
+    v[0] = __uint_as_float((uint32_t)x);
+    v[1] = __uint_as_float((uint32_t)y);
+    v[2] = __uint_as_float(((uint32_t)(x >> 32) & 0xFFFFu) | (uint32_t)(y >> 32) << 16);
+  }
+  static __device__ __forceinline__ void pack(const float* v, uint32_t turn, unsigned long long* w) {
+    const uint32_t o = __float_as_uint(v[2]);
+    w[0] = __float_as_uint(v[0]) | (unsigned long long)((o & 0xFFFFu) | turn << 16) << 32;
+    w[1] = __float_as_uint(v[1]) | (unsigned long long)((o >> 16) | turn << 16) << 32;
+  }
+  // waits for the manifold's turn on both its bodies
+  __device__ __forceinline__ void wait(const ManF& m, int pass) const {
+    const Turns t = unpack_turns(m.turns);
+    const uint32_t ta = (uint32_t)(pass * t.of_a + t.at_a) & 0xFFFFu,
+                   tb = (uint32_t)(pass * t.of_b + t.at_b) & 0xFFFFu;
+    const unsigned long long *pa = c->flow_vel + FLOW_LINE * (long)m.ga,
+                             *pb = c->flow_vel + FLOW_LINE * (long)m.gb;
+    for (int n = 1;; ++n) {
+      u32x4 x, y;
+      asm volatile(
+          "global_load_dwordx4 %0, %2, off sc1\n\t"
+          "global_load_dwordx4 %1, %3, off sc1\n\t"
+          "s_waitcnt vmcnt(0)"
+          : "=&v"(x), "=&v"(y)
+          : "v"(pa), "v"(pb)
+          : "memory");
+      w[0] = x[0] | (unsigned long long)x[1] << 32;
+      w[1] = x[2] | (unsigned long long)x[3] << 32;
+      w[2] = y[0] | (unsigned long long)y[1] << 32;
+      w[3] = y[2] | (unsigned long long)y[3] << 32;
+      const bool a = t.of_a == 0 || ((uint32_t)(w[0] >> 48) == ta && (uint32_t)(w[1] >> 48) == ta);
+      const bool b = t.of_b == 0 || ((uint32_t)(w[2] >> 48) == tb && (uint32_t)(w[3] >> 48) == tb);
+      if ((a && b) || dead) break;
+      if (n % 256 == 0) {
+        if (n >= FLOW_POLLS) {
+          atomicOr(&c->counters[CNT_FLAGS], SHP_FLAG_STALL);
+          poke(abort, 1);
+        }
+        dead = peek(abort) != 0;
+      }
+    }
+  }
+  __device__ __forceinline__ void load(const ManF&, float* v) const {
+    unpack(w[0], w[1], v);
+    unpack(w[2], w[3], v + 3);
+  }
+  __device__ __forceinline__ void store(const ManF& m, const float* v, bool changed) const {
+    const Turns t = unpack_turns(m.turns);
+    auto hand_on = [&](int g, const unsigned long long* old, const float* x, bool keep) {
+      const uint32_t turn = ((uint32_t)(old[0] >> 48) + 1u) & 0xFFFFu;
+      unsigned long long n[2];
+      float y[3];
+      unpack(old[0], old[1], y);
+      pack(keep ? y : x, turn, n);
+      const u32x4 x4 = {(uint32_t)n[0], (uint32_t)(n[0] >> 32), (uint32_t)n[1], (uint32_t)(n[1] >> 32)};
+      asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1"
+                   :
+                   : "v"(c->flow_vel + FLOW_LINE * (long)g), "v"(x4)
+                   : "memory");
+    };
+    if (t.of_a) hand_on(m.ga, w, v, !changed || (m.flags & MFL_A_STATIC));
+    if (t.of_b) hand_on(m.gb, w + 2, v + 3, !changed || (m.flags & MFL_B_STATIC));
+  }
+};
+
 // One manifold: warm start (pass 0: useCache's applySln) or one sweep
 // (improveContactSln with FP32 velocities/rows and FP64 accumulators) of
-// its contacts in key order.  m_loc: the world-local manifold index for the
-// lagrangian stores.  The FP32 arithmetic is this solver's own: the bounce
+// its contacts in key order.  lambda(j): where contact j's lagrangians go.
+// The FP32 arithmetic is this solver's own: the bounce
 // term's closing velocity is the normal row times the velocities (the same
 // quantity as bounceB's, Solvers/Contact.hs), the effective masses enter as
 // reciprocals, and products with velocities are fused.
-template <bool VLDS>
-__device__ __forceinline__ void solve_man(const RecW& R, int m_loc, ManF& m, bool warm,
-                                          const VelF<VLDS>& V) {
+template <class Lambda, class Vel>
+__device__ __forceinline__ void solve_man(Lambda lambda, ManF& m, bool warm, const Vel& V) {
   float v[6];
-  V.load(m.ga, v);
-  V.load(m.gb, v + 3);
+  V.load(m, v);
   const int nk = (m.flags & MFL_TWO) ? 2 : 1;
   bool changed = false;
 #pragma unroll
@@ -220,14 +349,11 @@ __device__ __forceinline__ void solve_man(const RecW& R, int m_loc, ManF& m, boo
     k.lt = accp;
     changed = true;
   }
-  if (!changed) return;
-  if (!warm) {  // the solved contacts' lagrangians
-    *(double2*)(rec_of(R.rec, R.p0 + m_loc) + 6 * RB) = make_double2(m.k[0].ln, m.k[0].lt);
-    if (nk > 1)
-      *(double2*)(rec2_of(R.rec2, R.p0 + m_loc) + 3 * RB) = make_double2(m.k[1].ln, m.k[1].lt);
+  V.store(m, v, changed);
+  if (changed && !warm) {  // the solved contacts' lagrangians
+    *lambda(0) = make_double2(m.k[0].ln, m.k[0].lt);
+    if (nk > 1) *lambda(1) = make_double2(m.k[1].ln, m.k[1].lt);
   }
-  if (!(m.flags & MFL_A_STATIC)) V.store(m.ga, v);
-  if (!(m.flags & MFL_B_STATIC)) V.store(m.gb, v + 3);
 }
 
 // Colours per pair, in global memory: -1 uncoloured, -2 no contacts.
@@ -292,7 +418,7 @@ __device__ void assign_slots(int p0, int np, const CT* colour, int* scur, int ta
 }
 
 // Warm-start pass and sweeps, colour by colour, with prefetching.  Phase
-// h = pass * ncol + l; lane t of STEP takes manifolds off[l] + t, + STEP,
+// h = pass * ncol + l; lane t of `step` takes manifolds off[l] + t, + step,
 // ... of colour l (the last colour serially by lane 0 when colouring
 // stopped after JP_ROUNDS), and `sync` ends each phase.  Two records per
 // lane: the lane's next manifold of a colour loads into the other record
@@ -301,24 +427,26 @@ __device__ void assign_slots(int p0, int np, const CT* colour, int* scur, int ta
 // just solved, whose lagrangians the pass changes).  The colour bounds of
 // this phase (cs, ce) and the next (ns, ne) stay in registers; those of
 // the phase after next are read early in the phase.
-template <bool VLDS, int STEP, class Sync>
+template <class Vel, class Sync>
 __device__ __forceinline__ void sweep_prefetched(const Ctx& c, const RecW& R, int ncol,
                                                  bool serial_tail, const int* off, int lane,
-                                                 const VelF<VLDS>& V, Sync sync) {
+                                                 const int step, const Vel& V, Sync sync) {
   const int phases = (c.iterations + 1) * ncol;
   auto first_of = [&](int l, int b0_, int b1_) {
     const bool tail = serial_tail && l == ncol - 1;
     return tail ? (lane == 0 ? b0_ : b1_) : b0_ + lane;
   };
+  auto next = [&](int l) { return l + 1 == ncol ? 0 : l + 1; };
+  int l = 0, l1 = next(0);
   int cs = off[0], ce = off[1];
-  int ns = off[1 % ncol], ne = off[1 % ncol + 1];
+  int ns = off[l1], ne = off[l1 + 1];
   ManF m, n;
   bool loaded = false;
   for (int h = 0; h < phases; ++h) {
-    const int l = h % ncol, l1 = (h + 1) % ncol, l2 = (h + 2) % ncol;
+    const int l2 = next(l1);
     const int s2 = off[l2], e2 = off[l2 + 1];
     const bool warm = h < ncol;
-    const int di = serial_tail && l == ncol - 1 ? 1 : STEP;
+    const int di = serial_tail && l == ncol - 1 ? 1 : step;
     const int end = ce;
     int i = first_of(l, cs, ce);
     if (i < end && !loaded) load_man(R, i, m);
@@ -326,13 +454,13 @@ __device__ __forceinline__ void sweep_prefetched(const Ctx& c, const RecW& R, in
       int inext = i + di;
       bool more = inext < end;
       if (more) load_man(R, inext, n);
-      solve_man<VLDS>(R, i, m, warm, V);
+      solve_man([&](int j) { return lambda_of(R, i, j); }, m, warm, V);
       if (!more) break;
       i = inext;
       inext = i + di;
       more = inext < end;
       if (more) load_man(R, inext, m);
-      solve_man<VLDS>(R, i, n, warm, V);
+      solve_man([&](int j) { return lambda_of(R, i, j); }, n, warm, V);
       if (!more) break;
       i = inext;
     }
@@ -349,6 +477,8 @@ __device__ __forceinline__ void sweep_prefetched(const Ctx& c, const RecW& R, in
     ce = ne;
     ns = s2;
     ne = e2;
+    l = l1;
+    l1 = l2;
   }
 }
 
@@ -356,8 +486,8 @@ __device__ __forceinline__ void sweep_prefetched(const Ctx& c, const RecW& R, in
 template <bool VLDS, int T>
 __device__ void sweep_colours(const Ctx& c, const RecW& R, int ncol, bool serial_tail,
                               const int* s_off, const VelF<VLDS>& V) {
-  sweep_prefetched<VLDS, T>(c, R, ncol, serial_tail, s_off, (int)threadIdx.x, V,
-                            [] { __syncthreads(); });
+  sweep_prefetched(c, R, ncol, serial_tail, s_off, (int)threadIdx.x, T, V,
+                   [] { __syncthreads(); });
 }
 
 // Colour-order bookkeeping shared by both kernels: per-colour counts of the
@@ -428,7 +558,7 @@ __device__ void colour_finish(const Ctx& c, int w, int p0, int np, const CT* col
   assign_slots<T>(p0, np, colour, s_cur, serial_tail ? ncol - 1 : -1, c.sched_order + p0);
   int* off = c.col_off + (long)w * (COLOR_CAP + 3);
   for (int l = threadIdx.x; l <= ncol; l += T) off[l] = s_off[l];
-  if (threadIdx.x == 0) c.col_info[w] = ncol | (serial_tail ? 1 << 16 : 0);
+  if (threadIdx.x == 0) c.col_info[w] = ncol | (serial_tail ? COL_TAIL : 0);
 }
 
 // Number of manifolds (pairs with stored contacts) of a world, summed over
@@ -945,7 +1075,7 @@ __device__ __forceinline__ void wave_sync() {
 // sweep_world, so the same results.
 __global__ __launch_bounds__(64 * SWEEP_WAVES) void k_sweep_waves(Ctx c, int first_world,
                                                                   int slice_floats) {
-  extern __shared__ int lds[];
+  extern __shared__ __align__(16) int lds[];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int k = first_world + (int)blockIdx.x * SWEEP_WAVES + wave;
   if (k >= c.W) return;  // this wavefront only: no workgroup barrier follows
@@ -953,7 +1083,7 @@ __global__ __launch_bounds__(64 * SWEEP_WAVES) void k_sweep_waves(Ctx c, int fir
   const int info = c.col_info[w];
   const int ncol = info & 0xFFFF;
   if (ncol == 0) return;
-  const bool serial_tail = (info >> 16) & 1;
+  const bool serial_tail = info & COL_TAIL;
   const int p0 = c.wpair_off[w];
   const int b0 = c.body_off[w], nb = c.body_off[w + 1] - b0;
   const int* off = c.col_off + (long)w * (COLOR_CAP + 3);
@@ -968,8 +1098,8 @@ __global__ __launch_bounds__(64 * SWEEP_WAVES) void k_sweep_waves(Ctx c, int fir
   }
   wave_sync();
   const PackF P = packf(c);
-  sweep_prefetched<true, 64>(c, recw(c, P, p0), ncol, serial_tail, off, lane, V,
-                             [] { wave_sync(); });
+  sweep_prefetched(c, recw(c, P, p0), ncol, serial_tail, off, lane, 64, V,
+                   [] { wave_sync(); });
   for (int i = lane; i < nb; i += 64) {
     float v[3];
     V.load(b0 + i, v);
@@ -977,28 +1107,16 @@ __global__ __launch_bounds__(64 * SWEEP_WAVES) void k_sweep_waves(Ctx c, int fir
   }
 }
 
-// Colouring, one workgroup per world, the largest worlds first: in LDS when
-// the world's colouring fits (by its pair count, else by its manifold
-// count), else with the bodies in LDS and the manifold lists in global
-// memory when the bodies fit, else in global memory.
+// Colouring of world w by one workgroup: in LDS when the world's colouring
+// fits (by its pair count, else by its manifold count), else with the bodies
+// in LDS and the manifold lists in global memory when the bodies fit, else in
+// global memory.
 template <int T>
-__global__ __launch_bounds__(T) void k_colour(Ctx c, int pool_bytes) {
-  extern __shared__ int lds[];
+__device__ void colour_world(const Ctx& c, int w, int p0, int np, int pool_bytes, int* lds, int* sm) {
   int* s_off = lds;                      // COLOR_CAP + 3
   int* s_cur = lds + (COLOR_CAP + 3);    // COLOR_CAP + 3
   unsigned char* pool = (unsigned char*)(lds + 2 * (COLOR_CAP + 3) + 2);
-  __shared__ int sm[4];
-  const int w = c.world_order[blockIdx.x], tid = threadIdx.x;
-  // the world's pairs (k_world_ranges computes the same offsets beside
-  // this kernel)
   const int b0 = c.body_off[w], nb = c.body_off[w + 1] - b0;
-  const int p0 = min(c.off_rank[b0], c.pair_cap), p1 = min(c.off_rank[b0 + nb], c.pair_cap);
-  const int np = p1 - p0;
-  if (np == 0) {  // nothing to solve
-    if (tid == 0) c.col_info[w] = 0;
-    return;
-  }
-  tmark(c, 0);
   // room for every pair as a manifold, or else for the manifolds counted
   int cap = np;
   bool in_lds = colour_fits_lds(nb, np, np, pool_bytes);
@@ -1014,6 +1132,286 @@ __global__ __launch_bounds__(T) void k_colour(Ctx c, int pool_bytes) {
     colour_world_hybrid<T, false>(c, w, p0, np, b0, nb, pool, s_off, s_cur, sm);
   else
     colour_world_global<T>(c, w, p0, np, b0, nb, s_off, s_cur, sm);
+}
+
+// ---- one world on several CUs ----------------------------------------------
+//
+// The workgroups that share a world wait for each other's results, so each of
+// them must be running.  They join by a counter; the first to come closes it
+// once all `want` have joined or after a bounded wait (on a GPU busy with
+// other streams some may not have started), and those that come later leave.
+// Returns the caller's seat and their number in *groups (-1: leave).  Seats
+// follow each other in space (pairs are in the order of their bodies), so
+// when all have come, those of an XCD, to which workgroups go in turn, are
+// consecutive: what neighbours exchange stays in its L2.
+constexpr int FLOW_JOIN_POLLS = 4096;  // about 0.5 ms
+enum { FLOW_CLOSED = 1 << 30 };
+
+constexpr int XCDS = 8;
+
+__device__ __forceinline__ int flow_join(int* seats, int* groups_word, int blk, int want, int* s_tmp,
+                                         int* groups) {
+  if (threadIdx.x == 0) {
+    constexpr int AGENT = __HIP_MEMORY_SCOPE_AGENT;
+    int s = __hip_atomic_fetch_add(seats, 1, __ATOMIC_RELAXED, AGENT), g = 0;
+    if (s & FLOW_CLOSED) {
+      s = -1;
+    } else if (s == 0) {
+      for (int n = 0; n < FLOW_JOIN_POLLS && peek(seats) < want; ++n) __builtin_amdgcn_s_sleep(1);
+      g = __hip_atomic_fetch_or(seats, FLOW_CLOSED, __ATOMIC_RELAXED, AGENT);
+      poke(groups_word, g);
+    } else {  // the first one runs and always writes it
+      for (int n = 0; n < FLOW_POLLS && (g = peek(groups_word)) == 0; ++n) __builtin_amdgcn_s_sleep(1);
+      if (g == 0) s = -1;
+    }
+    if (g == want) s = blk % XCDS * (want / XCDS) + min(blk % XCDS, want % XCDS) + blk / XCDS;
+    s_tmp[0] = s;
+    s_tmp[1] = g;
+  }
+  __syncthreads();
+  *groups = s_tmp[1];
+  const int seat = s_tmp[0];
+  __syncthreads();
+  return seat;
+}
+
+// Workgroups of world w, of at most `groups`.
+__device__ __forceinline__ int flow_want(const Ctx& c, int w, int groups) {
+  const int nb = c.body_off[w + 1] - c.body_off[w];
+  return min(groups, (nb + FLOW_GROUP_BODIES - 1) / FLOW_GROUP_BODIES);
+}
+
+// The rounds' colouring of a world without rounds, by several workgroups of T
+// lanes with FLOW_ITEMS / T pairs each.  In the rounds a manifold is coloured
+// once every manifold of higher priority on its bodies is; here it waits for
+// just those.  The lists k_sat made give each manifold its rank by priority
+// among its body's; a body's word (colours used | manifolds coloured << 32 |
+// round << 48) says whose turn it is and holds all that the colour depends
+// on: the next manifold of both its bodies takes the same colour as in the
+// rounds, and its round is one past the latest on its bodies.  A lane keeps
+// its manifolds in registers and looks at all that are left in turn, so the
+// time is that of the longest chain of priorities (about 20 hand-overs)
+// instead of 3 barriers and a scan of the lists for each of the rounds, on
+// one CU: one pile of 32768 polygons 40 us (about 20 of them joining, ranking
+// and the places in the colours), 496 before; of 8192 30, 113 before.
+//
+// Returns true when the world's colours are complete (its last workgroup has
+// written col_off, col_info and flow_cnt, and flow_slot holds each pair's
+// colour and its place among those of its workgroup).  A world with a body of more than FLOW_DEGREE manifolds, more pairs
+// than the lanes hold, or colours past FLOW_DEGREE is left to one workgroup:
+// *last tells the one that has to colour it.
+constexpr int FLOW_ITEMS = 8192, FLOW_COLOUR_LANES = 256;
+
+__device__ void colour_flow(const Ctx& c, int w, int p0, int np, int seat, int groups, int rows,
+                            int* lds, bool* last) {
+  constexpr int AGENT = __HIP_MEMORY_SCOPE_AGENT, T = FLOW_COLOUR_LANES;
+  int* s_cnt = lds;                 // FLOW_DEGREE
+  int* s_last = lds + FLOW_DEGREE;
+  // per pair its bodies, rank on a | rank on b << 8, and its colour; the first
+  // T lanes wait for them, tid + k T each
+  uint32_t* s_ab = (uint32_t*)(lds + 2 * FLOW_DEGREE);
+  uint16_t* s_rank = (uint16_t*)(s_ab + FLOW_ITEMS);
+  uint8_t* s_col = (uint8_t*)(s_rank + FLOW_ITEMS);
+  int* ctl = c.flow_ctl + (long)w * FLOW_CTL;
+  const int tid = threadIdx.x, b0 = c.body_off[w];
+  const int per = ((np + groups - 1) / groups + 63) & ~63;
+  const int q0 = seat * per, n = min(per, np - q0);
+  const bool fits = per <= FLOW_ITEMS;
+  if (tid < FLOW_DEGREE) s_cnt[tid] = 0;
+  if (fits && peek(ctl + FC_BAD) == 0) {
+    auto key = [&](uint32_t q) {  // orders like prio64
+      return (unsigned long long)(mix32(q * 0x9E3779B9u + (uint32_t)w) & 0x7FFFu) << 32 | q;
+    };
+    const int lanes = (int)blockDim.x;
+    for (int i = tid; i < n; i += lanes) {
+      const uint32_t ab = c.pair_ab[p0 + q0 + i];
+      s_ab[i] = ab;
+      s_col[i] = 0xFFu;
+      if (ab == NO_PAIR) continue;
+      const unsigned long long mine = key((uint32_t)(q0 + i));
+      int r[2], m[2];
+      const int4* row[2];
+      int4 e[2][2];
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        const uint32_t loc = s ? ab >> 16 : ab & 0xFFFFu;
+        const int g = b0 + (loc == NO_BODY ? 0 : (int)loc);
+        row[s] = (const int4*)(c.adj + (long)g * FLOW_DEGREE);
+        m[s] = loc == NO_BODY ? 0 : c.adj_n[g];
+        e[s][0] = row[s][0];
+        e[s][1] = row[s][1];
+      }
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        r[s] = 0;
+        auto count = [&](int4 x, int at) {
+          const int y[4] = {x.x, x.y, x.z, x.w};
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+            if (at + j < m[s] && key((uint32_t)(y[j] - p0)) > mine) ++r[s];
+        };
+        count(e[s][0], 0);
+        if (m[s] > 4) count(e[s][1], 4);
+        for (int at = 8; at < m[s]; at += 4) count(row[s][at / 4], at);
+      }
+      s_rank[i] = (uint16_t)(r[0] | r[1] << 8);
+    }
+    __syncthreads();
+    uint32_t alive = 0;
+    static_assert(FLOW_ITEMS / T <= 32, "a lane's pairs are bits of a word");
+    if (tid < T)
+      for (int i = tid, k = 0; i < n; i += T, ++k) alive |= (s_ab[i] != NO_PAIR ? 1u : 0u) << k;
+    bool bad = false;
+    for (int polls = 1; alive; ++polls) {
+      // the lane's next manifolds, two at a time
+      for (uint32_t rest = alive; rest;) {
+        int k[2];
+        uint32_t ab[2], rank[2];
+        unsigned long long wa[2], wb[2];
+        k[0] = __builtin_ctz(rest);
+        rest &= rest - 1;
+        k[1] = rest ? __builtin_ctz(rest) : k[0];
+        rest &= rest - 1;
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          const int i = tid + k[j] * T;
+          ab[j] = s_ab[i];
+          rank[j] = s_rank[i];
+          const uint32_t a = ab[j] & 0xFFFFu, b = ab[j] >> 16;
+          wa[j] = a != NO_BODY ? peek(c.flow_col + FLOW_LINE * (long)(b0 + a)) : 0ull;
+          wb[j] = b != NO_BODY ? peek(c.flow_col + FLOW_LINE * (long)(b0 + b)) : 0ull;
+        }
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          if (j == 1 && k[1] == k[0]) continue;
+          if (((uint32_t)(wa[j] >> 32) & 0xFFFFu) != (rank[j] & 0xFFu) ||
+              ((uint32_t)(wb[j] >> 32) & 0xFFFFu) != rank[j] >> 8)
+            continue;
+          const int round = max((int)(wa[j] >> 48), (int)(wb[j] >> 48));
+          const int l = greedy_colour((uint32_t)(wa[j] | wb[j]) & 0xFFFFu, round);
+          const bool ok = l < FLOW_DEGREE && round < JP_ROUNDS;
+          bad |= !ok;
+          s_col[tid + k[j] * T] = (uint8_t)(ok ? l : 0);
+          alive &= ~(1u << k[j]);
+          const unsigned long long up = (unsigned long long)min(round + 1, JP_ROUNDS) << 48;
+          auto hand_on = [&](uint32_t loc, unsigned long long x) {
+            if (loc == NO_BODY) return;
+            poke(c.flow_col + FLOW_LINE * (long)(b0 + loc), up | ((((x >> 32) & 0xFFFFull) + 1ull) << 32) |
+                                            (uint32_t)(x | (ok ? 1ull << l : 0ull)));
+          };
+          hand_on(ab[j] & 0xFFFFu, wa[j]);
+          hand_on(ab[j] >> 16, wb[j]);
+        }
+      }
+      if (polls % 64 == 0) {
+        if (polls >= FLOW_POLLS) {
+          atomicOr(&c.counters[CNT_FLAGS], SHP_FLAG_STALL);
+          bad = true;
+        }
+        if (bad || peek(ctl + FC_BAD) != 0) break;
+      }
+    }
+    if (bad) poke(ctl + FC_BAD, 1);
+    __syncthreads();
+    // places within the colours: consecutive for a wavefront's pairs of a
+    // colour, so that the sweeps' lanes stay near each other
+    for (int i0 = 0; i0 < n; i0 += lanes) {
+      const int i = i0 + tid;
+      const int at = wave_count(s_cnt, i < n && s_col[i] != 0xFFu ? (int)s_col[i] : -1);
+      if (i < n) s_ab[i] = (uint32_t)at;
+    }
+    __syncthreads();
+    if (tid < FLOW_DEGREE) poke(c.flow_cnt + (rows + seat) * FLOW_DEGREE + tid, s_cnt[tid]);
+    for (int i = tid; i < n; i += lanes) {
+      const int l = s_col[i];
+      c.flow_slot[p0 + q0 + i] = l == 0xFF ? -1 : (int)s_ab[i] << 5 | l;
+    }
+  }
+  // the last workgroup (the others' counts and flags are in: their stores were
+  // complete before their additions)
+  __builtin_amdgcn_s_waitcnt(0);
+  __syncthreads();
+  if (tid == 0)
+    *s_last = __hip_atomic_fetch_add(ctl + FC_DONE, 1, __ATOMIC_RELAXED, AGENT) == groups - 1
+                  ? 1 + (fits && peek(ctl + FC_BAD) == 0)
+                  : 0;
+  __syncthreads();
+  const int what = *s_last;
+  __syncthreads();
+  *last = what == 1;
+  if (what != 2) return;
+  // the colours' offsets, and within each those of the workgroups' manifolds,
+  // in the order of the seats: FLOW_DEGREE columns, a run of seats to a lane
+  const int l = tid % FLOW_DEGREE, runs = (int)blockDim.x / FLOW_DEGREE, run = tid / FLOW_DEGREE;
+  const int len = (groups + runs - 1) / runs, s0 = min(run * len, groups), s1 = min(s0 + len, groups);
+  int* s_run = (int*)s_ab;  // runs x FLOW_DEGREE
+  int32_t* cnt = c.flow_cnt + rows * FLOW_DEGREE + l;
+  int sum = 0;
+  for (int s = s0; s < s1; ++s) sum += peek(cnt + s * FLOW_DEGREE);
+  s_run[tid] = sum;
+  __syncthreads();
+  int before = 0, all = 0;
+  for (int r = 0; r < runs; ++r) {
+    const int x = s_run[r * FLOW_DEGREE + l];
+    before += r < run ? x : 0;
+    all += x;
+  }
+  for (int s = s0; s < s1; ++s) {
+    const int x = peek(cnt + s * FLOW_DEGREE);
+    cnt[s * FLOW_DEGREE] = before;
+    before += x;
+  }
+  if (tid >= 64) return;
+  const int have = tid < FLOW_DEGREE ? all : 0;
+  int upto = have;
+  for (int o = 1; o < 64; o <<= 1) {
+    const int x = __shfl_up(upto, o);
+    if (tid >= o) upto += x;
+  }
+  const unsigned long long used = __ballot(have > 0);
+  const int ncol = used ? 64 - __builtin_clzll(used) : 0;
+  int* off = c.col_off + (long)w * (COLOR_CAP + 3);
+  if (tid <= ncol) off[tid] = upto - have;
+  if (tid == 0) {
+    ctl[FC_ROWS] = rows;
+    ctl[FC_SHARE] = per;
+    c.col_info[w] = ncol | COL_FLOW;  // also without a manifold: flow_slot says so
+    atomicMax(&c.counters[CNT_LEVELS], ncol);
+  }
+}
+
+// Colouring: the flow worlds' workgroups, then one per world, the largest
+// worlds first.
+template <int T>
+__global__ __launch_bounds__(T) void k_colour(Ctx c, int pool_bytes) {
+  extern __shared__ __align__(16) int lds[];
+  __shared__ int sm[4];
+  const int flow_blocks = c.flow_worlds * c.flow_groups, blk = blockIdx.x;
+  const bool flow = blk < flow_blocks;
+  const int w = c.world_order[flow ? blk / c.flow_groups : blk - flow_blocks + c.flow_worlds];
+  // the world's pairs (k_world_ranges computes the same offsets beside
+  // this kernel)
+  const int b0 = c.body_off[w], b1 = c.body_off[w + 1];
+  const int p0 = min(c.off_rank[b0], c.pair_cap), p1 = min(c.off_rank[b1], c.pair_cap);
+  const int np = p1 - p0;
+  if (np == 0) {  // nothing to solve
+    if (threadIdx.x == 0) c.col_info[w] = 0;
+    return;
+  }
+  tmark(c, 0);
+  if (flow) {
+    int* ctl = c.flow_ctl + (long)w * FLOW_CTL;
+    const int want = flow_want(c, w, c.flow_groups);
+    if (blk % c.flow_groups >= want) return;
+    int groups;
+    const int seat = flow_join(ctl + FC_SEATS, ctl + FC_GROUPS, blk % c.flow_groups, want, sm,
+                               &groups);
+    if (seat < 0) return;
+    bool last;
+    colour_flow(c, w, p0, np, seat, groups, blk / c.flow_groups * c.flow_groups, lds, &last);
+    if (!last) return;
+  }
+  colour_world<T>(c, w, p0, np, pool_bytes, lds, sm);
   tmark(c, 1);
 }
 
@@ -1023,12 +1421,40 @@ __global__ __launch_bounds__(T) void k_colour(Ctx c, int pool_bytes) {
 __global__ void k_pack_manifolds(Ctx c) {
   const int tp = c.wpair_off[c.W];
   const PackF P = packf(c);
+  if (c.flow_worlds)  // the bodies' first velocity words
+    for (int g = blockIdx.x * blockDim.x + threadIdx.x; g < c.NB; g += gridDim.x * blockDim.x) {
+      const float v[3] = {(float)c.vx[g], (float)c.vy[g], (float)c.w[g]};
+      unsigned long long x[2];
+      VelFlow::pack(v, 0, x);
+      *(ulonglong2*)(c.flow_vel + FLOW_LINE * (long)g) = make_ulonglong2(x[0], x[1]);
+    }
   for (int p = blockIdx.x * blockDim.x + threadIdx.x; p < tp; p += gridDim.x * blockDim.x) {
-    const int M = c.sched_order[p];
+    int M, turns = 0;
+    const int w = c.flow_worlds ? c.body_world[c.pa[p]] : 0;
+    if (c.flow_worlds && (c.col_info[w] & COL_FLOW)) {
+      const int s = c.flow_slot[p], l = s & 31;
+      const int* ctl = c.flow_ctl + (long)w * FLOW_CTL;
+      const int p0 = c.wpair_off[w], row = ctl[FC_ROWS] + (p - p0) / ctl[FC_SHARE];
+      M = s < 0 ? -1
+                : p0 + c.col_off[(long)w * (COLOR_CAP + 3) + l] +
+                      c.flow_cnt[row * FLOW_DEGREE + l] + (s >> 5);
+      c.sched_order[p] = M;
+      auto turn = [&](int g, int& at, int& of) {
+        const uint32_t used = c.is_static[g] ? 0u : (uint32_t)c.flow_col[FLOW_LINE * (long)g];
+        at = __popc(used & ((1u << l) - 1u));
+        of = __popc(used);
+      };
+      Turns t;
+      turn(c.pa[p], t.at_a, t.of_a);
+      turn(c.pb[p], t.at_b, t.of_b);
+      turns = pack_turns(t);
+    } else {
+      M = c.sched_order[p];
+    }
     if (M < 0) continue;
     const int k0 = c.coff[p];
     if (k0 >= c.contact_cap) {
-      write_null_record(P, M, c.pa[p], c.pb[p]);
+      write_null_record(P, M, c.pa[p], c.pb[p], turns);
       continue;
     }
     const int cap = c.contact_cap - k0, nk = c.ccount[p] < cap ? c.ccount[p] : cap;
@@ -1050,7 +1476,7 @@ __global__ void k_pack_manifolds(Ctx c) {
       lt[j] = c.lt[k];
       warm |= (c.warm[k] ? 1 : 0) << j;
     }
-    write_record_head(c, P, M, ga, gb, u, ima, imb, nk, warm);
+    write_record_head(c, P, M, ga, gb, u, ima, imb, nk, warm, turns);
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       if (j >= nk) break;
@@ -1108,17 +1534,133 @@ __device__ void sweep_world(const Ctx& c, int w, int ncol, bool serial_tail, flo
   tmark(c, 5);
 }
 
-// One workgroup per world, the largest worlds first; velocities in LDS
-// when they fit.
+// The sweeps of a world by several workgroups, one wavefront of each, whose
+// manifolds wait for their own bodies only (VelFlow).  A wavefront has an even
+// share of every colour and takes its manifolds in colour order, so that what
+// any of its lanes waits for comes before all that the wavefront has left to
+// do.  Its records stay in LDS over the passes (its other wavefronts help to
+// bring them in and the lagrangians out), so that between two colours there
+// is only the velocities' way from CU to CU.  Few lanes to a CU, on many CUs:
+// the scattered velocity words cost a CU's address unit a cycle each.  One
+// pile of 32768 polygons, 4 iterations: 67 us (45 colours in turn, 1.4 us
+// each: a hand-over, 0.3 us of arithmetic, the slowest of a wavefront's
+// lanes), 1121 by one workgroup of 1024 lanes with a barrier after each
+// colour; of 8192, 8 iterations: 91 (72 colours), 270 before (velocities in
+// LDS).  With 256 lanes to a CU and the records read from L2 in each pass it
+// took 172 and 209.
+constexpr int FLOW_REC_BYTES = 16 * (REC_WORDS + REC2_WORDS);
+
+// The share of colour `lane` that seat `seat` has: [first, last), the
+// manifolds before it in the wavefront's records, and all of them; the most
+// that any seat has.
+struct FlowShare {
+  int first, last, start, all, most;
+};
+
+__device__ __forceinline__ FlowShare flow_share(const Ctx& c, int w, int ncol, int seat, int groups) {
+  const int lane = threadIdx.x & 63;
+  const int* offs = c.col_off + (long)w * (COLOR_CAP + 3) + min(lane, ncol - 1);
+  const int o0 = offs[0], o1 = offs[1], share = (o1 - o0 + groups - 1) / groups;
+  FlowShare f;
+  f.first = min(o0 + seat * share, o1);
+  f.last = min(f.first + share, o1);
+  const int n = lane < ncol ? f.last - f.first : 0;
+  int sum = n;
+  for (int o = 1; o < 64; o <<= 1) {
+    const int x = __shfl_up(sum, o);
+    if (lane >= o) sum += x;
+  }
+  f.start = sum - n;
+  f.all = __shfl(sum, 63);
+  f.most = wave_sum(lane < ncol ? share : 0);
+  return f;
+}
+
+__device__ void sweep_flow(const Ctx& c, int w, int ncol, const FlowShare f, float4* recs) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
+  const int step = f.all;  // between a record's words
+  const PackF P = packf(c);
+  const RecW R = recw(c, P, c.wpair_off[w]);
+  for (int l = wave; l < ncol; l += waves) {
+    const int i0 = __builtin_amdgcn_readlane(f.first, l), i1 = __builtin_amdgcn_readlane(f.last, l);
+    const int s0 = __builtin_amdgcn_readlane(f.start, l) - i0;
+    for (int i = i0 + lane; i < i1; i += 64) {
+      const float4 *r = rec_of(R.rec, R.p0 + i), *r2 = rec2_of(R.rec2, R.p0 + i);
+      float4 x[REC_WORDS + REC2_WORDS];
+#pragma unroll
+      for (int q = 0; q < REC_WORDS; ++q) x[q] = r[q * RB];
+#pragma unroll
+      for (int q = 0; q < REC2_WORDS; ++q) x[REC_WORDS + q] = r2[q * RB];
+#pragma unroll
+      for (int q = 0; q < REC_WORDS + REC2_WORDS; ++q) recs[q * step + s0 + i] = x[q];
+    }
+  }
+  __syncthreads();
+  if (wave == 0) {
+    const int passes = c.iterations + 1;
+    VelFlow V;
+    V.c = &c;
+    V.abort = c.flow_ctl + (long)w * FLOW_CTL + FS_ABORT;
+    V.dead = false;
+    for (int pass = 0; pass < passes; ++pass)
+      for (int l = 0; l < ncol; ++l) {
+        const int i0 = __builtin_amdgcn_readlane(f.first, l);
+        const int n = __builtin_amdgcn_readlane(f.last, l) - i0;
+        float4* r0 = recs + __builtin_amdgcn_readlane(f.start, l);
+        for (int i = lane; i < n; i += 64) {
+          ManF m;
+          load_head(r0 + i, step, m);
+          load_contact(r0 + i + 3 * step, step, m.k[0]);
+          load_contact(r0 + i + REC_WORDS * step, step, m.k[1]);
+          V.wait(m, pass);
+          solve_man([&](int j) { return (double2*)(r0 + i + (j ? REC_WORDS + 3 : 6) * step); }, m,
+                    pass == 0, V);
+        }
+      }
+  }
+  __syncthreads();
+  for (int l = wave; l < ncol; l += waves) {
+    const int i0 = __builtin_amdgcn_readlane(f.first, l), i1 = __builtin_amdgcn_readlane(f.last, l);
+    const int s0 = __builtin_amdgcn_readlane(f.start, l) - i0;
+    for (int i = i0 + lane; i < i1; i += 64) {
+      *(float4*)lambda_of(R, i, 0) = recs[6 * step + s0 + i];
+      *(float4*)lambda_of(R, i, 1) = recs[(REC_WORDS + 3) * step + s0 + i];
+    }
+  }
+}
+
+// The flow worlds' workgroups, then one workgroup per world, the largest
+// worlds first; velocities in LDS when they fit.
 template <int T>
 __global__ __launch_bounds__(T) void k_sweep_colours(Ctx c, int pool_bytes) {
-  extern __shared__ int lds[];
+  extern __shared__ __align__(16) int lds[];
   __shared__ int s_off[COLOR_CAP + 3];
-  const int w = c.world_order[blockIdx.x];
+  const int flow_blocks = c.flow_worlds * c.flow_groups, blk = blockIdx.x;
+  const bool flow = blk < flow_blocks;
+  const int w = c.world_order[flow ? blk / c.flow_groups : blk - flow_blocks + c.flow_worlds];
   const int info = c.col_info[w];
   const int ncol = info & 0xFFFF;
   if (ncol == 0) return;
-  const bool serial_tail = (info >> 16) & 1;
+  if (flow && (info & COL_FLOW)) {
+    int* ctl = c.flow_ctl + (long)w * FLOW_CTL;
+    const int want = flow_want(c, w, c.flow_groups);
+    if (blk % c.flow_groups >= want) return;
+    int groups;
+    const int seat = flow_join(ctl + FS_SEATS, ctl + FS_GROUPS, blk % c.flow_groups, want, s_off,
+                               &groups);
+    if (seat < 0) return;
+    const FlowShare f = flow_share(c, w, ncol, seat, groups);
+    if ((long)f.most * FLOW_REC_BYTES <= pool_bytes) {
+      sweep_flow(c, w, ncol, f, (float4*)lds);
+      return;
+    }
+    // records that do not fit in LDS: one workgroup
+    if (seat != 0) return;
+    if (threadIdx.x == 0) ctl[FS_ALONE] = 1;
+  } else if (flow && blk % c.flow_groups != 0) {
+    return;
+  }
+  const bool serial_tail = info & COL_TAIL;
   const int nb = c.body_off[w + 1] - c.body_off[w];
   if (vel_fits_lds(nb, pool_bytes))
     sweep_world<true, T>(c, w, ncol, serial_tail, (float*)lds, s_off);
@@ -1150,11 +1692,21 @@ __global__ void k_colour_unpack(Ctx c) {
     }
     if (t < c.NB) {
       const int g = (int)t;
-      if (!c.is_static[g] && (c.col_info[c.body_world[g]] & 0xFFFF) != 0) {
-        const float4 f = c.fv[g];
-        c.vx[g] = c.vx[g] + (double)(f.x - (float)c.vx[g]);
-        c.vy[g] = c.vy[g] + (double)(f.y - (float)c.vy[g]);
-        c.w[g] = c.w[g] + (double)(f.z - (float)c.w[g]);
+      const int info = c.col_info[c.body_world[g]];
+      if (!c.is_static[g] && (info & 0xFFFF) != 0) {
+        float f[3];
+        if ((info & COL_FLOW) && !c.flow_ctl[(long)c.body_world[g] * FLOW_CTL + FS_ALONE]) {
+          const ulonglong2 x = *(const ulonglong2*)(c.flow_vel + FLOW_LINE * (long)g);
+          VelFlow::unpack(x.x, x.y, f);
+        } else {
+          const float4 x = c.fv[g];
+          f[0] = x.x;
+          f[1] = x.y;
+          f[2] = x.z;
+        }
+        c.vx[g] = c.vx[g] + (double)(f[0] - (float)c.vx[g]);
+        c.vy[g] = c.vy[g] + (double)(f[1] - (float)c.vy[g]);
+        c.w[g] = c.w[g] + (double)(f[2] - (float)c.w[g]);
       }
     }
   }
@@ -1167,7 +1719,8 @@ __global__ void k_colour_unpack(Ctx c) {
 // needs more is coloured in global memory); the sweeps use the pool for
 // the FP32 velocities.  4 waves per world; a large world gets 8, and its
 // colouring 16 (light on registers).
-void plan_colored_solver(StepPlan* P, int solver_threads) {
+void plan_colored_solver(StepPlan* P, int solver_threads, const std::vector<int32_t>& body_off,
+                         const std::vector<int32_t>& order) {
   const long nb = P->max_nb;
   const long np = std::min<long>(32767, 8 * nb + 64);
   const long need = std::max(6 * nb + 2 + 7 * np, 12 * nb);
@@ -1186,6 +1739,25 @@ void plan_colored_solver(StepPlan* P, int solver_threads) {
   // worlds' colouring costs nothing there (one world: the contact kernel's
   // time) and smaller workgroups share CUs with it.
   P->records_in_contacts = P->color_threads >= 512 && P->W >= RECORDS_IN_CONTACTS_MIN_WORLDS;
+  // Worlds on several CUs, as many as there are CUs for: us a step, 6
+  // iterations, on several CUs against one (1024 lanes): one world of 1024
+  // bodies 183 / 181, 2048 193 / 217, 4096 210 / 268, 8192 223 / 364, 16384
+  // 265 / 765, 32768 325 / 1690; 8 of 4096 332 / 365, 16 of them 440 / 431,
+  // 4 of 8192 326 / 441, 8 429 / 509, 4 of 16384 414 / 889, 2 of 32768
+  // 417 / 1761.  (A workgroup's records fill its LDS at about 450 bodies, at
+  // 2 manifolds each.)
+  int big = 0;
+  while (big < P->W && body_off[order[big] + 1] - body_off[order[big]] > FLOW_MIN_BODIES) ++big;
+  if (big > 0 && !P->records_in_contacts) {
+    const long groups = std::min<long>((nb + FLOW_GROUP_BODIES - 1) / FLOW_GROUP_BODIES,
+                                       FLOW_MAX_GROUPS / big);
+    if (groups * FLOW_GROUP_MAX >= nb) {
+      P->flow_worlds = big;
+      P->flow_groups = (int)groups;
+      P->color_lds = LDS_MAX_BYTES;
+      P->color_pool = P->color_lds - fixed;
+    }
+  }
 }
 
 // k_colour: sm[4]; k_sweep_colours: s_off[COLOR_CAP + 3]
@@ -1230,10 +1802,11 @@ void launch_colouring(shp_batch* b, hipStream_t s) {
   const Ctx& c = b->ctx;
   const StepPlan& P = b->plan;
   const int pool = (int)P.color_pool;
+  const unsigned grid = (unsigned)(c.W + c.flow_worlds * (c.flow_groups - 1));
   if (P.color_threads >= 512)
-    k_colour<1024><<<c.W, 1024, P.color_lds, s>>>(c, pool);
+    k_colour<1024><<<grid, 1024, P.color_lds, s>>>(c, pool);
   else
-    k_colour<256><<<c.W, 256, P.color_lds, s>>>(c, pool);
+    k_colour<256><<<grid, 256, P.color_lds, s>>>(c, pool);
 }
 
 
@@ -1243,12 +1816,13 @@ void launch_colored_sweep(shp_batch* b) {
   const int pool = (int)P.color_pool;
   const unsigned big = (unsigned)P.sweep_big;
   if (big > 0) {
+    const unsigned grid = big + (unsigned)(c.flow_worlds * (c.flow_groups - 1));
     if (P.color_threads == 1024)
-      k_sweep_colours<1024><<<big, 1024, P.color_pool, b->stream>>>(c, pool);
+      k_sweep_colours<1024><<<grid, 1024, P.color_pool, b->stream>>>(c, pool);
     else if (P.color_threads == 512)
-      k_sweep_colours<512><<<big, 512, P.color_pool, b->stream>>>(c, pool);
+      k_sweep_colours<512><<<grid, 512, P.color_pool, b->stream>>>(c, pool);
     else
-      k_sweep_colours<256><<<big, 256, P.color_pool, b->stream>>>(c, pool);
+      k_sweep_colours<256><<<grid, 256, P.color_pool, b->stream>>>(c, pool);
   }
   if (P.g_sweep_waves > 0)
     k_sweep_waves<<<(unsigned)P.g_sweep_waves, 64 * SWEEP_WAVES,

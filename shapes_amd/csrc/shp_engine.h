@@ -38,6 +38,19 @@ constexpr size_t lds16(size_t bytes) { return (bytes + 15) & ~(size_t)15; }
 // contact, in blocks of 64 manifolds (PC manifolds)
 #define COLOR_PACK_FLOATS(PC) (44L * (((PC) + 63) / 64 * 64))
 
+// the coloured solver on several CUs (shp_colored.hip): worlds above
+// FLOW_MIN_BODIES, up to one workgroup per FLOW_GROUP_BODIES bodies and
+// FLOW_MAX_GROUPS workgroups in all, at least one per FLOW_GROUP_MAX bodies;
+// bodies of up to FLOW_DEGREE manifolds, as many colours; control words per
+// world (FC_*, FS_*)
+enum { FLOW_MIN_BODIES = 2048, FLOW_GROUP_BODIES = 64, FLOW_GROUP_MAX = 384,
+       FLOW_MAX_GROUPS = 256, FLOW_DEGREE = 32, FLOW_CTL = 32, FLOW_LINE = 16 };
+enum { FC_SEATS = 0, FC_GROUPS = 1, FC_DONE = 2, FC_BAD = 3, FS_SEATS = 4, FS_GROUPS = 5,
+       FS_ABORT = 6, FS_ALONE = 7, FC_ROWS = 8, FC_SHARE = 9 };
+// col_info: colours | serial tail << 16 | flow schedule << 17 (then the pairs'
+// slots come from flow_slot, and sched_order is written by the packing pass)
+enum { COL_TAIL = 1 << 16, COL_FLOW = 1 << 17 };
+
 // pair_ab words (coloured solver): world-local body ids a | b << 16, NO_BODY
 // for a static body, NO_PAIR for a pair without contacts
 #define NO_BODY 0xFFFFu
@@ -77,7 +90,8 @@ enum {
   SHP_FLAG_PAIR_OVERFLOW = 1,
   SHP_FLAG_CONTACT_OVERFLOW = 2,
   SHP_FLAG_NONFINITE = 4,
-  SHP_FLAG_SCHEDULE_OVERFLOW = 8
+  SHP_FLAG_SCHEDULE_OVERFLOW = 8,
+  SHP_FLAG_STALL = 16  // a wait between workgroups ran out (never in a correct run)
 };
 
 struct Ctx {
@@ -143,7 +157,17 @@ struct Ctx {
   uint2* col_list;     // 2 x pair_cap: uncoloured manifolds, pair index and body word
   uint32_t* pair_ab;             // per pair: world-local bodies for the colouring (k_sat)
   int32_t* col_off;   // per world: COLOR_CAP + 3 colour offsets (manifolds)
-  int32_t* col_info;  // per world: colours | serial tail << 16 (0: nothing to solve)
+  int32_t* col_info;  // per world: colours, COL_* flags (0: nothing to solve)
+  // worlds solved on several CUs: how many (the largest), the workgroups of
+  // the largest; control words per world; per body its manifolds' pairs and
+  // their number, the colouring's word and the velocity words (2 x NB); per
+  // pair its colour and place in it; per workgroup its manifolds by colour
+  int flow_worlds, flow_groups;
+  int32_t* flow_ctl;
+  uint32_t* adj;
+  int32_t* adj_n;
+  unsigned long long *flow_col, *flow_vel;
+  int32_t *flow_slot, *flow_cnt;
   // solver sub-phase timestamps of world 0 (wall_clock64), timing mode only
   unsigned long long* tstamp;
   unsigned long long* tstamp_store;
@@ -213,6 +237,9 @@ struct StepPlan {
   // coloured solver: lanes per world, dynamic LDS of the colouring, LDS pool
   int color_threads = 256;
   size_t color_lds = 0, color_pool = 0;
+  // the flow_worlds largest worlds are coloured and swept by up to
+  // flow_groups workgroups each
+  int flow_worlds = 0, flow_groups = 0;
   // the contact kernel writes the manifold records itself, after the
   // colouring, instead of beside it with a packing pass after both
   bool records_in_contacts = false;
@@ -314,7 +341,9 @@ shp_status solver_alloc(shp_batch* b);
 shp_status colored_alloc(shp_batch* b);
 // plan values of the solvers (lanes, LDS) from the largest world
 void plan_ordered_solver(StepPlan* P, int solver_threads);
-void plan_colored_solver(StepPlan* P, int solver_threads);
+// (order: worlds by descending size)
+void plan_colored_solver(StepPlan* P, int solver_threads, const std::vector<int32_t>& body_off,
+                         const std::vector<int32_t>& order);
 void launch_colored_pack(shp_batch* b);
 // static LDS of the solver kernels at `threads` lanes
 size_t ordered_static_lds(int threads);

@@ -75,6 +75,13 @@ __global__ void k_reset(Ctx c) {
   if (g < 8) c.counters[g] = 0;
   if (g < 3) c.quality[g] = 0ull;
   if (c.use_grid && g <= c.grid_buckets) c.bucket_cnt[g] = 0;
+  if (c.flow_worlds) {
+    if (g < (long)c.W * FLOW_CTL) c.flow_ctl[g] = 0;
+    if (g < c.NB) {
+      c.adj_n[g] = 0;
+      c.flow_col[FLOW_LINE * g] = 0ull;
+    }
+  }
 }
 
 // listToHull in local space (ConvexHull.hs:151-167): unit edge normals and
@@ -429,6 +436,15 @@ __device__ __forceinline__ void sat_pair(const Ctx& c, int p) {
       const uint32_t a = c.is_static[ga] ? NO_BODY : (uint32_t)(ga - b0) & 0xFFFFu;
       const uint32_t b = c.is_static[gb] ? NO_BODY : (uint32_t)(gb - b0) & 0xFFFFu;
       v = a | (b << 16);
+      const int w = c.body_world[ga];
+      if (c.flow_worlds && c.body_off[w + 1] - b0 > FLOW_MIN_BODIES) {
+        // the bodies' lists of manifolds
+        const int ia = a != NO_BODY ? atomicAdd(&c.adj_n[ga], 1) : 0;
+        const int ib = b != NO_BODY ? atomicAdd(&c.adj_n[gb], 1) : 0;
+        if (a != NO_BODY && ia < FLOW_DEGREE) c.adj[(long)ga * FLOW_DEGREE + ia] = (uint32_t)p;
+        if (b != NO_BODY && ib < FLOW_DEGREE) c.adj[(long)gb * FLOW_DEGREE + ib] = (uint32_t)p;
+        if (max(ia, ib) >= FLOW_DEGREE) c.flow_ctl[w * FLOW_CTL + FC_BAD] = 1;
+      }
     }
     c.pair_ab[p] = v;
   }
@@ -617,11 +633,11 @@ __device__ void contacts_of_pair(const Ctx& c, int p, int n, int& hits) {
   }
   if (M >= 0) {  // the manifold's words, from its first contact as stored above
     if (k0 >= c.contact_cap) {
-      write_null_record(P, M, ga, gb);
+      write_null_record(P, M, ga, gb, 0);
     } else {
       const int nk = n < c.contact_cap - k0 ? n : c.contact_cap - k0;
       const int warm = (c.warm[k0] ? 1 : 0) | (nk > 1 && c.warm[k0 + 1] ? 2 : 0);
-      write_record_head(c, P, M, ga, gb, row_normal(c, k0), im[0], im[3], nk, warm);
+      write_record_head(c, P, M, ga, gb, row_normal(c, k0), im[0], im[3], nk, warm, 0);
     }
   }
 }
@@ -1230,6 +1246,15 @@ static void batch_buffers(const StepPlan& P, Ctx& c, int32_t** scan_part, std::v
     add(&c.col_off, W * (COLOR_CAP + 3) * 4);
     add(&c.col_info, W * 4);
     add(&c.pair_ab, PC * 4);
+    if (P.flow_worlds > 0) {
+      add(&c.flow_ctl, W * FLOW_CTL * 4);
+      add(&c.adj, NB * FLOW_DEGREE * 4);
+      add(&c.adj_n, NB * 4);
+      add(&c.flow_col, NB * FLOW_LINE * 8);
+      add(&c.flow_vel, NB * FLOW_LINE * 8);
+      add(&c.flow_slot, PC * 4);
+      add(&c.flow_cnt, (size_t)P.flow_worlds * P.flow_groups * FLOW_DEGREE * 4);
+    }
   }
 }
 
@@ -1421,7 +1446,7 @@ shp_status plan_staged(const shp_config& cfg, HostBatch* hb) {
   if (cfg.solver == SHP_SOLVER_ORDERED_F64)
     plan_ordered_solver(&P, cfg.solver_threads);
   else
-    plan_colored_solver(&P, cfg.solver_threads);
+    plan_colored_solver(&P, cfg.solver_threads, body_off, hb->order);
   P.sweep_big = n_worlds;
   if (cfg.solver == SHP_SOLVER_COLORED_F32 && cfg.solver_threads == 64) {
     // worlds by descending size: the small ones form the tail of the order
@@ -1439,7 +1464,9 @@ shp_status plan_staged(const shp_config& cfg, HostBatch* hb) {
   }
 
   const long PC = P.pair_cap, CC = P.contact_cap;
-  P.g_reset = blocks(std::max<long>(64, P.use_grid ? P.grid_buckets + 1 : 0), 256);
+  P.g_reset = blocks(std::max({64L, P.use_grid ? P.grid_buckets + 1 : 0L,
+                               P.flow_worlds ? std::max(NB, (long)FLOW_CTL * n_worlds) : 0L}),
+                     256);
   P.g_bodies = blocks(NB, 256);
   P.g_pairs = P.grid_wide ? blocks(NB * 16, 256) : blocks(NB, 256);
   P.g_pairs_count = P.grid_wide ? P.g_pairs : blocks(NB * 4, 256);
@@ -1483,7 +1510,9 @@ void plan_launches(const StepPlan& P, bool infer, bool logging, std::vector<Laun
     add("k_broadphase", P.g_broadphase, 256, 0, 0);
   add("k_sat", P.g_sat, 256, 0, 0);
   const bool col = P.solver == SHP_SOLVER_COLORED_F32;
-  if (col) add("k_colour", P.W, P.color_threads >= 512 ? 1024 : 256, P.color_lds,
+  // workgroups beyond one to a world
+  const long flow_extra = (long)P.flow_worlds * (P.flow_groups - 1);
+  if (col) add("k_colour", P.W + flow_extra, P.color_threads >= 512 ? 1024 : 256, P.color_lds,
                colored_static_lds(false));
   scan_launches(P.scan_pairs, "scan_pairs", out);
   add("k_world_ranges", P.g_ranges, 256, 0, 0);
@@ -1492,7 +1521,7 @@ void plan_launches(const StepPlan& P, bool infer, bool logging, std::vector<Laun
   if (col) {
     if (!P.records_in_contacts) add("k_pack_manifolds", P.g_pack, 256, 0, 0);
     if (P.sweep_big > 0)
-      add("k_sweep_colours", P.sweep_big, P.color_threads, P.color_pool, colored_static_lds(true));
+      add("k_sweep_colours", P.sweep_big + flow_extra, P.color_threads, P.color_pool, colored_static_lds(true));
     if (P.g_sweep_waves > 0)
       add("k_sweep_waves", P.g_sweep_waves, 64 * SWEEP_WAVES,
           (size_t)SWEEP_WAVES * P.sweep_slice * 4, 0);
@@ -1673,6 +1702,8 @@ shp_status batch_alloc(shp_batch* b, const HostBatch& hb) {
   c.warm_mode = b->cfg.warm_start;
   c.use_grid = P.use_grid ? 1 : 0;
   c.records_in_contacts = P.records_in_contacts ? 1 : 0;
+  c.flow_worlds = P.flow_worlds;
+  c.flow_groups = P.flow_groups;
   c.grid_buckets = (int)P.grid_buckets;
   c.host_flags = (int32_t*)b->stage;
   b->h_body_off = hb.body_off;
@@ -1739,6 +1770,7 @@ static shp_status check_flags(shp_batch* b) {
   b->last_flags |= flags;
   if (b->last_flags & (SHP_FLAG_PAIR_OVERFLOW | SHP_FLAG_CONTACT_OVERFLOW))
     return fail(SHP_E_OVERFLOW, "pair/contact capacity exceeded; raise max_pairs_per_body");
+  if (b->last_flags & SHP_FLAG_STALL) return fail(SHP_E_HIP, "a wait between workgroups ran out");
   if (b->last_flags & SHP_FLAG_NONFINITE) return fail(SHP_E_NONFINITE, "non-finite body state");
   return SHP_OK;
 }

@@ -16,7 +16,8 @@ namespace shp {
 // rec[(M / RB) * 7 * RB + q * RB + M % RB] (blocks of RB manifolds)
 //   0  ux, uy, mu, e       the row normal (flip applied), materials
 //   1  ax, ay, bx, by      the normal times the inverse masses of a / b
-//   2  ga, gb, flags, 0    bodies (global ids), flags
+//   2  ga, gb, flags, turns  bodies (global ids), flags, and for a world
+//                          solved on several CUs the manifold's turns
 //   3  jn2, jn5, jt2, jt5  the first contact: angular entries of the
 //                          normal / friction rows
 //   4  bn, icn, ict, wn2   bias, reciprocal effective masses, angular
@@ -32,6 +33,17 @@ enum { REC_WORDS = 7, REC2_WORDS = 4 };
 constexpr int RB = 4;
 static_assert(16 * 64 * (REC_WORDS + REC2_WORDS) == 4 * COLOR_PACK_FLOATS(64),
               "record words differ from the buffer size");
+// a manifold's turn on a dynamic body: its place among the body's manifolds by
+// colour, and their number (0: a static body)
+struct Turns {
+  int at_a, of_a, at_b, of_b;
+};
+__host__ __device__ __forceinline__ int pack_turns(Turns t) {
+  return t.at_a | t.of_a << 8 | t.at_b << 16 | t.of_b << 24;
+}
+__host__ __device__ __forceinline__ Turns unpack_turns(int x) {
+  return Turns{x & 0xFF, (x >> 8) & 0xFF, (x >> 16) & 0xFF, (int)((unsigned)x >> 24)};
+}
 // manifold flags: 1 a static, 2 b static, 4 first contact warm, 8 second
 // contact present, 16 second contact warm
 enum { MFL_A_STATIC = 1, MFL_B_STATIC = 2, MFL_WARM0 = 4, MFL_TWO = 8, MFL_WARM1 = 16 };
@@ -86,7 +98,7 @@ __device__ __forceinline__ void write_record_lambda(const PackF& P, int M, int j
 // nk (1 or 2) stored contacts, bit j of `warm` set when contact j is warm.
 __device__ __forceinline__ void write_record_head(const Ctx& c, const PackF& P, int M, int ga,
                                                   int gb, d2 u, double ima, double imb, int nk,
-                                                  int warm) {
+                                                  int warm, int turns) {
   const int flags = (c.is_static[ga] ? MFL_A_STATIC : 0) | (c.is_static[gb] ? MFL_B_STATIC : 0) |
                     ((warm & 1) ? MFL_WARM0 : 0) | (nk > 1 ? MFL_TWO : 0) |
                     (nk > 1 && (warm & 2) ? MFL_WARM1 : 0);
@@ -95,17 +107,18 @@ __device__ __forceinline__ void write_record_head(const Ctx& c, const PackF& P, 
                      (float)hs_min(c.e[ga], c.e[gb]));
   r[RB] = make_float4((float)(ima * u.x), (float)(ima * u.y), (float)(imb * u.x),
                       (float)(imb * u.y));
-  *(int4*)(r + 2 * RB) = make_int4(ga, gb, flags, 0);
+  *(int4*)(r + 2 * RB) = make_int4(ga, gb, flags, turns);
 }
 
 // A manifold whose contacts lie beyond the contact capacity (the step then
 // reports the overflow): a record that touches no velocity and no contact.
-__device__ __forceinline__ void write_null_record(const PackF& P, int M, int ga, int gb) {
+__device__ __forceinline__ void write_null_record(const PackF& P, int M, int ga, int gb,
+                                                  int turns) {
   float4* r = rec_of(P.rec, M);
   const float4 z = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
   r[0] = z;
   r[RB] = z;
-  *(int4*)(r + 2 * RB) = make_int4(ga, gb, MFL_A_STATIC | MFL_B_STATIC, 0);
+  *(int4*)(r + 2 * RB) = make_int4(ga, gb, MFL_A_STATIC | MFL_B_STATIC, turns);
   r[3 * RB] = z;
   r[4 * RB] = z;
   r[5 * RB] = z;
