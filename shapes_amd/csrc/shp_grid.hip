@@ -31,21 +31,14 @@ __device__ __forceinline__ int cell_of(double x, double h) {
   return (int)q;
 }
 
-// Bucket of cell (cx, cy): the low 16 bits of each coordinate interleaved
-// (Morton order), masked to the world's table.  Nearby cells land in
-// nearby buckets, so a body's 3x3 neighbourhood reads a few cache lines of
-// the table; cells that alias share a bucket and are told apart by their
-// stored cell coordinates.
-__device__ __forceinline__ uint32_t spread_bits(uint32_t x) {
-  x &= 0xFFFFu;
-  x = (x | (x << 8)) & 0x00FF00FFu;
-  x = (x | (x << 4)) & 0x0F0F0F0Fu;
-  x = (x | (x << 2)) & 0x33333333u;
-  x = (x | (x << 1)) & 0x55555555u;
-  return x;
-}
+// Bucket of cell (cx, cy): a row's cells are consecutive buckets, rows lie
+// spread over the world's table (a golden-ratio step), so the 3 cells of a
+// row that hold a body's partners are one run of records, and bodies in
+// bucket order walk the same runs; cells that alias share a bucket and are
+// told apart by their stored cell coordinates.
 __device__ __forceinline__ uint32_t cell_hash(int cx, int cy, uint32_t mask) {
-  return (spread_bits((uint32_t)cx) | (spread_bits((uint32_t)cy) << 1)) & mask;
+  const uint32_t step = (uint32_t)(((uint64_t)mask * 40503u) >> 16) | 1u;
+  return ((uint32_t)cx + (uint32_t)cy * step) & mask;
 }
 
 __device__ __forceinline__ bool aabb_hit(const Ctx& c, double aminx, double amaxx, double aminy,
@@ -59,7 +52,12 @@ __device__ __forceinline__ bool aabb_hit(const Ctx& c, double aminx, double amax
 // (World.delete) get neither
 __global__ void k_grid_assign(Ctx c) {
   int g = blockIdx.x * blockDim.x + threadIdx.x;
-  if (g >= c.NB || c.dead[g]) return;
+  if (g >= c.NB) return;
+  if (c.dead[g]) {
+    const int w = c.body_world[g];
+    c.cnt_rank[c.body_off[w + 1] - 1 - (g - c.body_off[w])] = 0;
+    return;
+  }
   if (c.iml[g] != 0.0 && !c.probe) {
     c.vx[g] = c.vx[g] + c.gx * c.dt;
     c.vy[g] = c.vy[g] + c.gy * c.dt;
@@ -102,127 +100,164 @@ __global__ void k_grid_fill(Ctx c) {
   *(int4*)(p + 2) = make_int4(cx, cy, g, c.is_static[g] != 0);
 }
 
-// LANES lanes per body i (1, 4 or 16): count (fill = 0) or emit (fill = 1)
-// its pairs.  With one lane (or four, which count only, splitting the
-// cells), the count pass also keeps the first GRID_SLOTS partners, and the
-// one-lane emit pass writes those without a second visit when they are
-// all.  With 16, a small body's lanes 0..8 take one cell each of the
-// <= 3x3 cells that can hold a partner's min corner and lanes 9..15 the
-// world's large bodies, and a large body's lanes stride over every j < i:
-// for batches too small to fill the GPU with one lane per body (the
-// candidates are dependent loads).  With 1 lane per body the lane does all
-// of it: for large batches, where the GPU is full anyway.  Each lane visits
-// its candidates twice when emitting with 16 lanes (count, then write at
-// the group's prefix sum), once with 1; lane 0 then sorts the segment into
-// descending j.
+// The body whose pairs are sought, its cell (that of its min corner).
+struct GridBody {
+  double minx, maxx, miny, maxy;
+  int g, cx, cy;
+  bool st, large;
+};
+
+// LANES lanes per body i (1, 4 or 16) visit every j < i of its world with
+// which it makes a pair.  A small body's partners have their min corner in at
+// most 3 rows of 3 cells, each row one run of records: 5 lanes to a row (16
+// lanes), or one (4), and the last lane the world's large bodies; one lane
+// does all of it.  A large body's lanes stride over every j < i.
 template <int LANES, class F>
-__device__ __forceinline__ void grid_visit(const Ctx& c, int g, int sl, F&& hit) {
-  constexpr int CELL_LANES = LANES < 9 ? LANES : 9;
-  if (c.dead[g]) return;  // an empty slot has no pairs; empty slots are not binned
+__device__ __forceinline__ void grid_visit(const Ctx& c, const GridBody& a, int sl, F&& hit) {
+  constexpr int ROW_LANES = LANES == 16 ? 5 : 1;
+  const int g = a.g;
   const int w = c.body_world[g];
   const int b0 = c.body_off[w];
-  const bool si = c.is_static[g] != 0;
-  const double aminx = c.bminx[g], amaxx = c.bmaxx[g], aminy = c.bminy[g], amaxy = c.bmaxy[g];
-  const double h = c.cell_h[w];
-  const int cx0 = cell_of(aminx, h) - 1, cx1 = cell_of(amaxx, h);
-  const int cy0 = cell_of(aminy, h) - 1, cy1 = cell_of(amaxy, h);
-  const long ncx = (long)cx1 - cx0 + 1, ncy = (long)cy1 - cy0 + 1;
+  const double h = c.cell_h[w], slack = 1e-6 * h;
   // A large body scans every j < i of its world.  So does a body whose AABB
-  // is not finite (a small body's finite AABB spans at most 3 x 3 candidate
-  // cells; a non-finite one would span up to 2^62 of them): the same
-  // bounded work as a large body, by all lanes.
-  const double span = (amaxx - aminx) + (amaxy - aminy);
-  if (c.is_large[g] || !(span - span == 0.0) || ncx > 3 || ncy > 3) {
+  // is not finite or, from rounding far out, wider than a cell (a small body's
+  // AABB spans at most 3 x 3 candidate cells; a non-finite one would span up
+  // to 2^62 of them): the same bounded work as a large body, by all lanes.
+  const double span = (a.maxx - a.minx) + (a.maxy - a.miny);
+  // does it reach n cells on? (within the rounding of x / h; a cell too many
+  // only costs its candidates' tests)
+  auto reaches = [&](double max, int cell, int n) { return max >= (double)(cell + n) * h - slack; };
+  if (a.large || !(span - span == 0.0) || reaches(a.maxx, a.cx, 2) || reaches(a.maxy, a.cy, 2)) {
     for (int gj = g - 1 - sl; gj >= b0; gj -= LANES)
-      if (!(si && c.is_static[gj]) && !c.dead[gj] && aabb_hit(c, aminx, amaxx, aminy, amaxy, gj))
+      if (!(a.st && c.is_static[gj]) && !c.dead[gj] &&
+          aabb_hit(c, a.minx, a.maxx, a.miny, a.maxy, gj))
         hit(gj);
     return;
   }
-  // the world's large bodies: lanes 9.. with 16 lanes, else the last lane
-  // (which also takes its share of the cells)
-  constexpr bool LARGE_LANES = LANES > CELL_LANES;
-  if (LARGE_LANES ? sl >= CELL_LANES : sl == LANES - 1) {
-    const int l0 = LARGE_LANES ? sl - CELL_LANES : 0, ls = LARGE_LANES ? LANES - CELL_LANES : 1;
-    for (int q = c.large_off[w] + l0; q < c.large_off[w + 1]; q += ls) {
+  const int cx0 = a.cx - 1, cx1 = a.cx + reaches(a.maxx, a.cx, 1);
+  const int cy0 = a.cy - 1, ncx = cx1 - cx0 + 1, ncy = 2 + reaches(a.maxy, a.cy, 1);
+  if (sl == LANES - 1) {
+    for (int q = c.large_off[w]; q < c.large_off[w + 1]; ++q) {
       const int gj = c.large_ids[q];
       if (gj >= g) break;  // ascending
-      if (!(si && c.is_static[gj]) && !c.dead[gj] && aabb_hit(c, aminx, amaxx, aminy, amaxy, gj))
+      if (!(a.st && c.is_static[gj]) && !c.dead[gj] &&
+          aabb_hit(c, a.minx, a.maxx, a.miny, a.maxy, gj))
         hit(gj);
     }
-    if (LARGE_LANES) return;
+    if (LANES > 1) return;
   }
   const int t0 = c.tab_off[w];
   const uint32_t mask = (uint32_t)(c.tab_off[w + 1] - t0 - 1);
-  for (long ci = sl; ci < ncx * ncy; ci += CELL_LANES) {
-    const int cx = (int)(cx0 + ci % ncx), cy = (int)(cy0 + ci / ncx);
-    const int b = t0 + cell_hash(cx, cy, mask);
-    for (int q = c.bucket_start[b]; q < c.bucket_start[b + 1]; ++q) {
-      const GridRec r = load_rec(c, q);
-      if (r.g >= g || r.cx != cx || r.cy != cy) continue;
-      if (!(si && r.st) && !(r.minx > amaxx || r.maxx < aminx) && !(r.miny > amaxy || r.maxy < aminy))
-        hit(r.g);
+  const int* at = c.bucket_start + t0;
+  for (int row = LANES == 1 ? 0 : sl / ROW_LANES; row < ncy; row += LANES == 1 ? 1 : 3) {
+    const int cy = cy0 + row;
+    const uint32_t first = cell_hash(cx0, cy, mask), last = first + (uint32_t)ncx - 1u;
+    int from = at[first], to = at[min(last, mask) + 1];
+    bool past = last > mask;  // the run goes on at the start of the world's table
+    for (;;) {
+      // four records' cells and indices in flight, then the boxes of those
+      // that are in the row and below the body
+      for (int q = from + sl % ROW_LANES; q < to; q += 4 * ROW_LANES) {
+        int4 m[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+          m[k] = *(const int4*)(c.grid_rec + 6L * min(q + k * ROW_LANES, to - 1) + 4);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          if (q + k * ROW_LANES >= to || m[k].z >= g || m[k].y != cy || m[k].x < cx0 || m[k].x > cx1)
+            continue;
+          const double2* p = (const double2*)(c.grid_rec + 6L * (q + k * ROW_LANES));
+          const double2 x = p[0], y = p[1];
+          if (!(a.st && m[k].w) && !(x.x > a.maxx || x.y < a.minx) &&
+              !(y.x > a.maxy || y.y < a.miny))
+            hit(m[k].z);
+        }
+      }
+      if (!past) break;
+      past = false;
+      from = at[0];
+      to = at[last - mask];
     }
   }
 }
 
+// The pairs' counts (fill = 0, 4 or 16 lanes per body) and the pairs (fill =
+// 1, 1 or 16 lanes).  The count pass takes the bodies in bucket order, in
+// which a wavefront's bodies walk the same few runs of records (in body order,
+// a cell to a lane or two and 2 bucket bounds to a cell, it took 307 us for
+// 1.14 M bodies, bound by its 8.8 M scattered loads; 172 now), then the large
+// bodies, and keeps each body's first GRID_SLOTS partners; the emit pass
+// writes those without a second visit when they are all, and in descending j
+// either way.
 template <int LANES>
 __global__ void k_grid_pairs(Ctx c, int fill) {
   const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  const int g = (int)(t / LANES);  // the same for the LANES lanes of a group
   const int sl = (int)(t % LANES);
+  int g = (int)(t / LANES);  // the same for the LANES lanes of a group
   if (g >= c.NB) return;
-  const int w = c.body_world[g];
-  const int b0 = c.body_off[w];
-  const int nw = c.body_off[w + 1] - b0;
-  const int rank = b0 + (nw - 1 - (g - b0));
-  int base = 0, pos = 0, total = 0;
-  int32_t* slots = c.grid_slots + (long)g * GRID_SLOTS;
-  if (LANES == 1 && !fill) {
-    int count = 0;
-    grid_visit<LANES>(c, g, sl, [&](int gj) {
-      if (count < GRID_SLOTS) slots[count] = gj;
-      ++count;
-    });
-    c.cnt_rank[rank] = count;
-    return;
-  }
-  if (LANES == 4) {  // count pass only: the cells split over 4 lanes
-    int count = 0, kept[GRID_SLOTS];
-    grid_visit<LANES>(c, g, sl, [&](int gj) {
+  auto rank_of = [&](int body) {
+    const int w = c.body_world[body];
+    return c.body_off[w + 1] - 1 - (body - c.body_off[w]);
+  };
+  auto body_of = [&](int body) {
+    const bool large = c.is_large[body];  // not binned: no cell
+    return GridBody{c.bminx[body], c.bmaxx[body], c.bminy[body], c.bmaxy[body], body,
+                    large ? 0 : c.body_cell[2 * body], large ? 0 : c.body_cell[2 * body + 1],
+                    c.is_static[body] != 0, large};
+  };
+  auto upto = [&](int n) {  // the sum over the group's lanes up to this one
+    for (int o = 1; o < LANES; o <<= 1) {
+      const int y = __shfl_up(n, o, LANES);
+      if (sl >= o) n += y;
+    }
+    return n;
+  };
+  if (!fill) {
+    if constexpr (LANES > 1) {
+      const int binned = c.bucket_start[c.grid_buckets];
+      GridBody a;
+      if (g < binned) {
+        const GridRec r = load_rec(c, g);
+        a = GridBody{r.minx, r.maxx, r.miny, r.maxy, r.g, r.cx, r.cy, r.st != 0, false};
+      } else {
+        if (g - binned >= c.large_off[c.W]) return;
+        g = c.large_ids[g - binned];
+        if (c.dead[g]) return;  // k_grid_assign counts none
+        a = body_of(g);
+      }
+      int count = 0, kept[GRID_SLOTS];
+      grid_visit<LANES>(c, a, sl, [&](int gj) {
+#pragma unroll
+        for (int k = 0; k < GRID_SLOTS; ++k)
+          if (k == count) kept[k] = gj;
+        ++count;
+      });
+      const int incl = upto(count), first = incl - count;
+      const int total = __shfl(incl, LANES - 1, LANES);
+      // the first GRID_SLOTS partners of the body, lane by lane
+      int32_t* slots = c.grid_slots + (long)a.g * GRID_SLOTS;
 #pragma unroll
       for (int k = 0; k < GRID_SLOTS; ++k)
-        if (k == count) kept[k] = gj;
-      ++count;
-    });
-    int incl = count;
-    for (int o = 1; o < LANES; o <<= 1) {
-      const int y = __shfl_up(incl, o, LANES);
-      if (sl >= o) incl += y;
+        if (k < count && first + k < GRID_SLOTS) slots[first + k] = kept[k];
+      if (sl == 0) c.cnt_rank[rank_of(a.g)] = total;
     }
-    const int total = __shfl(incl, LANES - 1, LANES);
-    // the first GRID_SLOTS partners of the body, lane by lane
-    const int first = incl - count;
-#pragma unroll
-    for (int k = 0; k < GRID_SLOTS; ++k)
-      if (k < count && first + k < GRID_SLOTS) slots[first + k] = kept[k];
-    if (sl == 0) c.cnt_rank[rank] = total;
     return;
   }
   // Past the capacity the step reports an overflow; the slots below it are
   // still all written (a segment that straddles the capacity keeps its
   // first pairs), so no later kernel of the step reads an unwritten slot.
-  if (LANES == 1) {
-    // one lane: the count pass sized the segment
-    base = c.off_rank[rank];
-    total = c.cnt_rank[rank];
-    if ((long)base + total > c.pair_cap) atomicOr(&c.counters[CNT_FLAGS], SHP_FLAG_PAIR_OVERFLOW);
-    if (base >= c.pair_cap) return;
-    total = min(total, c.pair_cap - base);
-    if (total <= GRID_SLOTS && c.cnt_rank[rank] <= GRID_SLOTS) {
-      // the kept partners, in descending order
+  const int rank = rank_of(g);
+  const int base = c.off_rank[rank], all = c.cnt_rank[rank];
+  if ((long)base + all > c.pair_cap && sl == 0)
+    atomicOr(&c.counters[CNT_FLAGS], SHP_FLAG_PAIR_OVERFLOW);
+  if (all == 0 || base >= c.pair_cap) return;  // the same for the group's lanes
+  const int total = min(all, c.pair_cap - base), end = base + total;
+  if (all <= GRID_SLOTS) {  // the kept partners, in descending order
+    const int32_t* slots = c.grid_slots + (long)g * GRID_SLOTS;
+    if constexpr (LANES == 1) {
       int v[GRID_SLOTS];
 #pragma unroll
-      for (int k = 0; k < GRID_SLOTS; ++k) v[k] = k < total ? slots[k] : -1;
+      for (int k = 0; k < GRID_SLOTS; ++k) v[k] = k < all ? slots[k] : -1;
 #pragma unroll
       for (int a = 1; a < GRID_SLOTS; ++a)
 #pragma unroll
@@ -238,53 +273,40 @@ __global__ void k_grid_pairs(Ctx c, int fill) {
           c.pa[base + k] = g;
           c.pb[base + k] = v[k];
         }
-      return;
-    }
-    pos = base;
-    const int end = base + total;
-    grid_visit<LANES>(c, g, sl, [&](int gj) {
-      if (pos < end) {
-        c.pa[pos] = g;
-        c.pb[pos] = gj;
+    } else {
+      const int v = sl < all ? slots[sl] : -1;
+      int at = 0;
+#pragma unroll
+      for (int k = 0; k < GRID_SLOTS; ++k) at += __shfl(v, k, LANES) > v ? 1 : 0;
+      if (sl < all && at < total) {
+        c.pa[base + at] = g;
+        c.pb[base + at] = v;
       }
-      ++pos;
-    });
-  } else {
-    int count = 0;
-    grid_visit<LANES>(c, g, sl, [&](int) { ++count; });
-    int incl = count;
-    for (int o = 1; o < LANES; o <<= 1) {
-      const int y = __shfl_up(incl, o, LANES);
-      if (sl >= o) incl += y;
     }
-    total = LANES == 1 ? incl : __shfl(incl, LANES - 1, LANES);
-    if (!fill) {
-      if (sl == 0) c.cnt_rank[rank] = total;
-      return;
-    }
-    base = c.off_rank[rank];
-    if ((long)base + total > c.pair_cap && sl == 0)
-      atomicOr(&c.counters[CNT_FLAGS], SHP_FLAG_PAIR_OVERFLOW);
-    if (base >= c.pair_cap) return;  // the same for the group's lanes
-    total = min(total, c.pair_cap - base);
-    const int end = base + total;
-    pos = base + incl - count;
-    grid_visit<LANES>(c, g, sl, [&](int gj) {
-      if (pos < end) {
-        c.pa[pos] = g;
-        c.pb[pos] = gj;
-      }
-      ++pos;
-    });
-    // the group's stores precede lane 0's sort in this wavefront's program
-    // order; the fence keeps the compiler from moving them
-    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    return;
   }
+  const GridBody a = body_of(g);
+  int pos = base;
+  if constexpr (LANES > 1) {
+    int count = 0;
+    grid_visit<LANES>(c, a, sl, [&](int) { ++count; });
+    pos += upto(count) - count;
+  }
+  grid_visit<LANES>(c, a, sl, [&](int gj) {
+    if (pos < end) {
+      c.pa[pos] = g;
+      c.pb[pos] = gj;
+    }
+    ++pos;
+  });
+  // the group's stores precede lane 0's sort in this wavefront's program
+  // order; the fence keeps the compiler from moving them
+  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
   if (sl != 0) return;
   // the segment in descending j (insertion sort; segments are short)
-  for (int a = base + 1; a < base + total; ++a) {
-    const int v = c.pb[a];
-    int q = a - 1;
+  for (int k = base + 1; k < end; ++k) {
+    const int v = c.pb[k];
+    int q = k - 1;
     while (q >= base && c.pb[q] < v) {
       c.pb[q + 1] = c.pb[q];
       --q;
