@@ -86,6 +86,8 @@ enum {
   Q_STEPS = 9,
   Q_ENTRIES = 10
 };
+// most workgroups whose results the step's last kernel adds up
+enum { MAX_PARTS = 4096 };
 enum {
   SHP_FLAG_PAIR_OVERFLOW = 1,
   SHP_FLAG_CONTACT_OVERFLOW = 2,
@@ -209,6 +211,10 @@ struct Ctx {
   int32_t* counters;  // 8 ints: flags, warm hits, learned starts, levels
   int32_t* host_flags;  // pinned host memory: the last step's flags
   unsigned long long* quality;  // Q_ENTRIES entries, see Q_*
+  // per workgroup of k_finish its quality maxima (3 x MAX_PARTS), of
+  // k_contacts its warm hits and manifolds (MAX_PARTS)
+  unsigned long long* part_q;
+  int2* part_n;
 };
 
 // ---- launch plan ----------------------------------------------------------

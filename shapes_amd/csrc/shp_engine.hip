@@ -119,30 +119,48 @@ __global__ void k_init_hulls(Ctx c) {
 // was emptied.  Without (placement at creation or after a mutation), every
 // slot is placed from its state, which for an empty slot reproduces the
 // shape it was left with.
-// A workgroup takes 256 consecutive bodies: one lane per body builds the
+// A workgroup takes 128 consecutive bodies: one lane per body builds the
 // transform, one lane per vertex transforms it into LDS, then one lane per
 // vertex writes the vertex, its edge's normal and the hull's extent along
 // that normal (coalesced), and one lane per body folds its AABB in vertex
-// order from LDS.
+// order from LDS.  The vertices load while the transforms are built, and half
+// the bodies of a workgroup's lanes take half the LDS, so that six workgroups
+// share a CU instead of three (1.14 M bodies with 1.95 M contacts: 297 us
+// before, 273 with this, 194 with the quality's maxima left to the next kernel).
 constexpr int INTEGRATE_THREADS = 256;
-constexpr int INTEGRATE_VERTS = INTEGRATE_THREADS * SHP_MAXV;
+constexpr int INTEGRATE_BODIES = 128;
+constexpr int INTEGRATE_VERTS = INTEGRATE_BODIES * SHP_MAXV;
 
-// The bodies [vb * INTEGRATE_THREADS, ...) of the batch (one workgroup).
+// The bodies [vb * INTEGRATE_BODIES, ...) of the batch (one workgroup).
 __device__ __forceinline__ void integrate_tile(const Ctx& c, int advance, int vb) {
-  __shared__ double s_m[6][INTEGRATE_THREADS];
+  __shared__ double s_m[6][INTEGRATE_BODIES];
   __shared__ double s_wx[INTEGRATE_VERTS], s_wy[INTEGRATE_VERTS];
   __shared__ uint8_t s_body[INTEGRATE_VERTS];
-  __shared__ int s_voff[INTEGRATE_THREADS + 1];
-  __shared__ uint8_t s_dead[INTEGRATE_THREADS];
+  __shared__ int s_voff[INTEGRATE_BODIES + 1];
+  __shared__ uint8_t s_dead[INTEGRATE_BODIES];
+  constexpr int ROUNDS = INTEGRATE_VERTS / INTEGRATE_THREADS;
   const int t = threadIdx.x;
-  const int g0 = vb * INTEGRATE_THREADS;
-  const int nbk = min(INTEGRATE_THREADS, c.NB - g0);
+  const int g0 = vb * INTEGRATE_BODIES;
+  const int nbk = min(INTEGRATE_BODIES, c.NB - g0);
   const int g = g0 + t;
   const double one = 1.0, zer = 0.0;
+  const int v0 = c.vert_off[g0], nv = c.vert_off[g0 + nbk] - v0;
+  double lx[ROUNDS], ly[ROUNDS];
+  int ex[ROUNDS];
+#pragma unroll
+  for (int k = 0; k < ROUNDS; ++k) {
+    const int i = t + k * INTEGRATE_THREADS;
+    if (i < nv) {
+      lx[k] = c.lx[v0 + i];
+      ly[k] = c.ly[v0 + i];
+      ex[k] = c.ext[v0 + i];
+    }
+  }
   if (t < nbk) {
     const bool dead = c.dead[g] != 0;
     s_dead[t] = dead && advance;
     double px = c.px[g], py = c.py[g], th = c.th[g];
+    const int o = c.vert_off[g] - v0, e = c.vert_off[g + 1] - v0;
     if (advance && !dead) {
       double dt = c.dt;
       px = (dt * c.vx[g]) + px;
@@ -160,36 +178,37 @@ __device__ __forceinline__ void integrate_tile(const Ctx& c, int advance, int vb
     s_m[3][t] = (zer * co + one * s) + py * zer;
     s_m[4][t] = (zer * (-s) + one * co) + py * zer;
     s_m[5][t] = (zer * zer + one * zer) + py * one;
-    s_voff[t] = c.vert_off[g];
-    if (t == nbk - 1) s_voff[nbk] = c.vert_off[g + 1];
+    s_voff[t] = o;
+    if (t == nbk - 1) s_voff[nbk] = e;
+    for (int i = o; i < e; ++i) s_body[i] = (uint8_t)t;
     double chk = px + py + th + c.vx[g] + c.vy[g] + c.w[g];
     if (!dead && !(chk - chk == 0.0)) atomicOr(&c.counters[CNT_FLAGS], SHP_FLAG_NONFINITE);
   }
   __syncthreads();
-  const int v0 = s_voff[0], nv = s_voff[nbk] - v0;
-  if (t < nbk)
-    for (int i = s_voff[t] - v0; i < s_voff[t + 1] - v0; ++i) s_body[i] = (uint8_t)t;
-  __syncthreads();
-  for (int i = t; i < nv; i += INTEGRATE_THREADS) {
+#pragma unroll
+  for (int k = 0; k < ROUNDS; ++k) {
+    const int i = t + k * INTEGRATE_THREADS;
+    if (i >= nv) continue;
     const int b = s_body[i];
     if (s_dead[b]) continue;
-    const double lx = c.lx[v0 + i], ly = c.ly[v0 + i];
-    s_wx[i] = (s_m[0][b] * lx + s_m[1][b] * ly) + s_m[2][b] * one;
-    s_wy[i] = (s_m[3][b] * lx + s_m[4][b] * ly) + s_m[5][b] * one;
+    s_wx[i] = (s_m[0][b] * lx[k] + s_m[1][b] * ly[k]) + s_m[2][b] * one;
+    s_wy[i] = (s_m[3][b] * lx[k] + s_m[4][b] * ly[k]) + s_m[5][b] * one;
   }
   __syncthreads();
   // From the world vertices in LDS: each edge's unit normal and the hull's
   // own extent along it (extentAlong, ConvexHull.hs:81-92, at the cached
   // extent vertices), the projections the SAT reads, once per step here.
-  for (int i = t; i < nv; i += INTEGRATE_THREADS) {
+#pragma unroll
+  for (int k = 0; k < ROUNDS; ++k) {
+    const int i = t + k * INTEGRATE_THREADS;
+    if (i >= nv) continue;
     const int b = s_body[i];
     if (s_dead[b]) continue;
-    const int ex = c.ext[v0 + i];
-    const int o = s_voff[b] - v0, last = s_voff[b + 1] - v0 - 1;
+    const int o = s_voff[b], last = s_voff[b + 1] - 1;
     const int i1 = i < last ? i + 1 : o;
     const double x = s_wx[i], y = s_wy[i];
     const d2 nn = normalize(clockwise(sub(mk(s_wx[i1], s_wy[i1]), mk(x, y))));
-    const int lo = o + (ex & 255), hi = o + (ex >> 8);
+    const int lo = o + (ex[k] & 255), hi = o + (ex[k] >> 8);
     // vertex and edge normal in one 32-byte record, the extent in 16 (coalesced)
     c.wv[v0 + i] = make_double4(x, y, nn.x, nn.y);
     c.wext[v0 + i] = make_double2(dot(mk(s_wx[lo], s_wy[lo]), nn), dot(mk(s_wx[hi], s_wy[hi]), nn));
@@ -208,7 +227,7 @@ __device__ __forceinline__ void integrate_tile(const Ctx& c, int advance, int vb
       c.bmaxy[g] = y + r;
       return;
     }
-    const int o = s_voff[t] - v0, e = s_voff[t + 1] - v0;
+    const int o = s_voff[t], e = s_voff[t + 1];
     if (e == o) return;  // no shape: a slot never filled since creation
     double bminx = s_wx[o], bmaxx = s_wx[o], bminy = s_wy[o], bmaxy = s_wy[o];
     for (int i = o + 1; i < e; ++i) {
@@ -229,7 +248,9 @@ __device__ __forceinline__ void integrate_tile(const Ctx& c, int advance, int vb
 // complementarity residual |min(lambda_n, Jn.v + b)| and friction residual
 // |lambda_t - clamp(lambda_t - Jt.v / mt, +-mu*lambda_n)|; maxima of the step
 // and of the run.  Non-negative doubles order like their bit patterns, so the
-// maxima are integer maxima, reduced per workgroup before one atomic each.
+// maxima are integer maxima, reduced per workgroup, and those by the next
+// kernel: six atomics from each of 2048 workgroups on one line held this one
+// for 50 us whatever its work (96 k bodies with 204 k contacts 63 us, 19 now).
 // Workgroup vb of nvb (grid-stride over the step's contacts).
 #define QUALITY_THREADS 256
 
@@ -272,7 +293,7 @@ __device__ __forceinline__ void quality_tile(const Ctx& c, int vb, int nvb) {
     qn = b > qn ? b : qn;
     qt = d > qt ? d : qt;
   }
-  // wavefront, then workgroup maxima: one set of atomics per workgroup
+  // wavefront, then workgroup maxima
   __shared__ unsigned long long s_q[3][QUALITY_THREADS / 64];
   const int wid = threadIdx.x >> 6;
   qd = wave_max_u64(qd);
@@ -284,20 +305,11 @@ __device__ __forceinline__ void quality_tile(const Ctx& c, int vb, int nvb) {
     s_q[2][wid] = qt;
   }
   __syncthreads();
-  if (threadIdx.x != 0) return;
-  for (int q = 1; q < QUALITY_THREADS / 64; ++q) {
-    qd = s_q[0][q] > qd ? s_q[0][q] : qd;
-    qn = s_q[1][q] > qn ? s_q[1][q] : qn;
-    qt = s_q[2][q] > qt ? s_q[2][q] : qt;
-  }
-  if (qd | qn | qt) {
-    atomicMax(&c.quality[Q_DEPTH], qd);
-    atomicMax(&c.quality[Q_NRES], qn);
-    atomicMax(&c.quality[Q_FRES], qt);
-    atomicMax(&c.quality[Q_RUN_DEPTH], qd);
-    atomicMax(&c.quality[Q_RUN_NRES], qn);
-    atomicMax(&c.quality[Q_RUN_FRES], qt);
-  }
+  if (threadIdx.x >= 3) return;
+  unsigned long long m = s_q[threadIdx.x][0];
+  for (int q = 1; q < QUALITY_THREADS / 64; ++q)
+    m = s_q[threadIdx.x][q] > m ? s_q[threadIdx.x][q] : m;
+  c.part_q[threadIdx.x * MAX_PARTS + vb] = m;
 }
 
 __global__ __launch_bounds__(INTEGRATE_THREADS) void k_integrate(Ctx c, int advance) {
@@ -477,7 +489,10 @@ __global__ void k_world_ranges(Ctx c) {
 // descending, finds exactly the element descZipVector (Utils/Descending.hs:
 // 47-71) would pair it with.  For the coloured solver, the pair's manifold
 // record too, at the slot the colouring gave it (none: no slot).
-__device__ void contacts_of_pair(const Ctx& c, int p, int n, int& hits) {
+// Contact k of the n of pair p, stored at dst (below the capacity); the
+// manifold's record rows when M >= 0 is its slot.  Returns whether it starts
+// warm.
+__device__ __forceinline__ bool contact_of_pair(const Ctx& c, int p, int k, int n, int dst, int M) {
   int ga = c.pa[p], gb = c.pb[p];
   int w = c.body_world[ga];
   int b0 = c.body_off[w];
@@ -485,178 +500,209 @@ __device__ void contacts_of_pair(const Ctx& c, int p, int n, int& hits) {
   double im[6] = {c.iml[ga], c.iml[ga], c.imr[ga], c.iml[gb], c.iml[gb], c.imr[gb]};
   int cache_lo = c.cache_woff[w], cache_hi = c.cache_woff[w + 1];
   int c_lo = c.wcont_off[w], c_hi = c.wcont_off[w + 1];
-  const int M = c.records_in_contacts ? c.sched_order[p] : -1;
-  const int k0 = c.coff[p];
   const PackF P = packf(c);
-  for (int k = 0; k < n; ++k) {
-    int dst = k0 + k;
-    if (dst >= c.contact_cap) continue;
-    int s = 2 * p + k;
-    int fa = c.s_feat[s] >> 8, fb = c.s_feat[s] & 255;
-    int flip = c.s_flip[s];
-    uint64_t key = pack_key(ga - b0, gb - b0, fa, fb);
-    d2 nn = mk(c.s_nx[s], c.s_ny[s]);
-    d2 pp = mk(c.s_px[s], c.s_py[s]);
-    double depth = c.s_depth[s];
-    c.key[dst] = key;
-    c.ga[dst] = ga;
-    c.gb[dst] = gb;
-    c.flip[dst] = (uint8_t)flip;
-    c.cnx[dst] = nn.x;
-    c.cny[dst] = nn.y;
-    c.cpx[dst] = pp.x;
-    c.cpy[dst] = pp.y;
-    c.depth[dst] = depth;
-    double jn[6], jt[6];
-    if (!flip) {
-      np_jacobian(nn, pp, xa, xb, jn);
-      f_jacobian(nn, pp, xa, xb, jt);
-    } else {  // flipMap + flipExtract: swapped pair, halves swapped back
-      double t[6];
-      np_jacobian(nn, pp, xb, xa, t);
-      for (int q = 0; q < 3; ++q) {
-        jn[q] = t[q + 3];
-        jn[q + 3] = t[q];
-      }
-      f_jacobian(nn, pp, xb, xa, t);
-      for (int q = 0; q < 3; ++q) {
-        jt[q] = t[q + 3];
-        jt[q + 3] = t[q];
-      }
+  int s = 2 * p + k;
+  int fa = c.s_feat[s] >> 8, fb = c.s_feat[s] & 255;
+  int flip = c.s_flip[s];
+  uint64_t key = pack_key(ga - b0, gb - b0, fa, fb);
+  d2 nn = mk(c.s_nx[s], c.s_ny[s]);
+  d2 pp = mk(c.s_px[s], c.s_py[s]);
+  double depth = c.s_depth[s];
+  c.key[dst] = key;
+  c.ga[dst] = ga;
+  c.gb[dst] = gb;
+  c.flip[dst] = (uint8_t)flip;
+  c.cnx[dst] = nn.x;
+  c.cny[dst] = nn.y;
+  c.cpx[dst] = pp.x;
+  c.cpy[dst] = pp.y;
+  c.depth[dst] = depth;
+  double jn[6], jt[6];
+  if (!flip) {
+    np_jacobian(nn, pp, xa, xb, jn);
+    f_jacobian(nn, pp, xa, xb, jt);
+  } else {  // flipMap + flipExtract: swapped pair, halves swapped back
+    double t[6];
+    np_jacobian(nn, pp, xb, xa, t);
+    for (int q = 0; q < 3; ++q) {
+      jn[q] = t[q + 3];
+      jn[q + 3] = t[q];
     }
-    // the other eight entries of the rows are +-n and +-cw(n), rebuilt
-    // exactly from the normal and flip (row_normal)
-    c.jx[dst] = make_double4(jn[2], jn[5], jt[2], jt[5]);
-    // baumgarte (NonPenetration.hs:48-56)
-    const double bn = depth > c.slop ? (c.beta / c.dt) * (c.slop - depth) : 0.0;
-    c.bn[dst] = bn;
-    // Restitution.constraintGen (Restitution.hs:21-31)
-    d2 ra = sub(pp, xa), rb = sub(pp, xb);
-    c.rax[dst] = ra.x;
-    c.ray[dst] = ra.y;
-    c.rbx[dst] = rb.x;
-    c.rby[dst] = rb.y;
-    const double mcn = eff_mass(jn, im), mct = eff_mass(jt, im);
-    c.mcn[dst] = mcn;
-    c.mct[dst] = mct;
-    if (M >= 0) write_record_rows(P, M, k, im[2], im[5], jn[2], jn[5], jt[2], jt[5], bn, mcn, mct);
-    if (c.solver == SHP_SOLVER_ORDERED_F64) {
-      if (k == 0) {
-        const bool two = n > 1 && dst + 1 < c.contact_cap;
-        write_flow_head(c, dst, ga, gb, b0, flip ? neg(nn) : nn, im, two);
-      } else {
-        c.sch_ab[dst] = make_int2(-1, -1);
-      }
-      write_flow_con(c, dst, jn[2], jn[5], jt[2], jt[5], bn, mcn, mct);
+    f_jacobian(nn, pp, xb, xa, t);
+    for (int q = 0; q < 3; ++q) {
+      jt[q] = t[q + 3];
+      jt[q + 3] = t[q];
     }
-    // warm start lookup in the descending cache segment [cache_lo,
-    // cache_hi): the first entry <= key, then equality.  This frame's
-    // contacts come in the same order and mostly persist, so the search
-    // starts at the contact's proportional position and gallops outwards.
-    int found = -1;
-    if (cache_hi > cache_lo) {
-      const int nc = cache_hi - cache_lo, nw = c_hi - c_lo;
-      int g = cache_lo + (int)((long)(dst - c_lo) * nc / (nw > 0 ? nw : 1));
-      g = g < cache_lo ? cache_lo : (g >= cache_hi ? cache_hi - 1 : g);
-      int L, R;  // the first entry <= key lies in [L, R] (R = cache_hi: none)
-      if (c.cache_key[g] > key) {
-        L = g + 1;
-        R = cache_hi;
-        for (int step = 1;; step <<= 1) {
-          const int t = g + step;
-          if (t >= cache_hi) break;
-          if (c.cache_key[t] <= key) {
-            R = t;
-            break;
-          }
-          L = t + 1;
-        }
-      } else {
-        L = cache_lo;
-        R = g;
-        for (int step = 1;; step <<= 1) {
-          const int t = g - step;
-          if (t < cache_lo) break;
-          if (c.cache_key[t] > key) {
-            L = t + 1;
-            break;
-          }
+  }
+  // the other eight entries of the rows are +-n and +-cw(n), rebuilt
+  // exactly from the normal and flip (row_normal)
+  c.jx[dst] = make_double4(jn[2], jn[5], jt[2], jt[5]);
+  // baumgarte (NonPenetration.hs:48-56)
+  const double bn = depth > c.slop ? (c.beta / c.dt) * (c.slop - depth) : 0.0;
+  c.bn[dst] = bn;
+  // Restitution.constraintGen (Restitution.hs:21-31)
+  d2 ra = sub(pp, xa), rb = sub(pp, xb);
+  c.rax[dst] = ra.x;
+  c.ray[dst] = ra.y;
+  c.rbx[dst] = rb.x;
+  c.rby[dst] = rb.y;
+  const double mcn = eff_mass(jn, im), mct = eff_mass(jt, im);
+  c.mcn[dst] = mcn;
+  c.mct[dst] = mct;
+  if (M >= 0) write_record_rows(P, M, k, im[2], im[5], jn[2], jn[5], jt[2], jt[5], bn, mcn, mct);
+  if (c.solver == SHP_SOLVER_ORDERED_F64) {
+    if (k == 0) {
+      const bool two = n > 1 && dst + 1 < c.contact_cap;
+      write_flow_head(c, dst, ga, gb, b0, flip ? neg(nn) : nn, im, two);
+    } else {
+      c.sch_ab[dst] = make_int2(-1, -1);
+    }
+    write_flow_con(c, dst, jn[2], jn[5], jt[2], jt[5], bn, mcn, mct);
+  }
+  // warm start lookup in the descending cache segment [cache_lo,
+  // cache_hi): the first entry <= key, then equality.  This frame's
+  // contacts come in the same order and mostly persist, so the search
+  // starts at the contact's proportional position and gallops outwards.
+  int found = -1;
+  if (cache_hi > cache_lo) {
+    const int nc = cache_hi - cache_lo, nw = c_hi - c_lo;
+    int g = cache_lo + (int)((long)(dst - c_lo) * nc / (nw > 0 ? nw : 1));
+    g = g < cache_lo ? cache_lo : (g >= cache_hi ? cache_hi - 1 : g);
+    int L, R;  // the first entry <= key lies in [L, R] (R = cache_hi: none)
+    if (c.cache_key[g] > key) {
+      L = g + 1;
+      R = cache_hi;
+      for (int step = 1;; step <<= 1) {
+        const int t = g + step;
+        if (t >= cache_hi) break;
+        if (c.cache_key[t] <= key) {
           R = t;
+          break;
         }
+        L = t + 1;
       }
-      while (L < R) {
-        const int mid = (L + R) >> 1;
-        if (c.cache_key[mid] > key) L = mid + 1;
-        else R = mid;
-      }
-      if (R < cache_hi && c.cache_key[R] == key) found = R;
-    }
-    double ln = 0.0, lt = 0.0;
-    if (found >= 0) {
-      ln = c.cache_ln[found];
-      lt = c.cache_lt[found];
-    }
-    if (M >= 0) write_record_lambda(P, M, k, ln, lt);
-    if (found >= 0) {
-      c.ln[dst] = ln;
-      c.lt[dst] = lt;
-      c.warm[dst] = 1;
-      ++hits;
     } else {
-      // newCache (Solvers/Contact.hs:91-99): zero start; the learned warm
-      // start may replace it before the solve (and patch the record)
-      c.ln[dst] = 0.0;
-      c.lt[dst] = 0.0;
-      c.warm[dst] = 0;
-      if (c.collect_misses) {
-        // one atomic per wavefront for the lanes that miss together
-        const unsigned long long act = __ballot(1);
-        const int lane = threadIdx.x & 63, leader = __ffsll((long long)act) - 1;
-        int base = 0;
-        if (lane == leader) base = atomicAdd(&c.counters[CNT_MISS], (int)__popcll(act));
-        const int slot = __shfl(base, leader) + (int)__popcll(act & ((1ull << lane) - 1ull));
-        if (slot < c.miss_cap) {
-          c.miss_idx[slot] = dst;
-          c.miss_rec[slot] = M >= 0 ? (M << 1) | k : -1;
+      L = cache_lo;
+      R = g;
+      for (int step = 1;; step <<= 1) {
+        const int t = g - step;
+        if (t < cache_lo) break;
+        if (c.cache_key[t] > key) {
+          L = t + 1;
+          break;
         }
-        // the features here only for the training log (which reads them
-        // after the solve); else the inference computes them from the
-        // stored contact, off this kernel's divergent path
-        if (slot < c.miss_cap && c.features_in_contacts) {
-          double v[6] = {c.vx[ga], c.vy[ga], c.w[ga], c.vx[gb], c.vy[gb], c.w[gb]};
-          double sgn = flip ? -1.0 : 1.0;
-          mlp_features(sgn * nn.x, sgn * nn.y, depth, v, ra.x, ra.y, rb.x, rb.y, c.iml[ga], c.iml[gb],
-                       c.imr[ga], c.imr[gb], (c.mu[ga] + c.mu[gb]) / 2.0, c.miss_feat + (size_t)slot * MLP_IN);
-        }
+        R = t;
+      }
+    }
+    while (L < R) {
+      const int mid = (L + R) >> 1;
+      if (c.cache_key[mid] > key) L = mid + 1;
+      else R = mid;
+    }
+    if (R < cache_hi && c.cache_key[R] == key) found = R;
+  }
+  double ln = 0.0, lt = 0.0;
+  if (found >= 0) {
+    ln = c.cache_ln[found];
+    lt = c.cache_lt[found];
+  }
+  if (M >= 0) write_record_lambda(P, M, k, ln, lt);
+  if (found >= 0) {
+    c.ln[dst] = ln;
+    c.lt[dst] = lt;
+    c.warm[dst] = 1;
+  } else {
+    // newCache (Solvers/Contact.hs:91-99): zero start; the learned warm
+    // start may replace it before the solve (and patch the record)
+    c.ln[dst] = 0.0;
+    c.lt[dst] = 0.0;
+    c.warm[dst] = 0;
+    if (c.collect_misses) {
+      // one atomic per wavefront for the lanes that miss together
+      const unsigned long long act = __ballot(1);
+      const int lane = threadIdx.x & 63, leader = __ffsll((long long)act) - 1;
+      int base = 0;
+      if (lane == leader) base = atomicAdd(&c.counters[CNT_MISS], (int)__popcll(act));
+      const int slot = __shfl(base, leader) + (int)__popcll(act & ((1ull << lane) - 1ull));
+      if (slot < c.miss_cap) {
+        c.miss_idx[slot] = dst;
+        c.miss_rec[slot] = M >= 0 ? (M << 1) | k : -1;
+      }
+      // the features here only for the training log (which reads them
+      // after the solve); else the inference computes them from the
+      // stored contact, off this kernel's divergent path
+      if (slot < c.miss_cap && c.features_in_contacts) {
+        double v[6] = {c.vx[ga], c.vy[ga], c.w[ga], c.vx[gb], c.vy[gb], c.w[gb]};
+        double sgn = flip ? -1.0 : 1.0;
+        mlp_features(sgn * nn.x, sgn * nn.y, depth, v, ra.x, ra.y, rb.x, rb.y, c.iml[ga], c.iml[gb],
+                     c.imr[ga], c.imr[gb], (c.mu[ga] + c.mu[gb]) / 2.0, c.miss_feat + (size_t)slot * MLP_IN);
       }
     }
   }
-  if (M >= 0) {  // the manifold's words, from its first contact as stored above
-    if (k0 >= c.contact_cap) {
-      write_null_record(P, M, ga, gb, 0);
-    } else {
-      const int nk = n < c.contact_cap - k0 ? n : c.contact_cap - k0;
-      const int warm = (c.warm[k0] ? 1 : 0) | (nk > 1 && c.warm[k0 + 1] ? 2 : 0);
-      write_record_head(c, P, M, ga, gb, row_normal(c, k0), im[0], im[3], nk, warm, 0);
-    }
-  }
+  return found >= 0;
 }
 
+// A lane to a contact: a workgroup takes CONTACT_PAIRS pairs, lists their
+// contacts in LDS and gives each lane one, so that neighbouring lanes store
+// neighbouring contacts.  (A lane to a pair, its contacts in turn, left a
+// third of the lanes idle for the first contact and 85% for the second, each
+// with all its loads and stores: 643 us for 2.5 M pairs with 1.95 M contacts,
+// bound by the CUs' address units; 476 with this, 385 with the workgroups'
+// counts added up by the step's last kernel instead of by two atomics each.)
+constexpr int CONTACT_PAIRS = 256;
+constexpr size_t CONTACTS_STATIC_LDS = lds16(4 * CONTACT_PAIRS) + lds16(CONTACT_PAIRS) +
+                                       lds16(2 * CONTACT_PAIRS) + lds16(CONTACT_PAIRS / 16) +
+                                       lds16(8);
 
-// 256-lane workgroups: 144 VGPRs and three waves per SIMD without spills
-// (the default bound of 1024 lanes held it to 128 with 20 bytes per lane in
-// scratch; a 1024-pile step 4.81 against 4.83 ms in this kernel)
-__global__ __launch_bounds__(256) void k_contacts(Ctx c) {
-  int tp = total_pairs(c);
+__global__ __launch_bounds__(CONTACT_PAIRS) void k_contacts(Ctx c) {
+  __shared__ uint16_t s_item[2 * CONTACT_PAIRS];  // pair of the tile << 1 | contact
+  __shared__ uint8_t s_n[CONTACT_PAIRS], s_warm[2 * CONTACT_PAIRS];
+  __shared__ int s_sum[CONTACT_PAIRS / 64];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tp = total_pairs(c);
+  const PackF P = packf(c);
   int hits = 0, mans = 0;
-  for (int p = blockIdx.x * blockDim.x + threadIdx.x; p < tp; p += gridDim.x * blockDim.x) {
-    int n = c.ccount[p];
-    if (n > 0) {
-      contacts_of_pair(c, p, n, hits);
-      mans += c.coff[p] < c.contact_cap;  // a manifold with stored contacts
+  for (long p0 = (long)blockIdx.x * CONTACT_PAIRS; p0 < tp; p0 += (long)gridDim.x * CONTACT_PAIRS) {
+    const int n = p0 + tid < tp ? c.ccount[p0 + tid] : 0;
+    // the pairs' places in the tile's list: lanes with one contact or two,
+    // lanes with two
+    const unsigned long long below = (1ull << lane) - 1ull;
+    const unsigned long long some = __ballot(n > 0), two = __ballot(n > 1);
+    if (lane == 0) s_sum[wave] = (int)(__popcll(some) + __popcll(two));
+    s_n[tid] = (uint8_t)n;
+    __syncthreads();
+    int at = (int)(__popcll(some & below) + __popcll(two & below)), all = 0;
+    for (int q = 0; q < CONTACT_PAIRS / 64; ++q) {
+      if (q < wave) at += s_sum[q];
+      all += s_sum[q];
+    }
+    for (int k = 0; k < n; ++k) s_item[at + k] = (uint16_t)(tid << 1 | k);
+    __syncthreads();
+    for (int i = tid; i < all; i += CONTACT_PAIRS) {
+      const int it = s_item[i], k = it & 1;
+      const int p = (int)p0 + (it >> 1), k0 = c.coff[p];
+      const bool stored = k0 + k < c.contact_cap;
+      const int M = c.records_in_contacts ? c.sched_order[p] : -1;
+      const bool warm = stored && contact_of_pair(c, p, k, s_n[it >> 1], k0 + k, M);
+      hits += warm;
+      mans += k == 0 && stored;  // a manifold with stored contacts
+      s_warm[i] = warm;
+    }
+    __syncthreads();
+    if (c.records_in_contacts && n > 0) {  // the manifold's words
+      const int p = (int)p0 + tid, M = c.sched_order[p];
+      const int ga = c.pa[p], gb = c.pb[p], left = c.contact_cap - c.coff[p];
+      if (M >= 0 && left <= 0) {
+        write_null_record(P, M, ga, gb, 0);
+      } else if (M >= 0) {
+        const int nk = min(n, left), warm = s_warm[at] | (nk > 1 ? s_warm[at + 1] << 1 : 0);
+        const d2 nn = mk(c.s_nx[2 * p], c.s_ny[2 * p]);
+        write_record_head(c, P, M, ga, gb, c.s_flip[2 * p] ? neg(nn) : nn, c.iml[ga], c.iml[gb], nk,
+                          warm, 0);
+      }
     }
   }
-  // one atomic per workgroup for the warm-start hit and manifold counters
+  // the workgroup's warm-start hits and manifolds
   __shared__ int s_cnt[2];
   if (threadIdx.x < 2) s_cnt[threadIdx.x] = 0;
   __syncthreads();
@@ -667,24 +713,74 @@ __global__ __launch_bounds__(256) void k_contacts(Ctx c) {
   if ((threadIdx.x & 63) == 0 && hits) atomicAdd(&s_cnt[0], hits);
   if ((threadIdx.x & 63) == 0 && mans) atomicAdd(&s_cnt[1], mans);
   __syncthreads();
-  if (threadIdx.x == 0 && s_cnt[0]) atomicAdd(&c.counters[CNT_WARM], s_cnt[0]);
-  if (threadIdx.x == 0 && s_cnt[1]) atomicAdd(&c.counters[CNT_MANIFOLDS], s_cnt[1]);
+  if (threadIdx.x != 0) return;
+  if (c.probe) {  // no kernel follows that adds up the workgroups' counts
+    if (s_cnt[0]) atomicAdd(&c.counters[CNT_WARM], s_cnt[0]);
+    if (s_cnt[1]) atomicAdd(&c.counters[CNT_MANIFOLDS], s_cnt[1]);
+  } else {
+    c.part_n[blockIdx.x] = make_int2(s_cnt[0], s_cnt[1]);
+  }
 }
 
 // This frame's lagrangians become the next frame's EngineCache
 // (Engine/Main.hs:32, wrapInitializer :61-69).
-__global__ void k_cache_store(Ctx c) {
-  // the step's quality maxima are final (k_finish ran before): add them to
-  // the run sums, whose means over the run are less sensitive to a single
-  // impact than the run maxima
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
-    for (int k = 0; k < 3; ++k) {
-      const double m = __longlong_as_double((long long)c.quality[Q_DEPTH + k]);
-      const double s = __longlong_as_double((long long)c.quality[Q_SUM_DEPTH + k]);
-      c.quality[Q_SUM_DEPTH + k] = (unsigned long long)__double_as_longlong(s + m);
+__global__ __launch_bounds__(256) void k_cache_store(Ctx c, int n_quality, int n_contacts) {
+  if (blockIdx.x == 0) {
+    // the step's quality maxima and contact counts from those of k_finish's and
+    // k_contacts' workgroups; the maxima also into the run's maxima and sums
+    // (whose means over the run are less sensitive to a single impact)
+    __shared__ unsigned long long s_max[3][4];
+    __shared__ int s_sum[2][4];
+    const int t = threadIdx.x;
+    unsigned long long m[3] = {0, 0, 0};
+    int n[2] = {0, 0};
+    // several loads in flight a lane (entries past the end: the last one again)
+    for (int i0 = t; i0 < n_quality; i0 += 4 * 256) {
+      unsigned long long x[4][3];
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int q = 0; q < 3; ++q)
+          x[u][q] = c.part_q[q * MAX_PARTS + min(i0 + u * 256, n_quality - 1)];
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int q = 0; q < 3; ++q) m[q] = x[u][q] > m[q] ? x[u][q] : m[q];
     }
-    c.quality[Q_STEPS] += 1;
-    *c.host_flags = c.counters[CNT_FLAGS];
+    for (int i0 = t; i0 < n_contacts; i0 += 8 * 256) {
+      int2 x[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) x[u] = c.part_n[min(i0 + u * 256, n_contacts - 1)];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        n[0] += i0 + u * 256 < n_contacts ? x[u].x : 0;
+        n[1] += i0 + u * 256 < n_contacts ? x[u].y : 0;
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < 3; ++q) m[q] = wave_max_u64(m[q]);
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+      for (int o = 32; o > 0; o >>= 1) n[q] += __shfl_xor(n[q], o);
+    if ((t & 63) == 0) {
+      for (int q = 0; q < 3; ++q) s_max[q][t >> 6] = m[q];
+      for (int q = 0; q < 2; ++q) s_sum[q][t >> 6] = n[q];
+    }
+    __syncthreads();
+    if (t < 3) {
+      unsigned long long x = s_max[t][0];
+      for (int q = 1; q < 4; ++q) x = s_max[t][q] > x ? s_max[t][q] : x;
+      c.quality[Q_DEPTH + t] = x;
+      if (x > c.quality[Q_RUN_DEPTH + t]) c.quality[Q_RUN_DEPTH + t] = x;
+      const double s = __longlong_as_double((long long)c.quality[Q_SUM_DEPTH + t]) +
+                       __longlong_as_double((long long)x);
+      c.quality[Q_SUM_DEPTH + t] = (unsigned long long)__double_as_longlong(s);
+    } else if (t == 3) {
+      c.counters[CNT_WARM] = (s_sum[0][0] + s_sum[0][1]) + (s_sum[0][2] + s_sum[0][3]);
+      c.counters[CNT_MANIFOLDS] = (s_sum[1][0] + s_sum[1][1]) + (s_sum[1][2] + s_sum[1][3]);
+      c.quality[Q_STEPS] += 1;
+      *c.host_flags = c.counters[CNT_FLAGS];
+    }
   }
   int stride = gridDim.x * blockDim.x;
   int tc = c.wcont_off[c.W];
@@ -1116,7 +1212,7 @@ static shp_status enqueue_step(shp_batch* b) {
   k_finish<<<P.g_finish_ni + P.g_finish_nq, INTEGRATE_THREADS, 0, s>>>(c, (int)P.g_finish_ni);
   mark(b, 13);
   // the run sums read the quality maxima
-  k_cache_store<<<P.g_cache, 256, 0, s>>>(c);
+  k_cache_store<<<P.g_cache, 256, 0, s>>>(c, (int)P.g_finish_nq, (int)P.g_contacts);
   mark(b, SHP_MAIN_PHASES);
   HIPCHK(hipGetLastError());
   return SHP_OK;
@@ -1150,8 +1246,8 @@ static shp_status accumulate_timing(shp_batch* b) {
 
 // static LDS of the engine's kernels (the __shared__ arrays they declare)
 constexpr size_t FINISH_STATIC_LDS =
-    lds16(6 * INTEGRATE_THREADS * 8) + 2 * lds16(INTEGRATE_VERTS * 8) + lds16(INTEGRATE_VERTS) +
-    lds16((INTEGRATE_THREADS + 1) * 4) + lds16(INTEGRATE_THREADS) +
+    lds16(6 * INTEGRATE_BODIES * 8) + 2 * lds16(INTEGRATE_VERTS * 8) + lds16(INTEGRATE_VERTS) +
+    lds16((INTEGRATE_BODIES + 1) * 4) + lds16(INTEGRATE_BODIES) +
     lds16(3 * (QUALITY_THREADS / 64) * 8);
 // 16 lanes per body in the grid's pair passes up to this many bodies
 #define GRID_WIDE_MAX_BODIES 131072
@@ -1213,6 +1309,8 @@ static void batch_buffers(const StepPlan& P, Ctx& c, int32_t** scan_part, std::v
   add(&c.log_count, 8);
   add(&c.counters, 8 * 4);
   add(&c.quality, Q_ENTRIES * 8);
+  add(&c.part_q, 3 * MAX_PARTS * 8);
+  add(&c.part_n, MAX_PARTS * 8);
   if (P.scan_parts_max > 0) add(scan_part, (size_t)P.scan_parts_max * 4);
   if (P.use_grid) {
     const size_t TB = P.grid_buckets;
@@ -1473,13 +1571,13 @@ shp_status plan_staged(const shp_config& cfg, HostBatch* hb) {
   P.g_broadphase = blocks(NB * 64, 256);
   P.g_sat = gs_blocks(PC);
   P.g_ranges = blocks(n_worlds + 1, 256);
-  P.g_contacts = gs_blocks(PC);
+  P.g_contacts = std::min<long>(gs_blocks(PC), MAX_PARTS);
   P.g_pack = gs_blocks(PC);
   P.g_infer = std::min<long>(std::max<long>(1, blocks(P.miss_cap, MLP_INFER_ROWS)), 512);
   P.g_unpack = std::max(1L, std::min(blocks(std::max(PC, NB), 256), 4096L));
   P.g_log = std::max<long>(1, blocks(P.miss_cap, 256));
-  P.g_finish_ni = blocks(NB, INTEGRATE_THREADS);
-  P.g_finish_nq = std::max(1L, std::min(blocks(CC, 256), 2048L));
+  P.g_finish_ni = blocks(NB, INTEGRATE_BODIES);
+  P.g_finish_nq = std::max(1L, std::min<long>(blocks(CC, 256), MAX_PARTS / 2));
   P.g_cache = gs_blocks(std::max<long>(CC, n_worlds + 1));
   P.device_bytes = footprint(P);
 
@@ -1516,7 +1614,7 @@ void plan_launches(const StepPlan& P, bool infer, bool logging, std::vector<Laun
                colored_static_lds(false));
   scan_launches(P.scan_pairs, "scan_pairs", out);
   add("k_world_ranges", P.g_ranges, 256, 0, 0);
-  add("k_contacts", P.g_contacts, 256, 0, lds16(4));
+  add("k_contacts", P.g_contacts, CONTACT_PAIRS, 0, CONTACTS_STATIC_LDS);
   if (infer) add("k_mlp_infer", P.g_infer, MLP_INFER_THREADS, 0, mlp_infer_static_lds());
   if (col) {
     if (!P.records_in_contacts) add("k_pack_manifolds", P.g_pack, 256, 0, 0);
@@ -1531,7 +1629,7 @@ void plan_launches(const StepPlan& P, bool infer, bool logging, std::vector<Laun
   }
   if (logging) add("k_mlp_log", P.g_log, 256, 0, 0);
   add("k_finish", P.g_finish_ni + P.g_finish_nq, INTEGRATE_THREADS, 0, FINISH_STATIC_LDS);
-  add("k_cache_store", P.g_cache, 256, 0, 0);
+  add("k_cache_store", P.g_cache, 256, 0, lds16(3 * 4 * 8) + lds16(2 * 4 * 4));
 }
 
 shp_status audit_plan(const StepPlan& P, const std::vector<LaunchRec>& L) {
@@ -1741,6 +1839,7 @@ shp_status batch_alloc(shp_batch* b, const HostBatch& hb) {
   }
   TRY(solver_alloc(b));
   TRY(check_static_lds((const void*)k_finish, FINISH_STATIC_LDS, "k_finish"));
+  TRY(check_static_lds((const void*)k_contacts, CONTACTS_STATIC_LDS, "k_contacts"));
 
   hipStream_t s = b->stream;
   k_fill_i32<<<1, 1, 0, s>>>(c.cnt_rank + NB, 0, 1);
@@ -1753,7 +1852,7 @@ shp_status batch_alloc(shp_batch* b, const HostBatch& hb) {
   // makeWorldObj places each shape with moveShape (World.hs:142-149)
   b->flags_on_device = true;
   k_init_hulls<<<blocks(NB, 256), 256, 0, s>>>(c);
-  k_integrate<<<blocks(NB, INTEGRATE_THREADS), INTEGRATE_THREADS, 0, s>>>(c, 0);
+  k_integrate<<<blocks(NB, INTEGRATE_BODIES), INTEGRATE_THREADS, 0, s>>>(c, 0);
   HIPCHK(hipGetLastError());
   HIPCHK(hipStreamSynchronize(s));
   return SHP_OK;
@@ -2252,7 +2351,7 @@ static shp_status write_slot_in_place(shp_batch* b, long g, const StagedBody& s)
   HIPCHK(hipMemcpy(c.dead + g, &zero, 1, hipMemcpyHostToDevice));
   b->flags_on_device = true;
   k_init_hulls<<<blocks(c.NB, 256), 256, 0, b->stream>>>(c);
-  k_integrate<<<blocks(c.NB, INTEGRATE_THREADS), INTEGRATE_THREADS, 0, b->stream>>>(c, 0);
+  k_integrate<<<blocks(c.NB, INTEGRATE_BODIES), INTEGRATE_THREADS, 0, b->stream>>>(c, 0);
   HIPCHK(hipGetLastError());
   HIPCHK(hipStreamSynchronize(b->stream));
   return SHP_OK;
