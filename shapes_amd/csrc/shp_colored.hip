@@ -42,6 +42,7 @@
 #include <algorithm>
 
 #include "shp_engine.h"
+#include "shp_flow.h"
 #include "shp_geom.h"
 #include "shp_records.h"
 #include "shp_solve_common.h"
@@ -197,22 +198,6 @@ struct VelF {
   }
 };
 
-// Agent-scope accesses of a single word, which other workgroups' wavefronts
-// read and write while this one runs.
-template <class X>
-__device__ __forceinline__ X peek(const X* p) {
-  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-template <class X>
-__device__ __forceinline__ void poke(X* p, X v) {
-  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-// Polls before a wait on another workgroup gives up and flags the step.  The
-// waits end by themselves: what one waits for is held by a wavefront that has
-// joined the world, so that it runs, and comes earlier in the schedule.
-constexpr int FLOW_POLLS = 1 << 20;
-
 // Velocities of a world swept by several workgroups: two words per body in
 // global memory, vx | omega's low half << 32 | turn << 48 and vy | omega's
 // high half << 32 | turn << 48, where `turn` counts the manifolds that have
@@ -229,8 +214,6 @@ constexpr int FLOW_POLLS = 1 << 20;
 // 0.70 and 0.86 us.  A body has a line of 128 bytes to itself: accesses to one
 // line from many CUs wait for each other (8192 polygons 114 us with 8 bodies to
 // a line, 96 with one; with the 16-byte accesses 88).
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-
 struct VelFlow {
   const Ctx* c;
   int* abort;
@@ -256,13 +239,7 @@ struct VelFlow {
                              *pb = c->flow_vel + FLOW_LINE * (long)m.gb;
     for (int n = 1;; ++n) {
       u32x4 x, y;
-      asm volatile(
-          "global_load_dwordx4 %0, %2, off sc1\n\t"
-          "global_load_dwordx4 %1, %3, off sc1\n\t"
-          "s_waitcnt vmcnt(0)"
-          : "=&v"(x), "=&v"(y)
-          : "v"(pa), "v"(pb)
-          : "memory");
+      load_pair(pa, pb, x, y);
       w[0] = x[0] | (unsigned long long)x[1] << 32;
       w[1] = x[2] | (unsigned long long)x[3] << 32;
       w[2] = y[0] | (unsigned long long)y[1] << 32;
@@ -292,10 +269,7 @@ struct VelFlow {
       unpack(old[0], old[1], y);
       pack(keep ? y : x, turn, n);
       const u32x4 x4 = {(uint32_t)n[0], (uint32_t)(n[0] >> 32), (uint32_t)n[1], (uint32_t)(n[1] >> 32)};
-      asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1"
-                   :
-                   : "v"(c->flow_vel + FLOW_LINE * (long)g), "v"(x4)
-                   : "memory");
+      store_16(c->flow_vel + FLOW_LINE * (long)g, x4);
     };
     if (t.of_a) hand_on(m.ga, w, v, !changed || (m.flags & MFL_A_STATIC));
     if (t.of_b) hand_on(m.gb, w + 2, v + 3, !changed || (m.flags & MFL_B_STATIC));
@@ -1135,51 +1109,6 @@ __device__ void colour_world(const Ctx& c, int w, int p0, int np, int pool_bytes
 }
 
 // ---- one world on several CUs ----------------------------------------------
-//
-// The workgroups that share a world wait for each other's results, so each of
-// them must be running.  They join by a counter; the first to come closes it
-// once all `want` have joined or after a bounded wait (on a GPU busy with
-// other streams some may not have started), and those that come later leave.
-// Returns the caller's seat and their number in *groups (-1: leave).  Seats
-// follow each other in space (pairs are in the order of their bodies), so
-// when all have come, those of an XCD, to which workgroups go in turn, are
-// consecutive: what neighbours exchange stays in its L2.
-constexpr int FLOW_JOIN_POLLS = 4096;  // about 0.5 ms
-enum { FLOW_CLOSED = 1 << 30 };
-
-constexpr int XCDS = 8;
-
-__device__ __forceinline__ int flow_join(int* seats, int* groups_word, int blk, int want, int* s_tmp,
-                                         int* groups) {
-  if (threadIdx.x == 0) {
-    constexpr int AGENT = __HIP_MEMORY_SCOPE_AGENT;
-    int s = __hip_atomic_fetch_add(seats, 1, __ATOMIC_RELAXED, AGENT), g = 0;
-    if (s & FLOW_CLOSED) {
-      s = -1;
-    } else if (s == 0) {
-      for (int n = 0; n < FLOW_JOIN_POLLS && peek(seats) < want; ++n) __builtin_amdgcn_s_sleep(1);
-      g = __hip_atomic_fetch_or(seats, FLOW_CLOSED, __ATOMIC_RELAXED, AGENT);
-      poke(groups_word, g);
-    } else {  // the first one runs and always writes it
-      for (int n = 0; n < FLOW_POLLS && (g = peek(groups_word)) == 0; ++n) __builtin_amdgcn_s_sleep(1);
-      if (g == 0) s = -1;
-    }
-    if (g == want) s = blk % XCDS * (want / XCDS) + min(blk % XCDS, want % XCDS) + blk / XCDS;
-    s_tmp[0] = s;
-    s_tmp[1] = g;
-  }
-  __syncthreads();
-  *groups = s_tmp[1];
-  const int seat = s_tmp[0];
-  __syncthreads();
-  return seat;
-}
-
-// Workgroups of world w, of at most `groups`.
-__device__ __forceinline__ int flow_want(const Ctx& c, int w, int groups) {
-  const int nb = c.body_off[w + 1] - c.body_off[w];
-  return min(groups, (nb + FLOW_GROUP_BODIES - 1) / FLOW_GROUP_BODIES);
-}
 
 // The rounds' colouring of a world without rounds, by several workgroups of T
 // lanes with FLOW_ITEMS / T pairs each.  In the rounds a manifold is coloured
@@ -1754,6 +1683,7 @@ void plan_colored_solver(StepPlan* P, int solver_threads, const std::vector<int3
     if (groups * FLOW_GROUP_MAX >= nb) {
       P->flow_worlds = big;
       P->flow_groups = (int)groups;
+      P->flow_min = FLOW_MIN_BODIES;
       P->color_lds = LDS_MAX_BYTES;
       P->color_pool = P->color_lds - fixed;
     }

@@ -38,6 +38,10 @@ constexpr size_t lds16(size_t bytes) { return (bytes + 15) & ~(size_t)15; }
 // contact, in blocks of 64 manifolds (PC manifolds)
 #define COLOR_PACK_FLOATS(PC) (44L * (((PC) + 63) / 64 * 64))
 
+// the ordered solver on several CUs (shp_solver.hip): worlds above
+// FLOW_ORDERED_MIN_BODIES, a workgroup per FLOW_ORDERED_PAIRS pairs, at most
+// FLOW_ORDERED_GROUPS workgroups in all
+enum { FLOW_ORDERED_MIN_BODIES = 3072, FLOW_ORDERED_PAIRS = 128, FLOW_ORDERED_GROUPS = 1024 };
 // the coloured solver on several CUs (shp_colored.hip): worlds above
 // FLOW_MIN_BODIES, up to one workgroup per FLOW_GROUP_BODIES bodies and
 // FLOW_MAX_GROUPS workgroups in all, at least one per FLOW_GROUP_MAX bodies;
@@ -164,7 +168,7 @@ struct Ctx {
   // the largest; control words per world; per body its manifolds' pairs and
   // their number, the colouring's word and the velocity words (2 x NB); per
   // pair its colour and place in it; per workgroup its manifolds by colour
-  int flow_worlds, flow_groups;
+  int flow_worlds, flow_groups, flow_min;
   int32_t* flow_ctl;
   uint32_t* adj;
   int32_t* adj_n;
@@ -243,9 +247,9 @@ struct StepPlan {
   // coloured solver: lanes per world, dynamic LDS of the colouring, LDS pool
   int color_threads = 256;
   size_t color_lds = 0, color_pool = 0;
-  // the flow_worlds largest worlds are coloured and swept by up to
+  // the flow_worlds largest worlds (above flow_min bodies) are solved by up to
   // flow_groups workgroups each
-  int flow_worlds = 0, flow_groups = 0;
+  int flow_worlds = 0, flow_groups = 0, flow_min = 0;
   // the contact kernel writes the manifold records itself, after the
   // colouring, instead of beside it with a packing pass after both
   bool records_in_contacts = false;
@@ -346,8 +350,9 @@ shp_status dalloc_bytes(shp_batch* b, void** p, size_t bytes);
 shp_status solver_alloc(shp_batch* b);
 shp_status colored_alloc(shp_batch* b);
 // plan values of the solvers (lanes, LDS) from the largest world
-void plan_ordered_solver(StepPlan* P, int solver_threads);
 // (order: worlds by descending size)
+void plan_ordered_solver(StepPlan* P, int solver_threads, const std::vector<int32_t>& body_off,
+                         const std::vector<int32_t>& order);
 void plan_colored_solver(StepPlan* P, int solver_threads, const std::vector<int32_t>& body_off,
                          const std::vector<int32_t>& order);
 void launch_colored_pack(shp_batch* b);

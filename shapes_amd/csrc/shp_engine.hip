@@ -43,6 +43,7 @@
 #include "shp_geom.h"
 #include "shp_trig.h"
 #include "shp_engine.h"
+#include "shp_flow.h"
 #include "shp_records.h"
 #include "shp_solve_common.h"
 
@@ -79,7 +80,7 @@ __global__ void k_reset(Ctx c) {
     if (g < (long)c.W * FLOW_CTL) c.flow_ctl[g] = 0;
     if (g < c.NB) {
       c.adj_n[g] = 0;
-      c.flow_col[FLOW_LINE * g] = 0ull;
+      if (c.flow_col) c.flow_col[FLOW_LINE * g] = 0ull;
     }
   }
 }
@@ -440,25 +441,22 @@ __device__ __forceinline__ void sat_pair(const Ctx& c, int p) {
     c.s_depth[s] = gm[k].depth;
   }
   c.ccount[p] = n;
+  if (c.solver != SHP_SOLVER_COLORED_F32 && c.flow_worlds == 0) return;
+  const int ga = c.pa[p], gb = c.pb[p];
+  const int w = c.body_world[ga], b0 = c.body_off[w];
+  const bool sa = c.is_static[ga] != 0, sb = c.is_static[gb] != 0;
   if (c.solver == SHP_SOLVER_COLORED_F32) {  // the pair's word for the colouring
-    const int ga = c.pa[p], gb = c.pb[p];
-    uint32_t v = NO_PAIR;
-    if (n > 0) {
-      const int b0 = c.body_off[c.body_world[ga]];
-      const uint32_t a = c.is_static[ga] ? NO_BODY : (uint32_t)(ga - b0) & 0xFFFFu;
-      const uint32_t b = c.is_static[gb] ? NO_BODY : (uint32_t)(gb - b0) & 0xFFFFu;
-      v = a | (b << 16);
-      const int w = c.body_world[ga];
-      if (c.flow_worlds && c.body_off[w + 1] - b0 > FLOW_MIN_BODIES) {
-        // the bodies' lists of manifolds
-        const int ia = a != NO_BODY ? atomicAdd(&c.adj_n[ga], 1) : 0;
-        const int ib = b != NO_BODY ? atomicAdd(&c.adj_n[gb], 1) : 0;
-        if (a != NO_BODY && ia < FLOW_DEGREE) c.adj[(long)ga * FLOW_DEGREE + ia] = (uint32_t)p;
-        if (b != NO_BODY && ib < FLOW_DEGREE) c.adj[(long)gb * FLOW_DEGREE + ib] = (uint32_t)p;
-        if (max(ia, ib) >= FLOW_DEGREE) c.flow_ctl[w * FLOW_CTL + FC_BAD] = 1;
-      }
-    }
-    c.pair_ab[p] = v;
+    const uint32_t a = sa ? NO_BODY : (uint32_t)(ga - b0) & 0xFFFFu;
+    const uint32_t b = sb ? NO_BODY : (uint32_t)(gb - b0) & 0xFFFFu;
+    c.pair_ab[p] = n > 0 ? a | (b << 16) : NO_PAIR;
+  }
+  if (n > 0 && c.flow_worlds && c.body_off[w + 1] - b0 > c.flow_min) {
+    // the dynamic bodies' lists of manifolds
+    const int ia = sa ? 0 : atomicAdd(&c.adj_n[ga], 1);
+    const int ib = sb ? 0 : atomicAdd(&c.adj_n[gb], 1);
+    if (!sa && ia < FLOW_DEGREE) c.adj[(long)ga * FLOW_DEGREE + ia] = (uint32_t)p;
+    if (!sb && ib < FLOW_DEGREE) c.adj[(long)gb * FLOW_DEGREE + ib] = (uint32_t)p;
+    if (max(ia, ib) >= FLOW_DEGREE) c.flow_ctl[w * FLOW_CTL + FC_BAD] = 1;
   }
 }
 
@@ -466,6 +464,15 @@ __device__ __forceinline__ void sat_pair(const Ctx& c, int p) {
 // at most 128 VGPRs, so that four waves per SIMD overlap their hull loads
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_sat(Ctx c) {
   int tp = total_pairs(c);
+  if (c.solver == SHP_SOLVER_ORDERED_F64 && c.flow_worlds)  // the bodies' first velocity words
+    for (int g = blockIdx.x * blockDim.x + threadIdx.x; g < c.NB; g += gridDim.x * blockDim.x) {
+      const double v[3] = {c.vx[g], c.vy[g], c.w[g]};
+      u32x4 x[2];
+      flow_pack(v, 0, x);
+      u32x4* to = (u32x4*)(c.flow_vel + FLOW_LINE * (long)g);
+      to[0] = x[0];
+      to[1] = x[1];
+    }
   for (int p = blockIdx.x * blockDim.x + threadIdx.x; p < tp; p += gridDim.x * blockDim.x) sat_pair(c, p);
 }
 
@@ -1345,14 +1352,16 @@ static void batch_buffers(const StepPlan& P, Ctx& c, int32_t** scan_part, std::v
     add(&c.col_info, W * 4);
     add(&c.pair_ab, PC * 4);
     if (P.flow_worlds > 0) {
-      add(&c.flow_ctl, W * FLOW_CTL * 4);
-      add(&c.adj, NB * FLOW_DEGREE * 4);
-      add(&c.adj_n, NB * 4);
       add(&c.flow_col, NB * FLOW_LINE * 8);
-      add(&c.flow_vel, NB * FLOW_LINE * 8);
       add(&c.flow_slot, PC * 4);
       add(&c.flow_cnt, (size_t)P.flow_worlds * P.flow_groups * FLOW_DEGREE * 4);
     }
+  }
+  if (P.flow_worlds > 0) {
+    add(&c.flow_ctl, W * FLOW_CTL * 4);
+    add(&c.adj, NB * FLOW_DEGREE * 4);
+    add(&c.adj_n, NB * 4);
+    add(&c.flow_vel, NB * FLOW_LINE * 8);
   }
 }
 
@@ -1542,7 +1551,7 @@ shp_status plan_staged(const shp_config& cfg, HostBatch* hb) {
   P.scan_parts_max =
       std::max({(long)P.scan_buckets.parts, (long)P.scan_bodies.parts, (long)P.scan_pairs.parts});
   if (cfg.solver == SHP_SOLVER_ORDERED_F64)
-    plan_ordered_solver(&P, cfg.solver_threads);
+    plan_ordered_solver(&P, cfg.solver_threads, body_off, hb->order);
   else
     plan_colored_solver(&P, cfg.solver_threads, body_off, hb->order);
   P.sweep_big = n_worlds;
@@ -1625,6 +1634,8 @@ void plan_launches(const StepPlan& P, bool infer, bool logging, std::vector<Laun
           (size_t)SWEEP_WAVES * P.sweep_slice * 4, 0);
     add("k_colour_unpack", P.g_unpack, 256, 0, 0);
   } else {
+    if (P.flow_worlds > 0)
+      add("k_solve_flow", (long)P.flow_worlds * P.flow_groups, 256, 0, lds16(2 * 4));
     add("k_solve_ordered", P.W, P.solve_threads, P.solve_lds, ordered_static_lds(P.solve_threads));
   }
   if (logging) add("k_mlp_log", P.g_log, 256, 0, 0);
@@ -1802,6 +1813,7 @@ shp_status batch_alloc(shp_batch* b, const HostBatch& hb) {
   c.records_in_contacts = P.records_in_contacts ? 1 : 0;
   c.flow_worlds = P.flow_worlds;
   c.flow_groups = P.flow_groups;
+  c.flow_min = P.flow_min;
   c.grid_buckets = (int)P.grid_buckets;
   c.host_flags = (int32_t*)b->stage;
   b->h_body_off = hb.body_off;

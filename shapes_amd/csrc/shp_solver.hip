@@ -38,6 +38,9 @@
 // The links and tokens are 16-bit LDS arrays when they fit (6 bytes a
 // contact), else 32-bit arrays in global memory: the same code.
 //
+// A large world with CUs to spare is solved by many workgroups instead, whose
+// items wait for their bodies rather than for a level (k_solve_flow).
+//
 // Measured (this kernel; before, items waited on per-body counters or ran
 // pass after pass): 55-box pyramid 72 us (159), 900 boxes 61 us (741), 512
 // worlds of 8-1024 bodies 183 us (752), 8192 polygons 1.48 ms (3.45; there
@@ -50,6 +53,7 @@
 #include <type_traits>
 
 #include "shp_engine.h"
+#include "shp_flow.h"
 #include "shp_geom.h"
 #include "shp_records.h"
 #include "shp_solve_common.h"
@@ -156,13 +160,15 @@ struct OState {
       ((double2*)(c->gvel + b0 + lb))[side] = side ? make_double2(v[2], 0.0) : make_double2(bx, by);
     }
   }
-  // this lane's lagrangian of contact k: the normal one in lane 1
-  __device__ __forceinline__ double load_lam(int k, int side) const {
+  // this lane's lagrangian of contact k + j: the normal one in lane 1
+  __device__ __forceinline__ double load_lam(int k, int j, int side) const {
+    k += j;
     if (LLDS) return lam[2 * k + 1 - side];
     const double2 l = c->glam[c0 + k];
     return side ? l.x : l.y;
   }
-  __device__ __forceinline__ void store_lam(int k, int side, double l) const {
+  __device__ __forceinline__ void store_lam(int k, int j, int side, double l) {
+    k += j;
     if (LLDS)
       lam[2 * k + 1 - side] = l;
     else
@@ -181,16 +187,16 @@ struct OState {
 // on: the even lane folds body a's three, the odd lane goes on with body
 // b's.  Without restitution the bounce term is min 0 (0 * x) = 0.
 // GENERAL: some lane of the wavefront is in pass 0 or has restitution.
-template <bool GENERAL, bool VLDS, bool LLDS>
-__device__ __forceinline__ void run_item(const ORec& r, int side, const OState<VLDS, LLDS>& S) {
+template <bool GENERAL, class State>
+__device__ __forceinline__ void run_item(const ORec& r, int side, State& S) {
   double v[3], lam[2];
   const int k = (int)(r.item & ~ITEM_WARM);
   const bool warm = GENERAL && (r.item & ITEM_WARM);
   const int id = orec_id(r, side), la = orec_id(r, 0) & FLOW_BODY, lb = orec_id(r, 1) & FLOW_BODY;
   const bool fixed = id < 0, two = (id & FLOW_TWO) != 0;  // FLOW_STATIC is the sign bit
   S.load(la, lb, side, v);
-  lam[0] = S.load_lam(k, side);
-  lam[1] = two ? S.load_lam(k + 1, side) : 0.0;
+  lam[0] = S.load_lam(k, 0, side);
+  lam[1] = two ? S.load_lam(k, 1, side) : 0.0;
   const int neg_a = side ? 0 : (int)0x80000000;
   const double sx = flip_sign(r.u.x, neg_a), sy = flip_sign(r.u.y, neg_a);
   const double iml = r.m.x, imr = r.m.y;
@@ -232,7 +238,7 @@ __device__ __forceinline__ void run_item(const ORec& r, int side, const OState<V
       app = l;
       apply = apply && ((r.warm >> (8 * j)) & 0xFF) != 0;
     }
-    S.store_lam(k + j, side, acc);
+    S.store_lam(k, j, side, acc);
     const double gn = from_b(app), gt = from_a(app);
     // applyLagrangian (Constraint.hs:182-221), normal first; a static side
     // keeps its velocity (the reference adds +-0 to it)
@@ -513,7 +519,7 @@ __device__ __forceinline__ void make_level(const Sched<L>& S, const Front<T, L>&
 // STEP items of a level at a time.
 template <int T, bool L, bool VLDS, bool LLDS>
 __device__ __forceinline__ void run_levels(const Ctx& c, const Sched<L>& Q,
-                                           const OState<VLDS, LLDS>& S, const Front<T, L>& fr) {
+                                           OState<VLDS, LLDS> S, const Front<T, L>& fr) {
   constexpr int NS = T / 256, NE = T / 64 - NS, STEP = NE * 32;
   static_assert(STEP <= Front<T, L>::CAP, "a level's first step reads its LDS slots");
   const int wave = threadIdx.x >> 6;
@@ -627,11 +633,11 @@ __device__ __forceinline__ void solve_world(const Ctx& c, const Sched<L>& Q, uns
   tmark(c, 2);
   tmark(c, 3);
   if (llds)
-    run_levels<T, L>(c, Q, OState<true, true>{vel, lam, &c, b0, c0}, fr);
+    run_levels<T, L, true, true>(c, Q, OState<true, true>{vel, lam, &c, b0, c0}, fr);
   else if (vlds)
-    run_levels<T, L>(c, Q, OState<true, false>{vel, lam, &c, b0, c0}, fr);
+    run_levels<T, L, true, false>(c, Q, OState<true, false>{vel, lam, &c, b0, c0}, fr);
   else
-    run_levels<T, L>(c, Q, OState<false, false>{vel, lam, &c, b0, c0}, fr);
+    run_levels<T, L, false, false>(c, Q, OState<false, false>{vel, lam, &c, b0, c0}, fr);
   __syncthreads();
   tmark(c, 4);
   for (int k = tid; k < n; k += T) {
@@ -661,6 +667,149 @@ __device__ __forceinline__ void solve_world(const Ctx& c, const Sched<L>& Q, uns
   tmark(c, 5);
 }
 
+// ---- one world on several CUs ----------------------------------------------
+//
+// Two lanes to a manifold for the whole solve, its record and lagrangians in
+// their registers, and no schedule: a lane of a manifold waits for the
+// manifold's turn on its body (flow_pack's words: pass * the body's manifolds +
+// the manifold's place among them in sequence order, from the lists k_sat
+// made), and the two run the item when both have it.  So the items run as in
+// the levels above, each as early as the latest earlier item on each of its
+// bodies allows, and a level costs a hand-over from CU to CU (about 1 us with
+// the item) whatever its width, where one CU runs the 600 items of a level of
+// an 8192-polygon pile in 7.5 us.  A lane that has seen its body several turns
+// away looks again only that many rounds later.  That pile, 8 iterations: 345
+// us, 1610 on one CU, and 2600 there once its schedule outgrew the LDS (from
+// about 19 k contacts).  Looking in every round 356; workgroups of 64 or 128
+// lanes instead of 256 the same.
+struct OFlow {
+  const Ctx* c;
+  int b0, c0;
+  u32x4 x, y;  // the body's words as loaded
+  double lam[2];
+  int g, last;  // the body; its last manifold's pass, else -1
+  int pass;
+  __device__ __forceinline__ void load(int, int, int, double* v) const {
+    flow_unpack(x, y, v);
+  }
+  __device__ __forceinline__ void store(int, int, int, bool fixed, const double* v) const {
+    if (fixed) return;
+    u32x4 n[2];
+    flow_pack(v, (x[1] >> 16) + 1u, n);
+    unsigned long long* to = c->flow_vel + FLOW_LINE * (long)g;
+    store_16(to, n[0]);
+    store_16(to + 2, n[1]);
+    if (pass == last) {
+      c->vx[g] = v[0];
+      c->vy[g] = v[1];
+      c->w[g] = v[2];
+    }
+  }
+  __device__ __forceinline__ double load_lam(int, int j, int) const { return lam[j]; }
+  __device__ __forceinline__ void store_lam(int, int j, int, double l) { lam[j] = l; }
+};
+
+__global__ __launch_bounds__(256) void k_solve_flow(Ctx c) {
+  __shared__ int s_tmp[2];
+  const int blk = blockIdx.x % c.flow_groups, w = c.world_order[blockIdx.x / c.flow_groups];
+  const int b0 = c.body_off[w];
+  const int p0 = c.wpair_off[w], np = c.wpair_off[w + 1] - p0;
+  int* ctl = c.flow_ctl + (long)w * FLOW_CTL;
+  const int want = (np + FLOW_ORDERED_PAIRS - 1) / FLOW_ORDERED_PAIRS;
+  if (np == 0) return;
+  // bodies of too many manifolds, too many pairs, or contacts beyond the
+  // capacity: k_solve_ordered
+  if (peek(ctl + FC_BAD) != 0 || want > c.flow_groups || c.coff[p0 + np] > c.contact_cap) {
+    if (blk == 0 && threadIdx.x == 0) ctl[FS_ALONE] = 1;
+    return;
+  }
+  if (blk >= want) return;
+  int groups;
+  const int seat = flow_join(ctl + FS_SEATS, ctl + FS_GROUPS, blk, want, s_tmp, &groups);
+  if (seat < 0) return;
+  if (groups < want) {
+    if (seat == 0 && threadIdx.x == 0) ctl[FS_ALONE] = 1;
+    return;
+  }
+  const int side = threadIdx.x & 1, q = seat * FLOW_ORDERED_PAIRS + ((int)threadIdx.x >> 1);
+  const int p = p0 + q, passes = c.iterations + 1;
+  ORec r;
+  OFlow S;
+  S.c = &c;
+  S.b0 = b0;
+  S.c0 = c.wcont_off[w];
+  S.pass = 0;
+  bool alive = q < np && c.ccount[p] > 0;
+  int k = 0, at = 0, of = 0, id = 0;
+  if (alive) {
+    k = c.coff[p] - S.c0;
+    load_orec(c, S.c0, (uint32_t)k, side, r);
+    id = orec_id(r, side);
+    S.g = b0 + (id & FLOW_BODY);
+    const double *ln = c.ln + S.c0 + k, *lt = c.lt + S.c0 + k;
+    S.lam[0] = side ? ln[0] : lt[0];
+    S.lam[1] = (id & FLOW_TWO) == 0 ? 0.0 : side ? ln[1] : lt[1];
+    if (id >= 0) {
+      of = c.adj_n[S.g];
+      const int4* row = (const int4*)(c.adj + (long)S.g * FLOW_DEGREE);
+      for (int e = 0; e < of; e += 4) {
+        const int4 x = row[e / 4];
+        at += x.x < p;
+        at += e + 1 < of && x.y < p;
+        at += e + 2 < of && x.z < p;
+        at += e + 3 < of && x.w < p;
+      }
+    } else {
+      const double v[3] = {c.vx[S.g], c.vy[S.g], c.w[S.g]};
+      u32x4 n[2];
+      flow_pack(v, 0, n);
+      S.x = n[0];
+      S.y = n[1];
+    }
+    S.last = at == of - 1 ? passes - 1 : -1;
+  }
+  const unsigned long long* word = c.flow_vel + FLOW_LINE * (long)(alive ? S.g : b0);
+  int rest = 0;
+  for (int polls = 1; __ballot(alive); ++polls) {
+    bool ready = alive && id < 0;
+    if (alive && id >= 0) {
+      if (rest > 0) {
+        --rest;
+      } else {
+        const uint32_t turn = (uint32_t)(S.pass * of + at) & 0xFFFFu;
+        load_pair(word, word + 2, S.x, S.y);
+        ready = S.x[1] >> 16 == turn && S.x[3] >> 16 == turn && S.y[1] >> 16 == turn &&
+                S.y[3] >> 16 == turn;
+        rest = ready ? 0 : min(((int)(turn - (S.x[1] >> 16)) & 0xFFFF) - 1, 7);
+      }
+    }
+    const int other = __builtin_amdgcn_mov_dpp((int)ready, 0xB1, 0xf, 0xf, true);
+    const bool run = ready && other;
+    r.item = (uint32_t)k | (S.pass == 0 ? ITEM_WARM : 0u);
+    if (__ballot(run)) {
+      if (__ballot(run && (S.pass == 0 || (id & FLOW_BOUNCE)))) {
+        if (run) run_item<true>(r, side, S);
+      } else {
+        if (run) run_item<false>(r, side, S);
+      }
+      if (run && ++S.pass == passes) {
+        alive = false;
+        double* l = (side ? c.ln : c.lt) + S.c0 + k;
+        l[0] = S.lam[0];
+        if (id & FLOW_TWO) l[1] = S.lam[1];
+      }
+      polls = 0;  // what remains to wait for has come nearer
+    }
+    if (polls % 256 == 255) {
+      if (polls >= FLOW_POLLS - 1) {
+        atomicOr(&c.counters[CNT_FLAGS], SHP_FLAG_STALL);
+        poke(ctl + FS_ABORT, 1);
+      }
+      if (peek(ctl + FS_ABORT) != 0) return;
+    }
+  }
+}
+
 template <int T>
 __global__ __launch_bounds__(T) void k_solve_ordered(Ctx c, int pool_bytes) {
   extern __shared__ __align__(16) unsigned char pool[];
@@ -671,6 +820,8 @@ __global__ __launch_bounds__(T) void k_solve_ordered(Ctx c, int pool_bytes) {
   const int tid = threadIdx.x;
   const int c0 = c.wcont_off[w], c1 = c.wcont_off[w + 1];
   if (c1 <= c0) return;
+  // solved by k_solve_flow?
+  if ((int)blockIdx.x < c.flow_worlds && c.flow_ctl[(long)w * FLOW_CTL + FS_ALONE] == 0) return;
   const int n = c1 - c0;
   const int b0 = c.body_off[w], nb = c.body_off[w + 1] - b0;
   tmark(c, 0);
@@ -709,10 +860,27 @@ size_t ordered_static_lds(int threads) {
 // as far as it goes.  4 waves per world; a world of more than
 // 512 bodies gets 8 (with 16, at 128 registers a lane, an 8192-polygon pile
 // took 1.93 ms instead of 1.64).
-void plan_ordered_solver(StepPlan* P, int solver_threads) {
+void plan_ordered_solver(StepPlan* P, int solver_threads, const std::vector<int32_t>& body_off,
+                         const std::vector<int32_t>& order) {
   P->solve_threads = solver_threads ? solver_threads : (P->max_nb > 512 ? 512 : 256);
   const size_t room = LDS_BYTES_PER_CU - ordered_static_lds(P->solve_threads) - 256;
   P->solve_lds = std::min<size_t>(room, 72UL * P->max_nb + 1024);
+  // Worlds on several CUs, while the lanes (two to a pair) fit the GPU at 110
+  // registers: us a step, 6 iterations, on several CUs against one: one world
+  // of 1024 bodies 327 / 246, 2048 412 / 333, 4096 527 / 681, 8192 653 / 1211,
+  // 16384 870 / 2751, 32768 1152 / 5004; 4 of 8192 754 / 1317.
+  int big = 0;
+  while (big < P->W && body_off[order[big] + 1] - body_off[order[big]] > FLOW_ORDERED_MIN_BODIES)
+    ++big;
+  if (big > 0) {
+    const long groups = std::min<long>((3 * P->max_nb + FLOW_ORDERED_PAIRS - 1) / FLOW_ORDERED_PAIRS,
+                                       FLOW_ORDERED_GROUPS / big);
+    if (groups * FLOW_ORDERED_PAIRS >= 2 * P->max_nb) {
+      P->flow_worlds = big;
+      P->flow_groups = (int)groups;
+      P->flow_min = FLOW_ORDERED_MIN_BODIES;
+    }
+  }
 }
 
 static const void* ordered_kernel(int threads) {
@@ -740,6 +908,8 @@ shp_status solver_alloc(shp_batch* b) {
 void launch_ordered_solver(shp_batch* b) {
   const StepPlan& P = b->plan;
   const Ctx& c = b->ctx;
+  if (P.flow_worlds > 0)
+    k_solve_flow<<<(unsigned)(P.flow_worlds * P.flow_groups), 256, 0, b->stream>>>(c);
   if (P.solve_threads == 512)
     k_solve_ordered<512><<<c.W, 512, P.solve_lds, b->stream>>>(c, (int)P.solve_lds);
   else
