@@ -42,7 +42,7 @@ typedef int32_t shp_status;
                                     FP64 impulse accumulators */
 
 /* Broadphase algorithms (same pair set and order) */
-#define SHP_BROADPHASE_AUTO 0 /* grid when a world has more than 2048 bodies */
+#define SHP_BROADPHASE_AUTO 0 /* grid for large worlds or many bodies in all */
 #define SHP_BROADPHASE_SCAN 1 /* one wavefront per body scans j < i */
 #define SHP_BROADPHASE_GRID 2 /* uniform grid + explicit large static bodies;
                                  16 lanes per body up to 131072 bodies, one

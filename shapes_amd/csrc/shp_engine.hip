@@ -1508,7 +1508,18 @@ shp_status plan_staged(const shp_config& cfg, HostBatch* hb) {
   // radius of its dynamic bodies; static bodies larger than a cell are
   // "large" and tested explicitly
   const int mode = cfg.broadphase;
-  P.use_grid = mode >= SHP_BROADPHASE_GRID || (mode == SHP_BROADPHASE_AUTO && max_nb > 2048);
+  // By default the grid where it is faster, steps of one iteration, us, scan /
+  // grid: one world of 2048 bodies 242 / 215; 4 of 1024 (pairs of bodies, sum of
+  // n^2: 4.2 M) 207 / 198, 8 222 / 204, 32 315 / 243; 16 of 512 (4.2 M) 155 /
+  // 155, 64 222 / 190; 64 of 256 (4.2 M) 141 / 145, 128 179 / 169; 512 of 64
+  // (2.2 M) 152 / 160.
+  double tests = 0.0;
+  for (int w = 0; w < n_worlds; ++w) {
+    const double n = body_off[w + 1] - body_off[w];
+    tests += n * n;
+  }
+  P.use_grid = mode >= SHP_BROADPHASE_GRID ||
+               (mode == SHP_BROADPHASE_AUTO && (max_nb > 1536 || tests > 6e6));
   if (P.use_grid) {
     std::vector<double> rmax(hb->rad);  // a circle's extent is its radius
     for (long gg = 0; gg < NB; ++gg)
