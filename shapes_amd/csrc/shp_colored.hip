@@ -1040,18 +1040,24 @@ __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// Worlds small enough for one wavefront each (world_order[first_world, W),
-// at most SWEEP_WAVE_MAX_BODIES bodies, FP32 velocities in the wavefront's
-// slice of LDS): the warm pass and the sweeps of sweep_prefetched with 64
-// lanes, colour by colour, with the wavefront's own ordering of its LDS
-// accesses between colours instead of workgroup barriers; SWEEP_WAVES
-// worlds per workgroup.  The same updates in the same colour order as
-// sweep_world, so the same results.
-__global__ __launch_bounds__(64 * SWEEP_WAVES) void k_sweep_waves(Ctx c, int first_world,
-                                                                  int slice_floats) {
+// Small worlds (world_order[first_world, W), at most SWEEP_WAVE_MAX_BODIES
+// bodies, FP32 velocities in the world's slice of LDS), SWEEP_WAVES of them to
+// a workgroup: the warm pass and the sweeps of sweep_prefetched, colour by
+// colour, by one wavefront with its own ordering of its LDS accesses between
+// colours, or, above SWEEP_ONE_WAVE_BODIES bodies, by SWEEP_PARTS wavefronts
+// that meet at a counter in LDS.  The same updates in the same colour order as
+// sweep_world, so the same results.  2048 worlds of 8 to 1024 bodies: 184 us,
+// 254 with one wavefront for each, the largest world's time; the rest is the
+// records, read again in each of 7 passes (0.6 GB).  Two wavefronts for the
+// larger worlds take 187; the line at 128 or 256 bodies makes no difference.
+__global__ __launch_bounds__(64 * SWEEP_WAVES * SWEEP_PARTS) void k_sweep_waves(Ctx c, int first_world,
+                                                                               int slice_floats) {
   extern __shared__ __align__(16) int lds[];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int k = first_world + (int)blockIdx.x * SWEEP_WAVES + wave;
+  __shared__ int s_met[SWEEP_WAVES];
+  if (threadIdx.x < SWEEP_WAVES) s_met[threadIdx.x] = 0;
+  __syncthreads();
+  const int wave = threadIdx.x >> 6, slot = wave % SWEEP_WAVES, part = wave / SWEEP_WAVES;
+  const int k = first_world + (int)blockIdx.x * SWEEP_WAVES + slot;
   if (k >= c.W) return;  // this wavefront only: no workgroup barrier follows
   const int w = c.world_order[k];
   const int info = c.col_info[w];
@@ -1060,21 +1066,39 @@ __global__ __launch_bounds__(64 * SWEEP_WAVES) void k_sweep_waves(Ctx c, int fir
   const bool serial_tail = info & COL_TAIL;
   const int p0 = c.wpair_off[w];
   const int b0 = c.body_off[w], nb = c.body_off[w + 1] - b0;
+  const int parts = nb > SWEEP_ONE_WAVE_BODIES ? SWEEP_PARTS : 1;
+  if (part >= parts) return;
+  const int lane = 64 * part + (int)(threadIdx.x & 63), lanes = 64 * parts;
   const int* off = c.col_off + (long)w * (COLOR_CAP + 3);
   VelF<true> V;
-  V.lds = (float*)lds + wave * slice_floats;
+  V.lds = (float*)lds + slot * slice_floats;
   V.c = &c;
   V.b0 = b0;
-  for (int i = lane; i < nb; i += 64) {
+  int meet = 0;
+  auto sync = [&] {
+    if (parts == 1) {
+      wave_sync();
+      return;
+    }
+    // every wavefront of the world runs (they are one workgroup's) and comes
+    // here as often
+    meet += SWEEP_PARTS;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    if ((threadIdx.x & 63) == 0)
+      __hip_atomic_fetch_add(&s_met[slot], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    while (__hip_atomic_load(&s_met[slot], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) < meet)
+      __builtin_amdgcn_s_sleep(1);
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+  };
+  for (int i = lane; i < nb; i += lanes) {
     const int g = b0 + i;
     const float v[3] = {(float)c.vx[g], (float)c.vy[g], (float)c.w[g]};
     V.store(g, v);
   }
-  wave_sync();
+  sync();
   const PackF P = packf(c);
-  sweep_prefetched(c, recw(c, P, p0), ncol, serial_tail, off, lane, 64, V,
-                   [] { wave_sync(); });
-  for (int i = lane; i < nb; i += 64) {
+  sweep_prefetched(c, recw(c, P, p0), ncol, serial_tail, off, lane, lanes, V, sync);
+  for (int i = lane; i < nb; i += lanes) {
     float v[3];
     V.load(b0 + i, v);
     c.fv[b0 + i] = make_float4(v[0], v[1], v[2], 0.0f);
@@ -1755,7 +1779,7 @@ void launch_colored_sweep(shp_batch* b) {
       k_sweep_colours<256><<<grid, 256, P.color_pool, b->stream>>>(c, pool);
   }
   if (P.g_sweep_waves > 0)
-    k_sweep_waves<<<(unsigned)P.g_sweep_waves, 64 * SWEEP_WAVES,
+    k_sweep_waves<<<(unsigned)P.g_sweep_waves, 64 * SWEEP_WAVES * SWEEP_PARTS,
                     (size_t)SWEEP_WAVES * P.sweep_slice * 4, b->stream>>>(c, (int)big,
                                                                          P.sweep_slice);
 }

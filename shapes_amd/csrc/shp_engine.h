@@ -22,10 +22,15 @@
 #define LDS_MAX_BYTES (LDS_BYTES_PER_CU - 512)
 // coloured solver: colour offsets per world
 #define COLOR_CAP 256
-// one wavefront per world in the coloured sweeps (solver_threads 64) for
-// worlds of up to this many bodies, SWEEP_WAVES wavefronts per workgroup
-#define SWEEP_WAVE_MAX_BODIES 1024
+// several worlds to a workgroup in the coloured sweeps (solver_threads 64) for
+// worlds of up to this many bodies (1024 and what they stand on: a single
+// world of 1025 had a launch of its own, 80 us): SWEEP_WAVES of them, one
+// wavefront each or,
+// above SWEEP_ONE_WAVE_BODIES bodies, SWEEP_PARTS
+#define SWEEP_WAVE_MAX_BODIES 1088
 #define SWEEP_WAVES 4
+#define SWEEP_PARTS 4
+#define SWEEP_ONE_WAVE_BODIES 256
 // the coloured solver keeps a world's FP32 velocities (12 B per body) in
 // LDS up to this many bodies; beyond, in global memory
 #define VEL_LDS_MAX_BODIES ((LDS_MAX_BYTES - (2 * (COLOR_CAP + 3) + 2) * 4) / 12)

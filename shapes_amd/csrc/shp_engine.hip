@@ -1641,8 +1641,8 @@ void plan_launches(const StepPlan& P, bool infer, bool logging, std::vector<Laun
     if (P.sweep_big > 0)
       add("k_sweep_colours", P.sweep_big + flow_extra, P.color_threads, P.color_pool, colored_static_lds(true));
     if (P.g_sweep_waves > 0)
-      add("k_sweep_waves", P.g_sweep_waves, 64 * SWEEP_WAVES,
-          (size_t)SWEEP_WAVES * P.sweep_slice * 4, 0);
+      add("k_sweep_waves", P.g_sweep_waves, 64 * SWEEP_WAVES * SWEEP_PARTS,
+          (size_t)SWEEP_WAVES * P.sweep_slice * 4, lds16(SWEEP_WAVES * 4));
     add("k_colour_unpack", P.g_unpack, 256, 0, 0);
   } else {
     if (P.flow_worlds > 0)
