@@ -185,13 +185,19 @@ __device__ __forceinline__ void grid_visit(const Ctx& c, const GridBody& a, int 
 // 1, 1 or 16 lanes).  The count pass takes the bodies in bucket order, in
 // which a wavefront's bodies walk the same few runs of records (in body order,
 // a cell to a lane or two and 2 bucket bounds to a cell, it took 307 us for
-// 1.14 M bodies, bound by its 8.8 M scattered loads; 172 now), then the large
+// 1.14 M bodies, bound by its 8.8 M scattered loads; 157 now), then the large
 // bodies, and keeps each body's first GRID_SLOTS partners; the emit pass
 // writes those without a second visit when they are all, and in descending j
 // either way.
+// Workgroups go to the 8 XCDs in turn: workgroup b of n as the one that makes
+// those of an XCD consecutive, so that the records of a region are in one L2.
+__device__ __forceinline__ int xcd_block(int b, int n) {
+  return b % 8 * (n / 8) + min(b % 8, n % 8) + b / 8;
+}
+
 template <int LANES>
 __global__ void k_grid_pairs(Ctx c, int fill) {
-  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  const long t = (long)xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
   const int sl = (int)(t % LANES);
   int g = (int)(t / LANES);  // the same for the LANES lanes of a group
   if (g >= c.NB) return;
