@@ -255,15 +255,15 @@ def roofline(instr, scene, word, broadphase="grid", threads=0):
     }
 
 
-# worlds of at most this many bodies sweep one wavefront each when the
+# worlds of at most this many bodies sweep several to a workgroup when the
 # coloured solver runs with 64 lanes
-SWEEP_WAVE_MAX_BODIES = 1024
+SWEEP_WAVE_MAX_BODIES = 1088
 
 
 def phase_kernel(phase, word, broadphase, threads=0, largest=0):
     """The kernel a single-kernel phase launches in this configuration (the
     coloured sweeps with 64 lanes: k_sweep_waves alone when every world
-    fits a wavefront's slice, else it and k_sweep_colours)."""
+    is small enough, else it and k_sweep_colours)."""
     if phase == "sweeps":
         if word == 8:
             return "k_solve_ordered"

@@ -1342,8 +1342,7 @@ __global__ __launch_bounds__(T) void k_colour(Ctx c, int pool_bytes) {
   const int flow_blocks = c.flow_worlds * c.flow_groups, blk = blockIdx.x;
   const bool flow = blk < flow_blocks;
   const int w = c.world_order[flow ? blk / c.flow_groups : blk - flow_blocks + c.flow_worlds];
-  // the world's pairs (k_world_ranges computes the same offsets beside
-  // this kernel)
+  // the world's pairs (k_contacts writes the same offsets beside this kernel)
   const int b0 = c.body_off[w], b1 = c.body_off[w + 1];
   const int p0 = min(c.off_rank[b0], c.pair_cap), p1 = min(c.off_rank[b1], c.pair_cap);
   const int np = p1 - p0;

@@ -226,6 +226,24 @@ struct Ctx {
   int2* part_n;
 };
 
+#ifdef __HIPCC__
+// The step's counters, quality maxima and the flow worlds' state, cleared by
+// its first kernel (all of its threads call this), which uses none of them: a
+// kernel of its own for that took 4 to 5 us of every step.
+__device__ __forceinline__ void begin_step(const Ctx& c) {
+  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t < 8) c.counters[t] = 0;
+  if (t < 3) c.quality[t] = 0ull;  // Q_DEPTH ..
+  if (c.flow_worlds == 0) return;
+  const long step = (long)gridDim.x * blockDim.x;
+  for (long i = t; i < (long)c.W * FLOW_CTL; i += step) c.flow_ctl[i] = 0;
+  for (long g = t; g < c.NB; g += step) {
+    c.adj_n[g] = 0;
+    if (c.flow_col) c.flow_col[FLOW_LINE * g] = 0ull;
+  }
+}
+#endif
+
 // ---- launch plan ----------------------------------------------------------
 // Every launch of a step takes its grid from the plan, which is computed on
 // the host from the worlds and the configuration before anything is
@@ -266,8 +284,7 @@ struct StepPlan {
   ScanPlan scan_buckets, scan_bodies, scan_pairs;
   long scan_parts_max = 0;  // scratch entries of the multi-workgroup scans
   // grids (workgroups) of the step's launches
-  long g_reset = 0, g_bodies = 0, g_pairs = 0, g_pairs_count = 0, g_broadphase = 0, g_sat = 0,
-       g_ranges = 0;
+  long g_bodies = 0, g_pairs = 0, g_pairs_count = 0, g_broadphase = 0, g_sat = 0;
   long g_contacts = 0, g_infer = 0, g_pack = 0, g_unpack = 0, g_log = 0, g_finish_ni = 0,
        g_finish_nq = 0, g_cache = 0;
   // device memory allocated at creation (bytes)

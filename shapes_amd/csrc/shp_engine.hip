@@ -3,18 +3,16 @@
 // One step (the reference's updateWorld, shapes/src/Physics/Engine/
 // Main.hs:71-86) is this sequence of launches on the batch's stream:
 //
-//   k_reset          clear per-step counters
 //   k_broadphase(0)  one wavefront per body: gravity (applyExternal) and the
 //                    count of its pairs (i, j<i); or the grid's binning and
-//                    count pass (shp_grid.hip)
+//                    count pass (shp_grid.hip); either clears the step's counters
 //   scan             exclusive sum of the counts, in descending body order
 //   k_broadphase(1)  same sweep, ballot/popcount compaction -> pairs in
 //                    descending (i, j) order (G.culledKeys); or the grid's
 //                    emit pass
 //   k_sat            one lane per pair: SAT + clipping -> <= 2 contacts
 //   scan             exclusive sum of contacts per pair
-//   k_world_ranges   per-world pair and contact ranges
-//   k_contacts       compaction, constraintGen, warm-start join; for the
+//   k_contacts       per-world pair and contact ranges, compaction, constraintGen, warm-start join; for the
 //                    coloured solver, after its k_colour (on a second
 //                    stream), also each manifold's record in colour order
 //   solve            warm-start application + Gauss-Seidel sweeps
@@ -69,21 +67,6 @@ __device__ __forceinline__ HullRef hull_of(const Ctx& c, int g) {
 }
 
 // ---------------------------------------------------------------- kernels
-
-// Per-step counters and quality maxima, and the grid's bucket counts.
-__global__ void k_reset(Ctx c) {
-  const long g = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (g < 8) c.counters[g] = 0;
-  if (g < 3) c.quality[g] = 0ull;
-  if (c.use_grid && g <= c.grid_buckets) c.bucket_cnt[g] = 0;
-  if (c.flow_worlds) {
-    if (g < (long)c.W * FLOW_CTL) c.flow_ctl[g] = 0;
-    if (g < c.NB) {
-      c.adj_n[g] = 0;
-      if (c.flow_col) c.flow_col[FLOW_LINE * g] = 0ull;
-    }
-  }
-}
 
 // listToHull in local space (ConvexHull.hs:151-167): unit edge normals and
 // the per-edge (min, max) extent vertex indices, first index on ties.
@@ -336,6 +319,7 @@ __global__ __launch_bounds__(INTEGRATE_THREADS) void k_finish(Ctx c, int ni) {
 // constantAccel, World/External.hs:23-28); pass 1 writes the pairs, in
 // descending j within descending i, using ballot + prefix popcount.
 __global__ void k_broadphase(Ctx c, int fill) {
+  if (!fill) begin_step(c);
   int wave = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
   int lane = threadIdx.x & 63;
   if (wave >= c.NB) return;
@@ -477,17 +461,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
 }
 
 
-// Per-world pair and contact ranges after the scans.
-__global__ void k_world_ranges(Ctx c) {
-  int w = blockIdx.x * blockDim.x + threadIdx.x;
-  if (w > c.W) return;
-  int ps = c.off_rank[c.body_off[w]];
-  if (ps > c.pair_cap) ps = c.pair_cap;
-  int cs = c.coff[ps];
-  if (cs > c.contact_cap) cs = c.contact_cap;
-  c.wpair_off[w] = ps;
-  c.wcont_off[w] = cs;
-  if (w == c.W && c.coff[ps] > c.contact_cap) atomicOr(&c.counters[CNT_FLAGS], SHP_FLAG_CONTACT_OVERFLOW);
+// Where the pairs and the contacts of world w (or of all, w = W) start and end.
+__device__ __forceinline__ int first_pair(const Ctx& c, int w) {
+  return min(c.off_rank[c.body_off[w]], c.pair_cap);
+}
+__device__ __forceinline__ int first_contact(const Ctx& c, int w) {
+  return min(c.coff[first_pair(c, w)], c.contact_cap);
 }
 
 // Compaction + constraintGen (Constraints/Contact.hs:60-72) + the warm
@@ -506,7 +485,7 @@ __device__ __forceinline__ bool contact_of_pair(const Ctx& c, int p, int k, int 
   d2 xa = mk(c.px[ga], c.py[ga]), xb = mk(c.px[gb], c.py[gb]);
   double im[6] = {c.iml[ga], c.iml[ga], c.imr[ga], c.iml[gb], c.iml[gb], c.imr[gb]};
   int cache_lo = c.cache_woff[w], cache_hi = c.cache_woff[w + 1];
-  int c_lo = c.wcont_off[w], c_hi = c.wcont_off[w + 1];
+  int c_lo = first_contact(c, w), c_hi = first_contact(c, w + 1);
   const PackF P = packf(c);
   int s = 2 * p + k;
   int fa = c.s_feat[s] >> 8, fb = c.s_feat[s] & 255;
@@ -668,6 +647,13 @@ __global__ __launch_bounds__(CONTACT_PAIRS) void k_contacts(Ctx c) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int tp = total_pairs(c);
   const PackF P = packf(c);
+  // the worlds' ranges, for the kernels that follow
+  for (int w = blockIdx.x * CONTACT_PAIRS + tid; w <= c.W; w += gridDim.x * CONTACT_PAIRS) {
+    const int ps = first_pair(c, w), cs = c.coff[ps];
+    c.wpair_off[w] = ps;
+    c.wcont_off[w] = min(cs, c.contact_cap);
+    if (w == c.W && cs > c.contact_cap) atomicOr(&c.counters[CNT_FLAGS], SHP_FLAG_CONTACT_OVERFLOW);
+  }
   int hits = 0, mans = 0;
   for (long p0 = (long)blockIdx.x * CONTACT_PAIRS; p0 < tp; p0 += (long)gridDim.x * CONTACT_PAIRS) {
     const int n = p0 + tid < tp ? c.ccount[p0 + tid] : 0;
@@ -1150,7 +1136,6 @@ static shp_status enqueue_front(shp_batch* b, bool fork) {
   const StepPlan& P = b->plan;
   hipStream_t s = b->stream;
   mark(b, 0);
-  k_reset<<<P.g_reset, 256, 0, s>>>(c);
   mark(b, 1);
   if (c.use_grid)
     HIPCHK(launch_grid_count(b));
@@ -1180,7 +1165,6 @@ static shp_status enqueue_front(shp_batch* b, bool fork) {
   HIPCHK(exclusive_sum(b, P.scan_pairs, c.ccount, c.coff, c.off_rank + c.NB, c.pair_cap, s));
   if (fork && P.records_in_contacts) TRY(fork_colouring(b));
   mark(b, 6);
-  k_world_ranges<<<P.g_ranges, 256, 0, s>>>(c);
   if (fork && P.records_in_contacts) HIPCHK(hipStreamWaitEvent(s, b->join_event, 0));
   mark(b, 7);
   k_contacts<<<P.g_contacts, 256, 0, s>>>(c);
@@ -1582,15 +1566,11 @@ shp_status plan_staged(const shp_config& cfg, HostBatch* hb) {
   }
 
   const long PC = P.pair_cap, CC = P.contact_cap;
-  P.g_reset = blocks(std::max({64L, P.use_grid ? P.grid_buckets + 1 : 0L,
-                               P.flow_worlds ? std::max(NB, (long)FLOW_CTL * n_worlds) : 0L}),
-                     256);
   P.g_bodies = blocks(NB, 256);
   P.g_pairs = P.grid_wide ? blocks(NB * 16, 256) : blocks(NB, 256);
   P.g_pairs_count = P.grid_wide ? P.g_pairs : blocks(NB * 4, 256);
   P.g_broadphase = blocks(NB * 64, 256);
   P.g_sat = gs_blocks(PC);
-  P.g_ranges = blocks(n_worlds + 1, 256);
   P.g_contacts = std::min<long>(gs_blocks(PC), MAX_PARTS);
   P.g_pack = gs_blocks(PC);
   P.g_infer = std::min<long>(std::max<long>(1, blocks(P.miss_cap, MLP_INFER_ROWS)), 512);
@@ -1612,7 +1592,6 @@ void plan_launches(const StepPlan& P, bool infer, bool logging, std::vector<Laun
   auto add = [&](const char* n, long g, int b, size_t dyn, size_t st) {
     out->push_back({n, g, b, dyn, st});
   };
-  add("k_reset", P.g_reset, 256, 0, 0);
   if (P.use_grid) {
     add("k_grid_assign", P.g_bodies, 256, 0, 0);
     scan_launches(P.scan_buckets, "scan_buckets", out);
@@ -1633,7 +1612,6 @@ void plan_launches(const StepPlan& P, bool infer, bool logging, std::vector<Laun
   if (col) add("k_colour", P.W + flow_extra, P.color_threads >= 512 ? 1024 : 256, P.color_lds,
                colored_static_lds(false));
   scan_launches(P.scan_pairs, "scan_pairs", out);
-  add("k_world_ranges", P.g_ranges, 256, 0, 0);
   add("k_contacts", P.g_contacts, CONTACT_PAIRS, 0, CONTACTS_STATIC_LDS);
   if (infer) add("k_mlp_infer", P.g_infer, MLP_INFER_THREADS, 0, mlp_infer_static_lds());
   if (col) {
@@ -1870,6 +1848,9 @@ shp_status batch_alloc(shp_batch* b, const HostBatch& hb) {
   k_fill_i32<<<blocks(n_worlds + 1, 256), 256, 0, s>>>(c.wcont_off, 0, n_worlds + 1);
   k_fill_i32<<<blocks(n_worlds + 1, 256), 256, 0, s>>>(c.wpair_off, 0, n_worlds + 1);
   k_fill_i32<<<1, 64, 0, s>>>(c.counters, 0, 8);
+  if (P.use_grid)  // k_grid_fill clears them for the next step
+    k_fill_i32<<<blocks(P.grid_buckets + 1, 256), 256, 0, s>>>(c.bucket_cnt, 0,
+                                                              (int)P.grid_buckets + 1);
   k_fill_i32<<<1, 64, 0, s>>>((int32_t*)c.quality, 0, 2 * Q_ENTRIES);
   k_fill_i32<<<1, 64, 0, s>>>((int32_t*)c.log_count, 0, 2);
   // makeWorldObj places each shape with moveShape (World.hs:142-149)

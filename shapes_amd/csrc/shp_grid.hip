@@ -51,6 +51,7 @@ __device__ __forceinline__ bool aabb_hit(const Ctx& c, double aminx, double amax
 // gravity (applyExternal) + binning of small bodies; empty slots
 // (World.delete) get neither
 __global__ void k_grid_assign(Ctx c) {
+  begin_step(c);
   int g = blockIdx.x * blockDim.x + threadIdx.x;
   if (g >= c.NB) return;
   if (c.dead[g]) {
@@ -87,6 +88,8 @@ __device__ __forceinline__ GridRec load_rec(const Ctx& c, int q) {
 
 __global__ void k_grid_fill(Ctx c) {
   int g = blockIdx.x * blockDim.x + threadIdx.x;
+  // the next step's bucket counts (this one's are summed)
+  for (long i = g; i <= c.grid_buckets; i += (long)gridDim.x * blockDim.x) c.bucket_cnt[i] = 0;
   if (g >= c.NB || c.is_large[g] || c.dead[g]) return;
   int w = c.body_world[g];
   int t0 = c.tab_off[w];
