@@ -262,6 +262,7 @@ struct StepPlan {
   long NB = 0, NV = 0, W = 0, max_nb = 0;
   long pair_cap = 0, contact_cap = 0, miss_cap = 0, grid_buckets = 0, n_large = 0;
   int ppb = 8;
+  bool small_front = false;  // the step up to the contacts in one launch
   bool use_grid = false, grid_wide = false;  // grid broadphase; 16 lanes per body
   int solver = 0, warm = 0;
   // ordered solver: lanes per world, dynamic LDS

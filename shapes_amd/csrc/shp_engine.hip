@@ -636,11 +636,13 @@ __device__ __forceinline__ bool contact_of_pair(const Ctx& c, int p, int k, int 
 // bound by the CUs' address units; 476 with this, 385 with the workgroups'
 // counts added up by the step's last kernel instead of by two atomics each.)
 constexpr int CONTACT_PAIRS = 256;
-constexpr size_t CONTACTS_STATIC_LDS = lds16(4 * CONTACT_PAIRS) + lds16(CONTACT_PAIRS) +
-                                       lds16(2 * CONTACT_PAIRS) + lds16(CONTACT_PAIRS / 16) +
-                                       lds16(8);
+constexpr size_t contacts_static_lds(int pairs) {
+  return lds16(4UL * pairs) + lds16(pairs) + lds16(2UL * pairs) + lds16(pairs / 16) + lds16(8);
+}
 
-__global__ __launch_bounds__(CONTACT_PAIRS) void k_contacts(Ctx c) {
+// (the whole workgroup, CONTACT_PAIRS lanes)
+template <int CONTACT_PAIRS>
+__device__ __forceinline__ void contact_tiles(const Ctx& c) {
   __shared__ uint16_t s_item[2 * CONTACT_PAIRS];  // pair of the tile << 1 | contact
   __shared__ uint8_t s_n[CONTACT_PAIRS], s_warm[2 * CONTACT_PAIRS];
   __shared__ int s_sum[CONTACT_PAIRS / 64];
@@ -714,6 +716,130 @@ __global__ __launch_bounds__(CONTACT_PAIRS) void k_contacts(Ctx c) {
     c.part_n[blockIdx.x] = make_int2(s_cnt[0], s_cnt[1]);
   }
 }
+
+__global__ __launch_bounds__(CONTACT_PAIRS) void k_contacts(Ctx c) {
+  contact_tiles<CONTACT_PAIRS>(c);
+}
+
+// ---- the front of a small batch's step in one launch ------------------------
+//
+// Gravity, the scan broadphase, SAT and contact generation by one workgroup,
+// the ordered solver's batches of up to FRONT_BODIES bodies: six launches of
+// 3.5 to 8 us each, of which a kernel's start and end are most.  The same pairs
+// in the same order.  us a step, separate launches / this one: pyramids of 16
+// bodies 80 / 72, 56 116 / 109, 121 158 / 148; heaps of 51 80 / 67, 101 88 /
+// 72.  (With two lanes to a body and up to 256 bodies it was no faster from
+// 121 bodies on: 158 / 161, 232 bodies 210 / 218.)
+constexpr int FRONT_T = 512, FRONT_BODIES = 128;
+
+// The exclusive sum of v over the workgroup, in thread order, and the total.
+__device__ __forceinline__ int front_sum(int v, int* s_sum, int* total) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  int incl = v;
+  for (int o = 1; o < 64; o <<= 1) {
+    const int y = __shfl_up(incl, o);
+    if (lane >= o) incl += y;
+  }
+  __syncthreads();  // s_sum is free
+  if (lane == 63) s_sum[wave] = incl;
+  __syncthreads();
+  int base = 0, all = 0;
+  for (int q = 0; q < FRONT_T / 64; ++q) {
+    if (q < wave) base += s_sum[q];
+    all += s_sum[q];
+  }
+  *total = all;
+  return base + incl - v;
+}
+
+__global__ __launch_bounds__(FRONT_T) void k_front_small(Ctx c) {
+  __shared__ double4 s_box[FRONT_BODIES];
+  __shared__ int s_cnt[FRONT_BODIES], s_part[4][FRONT_BODIES], s_sum[FRONT_T / 64];
+  __shared__ uint8_t s_flag[FRONT_BODIES];  // 1 dead, 2 static
+  const int tid = threadIdx.x;
+  begin_step(c);
+  if (tid < c.NB) {
+    const int g = tid;
+    const bool dead = c.dead[g] != 0;
+    // the constant acceleration (applyExternal)
+    if (c.iml[g] != 0.0 && !dead && !c.probe) {
+      c.vx[g] = c.vx[g] + c.gx * c.dt;
+      c.vy[g] = c.vy[g] + c.gy * c.dt;
+    }
+    s_box[g] = make_double4(c.bminx[g], c.bmaxx[g], c.bminy[g], c.bmaxy[g]);
+    s_flag[g] = (dead ? 1 : 0) | (body_static(c, g) ? 2 : 0);
+  }
+  // four lanes to a body i, each with a quarter of the bodies j: one bit for
+  // each that makes a pair (k_broadphase's test)
+  constexpr int QUARTER = FRONT_BODIES / 4;
+  static_assert(FRONT_T == 4 * FRONT_BODIES && QUARTER == 32, "a word of bits a lane");
+  const int g = tid % FRONT_BODIES, part = tid / FRONT_BODIES, jp = QUARTER * part;
+  const bool real = g < c.NB;
+  const int w = real ? c.body_world[g] : 0, b0 = c.body_off[w];
+  const int rank = c.body_off[w + 1] - 1 - (g - b0);
+  __syncthreads();
+  uint32_t hits = 0;
+  const double4 a = s_box[real ? g : 0];
+  const int fl = real ? s_flag[g] : 1, n = min(QUARTER, c.NB - jp);
+#pragma unroll 4
+  for (int k = 0; k < n; ++k) {
+    const int j = jp + k;
+    const double4 x = s_box[j];
+    const int fj = s_flag[j];
+    const bool hit = j >= b0 && j < g && !((fl | fj) & 1) && !(fl & fj & 2) &&
+                     !(x.x > a.y || x.y < a.x) && !(x.z > a.w || x.w < a.z);
+    hits |= (uint32_t)hit << k;
+  }
+  s_part[part][g] = __popc(hits);
+  __syncthreads();
+  if (part == 0 && real) s_cnt[rank] = (s_part[0][g] + s_part[1][g]) + (s_part[2][g] + s_part[3][g]);
+  __syncthreads();
+  {  // the segments, in descending body order
+    const int n = tid < c.NB ? s_cnt[tid] : 0;
+    int all;
+    const int off = front_sum(n, s_sum, &all);
+    if (tid < c.NB) {
+      c.cnt_rank[tid] = n;
+      c.off_rank[tid] = off;
+      s_cnt[tid] = off;
+    }
+    if (tid == 0) {
+      c.off_rank[c.NB] = all;
+      if (all > c.pair_cap) atomicOr(&c.counters[CNT_FLAGS], SHP_FLAG_PAIR_OVERFLOW);
+    }
+  }
+  __syncthreads();
+  if (real) {  // descending j
+    int pos = s_cnt[rank];
+    for (int q = 3; q > part; --q) pos += s_part[q][g];
+    for (uint32_t m = hits; m; ++pos) {
+      const int k = 31 - __builtin_clz(m);
+      m &= ~(1u << k);
+      if (pos < c.pair_cap) {
+        c.pa[pos] = g;
+        c.pb[pos] = jp + k;
+      }
+    }
+  }
+  __syncthreads();
+  const int tp = total_pairs(c);
+  int before = 0;
+  for (int p0 = 0; p0 < tp; p0 += FRONT_T) {
+    const int p = p0 + tid;
+    if (p < tp) sat_pair(c, p);
+    int all;
+    const int off = front_sum(p < tp ? c.ccount[p] : 0, s_sum, &all);
+    if (p < tp) c.coff[p] = before + off;
+    before += all;
+  }
+  if (tid == 0) c.coff[tp] = before;
+  __syncthreads();
+  contact_tiles<FRONT_T>(c);
+}
+constexpr size_t FRONT_STATIC_LDS = lds16(4 * FRONT_BODIES * 8) + lds16(FRONT_BODIES * 4) +
+                                    lds16(4 * FRONT_BODIES * 4) +
+                                    lds16(FRONT_T / 64 * 4) + lds16(FRONT_BODIES) +
+                                    contacts_static_lds(FRONT_T);
 
 // This frame's lagrangians become the next frame's EngineCache
 // (Engine/Main.hs:32, wrapInitializer :61-69).
@@ -1137,6 +1263,13 @@ static shp_status enqueue_front(shp_batch* b, bool fork) {
   hipStream_t s = b->stream;
   mark(b, 0);
   mark(b, 1);
+  if (P.small_front) {
+    for (int k = 2; k < 8; ++k) mark(b, k);
+    k_front_small<<<1, FRONT_T, 0, s>>>(c);
+    mark(b, 8);
+    HIPCHK(hipGetLastError());
+    return SHP_OK;
+  }
   if (c.use_grid)
     HIPCHK(launch_grid_count(b));
   else
@@ -1571,7 +1704,8 @@ shp_status plan_staged(const shp_config& cfg, HostBatch* hb) {
   P.g_pairs_count = P.grid_wide ? P.g_pairs : blocks(NB * 4, 256);
   P.g_broadphase = blocks(NB * 64, 256);
   P.g_sat = gs_blocks(PC);
-  P.g_contacts = std::min<long>(gs_blocks(PC), MAX_PARTS);
+  P.small_front = cfg.solver == SHP_SOLVER_ORDERED_F64 && !P.use_grid && NB <= FRONT_BODIES;
+  P.g_contacts = P.small_front ? 1 : std::min<long>(gs_blocks(PC), MAX_PARTS);
   P.g_pack = gs_blocks(PC);
   P.g_infer = std::min<long>(std::max<long>(1, blocks(P.miss_cap, MLP_INFER_ROWS)), 512);
   P.g_unpack = std::max(1L, std::min(blocks(std::max(PC, NB), 256), 4096L));
@@ -1592,27 +1726,31 @@ void plan_launches(const StepPlan& P, bool infer, bool logging, std::vector<Laun
   auto add = [&](const char* n, long g, int b, size_t dyn, size_t st) {
     out->push_back({n, g, b, dyn, st});
   };
-  if (P.use_grid) {
-    add("k_grid_assign", P.g_bodies, 256, 0, 0);
-    scan_launches(P.scan_buckets, "scan_buckets", out);
-    add("k_grid_fill", P.g_bodies, 256, 0, 0);
-    add("k_grid_pairs", P.g_pairs_count, 256, 0, 0);
-  } else {
-    add("k_broadphase", P.g_broadphase, 256, 0, 0);
-  }
-  scan_launches(P.scan_bodies, "scan_bodies", out);
-  if (P.use_grid)
-    add("k_grid_pairs", P.g_pairs, 256, 0, 0);
-  else
-    add("k_broadphase", P.g_broadphase, 256, 0, 0);
-  add("k_sat", P.g_sat, 256, 0, 0);
   const bool col = P.solver == SHP_SOLVER_COLORED_F32;
   // workgroups beyond one to a world
   const long flow_extra = (long)P.flow_worlds * (P.flow_groups - 1);
-  if (col) add("k_colour", P.W + flow_extra, P.color_threads >= 512 ? 1024 : 256, P.color_lds,
-               colored_static_lds(false));
-  scan_launches(P.scan_pairs, "scan_pairs", out);
-  add("k_contacts", P.g_contacts, CONTACT_PAIRS, 0, CONTACTS_STATIC_LDS);
+  if (P.small_front) {
+    add("k_front_small", 1, FRONT_T, 0, FRONT_STATIC_LDS);
+  } else {
+    if (P.use_grid) {
+      add("k_grid_assign", P.g_bodies, 256, 0, 0);
+      scan_launches(P.scan_buckets, "scan_buckets", out);
+      add("k_grid_fill", P.g_bodies, 256, 0, 0);
+      add("k_grid_pairs", P.g_pairs_count, 256, 0, 0);
+    } else {
+      add("k_broadphase", P.g_broadphase, 256, 0, 0);
+    }
+    scan_launches(P.scan_bodies, "scan_bodies", out);
+    if (P.use_grid)
+      add("k_grid_pairs", P.g_pairs, 256, 0, 0);
+    else
+      add("k_broadphase", P.g_broadphase, 256, 0, 0);
+    add("k_sat", P.g_sat, 256, 0, 0);
+    if (col) add("k_colour", P.W + flow_extra, P.color_threads >= 512 ? 1024 : 256, P.color_lds,
+                 colored_static_lds(false));
+    scan_launches(P.scan_pairs, "scan_pairs", out);
+    add("k_contacts", P.g_contacts, CONTACT_PAIRS, 0, contacts_static_lds(CONTACT_PAIRS));
+  }
   if (infer) add("k_mlp_infer", P.g_infer, MLP_INFER_THREADS, 0, mlp_infer_static_lds());
   if (col) {
     if (!P.records_in_contacts) add("k_pack_manifolds", P.g_pack, 256, 0, 0);
@@ -1840,7 +1978,8 @@ shp_status batch_alloc(shp_batch* b, const HostBatch& hb) {
   }
   TRY(solver_alloc(b));
   TRY(check_static_lds((const void*)k_finish, FINISH_STATIC_LDS, "k_finish"));
-  TRY(check_static_lds((const void*)k_contacts, CONTACTS_STATIC_LDS, "k_contacts"));
+  TRY(check_static_lds((const void*)k_contacts, contacts_static_lds(CONTACT_PAIRS), "k_contacts"));
+  TRY(check_static_lds((const void*)k_front_small, FRONT_STATIC_LDS, "k_front_small"));
 
   hipStream_t s = b->stream;
   k_fill_i32<<<1, 1, 0, s>>>(c.cnt_rank + NB, 0, 1);
