@@ -112,48 +112,80 @@ __device__ __forceinline__ void load_hull_v(const HullRef& h, HullV& r) {
     }
 }
 
-// overlap + minOverlap fold (Contact/SAT.hs:103-138): first separating
-// edge wins; otherwise the first strictly smallest depth.  Returns false if
-// separated.  se's own extent along each edge normal (extentAlong,
-// ConvexHull.hs:81-92) comes precomputed with the step's transform; every
-// edge's axis and extent are loaded before the first projection, so that a
-// pair waits on one round of loads per hull rather than on two per edge.
-__device__ __forceinline__ bool min_overlap(const HullRef& se, const HullV& sp, Overlap* out) {
+// A hull's edges held in registers: axes and the hull's own extents.
+struct HullE {
   double ax[SHP_MAXV], ay[SHP_MAXV], lo[SHP_MAXV], hi[SHP_MAXV];
+  int n;
+};
+
+__device__ __forceinline__ void load_hull_e(const HullRef& h, HullE& r) {
+  r.n = h.n;
 #pragma unroll
   for (int e = 0; e < SHP_MAXV; ++e)
-    if (e < se.n) {
-      const d2 d = se.nrm(e);
-      const double2 s = se.sx[e];
-      ax[e] = d.x;
-      ay[e] = d.y;
-      lo[e] = s.x;
-      hi[e] = s.y;
+    if (e < h.n) {
+      const d2 d = h.nrm(e);
+      const double2 s = h.sx[e];
+      r.ax[e] = d.x;
+      r.ay[e] = d.y;
+      r.lo[e] = s.x;
+      r.hi[e] = s.y;
     }
+}
+
+// overlap + minOverlap fold (Contact/SAT.hs:103-138): separated by any edge,
+// else the first strictly smallest depth.  Returns false if separated.  se's
+// own extent along each edge normal (extentAlong, ConvexHull.hs:81-92) comes
+// precomputed with the step's transform.  No lane leaves a loop on its own: a
+// missing vertex is vertex 0 once more, which no strict comparison prefers,
+// and a missing edge's outcome is dropped.  With branches for each lane's
+// number of vertices and edges (256 of them, 2.3 k vector instructions a
+// wavefront, a third of them selects of 64-bit minima) k_sat took, us before
+// and now: 900 boxes 9.4 / 8.1, piles of 8192 polygons 21 / 15 and of 32768
+// 27 / 21, 512 worlds of boxes 31 / 24, 2048 worlds 119 / 96, 256 piles (2.5 M
+// pairs) 341 / 294.  At 2.5 M pairs the CU's address unit bounds it, which
+// takes a cycle for each lane's line of a load; a wavefront's lanes loading
+// its hulls together, eight lanes to a hull, and passing them on through LDS
+// takes 281 there, but 108 and 31 for the 2048 and the 512 worlds.
+__device__ __forceinline__ bool min_overlap(const HullE& se, const HullV& sp, Overlap* out) {
+  double vx[SHP_MAXV], vy[SHP_MAXV];
+#pragma unroll
+  for (int k = 0; k < SHP_MAXV; ++k) {
+    vx[k] = k < sp.n ? sp.x[k] : sp.x[0];
+    vy[k] = k < sp.n ? sp.y[k] : sp.y[0];
+  }
+  const bool many = __ballot(sp.n > 4) != 0;
   Overlap best{0, 0, 0.0};
+  bool apart = false;
 #pragma unroll
   for (int e = 0; e < SHP_MAXV; ++e) {
-    if (e >= se.n) break;
-    const d2 dir = mk(ax[e], ay[e]);
-    const double smin = lo[e], smax = hi[e];
-    double pmin = dot(mk(sp.x[0], sp.y[0]), dir), pmax = pmin;
+    const bool edge = e < se.n;
+    if (__ballot(edge && !apart) == 0) break;
+    const d2 dir = mk(se.ax[e], se.ay[e]);
+    const double d0 = dot(mk(vx[0], vy[0]), dir);
+    double pmin = d0, pmax = d0;
     int imin = 0;
+    auto vertex = [&](int k) {
+      const double d = dot(mk(vx[k], vy[k]), dir);
+      imin = d < pmin ? k : imin;
+      pmin = __builtin_fmin(pmin, d);
+      pmax = __builtin_fmax(pmax, d);
+    };
 #pragma unroll
-    for (int k = 1; k < SHP_MAXV; ++k) {
-      if (k >= sp.n) break;
-      double d = dot(mk(sp.x[k], sp.y[k]), dir);
-      if (d < pmin) {
-        pmin = d;
-        imin = k;
-      }
-      if (d > pmax) pmax = d;
+    for (int k = 1; k < 4; ++k) vertex(k);
+    if (many) {
+#pragma unroll
+      for (int k = 4; k < SHP_MAXV; ++k) vertex(k);
     }
-    if (pmin > smax || pmax < smin) return false;
-    double depth = smax - pmin;
-    if (e == 0 || depth < best.depth) best = Overlap{e, imin, depth};
+    // comparisons with a d0 that is not a number are false
+    const bool number = d0 == d0;
+    imin = number ? imin : 0;
+    pmin = number ? pmin : d0;
+    apart = apart || (edge && (pmin > se.hi[e] || (number && pmax < se.lo[e])));
+    const double depth = se.hi[e] - pmin;
+    if (edge && (e == 0 || depth < best.depth)) best = Overlap{e, imin, depth};
   }
   *out = best;
-  return true;
+  return !apart;
 }
 
 struct Cgeom {
@@ -234,16 +266,18 @@ __device__ __forceinline__ int clip_contacts(const HullRef& se, const HullRef& s
 
 // HH.generateContacts via contactDebug + eitherBranchBoth (SAT.hs:238-249,
 // Utils/Utils.hs:230-235).  *flip_out: 0 Same (A penetrated), 1 Flip.
+// B's vertices against A's edges, then A's against B's.
 __device__ __forceinline__ int hull_contacts(const HullRef& A, const HullRef& B, Cgeom* out,
                                              int* flip_out) {
-  // one hull's vertices in registers at a time: B's against A's edges, then
-  // A's against B's edges (the same reads of the same values)
   Overlap oab, oba;
   HullV hv;
+  HullE he;
   load_hull_v(B, hv);
-  if (!min_overlap(A, hv, &oab)) return 0;
+  load_hull_e(A, he);
+  if (!min_overlap(he, hv, &oab)) return 0;
   load_hull_v(A, hv);
-  if (!min_overlap(B, hv, &oba)) return 0;
+  load_hull_e(B, he);
+  if (!min_overlap(he, hv, &oba)) return 0;
   if (oab.depth < oba.depth) {
     *flip_out = 0;
     return clip_contacts(A, B, oab, false, out);
