@@ -1171,7 +1171,11 @@ __device__ void colour_flow(const Ctx& c, int w, int p0, int np, int seat, int g
   const int q0 = seat * per, n = min(per, np - q0);
   const bool fits = per <= FLOW_ITEMS;
   if (tid < FLOW_DEGREE) s_cnt[tid] = 0;
-  if (fits && peek(ctl + FC_BAD) == 0) {
+  // read once: another workgroup may set it meanwhile, and all wavefronts have
+  // to take the same way past the barriers below
+  if (tid == 0) *s_last = peek(ctl + FC_BAD);
+  __syncthreads();
+  if (fits && *s_last == 0) {
     auto key = [&](uint32_t q) {  // orders like prio64
       return (unsigned long long)(mix32(q * 0x9E3779B9u + (uint32_t)w) & 0x7FFFu) << 32 | q;
     };
