@@ -330,6 +330,10 @@ __device__ __forceinline__ void solve_man(Lambda lambda, ManF& m, bool warm, con
   }
 }
 
+// The colouring's parts are inlined whatever their size: as a call, one of them
+// takes the kernel's arguments (1 KB) and its register arrays through scratch
+// memory (4097 worlds' step with k_colour<1024> 1930 us, 1300 inlined).
+
 // Colours per pair, in global memory: -1 uncoloured, -2 no contacts.
 __device__ __forceinline__ int colour_of(int x) { return x; }
 
@@ -375,8 +379,8 @@ __device__ __forceinline__ int wave_count(int* ctr, int key) {
 // inside a colour is free, except in the serial tail colour (tail >= 0),
 // whose manifolds may share bodies: thread 0 places those in pair order.
 template <int T, class CT>
-__device__ void assign_slots(int p0, int np, const CT* colour, int* scur, int tail,
-                             int32_t* slot) {
+__device__ __forceinline__ void assign_slots(int p0, int np, const CT* colour, int* scur, int tail,
+                                             int32_t* slot) {
   for (int q0 = 0; q0 < np; q0 += T) {
     const int q = q0 + threadIdx.x;
     const int cl = q < np ? colour_of(colour[q]) : -1;
@@ -467,7 +471,7 @@ __device__ void sweep_colours(const Ctx& c, const RecW& R, int ncol, bool serial
 // Colour-order bookkeeping shared by both kernels: per-colour counts of the
 // coloured manifolds -> s_off (exclusive) and s_cur (cursors).
 template <int T, class CT>
-__device__ void colour_offsets(const CT* colour, int np, int ncol, int* s_off, int* s_cur) {
+__device__ __forceinline__ void colour_offsets(const CT* colour, int np, int ncol, int* s_off, int* s_cur) {
   const int tid = threadIdx.x;
   for (int i = tid; i <= ncol + 1; i += T) s_cur[i] = 0;
   __syncthreads();
@@ -524,7 +528,7 @@ __device__ __forceinline__ unsigned long long prio64(int q, int w) {
 // top if any): per-colour offsets into col_off[w], the colour count into
 // col_info[w], and each pair's manifold slot into sched_order (pair index).
 template <int T, class CT>
-__device__ void colour_finish(const Ctx& c, int w, int p0, int np, const CT* colour, int top,
+__device__ __forceinline__ void colour_finish(const Ctx& c, int w, int p0, int np, const CT* colour, int top,
                               bool serial_tail, int* s_off, int* s_cur) {
   const int ncol = top + (serial_tail ? 1 : 0);
   if (threadIdx.x == 0) atomicMax(&c.counters[CNT_LEVELS], ncol);
@@ -538,7 +542,7 @@ __device__ void colour_finish(const Ctx& c, int w, int p0, int np, const CT* col
 // Number of manifolds (pairs with stored contacts) of a world, summed over
 // the workgroup; every thread gets it.
 template <int T>
-__device__ int count_manifolds(const Ctx& c, int p0, int np, int* s_cnt) {
+__device__ __forceinline__ int count_manifolds(const Ctx& c, int p0, int np, int* s_cnt) {
   if (threadIdx.x == 0) *s_cnt = 0;
   __syncthreads();
   int mine = 0;
@@ -559,7 +563,7 @@ __device__ int count_manifolds(const Ctx& c, int p0, int np, int* s_cnt) {
 // tail in pair order.
 #define COLOUR_REG_ITEMS 16
 template <int T>
-__device__ bool colour_regs(const Ctx& c, int w, int p0, int nm, int nb, uint32_t* s_best,
+__device__ __forceinline__ bool colour_regs(const Ctx& c, int w, int p0, int nm, int nb, uint32_t* s_best,
                             uint16_t* s_used, const uint32_t* m_ab, const uint16_t* m_q,
                             int32_t* colour, int* s_off, int* s_cur, int* sm) {
   int* s_tk = sm;  // [2]: taken this round, next round
@@ -683,7 +687,7 @@ __device__ bool colour_regs(const Ctx& c, int w, int p0, int nm, int nb, uint32_
 // 0xFF uncoloured), room for `cap` manifolds.  Colours go to sched_level per
 // pair (-2 for pairs without contacts).
 template <int T>
-__device__ void colour_world_lds(const Ctx& c, int w, int p0, int np, int b0, int nb,
+__device__ __forceinline__ void colour_world_lds(const Ctx& c, int w, int p0, int np, int b0, int nb,
                                  int cap, unsigned char* pool, int* s_off, int* s_cur, int* sm) {
   int &s_left = sm[0], &s_taken = sm[1], &s_top = sm[2], &s_fill = sm[3];
   const int tid = threadIdx.x;
@@ -808,7 +812,7 @@ __device__ void colour_world_lds(const Ctx& c, int w, int p0, int np, int b0, in
 // only on which manifolds are uncoloured and on their priorities, so the
 // colours are those of a round over every pair.
 template <int T>
-__device__ void colour_world_global(const Ctx& c, int w, int p0, int np, int b0, int nb,
+__device__ __forceinline__ void colour_world_global(const Ctx& c, int w, int p0, int np, int b0, int nb,
                                     int* s_off, int* s_cur, int* sm) {
   int &s_left = sm[0], &s_taken = sm[1], &s_top = sm[2], &s_fill = sm[3];
   const int tid = threadIdx.x;
@@ -921,7 +925,7 @@ __device__ void colour_world_global(const Ctx& c, int w, int p0, int np, int b0,
 // worlds whose bodies fit LDS but whose manifolds do not.  A mask is read
 // and written only by the manifold a round selects on the body.
 template <int T, bool MASKS_LDS>
-__device__ void colour_world_hybrid(const Ctx& c, int w, int p0, int np, int b0, int nb,
+__device__ __forceinline__ void colour_world_hybrid(const Ctx& c, int w, int p0, int np, int b0, int nb,
                                     unsigned char* pool, int* s_off, int* s_cur, int* sm) {
   int &s_left = sm[0], &s_taken = sm[1], &s_top = sm[2], &s_fill = sm[3];
   const int tid = threadIdx.x;
@@ -1110,7 +1114,7 @@ __global__ __launch_bounds__(64 * SWEEP_WAVES * SWEEP_PARTS) void k_sweep_waves(
 // in LDS and the manifold lists in global memory when the bodies fit, else in
 // global memory.
 template <int T>
-__device__ void colour_world(const Ctx& c, int w, int p0, int np, int pool_bytes, int* lds, int* sm) {
+__device__ __forceinline__ void colour_world(const Ctx& c, int w, int p0, int np, int pool_bytes, int* lds, int* sm) {
   int* s_off = lds;                      // COLOR_CAP + 3
   int* s_cur = lds + (COLOR_CAP + 3);    // COLOR_CAP + 3
   unsigned char* pool = (unsigned char*)(lds + 2 * (COLOR_CAP + 3) + 2);
@@ -1155,7 +1159,7 @@ __device__ void colour_world(const Ctx& c, int w, int p0, int np, int pool_bytes
 // *last tells the one that has to colour it.
 constexpr int FLOW_ITEMS = 8192, FLOW_COLOUR_LANES = 256;
 
-__device__ void colour_flow(const Ctx& c, int w, int p0, int np, int seat, int groups, int rows,
+__device__ __forceinline__ void colour_flow(const Ctx& c, int w, int p0, int np, int seat, int groups, int rows,
                             int* lds, bool* last) {
   constexpr int AGENT = __HIP_MEMORY_SCOPE_AGENT, T = FLOW_COLOUR_LANES;
   int* s_cnt = lds;                 // FLOW_DEGREE
