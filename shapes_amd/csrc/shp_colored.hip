@@ -1048,14 +1048,18 @@ __device__ __forceinline__ void wave_sync() {
 // bodies, FP32 velocities in the world's slice of LDS), SWEEP_WAVES of them to
 // a workgroup: the warm pass and the sweeps of sweep_prefetched, colour by
 // colour, by one wavefront with its own ordering of its LDS accesses between
-// colours, or, above SWEEP_ONE_WAVE_BODIES bodies, by SWEEP_PARTS wavefronts
-// that meet at a counter in LDS.  The same updates in the same colour order as
-// sweep_world, so the same results.  2048 worlds of 8 to 1024 bodies: 184 us,
-// 254 with one wavefront for each, the largest world's time; the rest is the
-// records, read again in each of 7 passes (0.6 GB).  Two wavefronts for the
-// larger worlds take 187; the line at 128 or 256 bodies makes no difference.
-__global__ __launch_bounds__(64 * SWEEP_WAVES * SWEEP_PARTS) void k_sweep_waves(Ctx c, int first_world,
-                                                                               int slice_floats) {
+// colours, or, above SWEEP_ONE_WAVE_BODIES bodies, by PARTS wavefronts that
+// meet at a counter in LDS (PARTS = 1: no world of the launch is that large).
+// The same updates in the same colour order as sweep_world, so the same
+// results.  2048 worlds of 8 to 1024 bodies: 184 us, 254 with one wavefront for
+// each, the largest world's time; the rest is the records, read again in each
+// of 7 passes (0.6 GB).  Two wavefronts for the larger worlds take 187; the
+// line at 128 or 256 bodies makes no difference there.  Without larger worlds
+// the other wavefronts would only hold places on the CUs: 4096 worlds of 64
+// bodies 95 us with PARTS = 1, 210 with 4.
+template <int PARTS>
+__global__ __launch_bounds__(64 * SWEEP_WAVES * PARTS) void k_sweep_waves(Ctx c, int first_world,
+                                                                         int slice_floats) {
   extern __shared__ __align__(16) int lds[];
   __shared__ int s_met[SWEEP_WAVES];
   if (threadIdx.x < SWEEP_WAVES) s_met[threadIdx.x] = 0;
@@ -1070,7 +1074,7 @@ __global__ __launch_bounds__(64 * SWEEP_WAVES * SWEEP_PARTS) void k_sweep_waves(
   const bool serial_tail = info & COL_TAIL;
   const int p0 = c.wpair_off[w];
   const int b0 = c.body_off[w], nb = c.body_off[w + 1] - b0;
-  const int parts = nb > SWEEP_ONE_WAVE_BODIES ? SWEEP_PARTS : 1;
+  const int parts = nb > SWEEP_ONE_WAVE_BODIES ? PARTS : 1;
   if (part >= parts) return;
   const int lane = 64 * part + (int)(threadIdx.x & 63), lanes = 64 * parts;
   const int* off = c.col_off + (long)w * (COLOR_CAP + 3);
@@ -1086,7 +1090,7 @@ __global__ __launch_bounds__(64 * SWEEP_WAVES * SWEEP_PARTS) void k_sweep_waves(
     }
     // every wavefront of the world runs (they are one workgroup's) and comes
     // here as often
-    meet += SWEEP_PARTS;
+    meet += PARTS;
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
     if ((threadIdx.x & 63) == 0)
       __hip_atomic_fetch_add(&s_met[slot], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
@@ -1687,8 +1691,8 @@ void plan_colored_solver(StepPlan* P, int solver_threads, const std::vector<int3
   const size_t fixed = (2 * (COLOR_CAP + 3) + 2) * 4;
   P->color_lds = std::min<size_t>(fixed + need, LDS_MAX_BYTES);
   P->color_pool = P->color_lds - fixed;
-  // 64: worlds of up to SWEEP_WAVE_MAX_BODIES sweep one wavefront each,
-  // the others (and the colouring) with 256 lanes
+  // 64: worlds of up to SWEEP_WAVE_MAX_BODIES sweep several to a workgroup, one
+  // wavefront each or a few, the others (and the colouring) with 256 lanes
   P->color_threads = solver_threads == 64 ? 256
                      : solver_threads     ? solver_threads
                                           : (nb > 2048 ? 512 : 256);
@@ -1732,8 +1736,10 @@ shp_status colored_alloc(shp_batch* b) {
                        : t == 512 ? (const void*)k_sweep_colours<512>
                                   : (const void*)k_sweep_colours<256>};
   const size_t ldsz[] = {P.color_lds, P.color_pool};
+  const void* waves = P.sweep_parts > 1 ? (const void*)k_sweep_waves<SWEEP_PARTS>
+                                        : (const void*)k_sweep_waves<1>;
   if (P.g_sweep_waves > 0 &&
-      hipFuncSetAttribute((const void*)k_sweep_waves, hipFuncAttributeMaxDynamicSharedMemorySize,
+      hipFuncSetAttribute(waves, hipFuncAttributeMaxDynamicSharedMemorySize,
                           (int)std::max<size_t>((size_t)SWEEP_WAVES * P.sweep_slice * 4, 16)) !=
           hipSuccess) {
     shp_set_error("hipFuncSetAttribute (wavefront sweeps LDS) failed");
@@ -1785,10 +1791,15 @@ void launch_colored_sweep(shp_batch* b) {
     else
       k_sweep_colours<256><<<grid, 256, P.color_pool, b->stream>>>(c, pool);
   }
-  if (P.g_sweep_waves > 0)
-    k_sweep_waves<<<(unsigned)P.g_sweep_waves, 64 * SWEEP_WAVES * SWEEP_PARTS,
-                    (size_t)SWEEP_WAVES * P.sweep_slice * 4, b->stream>>>(c, (int)big,
-                                                                         P.sweep_slice);
+  if (P.g_sweep_waves > 0) {
+    const size_t lds = (size_t)SWEEP_WAVES * P.sweep_slice * 4;
+    const unsigned grid = (unsigned)P.g_sweep_waves;
+    if (P.sweep_parts > 1)
+      k_sweep_waves<SWEEP_PARTS><<<grid, 64 * SWEEP_WAVES * SWEEP_PARTS, lds, b->stream>>>(
+          c, (int)big, P.sweep_slice);
+    else
+      k_sweep_waves<1><<<grid, 64 * SWEEP_WAVES, lds, b->stream>>>(c, (int)big, P.sweep_slice);
+  }
 }
 
 void launch_colored_unpack(shp_batch* b) {

@@ -23,10 +23,15 @@
 // coloured solver: colour offsets per world
 #define COLOR_CAP 256
 // several worlds to a workgroup in the coloured sweeps (solver_threads 64) for
-// worlds of up to this many bodies (1024 and what they stand on: a single
-// world of 1025 had a launch of its own, 80 us): SWEEP_WAVES of them, one
-// wavefront each or,
-// above SWEEP_ONE_WAVE_BODIES bodies, SWEEP_PARTS
+// worlds of up to SWEEP_WAVE_MAX_BODIES bodies: SWEEP_WAVES of them, one
+// wavefront each or, above SWEEP_ONE_WAVE_BODIES bodies, SWEEP_PARTS.  The line
+// takes in worlds of 1024 bodies and what they stand on.  Alone they would
+// rather have workgroups of their own (us a step, in this launch / in their
+// own, 1, 16, 64, 256 and 512 worlds of 1025 bodies: 223 / 215, 281 / 251, 330 /
+// 301, 514 / 463, 797 / 777; of 1600 bodies 276 / 268, 370 / 325, 441 / 393, 745
+// / 670, 1267 / 1270), but beside smaller worlds, whose launch this is, a second
+// one costs more: 1 of 1060 bodies and 255 of 600 370 / 437, 64 and 192 436 /
+// 480, 256 and 256 681 / 718, 256 and 64 553 / 600.
 #define SWEEP_WAVE_MAX_BODIES 1088
 #define SWEEP_WAVES 4
 #define SWEEP_PARTS 4
@@ -278,10 +283,11 @@ struct StepPlan {
   // colouring, instead of beside it with a packing pass after both
   bool records_in_contacts = false;
   // with solver_threads 64: the worlds of at most SWEEP_WAVE_MAX_BODIES
-  // bodies (world_order[sweep_big, W)) sweep one wavefront each, several
-  // per workgroup, velocities in the wavefront's LDS slice (floats)
+  // bodies (world_order[sweep_big, W)) sweep several to a workgroup, velocities
+  // in the world's LDS slice (floats), each by one wavefront, the larger ones
+  // of them by sweep_parts
   long sweep_big = 0, g_sweep_waves = 0;
-  int sweep_slice = 0;
+  int sweep_slice = 0, sweep_parts = 1;
   ScanPlan scan_buckets, scan_bodies, scan_pairs;
   long scan_parts_max = 0;  // scratch entries of the multi-workgroup scans
   // grids (workgroups) of the step's launches

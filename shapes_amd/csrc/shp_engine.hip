@@ -1695,6 +1695,7 @@ shp_status plan_staged(const shp_config& cfg, HostBatch* hb) {
     }
     P.sweep_big = big;
     P.sweep_slice = (int)((3 * small_max + 3) & ~3L);
+    P.sweep_parts = small_max > SWEEP_ONE_WAVE_BODIES ? SWEEP_PARTS : 1;
     P.g_sweep_waves = (n_worlds - big + SWEEP_WAVES - 1) / SWEEP_WAVES;
   }
 
@@ -1757,7 +1758,7 @@ void plan_launches(const StepPlan& P, bool infer, bool logging, std::vector<Laun
     if (P.sweep_big > 0)
       add("k_sweep_colours", P.sweep_big + flow_extra, P.color_threads, P.color_pool, colored_static_lds(true));
     if (P.g_sweep_waves > 0)
-      add("k_sweep_waves", P.g_sweep_waves, 64 * SWEEP_WAVES * SWEEP_PARTS,
+      add("k_sweep_waves", P.g_sweep_waves, 64 * SWEEP_WAVES * P.sweep_parts,
           (size_t)SWEEP_WAVES * P.sweep_slice * 4, lds16(SWEEP_WAVES * 4));
     add("k_colour_unpack", P.g_unpack, 256, 0, 0);
   } else {

@@ -44,3 +44,13 @@ def test_colours_past_the_limit(orc):
     b.step(4)
     assert b.stats()["flags"] == 0 and b.stats()["max_levels"] > 32
     b.close()
+
+
+@pytest.mark.parametrize("sizes", [(256, 2, 255, 90, 17), (3,), (1200, 250, 40)])
+def test_small_worlds_without_larger_ones(orc, sizes):
+    """The small worlds' sweeps when none of them takes more than a wavefront,
+    alone and beside a world with a workgroup of its own."""
+    worlds = [scenes.random_world(50 + k, count=n - 1, cols=max(4, int(n ** 0.5)))
+              for k, n in enumerate(sizes)]
+    print(f"worlds of {sizes} bodies", flush=True)
+    _colored_vs_restatement(orc, worlds, scenes.SceneConfig(iterations=5), steps=40, every=20, threads=64)
