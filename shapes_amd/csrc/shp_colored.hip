@@ -248,7 +248,7 @@ struct VelFlow {
       const bool b = t.of_b == 0 || ((uint32_t)(w[2] >> 48) == tb && (uint32_t)(w[3] >> 48) == tb);
       if ((a && b) || dead) break;
       if (n % 256 == 0) {
-        if (n >= FLOW_POLLS) {
+        if (n >= c->flow_polls) {
           atomicOr(&c->counters[CNT_FLAGS], SHP_FLAG_STALL);
           poke(abort, 1);
         }
@@ -1156,15 +1156,17 @@ __device__ __forceinline__ void colour_world(const Ctx& c, int w, int p0, int np
 // one CU: one pile of 32768 polygons 40 us (about 20 of them joining, ranking
 // and the places in the colours), 496 before; of 8192 30, 113 before.
 //
-// Returns true when the world's colours are complete (its last workgroup has
-// written col_off, col_info and flow_cnt, and flow_slot holds each pair's
-// colour and its place among those of its workgroup).  A world with a body of more than FLOW_DEGREE manifolds, more pairs
-// than the lanes hold, or colours past FLOW_DEGREE is left to one workgroup:
-// *last tells the one that has to colour it.
+// The world's last workgroup writes col_off, col_info and flow_cnt when all of
+// its colours are there; flow_slot holds each pair's colour and its place among
+// those of its workgroup.  A world with a body of more than FLOW_DEGREE
+// manifolds, more pairs than the lanes hold, or colours past FLOW_DEGREE is left
+// to one workgroup: *last tells the one that has to colour it.
 constexpr int FLOW_ITEMS = 8192, FLOW_COLOUR_LANES = 256;
 
-__device__ __forceinline__ void colour_flow(const Ctx& c, int w, int p0, int np, int seat, int groups, int rows,
-                            int* lds, bool* last) {
+// given_up: FC_BAD as one lane has read it for the workgroup; another one may set
+// it meanwhile, and all wavefronts have to take the same way past the barriers.
+__device__ __forceinline__ void colour_flow(const Ctx& c, int w, int p0, int np, int seat, int groups,
+                                            int rows, bool given_up, int* lds, bool* last) {
   constexpr int AGENT = __HIP_MEMORY_SCOPE_AGENT, T = FLOW_COLOUR_LANES;
   int* s_cnt = lds;                 // FLOW_DEGREE
   int* s_last = lds + FLOW_DEGREE;
@@ -1179,11 +1181,7 @@ __device__ __forceinline__ void colour_flow(const Ctx& c, int w, int p0, int np,
   const int q0 = seat * per, n = min(per, np - q0);
   const bool fits = per <= FLOW_ITEMS;
   if (tid < FLOW_DEGREE) s_cnt[tid] = 0;
-  // read once: another workgroup may set it meanwhile, and all wavefronts have
-  // to take the same way past the barriers below
-  if (tid == 0) *s_last = peek(ctl + FC_BAD);
-  __syncthreads();
-  if (fits && *s_last == 0) {
+  if (fits && !given_up) {
     auto key = [&](uint32_t q) {  // orders like prio64
       return (unsigned long long)(mix32(q * 0x9E3779B9u + (uint32_t)w) & 0x7FFFu) << 32 | q;
     };
@@ -1269,7 +1267,7 @@ __device__ __forceinline__ void colour_flow(const Ctx& c, int w, int p0, int np,
         }
       }
       if (polls % 64 == 0) {
-        if (polls >= FLOW_POLLS) {
+        if (polls >= c.flow_polls) {
           atomicOr(&c.counters[CNT_FLAGS], SHP_FLAG_STALL);
           bad = true;
         }
@@ -1368,11 +1366,14 @@ __global__ __launch_bounds__(T) void k_colour(Ctx c, int pool_bytes) {
     const int want = flow_want(c, w, c.flow_groups);
     if (blk % c.flow_groups >= want) return;
     int groups;
-    const int seat = flow_join(ctl + FC_SEATS, ctl + FC_GROUPS, blk % c.flow_groups, want, sm,
+    const int bad = threadIdx.x == 0 ? peek(ctl + FC_BAD) : 0;  // on its way while they join
+    const int seat = flow_join(c, ctl + FC_SEATS, ctl + FC_GROUPS, blk % c.flow_groups, want, sm,
                                &groups);
     if (seat < 0) return;
+    if (threadIdx.x == 0) sm[2] = bad;
+    __syncthreads();
     bool last;
-    colour_flow(c, w, p0, np, seat, groups, blk / c.flow_groups * c.flow_groups, lds, &last);
+    colour_flow(c, w, p0, np, seat, groups, blk / c.flow_groups * c.flow_groups, sm[2] != 0, lds, &last);
     if (!last) return;
   }
   colour_world<T>(c, w, p0, np, pool_bytes, lds, sm);
@@ -1395,6 +1396,10 @@ __global__ void k_pack_manifolds(Ctx c) {
   for (int p = blockIdx.x * blockDim.x + threadIdx.x; p < tp; p += gridDim.x * blockDim.x) {
     int M, turns = 0;
     const int w = c.flow_worlds ? c.body_world[c.pa[p]] : 0;
+    if (c.flow_worlds && c.col_info[w] == 0) {  // nothing to solve, or its colouring gave up
+      c.sched_order[p] = -1;
+      continue;
+    }
     if (c.flow_worlds && (c.col_info[w] & COL_FLOW)) {
       const int s = c.flow_slot[p], l = s & 31;
       const int* ctl = c.flow_ctl + (long)w * FLOW_CTL;
@@ -1610,7 +1615,7 @@ __global__ __launch_bounds__(T) void k_sweep_colours(Ctx c, int pool_bytes) {
     const int want = flow_want(c, w, c.flow_groups);
     if (blk % c.flow_groups >= want) return;
     int groups;
-    const int seat = flow_join(ctl + FS_SEATS, ctl + FS_GROUPS, blk % c.flow_groups, want, s_off,
+    const int seat = flow_join(c, ctl + FS_SEATS, ctl + FS_GROUPS, blk % c.flow_groups, want, s_off,
                                &groups);
     if (seat < 0) return;
     const FlowShare f = flow_share(c, w, ncol, seat, groups);

@@ -179,6 +179,7 @@ struct Ctx {
   // their number, the colouring's word and the velocity words (2 x NB); per
   // pair its colour and place in it; per workgroup its manifolds by colour
   int flow_worlds, flow_groups, flow_min;
+  int flow_seats, flow_polls;  // most workgroups that join a world; polls of a wait (shp_flow.h)
   int32_t* flow_ctl;
   uint32_t* adj;
   int32_t* adj_n;
@@ -242,6 +243,10 @@ __device__ __forceinline__ void begin_step(const Ctx& c) {
   if (c.flow_worlds == 0) return;
   const long step = (long)gridDim.x * blockDim.x;
   for (long i = t; i < (long)c.W * FLOW_CTL; i += step) c.flow_ctl[i] = 0;
+  // nothing to solve until a colouring has ended: a step whose colouring gives
+  // up must not take the last step's slots for its own
+  if (c.flow_col)
+    for (long k = t; k < c.flow_worlds; k += step) c.col_info[c.world_order[k]] = 0;
   for (long g = t; g < c.NB; g += step) {
     c.adj_n[g] = 0;
     if (c.flow_col) c.flow_col[FLOW_LINE * g] = 0ull;

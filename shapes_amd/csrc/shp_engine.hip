@@ -1942,6 +1942,8 @@ shp_status batch_alloc(shp_batch* b, const HostBatch& hb) {
   c.flow_worlds = P.flow_worlds;
   c.flow_groups = P.flow_groups;
   c.flow_min = P.flow_min;
+  c.flow_seats = FLOW_ANY_SEATS;
+  c.flow_polls = FLOW_POLLS;
   c.grid_buckets = (int)P.grid_buckets;
   c.host_flags = (int32_t*)b->stage;
   b->h_body_off = hb.body_off;
@@ -2084,6 +2086,17 @@ static shp_status capture_graph(shp_batch* b) {
 }
 
 extern "C" {
+
+// For the tests of worlds shared by workgroups: at most `seats` workgroups
+// join a world (the others leave as if they had come too late), and a wait
+// gives up after `polls`.
+shp_status shp_batch_flow_limits(shp_batch* b, int32_t seats, int32_t polls) {
+  if (!b || seats < 1 || polls < 0) return fail(SHP_E_INVAL, "bad argument");
+  b->ctx.flow_seats = std::min(seats, FLOW_ANY_SEATS);
+  b->ctx.flow_polls = polls;
+  b->graph_ready = false;  // kernel arguments changed
+  return SHP_OK;
+}
 
 shp_status shp_batch_destroy(shp_batch* b) {
   if (!b) return SHP_OK;

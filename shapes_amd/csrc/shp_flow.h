@@ -21,10 +21,13 @@ __device__ __forceinline__ void poke(X* p, X v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Polls before a wait on another workgroup gives up and flags the step.  The
-// waits end by themselves: what one waits for is held by a wavefront that has
-// joined the world, so that it runs, and comes earlier in the schedule.
+// Polls before a wait on another workgroup gives up and flags the step
+// (SHP_FLAG_STALL).  The waits end by themselves: what one waits for is held by
+// a wavefront that has joined the world, so that it runs, and comes earlier in
+// the schedule.
 constexpr int FLOW_POLLS = 1 << 20;
+// seats of a world beyond any grid's
+constexpr int FLOW_ANY_SEATS = 1 << 29;
 
 // 16 bytes past the L1 cache (sc1, as agent-scope atomics compile to; there is
 // none of 16 bytes): from two addresses, waiting for both, and to one.  A lane
@@ -50,7 +53,8 @@ __device__ __forceinline__ void store_16(void* p, u32x4 x) {
 // them must be running.  They join by a counter; the first to come closes it
 // once all `want` have joined or after a bounded wait (on a GPU busy with
 // other streams some may not have started), and those that come later leave.
-// Returns the caller's seat and their number in *groups (-1: leave).  Seats
+// Returns the caller's seat and their number in *groups (-1: leave; the seats
+// from c.flow_seats on leave too, as if they had come too late).  Seats
 // follow each other in space (pairs are in the order of their bodies), so
 // when all have come, those of an XCD, to which workgroups go in turn, are
 // consecutive: what neighbours exchange stays in its L2.
@@ -59,20 +63,25 @@ enum { FLOW_CLOSED = 1 << 30 };
 
 constexpr int XCDS = 8;
 
-static __device__ __forceinline__ int flow_join(int* seats, int* groups_word, int blk, int want, int* s_tmp,
-                                         int* groups) {
+static __device__ __forceinline__ int flow_join(const Ctx& c, int* seats, int* groups_word, int blk,
+                                                int want, int* s_tmp, int* groups) {
   if (threadIdx.x == 0) {
     constexpr int AGENT = __HIP_MEMORY_SCOPE_AGENT;
     int s = __hip_atomic_fetch_add(seats, 1, __ATOMIC_RELAXED, AGENT), g = 0;
-    if (s & FLOW_CLOSED) {
+    if (s >= c.flow_seats) {  // closed, or one too many
       s = -1;
     } else if (s == 0) {
-      for (int n = 0; n < FLOW_JOIN_POLLS && peek(seats) < want; ++n) __builtin_amdgcn_s_sleep(1);
-      g = __hip_atomic_fetch_or(seats, FLOW_CLOSED, __ATOMIC_RELAXED, AGENT);
+      for (int n = 0; n < FLOW_JOIN_POLLS && peek(seats) < min(want, c.flow_seats); ++n)
+        __builtin_amdgcn_s_sleep(1);
+      g = min(__hip_atomic_fetch_or(seats, FLOW_CLOSED, __ATOMIC_RELAXED, AGENT), c.flow_seats);
       poke(groups_word, g);
     } else {  // the first one runs and always writes it
-      for (int n = 0; n < FLOW_POLLS && (g = peek(groups_word)) == 0; ++n) __builtin_amdgcn_s_sleep(1);
-      if (g == 0) s = -1;
+      for (int n = 0; n < c.flow_polls && (g = peek(groups_word)) == 0; ++n)
+        __builtin_amdgcn_s_sleep(1);
+      if (g == 0) {  // counted in, and now missing
+        atomicOr(&c.counters[CNT_FLAGS], SHP_FLAG_STALL);
+        s = -1;
+      }
     }
     if (g == want) s = blk % XCDS * (want / XCDS) + min(blk % XCDS, want % XCDS) + blk / XCDS;
     s_tmp[0] = s;

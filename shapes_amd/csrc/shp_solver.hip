@@ -725,7 +725,7 @@ __global__ __launch_bounds__(256) void k_solve_flow(Ctx c) {
   }
   if (blk >= want) return;
   int groups;
-  const int seat = flow_join(ctl + FS_SEATS, ctl + FS_GROUPS, blk, want, s_tmp, &groups);
+  const int seat = flow_join(c, ctl + FS_SEATS, ctl + FS_GROUPS, blk, want, s_tmp, &groups);
   if (seat < 0) return;
   if (groups < want) {
     if (seat == 0 && threadIdx.x == 0) ctl[FS_ALONE] = 1;
@@ -801,7 +801,7 @@ __global__ __launch_bounds__(256) void k_solve_flow(Ctx c) {
       polls = 0;  // what remains to wait for has come nearer
     }
     if (polls % 256 == 255) {
-      if (polls >= FLOW_POLLS - 1) {
+      if (polls >= c.flow_polls - 1) {
         atomicOr(&c.counters[CNT_FLAGS], SHP_FLAG_STALL);
         poke(ctl + FS_ABORT, 1);
       }

@@ -1,5 +1,8 @@
 """Worlds solved by several workgroups where that path ends: colours past its
-limit, told by one workgroup while others of the world still start."""
+limit, fewer workgroups than wanted, records that fill a workgroup's LDS, waits
+that give up; and batches that they share the GPU or the launch with."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -54,3 +57,87 @@ def test_small_worlds_without_larger_ones(orc, sizes):
               for k, n in enumerate(sizes)]
     print(f"worlds of {sizes} bodies", flush=True)
     _colored_vs_restatement(orc, worlds, scenes.SceneConfig(iterations=5), steps=40, every=20, threads=64)
+
+
+def _pile(n, seed=78, cols=60):
+    rng = np.random.Generator(np.random.Philox(seed))
+    return scenes.grid_world(rng, n, cols=cols, spacing=1.05, y0=1.0, square_frac=0.5, vel=0.3)
+
+
+def _limit(batch, seats=1 << 29, polls=1 << 20):
+    f = batch._L.shp_batch_flow_limits  # for tests: not in the header
+    f.argtypes = [C.c_void_p, C.c_int32, C.c_int32]
+    assert f(batch._h, seats, polls) == 0
+
+
+def _bits(worlds, cfg, steps, limit=None, **kw):
+    b = engine.make_batch(worlds, cfg, **kw)
+    if limit is not None:
+        _limit(b, seats=limit)
+    for k in range(2):
+        b.step_async(steps, use_graph=k == 1)
+        b.sync()
+        assert b.stats()["flags"] == 0
+    out = [(b.bodies(k).view(np.uint64), b.contacts(k)["lam"].view(np.uint64)) for k in range(len(worlds))]
+    b.close()
+    return out
+
+
+@pytest.mark.parametrize("solver", [engine.SOLVER_ORDERED_F64, engine.SOLVER_COLORED_F32])
+@pytest.mark.parametrize("n,n2", [(4096, 3300), (20000, 3300)])
+def test_fewer_workgroups_than_wanted(solver, n, n2):
+    """As many workgroups join as a busy GPU has room for: the ordered solver
+    leaves the world to one, the coloured colours and sweeps it with those,
+    or with one when their records do not fit in LDS."""
+    worlds, cfg = [_pile(n), _pile(30, 5, 8), _pile(n2, 4)], scenes.SceneConfig(iterations=3)
+    st, msg, _, rows = engine.plan(worlds, cfg, solver=solver)
+    r = {x["name"]: x["workgroups"] for x in rows}
+    assert st == 0 and (r.get("k_solve_flow", 0) > 40 or r["k_colour"] > 40), msg
+    want = _bits(worlds, cfg, 6, solver=solver)
+    for seats in (1, 2, 7, 33):
+        print(f"{n} bodies, solver {solver}, {seats} seats", flush=True)
+        got = _bits(worlds, cfg, 6, limit=seats, solver=solver)
+        for (a, b), (x, y) in zip(want, got):
+            assert len(b) and np.array_equal(a, x) and np.array_equal(b, y), seats
+
+
+@pytest.mark.parametrize("solver", [engine.SOLVER_ORDERED_F64, engine.SOLVER_COLORED_F32])
+def test_a_wait_that_gives_up_is_reported(solver):
+    """A workgroup that leaves its world after it was counted in (the waits end
+    at once here): the others' waits end too, and the step says so."""
+    b = engine.make_batch([_pile(4096)], scenes.SceneConfig(iterations=2), solver=solver)
+    _limit(b, polls=0)
+    print(f"waits that give up, solver {solver}", flush=True)
+    with pytest.raises(engine.ShapesError, match="wait between workgroups"):
+        b.step(1)
+    assert b.stats()["flags"] & 16
+    b.close()
+
+
+def test_batches_on_the_gpu_at_once():
+    """Batches whose shared worlds want every CU, stepped on their streams at
+    the same time."""
+    cfg = scenes.SceneConfig(iterations=3)
+    kinds = [(engine.SOLVER_COLORED_F32, 24000), (engine.SOLVER_ORDERED_F64, 12000),
+             (engine.SOLVER_COLORED_F32, 16000)]
+    want = [_bits([_pile(n)], cfg, 6, solver=s) for s, n in kinds]
+    print("three batches at once", flush=True)
+    bs = [engine.make_batch([_pile(n)], cfg, solver=s) for s, n in kinds]
+    for k in range(12):
+        for b in bs:
+            b.step_async(1, use_graph=k >= 6)
+    for b, ((x, lam),) in zip(bs, want):
+        b.sync()
+        assert b.stats()["flags"] == 0
+        assert np.array_equal(b.bodies(0).view(np.uint64), x)
+        assert np.array_equal(b.contacts(0)["lam"].view(np.uint64), lam)
+        b.close()
+
+
+def test_shared_world_beside_small_worlds_sweeps(orc):
+    """solver_threads 64 with a world for several workgroups, one for one, and
+    small ones of both forms."""
+    worlds = [scenes.random_world(60, count=300, cols=18), _pile(2600, 2, 40),
+              scenes.random_world(61, count=40), _pile(1500, 3, 30)]
+    print("shared, single and small worlds", flush=True)
+    _colored_vs_restatement(orc, worlds, scenes.SceneConfig(iterations=4), steps=8, every=4, threads=64)
