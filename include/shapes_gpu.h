@@ -136,7 +136,9 @@ typedef struct shp_step_stats {
   int64_t misses;       /* contacts absent from last frame's cache */
   int32_t max_levels;   /* most colours of a world (coloured solver) */
   int32_t flags;        /* bit 0 pair overflow, 1 contact overflow,
-                           2 non-finite, 3 coloured schedule overflow */
+                           2 non-finite, 3 coloured schedule overflow,
+                           4 a wait between workgroups ran out (a defect);
+                           with those that earlier calls have reported */
   /* Solve quality after the last sweep (FP64 state), maxima over contacts
    * of: penetration depth, |min(lambda_n, Jn.v + b)| and
    * |lambda_t - clamp(lambda_t - Jt.v / mt, +-mu*lambda_n)|; for the last
@@ -168,8 +170,9 @@ shp_status shp_batch_destroy(shp_batch* b);
 shp_status shp_batch_step(shp_batch* b, int32_t n_steps);
 
 /* Enqueue n_steps on the handle's stream without waiting; shp_batch_sync
- * waits and reports deferred errors.  With use_graph != 0 each step is
- * replayed from a captured HIP graph. */
+ * waits and reports deferred errors, those of any step since the last
+ * call that waited.  With use_graph != 0 each step is replayed from a
+ * captured HIP graph. */
 shp_status shp_batch_step_async(shp_batch* b, int32_t n_steps,
                                 int32_t use_graph);
 shp_status shp_batch_sync(shp_batch* b);

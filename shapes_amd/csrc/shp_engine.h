@@ -76,7 +76,9 @@ enum { COL_TAIL = 1 << 16, COL_FLOW = 1 << 17 };
 
 // bytes before the rows in a batch's pinned readback memory
 enum { STAGE_FLAGS = 64 };
-enum { CNT_FLAGS = 0, CNT_WARM = 1, CNT_LEARNED = 2, CNT_LEVELS = 3, CNT_MISS = 4, CNT_MANIFOLDS = 5 };
+// (CNT_SEEN: the flags of all steps so far)
+enum { CNT_FLAGS = 0, CNT_WARM = 1, CNT_LEARNED = 2, CNT_LEVELS = 3, CNT_MISS = 4, CNT_MANIFOLDS = 5,
+       CNT_SEEN = 6 };
 // grid broadphase: partners per body kept by the count pass for the emit
 // pass (bodies with more are visited again)
 enum { GRID_SLOTS = 8 };
@@ -224,7 +226,7 @@ struct Ctx {
   int32_t* grid_slots;
   int32_t *large_off, *large_ids;
   int32_t* counters;  // 8 ints: flags, warm hits, learned starts, levels
-  int32_t* host_flags;  // pinned host memory: the last step's flags
+  int32_t* host_flags;  // pinned host memory: the flags of all steps so far
   unsigned long long* quality;  // Q_ENTRIES entries, see Q_*
   // per workgroup of k_finish its quality maxima (3 x MAX_PARTS), of
   // k_contacts its warm hits and manifolds (MAX_PARTS)
@@ -238,7 +240,7 @@ struct Ctx {
 // kernel of its own for that took 4 to 5 us of every step.
 __device__ __forceinline__ void begin_step(const Ctx& c) {
   const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t < 8) c.counters[t] = 0;
+  if (t < 8 && t != CNT_SEEN) c.counters[t] = 0;
   if (t < 3) c.quality[t] = 0ull;  // Q_DEPTH ..
   if (c.flow_worlds == 0) return;
   const long step = (long)gridDim.x * blockDim.x;
@@ -357,11 +359,11 @@ struct shp_batch {
   bool graph_ready = false;  // ... and it matches the current kernel arguments
   int32_t last_flags = 0;
   std::vector<void*> allocs;
-  // pinned host memory the readback kernels write: the last step's flags
-  // (STAGE_FLAGS bytes), then stage_bytes for one call's rows
+  // pinned host memory the kernels write: the steps' flags (STAGE_FLAGS
+  // bytes), then stage_bytes for one call's rows
   unsigned char* stage = nullptr;
   size_t stage_bytes = 0;
-  // the device's flags are newer than the pinned copy (a placement or a probe
+  // the device has flags that the pinned copy lacks (a placement or a probe
   // since the last step)
   bool flags_on_device = false;
   // per-phase event timing (shp_batch_set_timing)

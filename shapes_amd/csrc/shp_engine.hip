@@ -898,7 +898,8 @@ __global__ __launch_bounds__(256) void k_cache_store(Ctx c, int n_quality, int n
       c.counters[CNT_WARM] = (s_sum[0][0] + s_sum[0][1]) + (s_sum[0][2] + s_sum[0][3]);
       c.counters[CNT_MANIFOLDS] = (s_sum[1][0] + s_sum[1][1]) + (s_sum[1][2] + s_sum[1][3]);
       c.quality[Q_STEPS] += 1;
-      *c.host_flags = c.counters[CNT_FLAGS];
+      // a flag stays up through the steps of a call, until the host reads it
+      *c.host_flags = c.counters[CNT_SEEN] |= c.counters[CNT_FLAGS];
     }
   }
   int stride = gridDim.x * blockDim.x;
@@ -2004,15 +2005,15 @@ shp_status batch_alloc(shp_batch* b, const HostBatch& hb) {
   return SHP_OK;
 }
 
-// Waits for the batch's stream and reports what the flags say: the last
-// step's, which its last kernel wrote to the pinned memory, or the device's
+// Waits for the batch's stream and reports what the flags say: those of the
+// steps, which their last kernel wrote to the pinned memory, and the device's
 // own after a placement or a probe, which end before that kernel.
 static shp_status check_flags(shp_batch* b) {
   HIPCHK(hipStreamSynchronize(b->stream));
-  int32_t flags = *(volatile int32_t*)b->stage;
+  int32_t placed = 0;
   if (b->flags_on_device)
-    HIPCHK(hipMemcpy(&flags, b->ctx.counters + CNT_FLAGS, 4, hipMemcpyDeviceToHost));
-  b->last_flags |= flags;
+    HIPCHK(hipMemcpy(&placed, b->ctx.counters + CNT_FLAGS, 4, hipMemcpyDeviceToHost));
+  b->last_flags |= *(volatile int32_t*)b->stage | placed;
   if (b->last_flags & (SHP_FLAG_PAIR_OVERFLOW | SHP_FLAG_CONTACT_OVERFLOW))
     return fail(SHP_E_OVERFLOW, "pair/contact capacity exceeded; raise max_pairs_per_body");
   if (b->last_flags & SHP_FLAG_STALL) return fail(SHP_E_HIP, "a wait between workgroups ran out");
@@ -2582,6 +2583,7 @@ static shp_status rebuild_with(shp_batch* b, long g, const StagedBody& s) {
   unsigned long long q[Q_ENTRIES], logc = 0;
   HIPCHK(hipMemcpy(q, c.quality, sizeof(q), hipMemcpyDeviceToHost));
   HIPCHK(hipMemcpy(&logc, c.log_count, 8, hipMemcpyDeviceToHost));
+  b->last_flags |= *(volatile int32_t*)b->stage;  // unread; the counters start again
   const Ctx keep = c;
   const StepPlan old_plan = P;
 
