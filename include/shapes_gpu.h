@@ -356,8 +356,8 @@ shp_status shp_mlp_train(shp_mlp* m, const int32_t* indices, int32_t steps,
  * 1 broadphase count (with gravity), 2 pair scan, 3 broadphase fill, 4 SAT,
  * 5 contact scan, 6 world ranges, 7 contacts (constraintGen + warm-start
  * join), 8 learned inference, 9 solve set-up (the coloured solver: the wait
- * for the colouring and the manifold packing), 10 sweeps (k_sweep_colours or
- * k_solve_ordered), 11 solve write-back (coloured: k_colour_unpack), 12 advance
+ * for the colouring and the manifold packing), 10 sweeps (k_sweep_colours
+ * and k_sweep_waves, or k_solve_flow and k_solve_ordered), 11 solve write-back (coloured: k_colour_unpack), 12 advance
  * + moveShapes + AABBs + solve quality (k_finish), 13 cache store; and 14
  * the coloured solver's colouring (k_colour), timed on the second stream,
  * where it overlaps phases 5-9. */
@@ -369,10 +369,14 @@ shp_status shp_batch_set_timing(shp_batch* b, int32_t enable);
 /* Accumulated milliseconds per phase and the number of timed steps. */
 shp_status shp_batch_read_timing(shp_batch* b, double* ms_per_phase,
                                  int32_t* steps);
-/* Average microseconds per timed step of the solve's sub-phases in world 0:
- * ordered: 0 the schedule's links, 1 velocity and lagrangian staging, 2 -, 3
- * warm-start pass and sweeps, 4 write-back; coloured: 0 colouring, 1 bucketing + packing +
- * velocity staging, 2 warm-start pass, 3 sweeps, 4 write-back. */
+/* Average microseconds per timed step of the solve's sub-phases in the largest
+ * world: ordered: 0 the schedule's links, 1 velocity and lagrangian staging,
+ * 2 -, 3 warm-start pass and sweeps, 4 write-back; coloured: 0 colouring, 1 from
+ * its end to the sweeps' start (packing, velocity staging), 2 -, 3 warm-start
+ * pass and sweeps, 4 write-back.  A world solved by several workgroups: from the
+ * first one's start to the last one's end; ordered: 0 is the loading of the
+ * records, 1 and 4 are 0.  All 0 for a world whose sweeps share a workgroup
+ * with others (solver_threads 64). */
 shp_status shp_batch_read_solve_profile(shp_batch* b, double* us5);
 
 /* ---- plan and audit of a batch (no counterpart in the reference) -------

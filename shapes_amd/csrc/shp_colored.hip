@@ -1340,6 +1340,7 @@ __device__ __forceinline__ void colour_flow(const Ctx& c, int w, int p0, int np,
     ctl[FC_SHARE] = per;
     c.col_info[w] = ncol | COL_FLOW;  // also without a manifold: flow_slot says so
     atomicMax(&c.counters[CNT_LEVELS], ncol);
+    tmark(c, w, 1);
   }
 }
 
@@ -1360,7 +1361,7 @@ __global__ __launch_bounds__(T) void k_colour(Ctx c, int pool_bytes) {
     if (threadIdx.x == 0) c.col_info[w] = 0;
     return;
   }
-  tmark(c, 0);
+  if (!flow || blk % c.flow_groups == 0) tmark(c, w, 0);
   if (flow) {
     int* ctl = c.flow_ctl + (long)w * FLOW_CTL;
     const int want = flow_want(c, w, c.flow_groups);
@@ -1377,7 +1378,7 @@ __global__ __launch_bounds__(T) void k_colour(Ctx c, int pool_bytes) {
     if (!last) return;
   }
   colour_world<T>(c, w, p0, np, pool_bytes, lds, sm);
-  tmark(c, 1);
+  tmark(c, w, 1);
 }
 
 // Every coloured pair's <= 2 contacts become its manifold record, over the
@@ -1486,11 +1487,11 @@ __device__ void sweep_world(const Ctx& c, int w, int ncol, bool serial_tail, flo
       if (i0 + u * T < nb) V.store(b0 + i0 + u * T, x[u]);
   }
   __syncthreads();
-  tmark(c, 2);
-  tmark(c, 3);
+  tmark(c, w, 2);
+  tmark(c, w, 3);
   const PackF P = packf(c);
   sweep_colours<VLDS, T>(c, recw(c, P, p0), ncol, serial_tail, s_off, V);
-  tmark(c, 4);
+  tmark(c, w, 4);
   // (every phase ends with a barrier) the final FP32 velocities to global
   // memory, for k_colour_unpack
   if (VLDS) {
@@ -1500,7 +1501,7 @@ __device__ void sweep_world(const Ctx& c, int w, int ncol, bool serial_tail, flo
       c.fv[b0 + i] = make_float4(v[0], v[1], v[2], 0.0f);
     }
   }
-  tmark(c, 5);
+  tmark(c, w, 5);
 }
 
 // The sweeps of a world by several workgroups, one wavefront of each, whose
@@ -1545,7 +1546,7 @@ __device__ __forceinline__ FlowShare flow_share(const Ctx& c, int w, int ncol, i
   return f;
 }
 
-__device__ void sweep_flow(const Ctx& c, int w, int ncol, const FlowShare f, float4* recs) {
+__device__ void sweep_flow(const Ctx& c, int w, int ncol, int seat, const FlowShare f, float4* recs) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
   const int step = f.all;  // between a record's words
   const PackF P = packf(c);
@@ -1565,6 +1566,8 @@ __device__ void sweep_flow(const Ctx& c, int w, int ncol, const FlowShare f, flo
     }
   }
   __syncthreads();
+  if (seat == 0)
+    for (int k = 2; k < 4; ++k) tmark(c, w, k);
   if (wave == 0) {
     const int passes = c.iterations + 1;
     VelFlow V;
@@ -1588,6 +1591,7 @@ __device__ void sweep_flow(const Ctx& c, int w, int ncol, const FlowShare f, flo
       }
   }
   __syncthreads();
+  if (wave == 0) tmark_last(c, w, 4);
   for (int l = wave; l < ncol; l += waves) {
     const int i0 = __builtin_amdgcn_readlane(f.first, l), i1 = __builtin_amdgcn_readlane(f.last, l);
     const int s0 = __builtin_amdgcn_readlane(f.start, l) - i0;
@@ -1596,6 +1600,7 @@ __device__ void sweep_flow(const Ctx& c, int w, int ncol, const FlowShare f, flo
       *(float4*)lambda_of(R, i, 1) = recs[(REC_WORDS + 3) * step + s0 + i];
     }
   }
+  tmark_last(c, w, 5);
 }
 
 // The flow worlds' workgroups, then one workgroup per world, the largest
@@ -1620,7 +1625,7 @@ __global__ __launch_bounds__(T) void k_sweep_colours(Ctx c, int pool_bytes) {
     if (seat < 0) return;
     const FlowShare f = flow_share(c, w, ncol, seat, groups);
     if ((long)f.most * FLOW_REC_BYTES <= pool_bytes) {
-      sweep_flow(c, w, ncol, f, (float4*)lds);
+      sweep_flow(c, w, ncol, seat, f, (float4*)lds);
       return;
     }
     // records that do not fit in LDS: one workgroup

@@ -15,11 +15,15 @@ namespace shp {
 
 __device__ __forceinline__ bool body_static(const Ctx& c, int g) { return c.is_static[g] != 0; }
 
-// Solver sub-phase timestamp k of world 0 (timing mode only).
-__device__ __forceinline__ void tmark(const Ctx& c, int k) {
-  if (c.tstamp && blockIdx.x == 0 && threadIdx.x == 0) c.tstamp[k] = wall_clock64();
+// Solver sub-phase timestamp k of the largest world (timing mode only): the
+// lane's time, if w is that world, and the latest of several wavefronts'.
+__device__ __forceinline__ void tmark(const Ctx& c, int w, int k) {
+  if (c.tstamp && threadIdx.x == 0 && w == c.world_order[0]) c.tstamp[k] = wall_clock64();
 }
-
+__device__ __forceinline__ void tmark_last(const Ctx& c, int w, int k) {
+  if (c.tstamp && (threadIdx.x & 63) == 0 && w == c.world_order[0])
+    atomicMax(c.tstamp + k, (unsigned long long)wall_clock64());
+}
 
 __device__ __forceinline__ void load_vel(const Ctx& c, int ga, int gb, double* v) {
   v[0] = c.vx[ga];

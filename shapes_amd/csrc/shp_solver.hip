@@ -578,7 +578,7 @@ __device__ __forceinline__ void run_levels(const Ctx& c, const Sched<L>& Q,
 
 template <int T, bool L>
 __device__ __forceinline__ void solve_world(const Ctx& c, const Sched<L>& Q, unsigned char* pool,
-                                            long pool_bytes, int c0, int n, int b0, int nb,
+                                            long pool_bytes, int w, int c0, int n, int b0, int nb,
                                             const Front<T, L>& fr, int* wsum) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int2* ab = c.sch_ab + c0;
@@ -602,7 +602,7 @@ __device__ __forceinline__ void solve_world(const Ctx& c, const Sched<L>& Q, uns
       fr.put(0, base + (int)__popcll(bal & ((1ull << lane) - 1ull)), t & ~Sched<L>::ONE, true);
   }
   __syncthreads();
-  tmark(c, 1);
+  tmark(c, w, 1);
   // velocities, then lagrangians, in the rest of the LDS pool (over the
   // build's per-body arrays)
   const bool vlds = 24L * nb <= pool_bytes;
@@ -630,8 +630,8 @@ __device__ __forceinline__ void solve_world(const Ctx& c, const Sched<L>& Q, uns
     }
   }
   __syncthreads();
-  tmark(c, 2);
-  tmark(c, 3);
+  tmark(c, w, 2);
+  tmark(c, w, 3);
   if (llds)
     run_levels<T, L, true, true>(c, Q, OState<true, true>{vel, lam, &c, b0, c0}, fr);
   else if (vlds)
@@ -639,7 +639,7 @@ __device__ __forceinline__ void solve_world(const Ctx& c, const Sched<L>& Q, uns
   else
     run_levels<T, L, false, false>(c, Q, OState<false, false>{vel, lam, &c, b0, c0}, fr);
   __syncthreads();
-  tmark(c, 4);
+  tmark(c, w, 4);
   for (int k = tid; k < n; k += T) {
     double2 l;
     if (llds)
@@ -664,7 +664,7 @@ __device__ __forceinline__ void solve_world(const Ctx& c, const Sched<L>& Q, uns
     }
   }
   __syncthreads();
-  tmark(c, 5);
+  tmark(c, w, 5);
 }
 
 // ---- one world on several CUs ----------------------------------------------
@@ -731,6 +731,7 @@ __global__ __launch_bounds__(256) void k_solve_flow(Ctx c) {
     if (seat == 0 && threadIdx.x == 0) ctl[FS_ALONE] = 1;
     return;
   }
+  if (seat == 0) tmark(c, w, 0);
   const int side = threadIdx.x & 1, q = seat * FLOW_ORDERED_PAIRS + ((int)threadIdx.x >> 1);
   const int p = p0 + q, passes = c.iterations + 1;
   ORec r;
@@ -770,6 +771,8 @@ __global__ __launch_bounds__(256) void k_solve_flow(Ctx c) {
   }
   const unsigned long long* word = c.flow_vel + FLOW_LINE * (long)(alive ? S.g : b0);
   int rest = 0;
+  if (seat == 0)
+    for (int k = 1; k < 4; ++k) tmark(c, w, k);
   for (int polls = 1; __ballot(alive); ++polls) {
     bool ready = alive && id < 0;
     if (alive && id >= 0) {
@@ -808,6 +811,8 @@ __global__ __launch_bounds__(256) void k_solve_flow(Ctx c) {
       if (peek(ctl + FS_ABORT) != 0) return;
     }
   }
+  tmark_last(c, w, 4);  // (a manifold's last item has written its results back)
+  tmark_last(c, w, 5);
 }
 
 template <int T>
@@ -824,7 +829,7 @@ __global__ __launch_bounds__(T) void k_solve_ordered(Ctx c, int pool_bytes) {
   if ((int)blockIdx.x < c.flow_worlds && c.flow_ctl[(long)w * FLOW_CTL + FS_ALONE] == 0) return;
   const int n = c1 - c0;
   const int b0 = c.body_off[w], nb = c.body_off[w + 1] - b0;
-  tmark(c, 0);
+  tmark(c, w, 0);
   if (tid < 2 * RING) s_width[tid] = 0;
   for (int i = tid; i < front_bytes(T) / 4; i += T) s_front[i] = 0;
   uint32_t* glob = c.sch_glob + (3L + RING) * c0;
@@ -838,7 +843,7 @@ __global__ __launch_bounds__(T) void k_solve_ordered(Ctx c, int pool_bytes) {
     Q.cnt = Q.next + 2 * n;
     Q.off = (uint16_t*)(pool + hot);
     Q.first = (uint16_t*)(pool + hot + body2);
-    solve_world<T, true>(c, Q, pool + hot, pool_bytes - hot, c0, n, b0, nb,
+    solve_world<T, true>(c, Q, pool + hot, pool_bytes - hot, w, c0, n, b0, nb,
                          Front<T, true>{(uint16_t*)s_front, glob + 3L * n, s_width, n}, wsum);
   } else {
     Sched<false> Q;
@@ -846,7 +851,7 @@ __global__ __launch_bounds__(T) void k_solve_ordered(Ctx c, int pool_bytes) {
     Q.cnt = glob + 2L * n;
     Q.off = (uint32_t*)c.sch_off + b0;
     Q.first = (uint32_t*)c.sch_first + b0;
-    solve_world<T, false>(c, Q, pool, pool_bytes, c0, n, b0, nb,
+    solve_world<T, false>(c, Q, pool, pool_bytes, w, c0, n, b0, nb,
                           Front<T, false>{(uint32_t*)s_front, glob + 3L * n, s_width, n}, wsum);
   }
 }

@@ -141,3 +141,23 @@ def test_shared_world_beside_small_worlds_sweeps(orc):
               scenes.random_world(61, count=40), _pile(1500, 3, 30)]
     print("shared, single and small worlds", flush=True)
     _colored_vs_restatement(orc, worlds, scenes.SceneConfig(iterations=4), steps=8, every=4, threads=64)
+
+
+@pytest.mark.parametrize("solver", [engine.SOLVER_ORDERED_F64, engine.SOLVER_COLORED_F32])
+@pytest.mark.parametrize("seats", [1 << 29, 3])
+def test_solve_profile_of_a_shared_world(solver, seats):
+    """The solve's sub-phases are timed whoever solves the largest world, which
+    is the second here."""
+    b = engine.make_batch([_pile(40, 3, 8), _pile(5000)], scenes.SceneConfig(iterations=6), solver=solver)
+    _limit(b, seats=seats)
+    b.step(10)
+    b.set_timing(True)
+    print(f"solve profile, solver {solver}, {seats} seats", flush=True)
+    b.step(20)
+    us, ms = b.solve_profile(), b.timing()
+    b.close()
+    assert us[3] > 5 and us[0] > 0
+    coloured = solver == engine.SOLVER_COLORED_F32
+    assert us[3] + us[4] <= 1e3 * ms["sweeps"] + 1
+    if coloured:
+        assert us[0] <= 1e3 * ms["colouring"] + 1
