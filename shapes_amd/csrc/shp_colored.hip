@@ -216,6 +216,7 @@ struct VelF {
 // a line, 96 with one; with the 16-byte accesses 88).
 struct VelFlow {
   const Ctx* c;
+  unsigned long long* vel;  // the line of body 0, whose world's bodies have theirs
   int* abort;
   mutable bool dead;
   mutable unsigned long long w[4];  // the words as loaded
@@ -235,8 +236,7 @@ struct VelFlow {
     const Turns t = unpack_turns(m.turns);
     const uint32_t ta = (uint32_t)(pass * t.of_a + t.at_a) & 0xFFFFu,
                    tb = (uint32_t)(pass * t.of_b + t.at_b) & 0xFFFFu;
-    const unsigned long long *pa = c->flow_vel + FLOW_LINE * (long)m.ga,
-                             *pb = c->flow_vel + FLOW_LINE * (long)m.gb;
+    const unsigned long long *pa = vel + FLOW_LINE * (long)m.ga, *pb = vel + FLOW_LINE * (long)m.gb;
     for (int n = 1;; ++n) {
       u32x4 x, y;
       load_pair(pa, pb, x, y);
@@ -269,7 +269,7 @@ struct VelFlow {
       unpack(old[0], old[1], y);
       pack(keep ? y : x, turn, n);
       const u32x4 x4 = {(uint32_t)n[0], (uint32_t)(n[0] >> 32), (uint32_t)n[1], (uint32_t)(n[1] >> 32)};
-      store_16(c->flow_vel + FLOW_LINE * (long)g, x4);
+      store_16(vel + FLOW_LINE * (long)g, x4);
     };
     if (t.of_a) hand_on(m.ga, w, v, !changed || (m.flags & MFL_A_STATIC));
     if (t.of_b) hand_on(m.gb, w + 2, v + 3, !changed || (m.flags & MFL_B_STATIC));
@@ -1157,8 +1157,11 @@ __device__ __forceinline__ void colour_world(const Ctx& c, int w, int p0, int np
 // and the places in the colours), 496 before; of 8192 30, 113 before.
 //
 // The world's last workgroup writes col_off, col_info and flow_cnt when all of
-// its colours are there; flow_slot holds each pair's colour and its place among
-// those of its workgroup.  A world with a body of more than FLOW_DEGREE
+// its colours are there; sched_level then holds each pair's colour and its place
+// among those of its workgroup, from which the packing pass makes its slot in
+// sched_order.  (Not written here: the workgroup that colours the world alone
+// after all writes sched_order, and what another XCD's L2 still holds of an
+// array could come after it.)  A world with a body of more than FLOW_DEGREE
 // manifolds, more pairs than the lanes hold, or colours past FLOW_DEGREE is left
 // to one workgroup: *last tells the one that has to colour it.
 constexpr int FLOW_ITEMS = 8192, FLOW_COLOUR_LANES = 256;
@@ -1176,7 +1179,7 @@ __device__ __forceinline__ void colour_flow(const Ctx& c, int w, int p0, int np,
   uint16_t* s_rank = (uint16_t*)(s_ab + FLOW_ITEMS);
   uint8_t* s_col = (uint8_t*)(s_rank + FLOW_ITEMS);
   int* ctl = c.flow_ctl + (long)w * FLOW_CTL;
-  const int tid = threadIdx.x, b0 = c.body_off[w];
+  const int tid = threadIdx.x, f0 = c.body_off[w] + c.flow_shift[w];
   const int per = ((np + groups - 1) / groups + 63) & ~63;
   const int q0 = seat * per, n = min(per, np - q0);
   const bool fits = per <= FLOW_ITEMS;
@@ -1198,7 +1201,7 @@ __device__ __forceinline__ void colour_flow(const Ctx& c, int w, int p0, int np,
 #pragma unroll
       for (int s = 0; s < 2; ++s) {
         const uint32_t loc = s ? ab >> 16 : ab & 0xFFFFu;
-        const int g = b0 + (loc == NO_BODY ? 0 : (int)loc);
+        const int g = f0 + (loc == NO_BODY ? 0 : (int)loc);
         row[s] = (const int4*)(c.adj + (long)g * FLOW_DEGREE);
         m[s] = loc == NO_BODY ? 0 : c.adj_n[g];
         e[s][0] = row[s][0];
@@ -1241,8 +1244,8 @@ __device__ __forceinline__ void colour_flow(const Ctx& c, int w, int p0, int np,
           ab[j] = s_ab[i];
           rank[j] = s_rank[i];
           const uint32_t a = ab[j] & 0xFFFFu, b = ab[j] >> 16;
-          wa[j] = a != NO_BODY ? peek(c.flow_col + FLOW_LINE * (long)(b0 + a)) : 0ull;
-          wb[j] = b != NO_BODY ? peek(c.flow_col + FLOW_LINE * (long)(b0 + b)) : 0ull;
+          wa[j] = a != NO_BODY ? peek(c.flow_col + FLOW_LINE * (long)(f0 + a)) : 0ull;
+          wb[j] = b != NO_BODY ? peek(c.flow_col + FLOW_LINE * (long)(f0 + b)) : 0ull;
         }
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
@@ -1259,8 +1262,8 @@ __device__ __forceinline__ void colour_flow(const Ctx& c, int w, int p0, int np,
           const unsigned long long up = (unsigned long long)min(round + 1, JP_ROUNDS) << 48;
           auto hand_on = [&](uint32_t loc, unsigned long long x) {
             if (loc == NO_BODY) return;
-            poke(c.flow_col + FLOW_LINE * (long)(b0 + loc), up | ((((x >> 32) & 0xFFFFull) + 1ull) << 32) |
-                                            (uint32_t)(x | (ok ? 1ull << l : 0ull)));
+            poke(c.flow_col + FLOW_LINE * (long)(f0 + loc),
+                 up | ((((x >> 32) & 0xFFFFull) + 1ull) << 32) | (uint32_t)(x | (ok ? 1ull << l : 0ull)));
           };
           hand_on(ab[j] & 0xFFFFu, wa[j]);
           hand_on(ab[j] >> 16, wb[j]);
@@ -1287,7 +1290,7 @@ __device__ __forceinline__ void colour_flow(const Ctx& c, int w, int p0, int np,
     if (tid < FLOW_DEGREE) poke(c.flow_cnt + (rows + seat) * FLOW_DEGREE + tid, s_cnt[tid]);
     for (int i = tid; i < n; i += lanes) {
       const int l = s_col[i];
-      c.flow_slot[p0 + q0 + i] = l == 0xFF ? -1 : (int)s_ab[i] << 5 | l;
+      c.sched_level[p0 + q0 + i] = l == 0xFF ? -1 : (int)s_ab[i] << 5 | l;
     }
   }
   // the last workgroup (the others' counts and flags are in: their stores were
@@ -1338,7 +1341,7 @@ __device__ __forceinline__ void colour_flow(const Ctx& c, int w, int p0, int np,
   if (tid == 0) {
     ctl[FC_ROWS] = rows;
     ctl[FC_SHARE] = per;
-    c.col_info[w] = ncol | COL_FLOW;  // also without a manifold: flow_slot says so
+    c.col_info[w] = ncol | COL_FLOW;  // also without a manifold: sched_level says so
     atomicMax(&c.counters[CNT_LEVELS], ncol);
     tmark(c, w, 1);
   }
@@ -1388,11 +1391,12 @@ __global__ void k_pack_manifolds(Ctx c) {
   const int tp = c.wpair_off[c.W];
   const PackF P = packf(c);
   if (c.flow_worlds)  // the bodies' first velocity words
-    for (int g = blockIdx.x * blockDim.x + threadIdx.x; g < c.NB; g += gridDim.x * blockDim.x) {
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < c.flow_bodies; i += gridDim.x * blockDim.x) {
+      const int g = c.flow_body[i];
       const float v[3] = {(float)c.vx[g], (float)c.vy[g], (float)c.w[g]};
       unsigned long long x[2];
       VelFlow::pack(v, 0, x);
-      *(ulonglong2*)(c.flow_vel + FLOW_LINE * (long)g) = make_ulonglong2(x[0], x[1]);
+      *(ulonglong2*)(c.flow_vel + FLOW_LINE * (long)i) = make_ulonglong2(x[0], x[1]);
     }
   for (int p = blockIdx.x * blockDim.x + threadIdx.x; p < tp; p += gridDim.x * blockDim.x) {
     int M, turns = 0;
@@ -1402,15 +1406,16 @@ __global__ void k_pack_manifolds(Ctx c) {
       continue;
     }
     if (c.flow_worlds && (c.col_info[w] & COL_FLOW)) {
-      const int s = c.flow_slot[p], l = s & 31;
+      const int s = c.sched_level[p], l = s & 31;
       const int* ctl = c.flow_ctl + (long)w * FLOW_CTL;
       const int p0 = c.wpair_off[w], row = ctl[FC_ROWS] + (p - p0) / ctl[FC_SHARE];
       M = s < 0 ? -1
                 : p0 + c.col_off[(long)w * (COLOR_CAP + 3) + l] +
                       c.flow_cnt[row * FLOW_DEGREE + l] + (s >> 5);
       c.sched_order[p] = M;
+      const int shift = c.flow_shift[w];
       auto turn = [&](int g, int& at, int& of) {
-        const uint32_t used = c.is_static[g] ? 0u : (uint32_t)c.flow_col[FLOW_LINE * (long)g];
+        const uint32_t used = c.is_static[g] ? 0u : (uint32_t)c.flow_col[FLOW_LINE * (long)(g + shift)];
         at = __popc(used & ((1u << l) - 1u));
         of = __popc(used);
       };
@@ -1572,6 +1577,7 @@ __device__ void sweep_flow(const Ctx& c, int w, int ncol, int seat, const FlowSh
     const int passes = c.iterations + 1;
     VelFlow V;
     V.c = &c;
+    V.vel = c.flow_vel + FLOW_LINE * (long)c.flow_shift[w];
     V.abort = c.flow_ctl + (long)w * FLOW_CTL + FS_ABORT;
     V.dead = false;
     for (int pass = 0; pass < passes; ++pass)
@@ -1669,8 +1675,9 @@ __global__ void k_colour_unpack(Ctx c) {
       const int info = c.col_info[c.body_world[g]];
       if (!c.is_static[g] && (info & 0xFFFF) != 0) {
         float f[3];
-        if ((info & COL_FLOW) && !c.flow_ctl[(long)c.body_world[g] * FLOW_CTL + FS_ALONE]) {
-          const ulonglong2 x = *(const ulonglong2*)(c.flow_vel + FLOW_LINE * (long)g);
+        const int w = c.body_world[g];
+        if ((info & COL_FLOW) && !c.flow_ctl[(long)w * FLOW_CTL + FS_ALONE]) {
+          const ulonglong2 x = *(const ulonglong2*)(c.flow_vel + FLOW_LINE * (long)(g + c.flow_shift[w]));
           VelFlow::unpack(x.x, x.y, f);
         } else {
           const float4 x = c.fv[g];

@@ -61,8 +61,8 @@ enum { FLOW_MIN_BODIES = 2048, FLOW_GROUP_BODIES = 64, FLOW_GROUP_MAX = 384,
        FLOW_MAX_GROUPS = 256, FLOW_DEGREE = 32, FLOW_CTL = 32, FLOW_LINE = 16 };
 enum { FC_SEATS = 0, FC_GROUPS = 1, FC_DONE = 2, FC_BAD = 3, FS_SEATS = 4, FS_GROUPS = 5,
        FS_ABORT = 6, FS_ALONE = 7, FC_ROWS = 8, FC_SHARE = 9 };
-// col_info: colours | serial tail << 16 | flow schedule << 17 (then the pairs'
-// slots come from flow_slot, and sched_order is written by the packing pass)
+// col_info: colours | serial tail << 16 | flow schedule << 17 (then sched_level
+// holds colours and places, and sched_order is written by the packing pass)
 enum { COL_TAIL = 1 << 16, COL_FLOW = 1 << 17 };
 
 // pair_ab words (coloured solver): world-local body ids a | b << 16, NO_BODY
@@ -177,16 +177,18 @@ struct Ctx {
   int32_t* col_off;   // per world: COLOR_CAP + 3 colour offsets (manifolds)
   int32_t* col_info;  // per world: colours, COL_* flags (0: nothing to solve)
   // worlds solved on several CUs: how many (the largest), the workgroups of
-  // the largest; control words per world; per body its manifolds' pairs and
-  // their number, the colouring's word and the velocity words (2 x NB); per
-  // pair its colour and place in it; per workgroup its manifolds by colour
-  int flow_worlds, flow_groups, flow_min;
+  // the largest; control words per world; the bodies of those worlds, one world
+  // after another, and what a world's body ids are off by there; per such body
+  // its manifolds' pairs and their number, the colouring's word and the
+  // velocity words (a line each); per workgroup its manifolds by colour
+  int flow_worlds, flow_groups, flow_min, flow_bodies;
+  int32_t *flow_body, *flow_shift;
   int flow_seats, flow_polls;  // most workgroups that join a world; polls of a wait (shp_flow.h)
   int32_t* flow_ctl;
   uint32_t* adj;
   int32_t* adj_n;
   unsigned long long *flow_col, *flow_vel;
-  int32_t *flow_slot, *flow_cnt;
+  int32_t* flow_cnt;
   // solver sub-phase timestamps of world 0 (wall_clock64), timing mode only
   unsigned long long* tstamp;
   unsigned long long* tstamp_store;
@@ -249,9 +251,9 @@ __device__ __forceinline__ void begin_step(const Ctx& c) {
   // up must not take the last step's slots for its own
   if (c.flow_col)
     for (long k = t; k < c.flow_worlds; k += step) c.col_info[c.world_order[k]] = 0;
-  for (long g = t; g < c.NB; g += step) {
-    c.adj_n[g] = 0;
-    if (c.flow_col) c.flow_col[FLOW_LINE * g] = 0ull;
+  for (long i = t; i < c.flow_bodies; i += step) {
+    c.adj_n[i] = 0;
+    if (c.flow_col) c.flow_col[FLOW_LINE * i] = 0ull;
   }
 }
 #endif
@@ -286,6 +288,7 @@ struct StepPlan {
   // the flow_worlds largest worlds (above flow_min bodies) are solved by up to
   // flow_groups workgroups each
   int flow_worlds = 0, flow_groups = 0, flow_min = 0;
+  long flow_bodies = 0;  // of those worlds
   // the contact kernel writes the manifold records itself, after the
   // colouring, instead of beside it with a packing pass after both
   bool records_in_contacts = false;
@@ -321,6 +324,7 @@ struct HostBatch {
   std::vector<double> rad;    // circle radius, 0 for a hull
   std::vector<uint8_t> is_static, is_large, dead;
   std::vector<int32_t> body_world, vert_off, body_off, order, tab_off, large_off, large_ids;
+  std::vector<int32_t> flow_body, flow_shift;
   std::vector<double> lx, ly, cell;
 };
 

@@ -436,10 +436,11 @@ __device__ __forceinline__ void sat_pair(const Ctx& c, int p) {
   }
   if (n > 0 && c.flow_worlds && c.body_off[w + 1] - b0 > c.flow_min) {
     // the dynamic bodies' lists of manifolds
-    const int ia = sa ? 0 : atomicAdd(&c.adj_n[ga], 1);
-    const int ib = sb ? 0 : atomicAdd(&c.adj_n[gb], 1);
-    if (!sa && ia < FLOW_DEGREE) c.adj[(long)ga * FLOW_DEGREE + ia] = (uint32_t)p;
-    if (!sb && ib < FLOW_DEGREE) c.adj[(long)gb * FLOW_DEGREE + ib] = (uint32_t)p;
+    const int fa = ga + c.flow_shift[w], fb = gb + c.flow_shift[w];
+    const int ia = sa ? 0 : atomicAdd(&c.adj_n[fa], 1);
+    const int ib = sb ? 0 : atomicAdd(&c.adj_n[fb], 1);
+    if (!sa && ia < FLOW_DEGREE) c.adj[(long)fa * FLOW_DEGREE + ia] = (uint32_t)p;
+    if (!sb && ib < FLOW_DEGREE) c.adj[(long)fb * FLOW_DEGREE + ib] = (uint32_t)p;
     if (max(ia, ib) >= FLOW_DEGREE) c.flow_ctl[w * FLOW_CTL + FC_BAD] = 1;
   }
 }
@@ -449,11 +450,12 @@ __device__ __forceinline__ void sat_pair(const Ctx& c, int p) {
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_sat(Ctx c) {
   int tp = total_pairs(c);
   if (c.solver == SHP_SOLVER_ORDERED_F64 && c.flow_worlds)  // the bodies' first velocity words
-    for (int g = blockIdx.x * blockDim.x + threadIdx.x; g < c.NB; g += gridDim.x * blockDim.x) {
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < c.flow_bodies; i += gridDim.x * blockDim.x) {
+      const int g = c.flow_body[i];
       const double v[3] = {c.vx[g], c.vy[g], c.w[g]};
       u32x4 x[2];
       flow_pack(v, 0, x);
-      u32x4* to = (u32x4*)(c.flow_vel + FLOW_LINE * (long)g);
+      u32x4* to = (u32x4*)(c.flow_vel + FLOW_LINE * (long)i);
       to[0] = x[0];
       to[1] = x[1];
     }
@@ -1470,16 +1472,17 @@ static void batch_buffers(const StepPlan& P, Ctx& c, int32_t** scan_part, std::v
     add(&c.col_info, W * 4);
     add(&c.pair_ab, PC * 4);
     if (P.flow_worlds > 0) {
-      add(&c.flow_col, NB * FLOW_LINE * 8);
-      add(&c.flow_slot, PC * 4);
+      add(&c.flow_col, P.flow_bodies * FLOW_LINE * 8);
       add(&c.flow_cnt, (size_t)P.flow_worlds * P.flow_groups * FLOW_DEGREE * 4);
     }
   }
   if (P.flow_worlds > 0) {
     add(&c.flow_ctl, W * FLOW_CTL * 4);
-    add(&c.adj, NB * FLOW_DEGREE * 4);
-    add(&c.adj_n, NB * 4);
-    add(&c.flow_vel, NB * FLOW_LINE * 8);
+    add(&c.flow_shift, W * 4);
+    add(&c.flow_body, P.flow_bodies * 4);
+    add(&c.adj, P.flow_bodies * FLOW_DEGREE * 4);
+    add(&c.adj_n, P.flow_bodies * 4);
+    add(&c.flow_vel, P.flow_bodies * FLOW_LINE * 8);
   }
 }
 
@@ -1683,6 +1686,14 @@ shp_status plan_staged(const shp_config& cfg, HostBatch* hb) {
     plan_ordered_solver(&P, cfg.solver_threads, body_off, hb->order);
   else
     plan_colored_solver(&P, cfg.solver_threads, body_off, hb->order);
+  hb->flow_body.clear();
+  hb->flow_shift.assign(n_worlds, 0);
+  for (int k = 0; k < P.flow_worlds; ++k) {
+    const int w = hb->order[k];
+    hb->flow_shift[w] = (int32_t)hb->flow_body.size() - body_off[w];
+    for (int gg = body_off[w]; gg < body_off[w + 1]; ++gg) hb->flow_body.push_back(gg);
+  }
+  P.flow_bodies = (long)hb->flow_body.size();
   P.sweep_big = n_worlds;
   if (cfg.solver == SHP_SOLVER_COLORED_F32 && cfg.solver_threads == 64) {
     // worlds by descending size: the small ones form the tail of the order
@@ -1943,6 +1954,7 @@ shp_status batch_alloc(shp_batch* b, const HostBatch& hb) {
   c.flow_worlds = P.flow_worlds;
   c.flow_groups = P.flow_groups;
   c.flow_min = P.flow_min;
+  c.flow_bodies = (int)P.flow_bodies;
   c.flow_seats = FLOW_ANY_SEATS;
   c.flow_polls = FLOW_POLLS;
   c.grid_buckets = (int)P.grid_buckets;
@@ -1969,6 +1981,10 @@ shp_status batch_alloc(shp_batch* b, const HostBatch& hb) {
   HIPCHK(hipMemcpy(c.vert_off, hb.vert_off.data(), (NB + 1) * 4, hipMemcpyHostToDevice));
   HIPCHK(hipMemcpy(c.body_off, hb.body_off.data(), (n_worlds + 1) * 4, hipMemcpyHostToDevice));
   HIPCHK(hipMemcpy(c.world_order, hb.order.data(), n_worlds * 4, hipMemcpyHostToDevice));
+  if (P.flow_worlds > 0) {
+    HIPCHK(hipMemcpy(c.flow_shift, hb.flow_shift.data(), n_worlds * 4, hipMemcpyHostToDevice));
+    HIPCHK(hipMemcpy(c.flow_body, hb.flow_body.data(), hb.flow_body.size() * 4, hipMemcpyHostToDevice));
+  }
   HIPCHK(hipMemcpy(c.lx, hb.lx.data(), NV * 8, hipMemcpyHostToDevice));
   HIPCHK(hipMemcpy(c.ly, hb.ly.data(), NV * 8, hipMemcpyHostToDevice));
   if (P.use_grid) {

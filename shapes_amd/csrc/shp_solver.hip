@@ -688,6 +688,7 @@ struct OFlow {
   u32x4 x, y;  // the body's words as loaded
   double lam[2];
   int g, last;  // the body; its last manifold's pass, else -1
+  unsigned long long* word;  // the body's words
   int pass;
   __device__ __forceinline__ void load(int, int, int, double* v) const {
     flow_unpack(x, y, v);
@@ -696,9 +697,8 @@ struct OFlow {
     if (fixed) return;
     u32x4 n[2];
     flow_pack(v, (x[1] >> 16) + 1u, n);
-    unsigned long long* to = c->flow_vel + FLOW_LINE * (long)g;
-    store_16(to, n[0]);
-    store_16(to + 2, n[1]);
+    store_16(word, n[0]);
+    store_16(word + 2, n[1]);
     if (pass == last) {
       c->vx[g] = v[0];
       c->vy[g] = v[1];
@@ -733,7 +733,7 @@ __global__ __launch_bounds__(256) void k_solve_flow(Ctx c) {
   }
   if (seat == 0) tmark(c, w, 0);
   const int side = threadIdx.x & 1, q = seat * FLOW_ORDERED_PAIRS + ((int)threadIdx.x >> 1);
-  const int p = p0 + q, passes = c.iterations + 1;
+  const int p = p0 + q, passes = c.iterations + 1, shift = c.flow_shift[w];
   ORec r;
   OFlow S;
   S.c = &c;
@@ -751,8 +751,8 @@ __global__ __launch_bounds__(256) void k_solve_flow(Ctx c) {
     S.lam[0] = side ? ln[0] : lt[0];
     S.lam[1] = (id & FLOW_TWO) == 0 ? 0.0 : side ? ln[1] : lt[1];
     if (id >= 0) {
-      of = c.adj_n[S.g];
-      const int4* row = (const int4*)(c.adj + (long)S.g * FLOW_DEGREE);
+      of = c.adj_n[S.g + shift];
+      const int4* row = (const int4*)(c.adj + (long)(S.g + shift) * FLOW_DEGREE);
       for (int e = 0; e < of; e += 4) {
         const int4 x = row[e / 4];
         at += x.x < p;
@@ -769,7 +769,7 @@ __global__ __launch_bounds__(256) void k_solve_flow(Ctx c) {
     }
     S.last = at == of - 1 ? passes - 1 : -1;
   }
-  const unsigned long long* word = c.flow_vel + FLOW_LINE * (long)(alive ? S.g : b0);
+  S.word = c.flow_vel + FLOW_LINE * (long)((alive ? S.g : b0) + shift);
   int rest = 0;
   if (seat == 0)
     for (int k = 1; k < 4; ++k) tmark(c, w, k);
@@ -780,7 +780,7 @@ __global__ __launch_bounds__(256) void k_solve_flow(Ctx c) {
         --rest;
       } else {
         const uint32_t turn = (uint32_t)(S.pass * of + at) & 0xFFFFu;
-        load_pair(word, word + 2, S.x, S.y);
+        load_pair(S.word, S.word + 2, S.x, S.y);
         ready = S.x[1] >> 16 == turn && S.x[3] >> 16 == turn && S.y[1] >> 16 == turn &&
                 S.y[3] >> 16 == turn;
         rest = ready ? 0 : min(((int)(turn - (S.x[1] >> 16)) & 0xFFFF) - 1, 7);
