@@ -326,6 +326,8 @@ shp_status shp_mlp_forward(shp_mlp* m, const float* feats, int32_t n,
  * forbid hipMalloc): d_feats (n x 14 FP32) and d_out (n x 2 FP32) are
  * device pointers on the handle's GPU, n <= 65536.  One launch and no memory
  * of its own: the call allocates nothing, and calls on different streams may
+ * overlap.  The two buffers may share memory: then the outputs go through the
+ * handle's own (a second launch), and two such calls of one handle must not
  * overlap.  Enqueued on `stream` (a hipStream_t; NULL: the handle's stream)
  * and returns without waiting. */
 shp_status shp_mlp_forward_noalloc(shp_mlp* m, const float* d_feats,

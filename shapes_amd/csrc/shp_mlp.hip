@@ -567,6 +567,14 @@ __global__ __launch_bounds__(512) void k_mlp_weights(const uint16_t* __restrict_
   if (e < 386) apply_gradient(step, i, g, true);
 }
 
+// outputs of a call on overlapping buffers, to where they belong
+__global__ void k_mlp_place(const float2* y, int n, float* out) {
+  const int r = blockIdx.x * blockDim.x + threadIdx.x;
+  if (r >= n) return;
+  out[2 * (size_t)r] = y[r].x;
+  out[2 * (size_t)r + 1] = y[r].y;
+}
+
 // 4 workgroups on each of 256 CUs
 void launch_eval(const MlpParams& p, const float* feats, int n, float* out, hipStream_t s) {
   const int tiles = (n + 15) / 16;
@@ -741,11 +749,15 @@ void mlp_launch_log(shp_batch* b) {
 
 // ---- training handle -------------------------------------------------------
 
+// rows of one shp_mlp_forward_noalloc call
+#define MLP_NOALLOC_MAX_ROWS 65536
+
 struct shp_mlp {
   int device = 0;  // the GPU the handle's weights live on
   hipStream_t stream = nullptr;
   MlpParams p{};
   float *mom = nullptr, *vel = nullptr, *grad = nullptr;
+  float2* staged = nullptr;  // MLP_NOALLOC_MAX_ROWS outputs
   // of cap_tiles training tiles: fragments and bias sums (k_mlp_rows)
   int cap_tiles = 0;
   uint16_t* frags = nullptr;
@@ -768,9 +780,6 @@ static shp_status mlp_fail(shp_status s, const char* m) {
   shp_set_error(m);
   return s;
 }
-
-// rows of one shp_mlp_forward_noalloc call
-#define MLP_NOALLOC_MAX_ROWS 65536
 
 #define MCHK(x) \
   do { if ((x) != hipSuccess) return mlp_fail(SHP_E_HIP, #x); } while (0)
@@ -833,7 +842,8 @@ shp_status shp_mlp_create(const float* params, shp_mlp** out) {
   if (st == SHP_OK) st = mlp_params_upload(&h->p, params, h->stream);
   if (st == SHP_OK) {
     if (hipMalloc(&h->mom, MLP_NPARAM_PAD * 4) != hipSuccess || hipMalloc(&h->vel, MLP_NPARAM_PAD * 4) != hipSuccess ||
-        hipMalloc(&h->grad, MLP_NPARAM_PAD * 4) != hipSuccess)
+        hipMalloc(&h->grad, MLP_NPARAM_PAD * 4) != hipSuccess ||
+        hipMalloc(&h->staged, MLP_NOALLOC_MAX_ROWS * sizeof(float2)) != hipSuccess)
       st = SHP_E_OOM;
   }
   if (st == SHP_OK) {
@@ -855,7 +865,7 @@ shp_status shp_mlp_destroy(shp_mlp* h) {
   if (!h) return SHP_OK;
   if (h->stream) (void)hipStreamSynchronize(h->stream);
   mlp_params_free(&h->p);
-  void* ptrs[] = {h->mom, h->vel, h->grad, h->frags, h->bsum, h->T, h->Fin,
+  void* ptrs[] = {h->mom, h->vel, h->grad, h->staged, h->frags, h->bsum, h->T, h->Fin,
                   h->out, h->didx, h->dX, h->dT};
   for (void* q : ptrs)
     if (q) (void)hipFree(q);
@@ -895,7 +905,12 @@ shp_status shp_mlp_forward_noalloc(shp_mlp* h, const float* d_feats, int32_t n, 
   int dev = -1;
   MCHK(hipGetDevice(&dev));
   if (dev != h->device) return mlp_fail(SHP_E_INVAL, "the current device is not the handle's");
-  launch_eval(h->p, d_feats, n, d_out, stream ? (hipStream_t)stream : h->stream);
+  const hipStream_t s = stream ? (hipStream_t)stream : h->stream;
+  // a workgroup's outputs must not reach rows that another one has yet to read
+  const uintptr_t in = (uintptr_t)d_feats, out = (uintptr_t)d_out;
+  const bool overlap = in < out + (size_t)n * 2 * 4 && out < in + (size_t)n * MLP_IN * 4;
+  launch_eval(h->p, d_feats, n, overlap ? (float*)h->staged : d_out, s);
+  if (overlap) k_mlp_place<<<(n + 255) / 256, 256, 0, s>>>(h->staged, n, d_out);
   MCHK(hipGetLastError());
   return SHP_OK;
 }
