@@ -16,8 +16,6 @@ CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "libshapes_gpu.so")
 SOURCES = ["shp_engine.hip", "shp_solver.hip", "shp_colored.hip", "shp_mlp.hip", "shp_grid.hip"]
-HEADERS = ["shp_engine.h", "shp_geom.h", "shp_trig.h", "shp_solve_common.h", "shp_mlp.h",
-           os.path.join("..", "..", "include", "shapes_gpu.h")]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = ["--offload-arch=gfx950"]

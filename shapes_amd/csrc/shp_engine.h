@@ -36,9 +36,6 @@
 #define SWEEP_WAVES 4
 #define SWEEP_PARTS 4
 #define SWEEP_ONE_WAVE_BODIES 256
-// the coloured solver keeps a world's FP32 velocities (12 B per body) in
-// LDS up to this many bodies; beyond, in global memory
-#define VEL_LDS_MAX_BODIES ((LDS_MAX_BYTES - (2 * (COLOR_CAP + 3) + 2) * 4) / 12)
 // the ordered solver's FP64 records (16-byte words per contact slot,
 // shp_records.h) and its global schedule scratch (words per contact slot)
 enum { FLOW_WORDS = 8, SCH_GLOB = 7 };
@@ -246,7 +243,8 @@ __device__ __forceinline__ void begin_step(const Ctx& c) {
   if (t < 3) c.quality[t] = 0ull;  // Q_DEPTH ..
   if (c.flow_worlds == 0) return;
   const long step = (long)gridDim.x * blockDim.x;
-  for (long i = t; i < (long)c.W * FLOW_CTL; i += step) c.flow_ctl[i] = 0;
+  for (long i = t; i < (long)c.flow_worlds * FLOW_CTL; i += step)
+    c.flow_ctl[(long)c.world_order[i / FLOW_CTL] * FLOW_CTL + i % FLOW_CTL] = 0;
   // nothing to solve until a colouring has ended: a step whose colouring gives
   // up must not take the last step's slots for its own
   if (c.flow_col)

@@ -34,12 +34,6 @@ __device__ __forceinline__ void load_vel(const Ctx& c, int ga, int gb, double* v
   v[5] = c.w[gb];
 }
 
-// applyLagrangian (Constraint.hs:182-221): v_k + ((j_k * l) * im_k)
-__device__ __forceinline__ void apply_lag(double l, const double* j, const double* im, double* v) {
-#pragma unroll
-  for (int k = 0; k < 6; ++k) v[k] = v[k] + ((j[k] * l) * im[k]);
-}
-
 // The row normal u of contact k: jn[3..4] as constraint generation computes
 // them, n for a pair in order and -n for a flipped one (whose halves are
 // swapped back).  Then jn = (-u, jn2, u, jn5) and jt = (-cw(u), jt2, cw(u),
