@@ -1364,7 +1364,7 @@ __global__ __launch_bounds__(T) void k_colour(Ctx c, int pool_bytes) {
     if (threadIdx.x == 0) c.col_info[w] = 0;
     return;
   }
-  if (!flow || blk % c.flow_groups == 0) tmark(c, w, 0);
+  if (blk == 0) tmark(c, w, 0);
   if (flow) {
     int* ctl = c.flow_ctl + (long)w * FLOW_CTL;
     const int want = flow_want(c, w, c.flow_groups);
@@ -1551,7 +1551,7 @@ __device__ __forceinline__ FlowShare flow_share(const Ctx& c, int w, int ncol, i
   return f;
 }
 
-__device__ void sweep_flow(const Ctx& c, int w, int ncol, int seat, const FlowShare f, float4* recs) {
+__device__ void sweep_flow(const Ctx& c, int w, int ncol, const FlowShare f, float4* recs) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
   const int step = f.all;  // between a record's words
   const PackF P = packf(c);
@@ -1571,8 +1571,6 @@ __device__ void sweep_flow(const Ctx& c, int w, int ncol, int seat, const FlowSh
     }
   }
   __syncthreads();
-  if (seat == 0)
-    for (int k = 2; k < 4; ++k) tmark(c, w, k);
   if (wave == 0) {
     const int passes = c.iterations + 1;
     VelFlow V;
@@ -1597,7 +1595,6 @@ __device__ void sweep_flow(const Ctx& c, int w, int ncol, int seat, const FlowSh
       }
   }
   __syncthreads();
-  if (wave == 0) tmark_last(c, w, 4);
   for (int l = wave; l < ncol; l += waves) {
     const int i0 = __builtin_amdgcn_readlane(f.first, l), i1 = __builtin_amdgcn_readlane(f.last, l);
     const int s0 = __builtin_amdgcn_readlane(f.start, l) - i0;
@@ -1606,7 +1603,6 @@ __device__ void sweep_flow(const Ctx& c, int w, int ncol, int seat, const FlowSh
       *(float4*)lambda_of(R, i, 1) = recs[(REC_WORDS + 3) * step + s0 + i];
     }
   }
-  tmark_last(c, w, 5);
 }
 
 // The flow worlds' workgroups, then one workgroup per world, the largest
@@ -1621,6 +1617,10 @@ __global__ __launch_bounds__(T) void k_sweep_colours(Ctx c, int pool_bytes) {
   const int info = c.col_info[w];
   const int ncol = info & 0xFFFF;
   if (ncol == 0) return;
+  // (a shared world's sweeps are timed from here to the next kernel's start:
+  // stamps inside them took 2 us)
+  if (blk == 0)
+    for (int k = 2; k < 4; ++k) tmark(c, w, k);
   if (flow && (info & COL_FLOW)) {
     int* ctl = c.flow_ctl + (long)w * FLOW_CTL;
     const int want = flow_want(c, w, c.flow_groups);
@@ -1631,7 +1631,7 @@ __global__ __launch_bounds__(T) void k_sweep_colours(Ctx c, int pool_bytes) {
     if (seat < 0) return;
     const FlowShare f = flow_share(c, w, ncol, seat, groups);
     if ((long)f.most * FLOW_REC_BYTES <= pool_bytes) {
-      sweep_flow(c, w, ncol, seat, f, (float4*)lds);
+      sweep_flow(c, w, ncol, f, (float4*)lds);
       return;
     }
     // records that do not fit in LDS: one workgroup
@@ -1655,6 +1655,9 @@ __global__ void k_colour_unpack(Ctx c) {
   const long tp = c.wpair_off[c.W];
   const long n = tp > c.NB ? tp : (long)c.NB;
   const PackF P = packf(c);
+  if (c.tstamp && blockIdx.x == 0 && (c.col_info[c.world_order[0]] & COL_FLOW) &&
+      !c.flow_ctl[(long)c.world_order[0] * FLOW_CTL + FS_ALONE])
+    for (int k = 4; k < 6; ++k) tmark(c, c.world_order[0], k);
   for (long t = blockIdx.x * (long)blockDim.x + threadIdx.x; t < n;
        t += (long)gridDim.x * blockDim.x) {
     if (t < tp) {
@@ -1735,7 +1738,6 @@ void plan_colored_solver(StepPlan* P, int solver_threads, const std::vector<int3
     if (groups * FLOW_GROUP_MAX >= nb) {
       P->flow_worlds = big;
       P->flow_groups = (int)groups;
-      P->flow_min = FLOW_MIN_BODIES;
       P->color_lds = LDS_MAX_BYTES;
       P->color_pool = P->color_lds - fixed;
     }

@@ -61,6 +61,8 @@ enum { FC_SEATS = 0, FC_GROUPS = 1, FC_DONE = 2, FC_BAD = 3, FS_SEATS = 4, FS_GR
 // col_info: colours | serial tail << 16 | flow schedule << 17 (then sched_level
 // holds colours and places, and sched_order is written by the packing pass)
 enum { COL_TAIL = 1 << 16, COL_FLOW = 1 << 17 };
+// flow_shift of a world that no several workgroups share
+constexpr int NOT_SHARED = -2147483647 - 1;
 
 // pair_ab words (coloured solver): world-local body ids a | b << 16, NO_BODY
 // for a static body, NO_PAIR for a pair without contacts
@@ -175,10 +177,11 @@ struct Ctx {
   int32_t* col_info;  // per world: colours, COL_* flags (0: nothing to solve)
   // worlds solved on several CUs: how many (the largest), the workgroups of
   // the largest; control words per world; the bodies of those worlds, one world
-  // after another, and what a world's body ids are off by there; per such body
+  // after another, and what a world's body ids are off by there (NOT_SHARED: a
+  // world without such bodies); per such body
   // its manifolds' pairs and their number, the colouring's word and the
   // velocity words (a line each); per workgroup its manifolds by colour
-  int flow_worlds, flow_groups, flow_min, flow_bodies;
+  int flow_worlds, flow_groups, flow_bodies;
   int32_t *flow_body, *flow_shift;
   int flow_seats, flow_polls;  // most workgroups that join a world; polls of a wait (shp_flow.h)
   int32_t* flow_ctl;
@@ -283,9 +286,8 @@ struct StepPlan {
   // coloured solver: lanes per world, dynamic LDS of the colouring, LDS pool
   int color_threads = 256;
   size_t color_lds = 0, color_pool = 0;
-  // the flow_worlds largest worlds (above flow_min bodies) are solved by up to
-  // flow_groups workgroups each
-  int flow_worlds = 0, flow_groups = 0, flow_min = 0;
+  // the flow_worlds largest worlds are solved by up to flow_groups workgroups each
+  int flow_worlds = 0, flow_groups = 0;
   long flow_bodies = 0;  // of those worlds
   // the contact kernel writes the manifold records itself, after the
   // colouring, instead of beside it with a packing pass after both

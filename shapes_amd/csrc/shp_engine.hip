@@ -428,15 +428,16 @@ __device__ __forceinline__ void sat_pair(const Ctx& c, int p) {
   if (c.solver != SHP_SOLVER_COLORED_F32 && c.flow_worlds == 0) return;
   const int ga = c.pa[p], gb = c.pb[p];
   const int w = c.body_world[ga], b0 = c.body_off[w];
+  const int shift = c.flow_worlds ? c.flow_shift[w] : NOT_SHARED;
   const bool sa = c.is_static[ga] != 0, sb = c.is_static[gb] != 0;
   if (c.solver == SHP_SOLVER_COLORED_F32) {  // the pair's word for the colouring
     const uint32_t a = sa ? NO_BODY : (uint32_t)(ga - b0) & 0xFFFFu;
     const uint32_t b = sb ? NO_BODY : (uint32_t)(gb - b0) & 0xFFFFu;
     c.pair_ab[p] = n > 0 ? a | (b << 16) : NO_PAIR;
   }
-  if (n > 0 && c.flow_worlds && c.body_off[w + 1] - b0 > c.flow_min) {
+  if (n > 0 && shift != NOT_SHARED) {
     // the dynamic bodies' lists of manifolds
-    const int fa = ga + c.flow_shift[w], fb = gb + c.flow_shift[w];
+    const int fa = ga + shift, fb = gb + shift;
     const int ia = sa ? 0 : atomicAdd(&c.adj_n[fa], 1);
     const int ib = sb ? 0 : atomicAdd(&c.adj_n[fb], 1);
     if (!sa && ia < FLOW_DEGREE) c.adj[(long)fa * FLOW_DEGREE + ia] = (uint32_t)p;
@@ -1687,7 +1688,7 @@ shp_status plan_staged(const shp_config& cfg, HostBatch* hb) {
   else
     plan_colored_solver(&P, cfg.solver_threads, body_off, hb->order);
   hb->flow_body.clear();
-  hb->flow_shift.assign(n_worlds, 0);
+  hb->flow_shift.assign(n_worlds, NOT_SHARED);
   for (int k = 0; k < P.flow_worlds; ++k) {
     const int w = hb->order[k];
     hb->flow_shift[w] = (int32_t)hb->flow_body.size() - body_off[w];
@@ -1953,7 +1954,6 @@ shp_status batch_alloc(shp_batch* b, const HostBatch& hb) {
   c.records_in_contacts = P.records_in_contacts ? 1 : 0;
   c.flow_worlds = P.flow_worlds;
   c.flow_groups = P.flow_groups;
-  c.flow_min = P.flow_min;
   c.flow_bodies = (int)P.flow_bodies;
   c.flow_seats = FLOW_ANY_SEATS;
   c.flow_polls = FLOW_POLLS;
