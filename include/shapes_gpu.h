@@ -375,10 +375,11 @@ shp_status shp_batch_read_timing(shp_batch* b, double* ms_per_phase,
  * world: ordered: 0 the schedule's links, 1 velocity and lagrangian staging,
  * 2 -, 3 warm-start pass and sweeps, 4 write-back; coloured: 0 colouring, 1 from
  * its end to the sweeps' start (packing, velocity staging), 2 -, 3 warm-start
- * pass and sweeps, 4 write-back.  A world solved by several workgroups: from the
- * first one's start to the last one's end; ordered: 0 is the loading of the
- * records, 1 and 4 are 0.  All 0 for a world whose sweeps share a workgroup
- * with others (solver_threads 64). */
+ * pass and sweeps, 4 write-back.  A world solved by several workgroups:
+ * ordered: 0 the first one's loading of the records, 3 from there to the last
+ * one's end; coloured: 3 from the sweeps' kernel's start to the next one's; the
+ * others 0.  2 to 4 are 0 for a world whose sweeps share a workgroup with
+ * others (solver_threads 64). */
 shp_status shp_batch_read_solve_profile(shp_batch* b, double* us5);
 
 /* ---- plan and audit of a batch (no counterpart in the reference) -------

@@ -679,9 +679,10 @@ __device__ __forceinline__ void solve_world(const Ctx& c, const Sched<L>& Q, uns
 // the item) whatever its width, where one CU runs the 600 items of a level of
 // an 8192-polygon pile in 7.5 us.  A lane that has seen its body several turns
 // away looks again only that many rounds later, and keeps the address of its
-// body's words (350 us without).  That pile, 8 iterations: 330 us, 1610 on one CU, and 2600 there once its schedule outgrew the LDS (from
-// about 19 k contacts).  Looking in every round took 11 us more; workgroups of 64
-// or 128 lanes instead of 256 the same.
+// body's words (350 us without).  That pile, 8 iterations: 330 us, 1610 on one
+// CU, and 2600 there once its schedule outgrew the LDS (from about 19 k
+// contacts).  Looking in every round took 11 us more; workgroups of 64 or 128
+// lanes instead of 256 the same.
 struct OFlow {
   const Ctx* c;
   int b0, c0;
