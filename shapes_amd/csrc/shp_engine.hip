@@ -918,11 +918,11 @@ __global__ __launch_bounds__(256) void k_cache_store(Ctx c, int n_quality, int n
 }
 
 // Readback of rows [first, first + n) of up to READ_COLS arrays into pinned
-// host memory: n (an int), then from byte 16 on every column, `cap` rows of
-// it (16-byte aligned).  range: when set, the rows are [range[0], range[1])
-// (a world's contacts, whose offsets are on the device); rows beyond `cap`
-// are left out and n says so.  One launch and one wait for what took a
-// blocking copy an array (a world's bodies: 13 us instead of 60).
+// host memory: n and first (ints), then from byte 16 on every column, `cap`
+// rows of it (16-byte aligned).  range: when set, the rows are [range[0],
+// range[1]) (a world's contacts, whose offsets are on the device); more than
+// `cap` rows are not copied, and n says so.  One launch and one wait for what
+// took a blocking copy an array (a world's bodies: 13 us instead of 60).
 enum { READ_COLS = 12 };
 struct ReadArgs {
   const void* src[READ_COLS];
@@ -941,9 +941,9 @@ __host__ __device__ inline size_t read_col_bytes(int bytes, int cap) {
 __global__ __launch_bounds__(256) void k_read_rows(ReadArgs a) {
   const long first = a.range ? a.range[0] : a.first;
   const int n = a.range ? a.range[1] - a.range[0] : a.n;
-  const int rows = n < a.cap ? n : a.cap;
+  const int rows = n <= a.cap ? n : 0;
   const int t0 = blockIdx.x * 256 + threadIdx.x, step = gridDim.x * 256;
-  if (t0 == 0) *(int*)a.out = n;
+  if (t0 == 0) *(int2*)a.out = make_int2(n, (int)first);
   unsigned char* o = a.out + 16;
   for (int k = 0; k < a.cols; ++k) {
     if (a.bytes[k] == 8) {
@@ -2283,8 +2283,7 @@ shp_status shp_batch_read_contacts(shp_batch* b, int32_t world, int32_t* count, 
   if (n == 0 || cols == 0) return SHP_OK;
   std::vector<uint8_t> big;
   if (!fits) {  // array by array
-    int32_t first = 0;
-    HIPCHK(hipMemcpy(&first, c.wcont_off + world, 4, hipMemcpyDeviceToHost));
+    const int32_t first = *(volatile int32_t*)(b->stage + STAGE_FLAGS + 4);
     size_t total = 0;
     for (int k = 0; k < cols; ++k) total += read_col_bytes(bytes[k], n);
     big.resize(total);
