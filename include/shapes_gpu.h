@@ -118,9 +118,10 @@ typedef struct shp_config {
   int32_t broadphase;         /* SHP_BROADPHASE_* */
   int32_t solver_threads;     /* lanes per world in the solve: 0 = by world
                                  size, or 256 or 512, or for the coloured
-                                 solver 1024, or 64: one wavefront per world
-                                 (several per workgroup) for worlds of at most
-                                 1024 bodies and 256 lanes for larger ones (a
+                                 solver 1024, or 64: one wavefront per world,
+                                 or a few, and several worlds per workgroup
+                                 for worlds of at most 1088 bodies, and 256
+                                 lanes for larger ones (a
                                  schedule choice; the results do not depend
                                  on it) */
 } shp_config;

@@ -12,9 +12,9 @@
 // hashed priority is the largest among the uncoloured manifolds on each of
 // its dynamic bodies is selected (the selected manifolds share no dynamic
 // body) and takes the smallest colour that no manifold on its dynamic
-// bodies has (a 16-bit mask per body; past 16 colours, colour 16 + round).  Velocities and constraint rows are FP32
-// (velocities staged in LDS when they fit); the accumulated lagrangians stay
-// FP64; each body's FP64 velocity receives the FP32 change of the solve, so
+// bodies has (a 16-bit mask per body; past 16 colours, colour 16 + round).
+// Velocities and constraint rows are FP32 (velocities staged in LDS when they
+// fit); the accumulated lagrangians stay FP64; each body's FP64 velocity receives the FP32 change of the solve, so
 // bodies without contacts keep their FP64 velocity exactly.
 //
 // Records are per manifold: the normal, materials, inverse masses and
@@ -557,8 +557,8 @@ __device__ __forceinline__ int count_manifolds(const Ctx& c, int p0, int np, int
 // lane + T, ...) held in registers with their bodies, priorities and
 // colours: a round reads only the bodies' priorities and colour masks, a
 // lane's coloured manifolds drop out of its later rounds, and the
-// per-colour counts and manifold slots come from the registers.  The taken count is double-buffered, so a round needs three
-// barriers.  Returns false (colours written to `colour` per pair instead)
+// per-colour counts and manifold slots come from the registers.  The taken
+// count is double-buffered, so a round needs three barriers.  Returns false (colours written to `colour` per pair instead)
 // when the rounds stopped at JP_ROUNDS: the caller then places the serial
 // tail in pair order.
 #define COLOUR_REG_ITEMS 16
