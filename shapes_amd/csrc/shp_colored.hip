@@ -14,8 +14,9 @@
 // body) and takes the smallest colour that no manifold on its dynamic
 // bodies has (a 16-bit mask per body; past 16 colours, colour 16 + round).
 // Velocities and constraint rows are FP32 (velocities staged in LDS when they
-// fit); the accumulated lagrangians stay FP64; each body's FP64 velocity receives the FP32 change of the solve, so
-// bodies without contacts keep their FP64 velocity exactly.
+// fit); the accumulated lagrangians stay FP64; each body's FP64 velocity
+// receives the FP32 change of the solve, so bodies without contacts keep their
+// FP64 velocity exactly.
 //
 // Records are per manifold: the normal, materials, inverse masses and
 // bodies once, then per contact the two cross terms of each row, bias,
@@ -558,9 +559,9 @@ __device__ __forceinline__ int count_manifolds(const Ctx& c, int p0, int np, int
 // colours: a round reads only the bodies' priorities and colour masks, a
 // lane's coloured manifolds drop out of its later rounds, and the
 // per-colour counts and manifold slots come from the registers.  The taken
-// count is double-buffered, so a round needs three barriers.  Returns false (colours written to `colour` per pair instead)
-// when the rounds stopped at JP_ROUNDS: the caller then places the serial
-// tail in pair order.
+// count is double-buffered, so a round needs three barriers.  Returns false
+// (colours written to `colour` per pair instead) when the rounds stopped at
+// JP_ROUNDS: the caller then places the serial tail in pair order.
 #define COLOUR_REG_ITEMS 16
 template <int T>
 __device__ __forceinline__ bool colour_regs(const Ctx& c, int w, int p0, int nm, int nb, uint32_t* s_best,
@@ -1118,7 +1119,8 @@ __global__ __launch_bounds__(64 * SWEEP_WAVES * PARTS) void k_sweep_waves(Ctx c,
 // in LDS and the manifold lists in global memory when the bodies fit, else in
 // global memory.
 template <int T>
-__device__ __forceinline__ void colour_world(const Ctx& c, int w, int p0, int np, int pool_bytes, int* lds, int* sm) {
+__device__ __forceinline__ void colour_world(const Ctx& c, int w, int p0, int np, int pool_bytes,
+                                             int* lds, int* sm) {
   int* s_off = lds;                      // COLOR_CAP + 3
   int* s_cur = lds + (COLOR_CAP + 3);    // COLOR_CAP + 3
   unsigned char* pool = (unsigned char*)(lds + 2 * (COLOR_CAP + 3) + 2);
@@ -1166,10 +1168,8 @@ __device__ __forceinline__ void colour_world(const Ctx& c, int w, int p0, int np
 // to one workgroup: *last tells the one that has to colour it.
 constexpr int FLOW_ITEMS = 8192, FLOW_COLOUR_LANES = 256;
 
-// given_up: FC_BAD as one lane has read it for the workgroup; another one may set
-// it meanwhile, and all wavefronts have to take the same way past the barriers.
 __device__ __forceinline__ void colour_flow(const Ctx& c, int w, int p0, int np, int seat, int groups,
-                                            int rows, bool given_up, int* lds, bool* last) {
+                                            int rows, int* lds, bool* last) {
   constexpr int AGENT = __HIP_MEMORY_SCOPE_AGENT, T = FLOW_COLOUR_LANES;
   int* s_cnt = lds;                 // FLOW_DEGREE
   int* s_last = lds + FLOW_DEGREE;
@@ -1182,9 +1182,12 @@ __device__ __forceinline__ void colour_flow(const Ctx& c, int w, int p0, int np,
   const int tid = threadIdx.x, f0 = c.body_off[w] + c.flow_shift[w];
   const int per = ((np + groups - 1) / groups + 63) & ~63;
   const int q0 = seat * per, n = min(per, np - q0);
-  const bool fits = per <= FLOW_ITEMS;
+  // The same for all wavefronts, whose barriers depend on it: FC_FULL is k_sat's
+  // and stays as it is during this kernel, while FC_BAD is set by any workgroup
+  // of the world at any time.
+  const bool fits = per <= FLOW_ITEMS && ctl[FC_FULL] == 0;
   if (tid < FLOW_DEGREE) s_cnt[tid] = 0;
-  if (fits && !given_up) {
+  if (fits) {
     auto key = [&](uint32_t q) {  // orders like prio64
       return (unsigned long long)(mix32(q * 0x9E3779B9u + (uint32_t)w) & 0x7FFFu) << 32 | q;
     };
@@ -1370,14 +1373,11 @@ __global__ __launch_bounds__(T) void k_colour(Ctx c, int pool_bytes) {
     const int want = flow_want(c, w, c.flow_groups);
     if (blk % c.flow_groups >= want) return;
     int groups;
-    const int bad = threadIdx.x == 0 ? peek(ctl + FC_BAD) : 0;  // on its way while they join
     const int seat = flow_join(c, ctl + FC_SEATS, ctl + FC_GROUPS, blk % c.flow_groups, want, sm,
                                &groups);
     if (seat < 0) return;
-    if (threadIdx.x == 0) sm[2] = bad;
-    __syncthreads();
     bool last;
-    colour_flow(c, w, p0, np, seat, groups, blk / c.flow_groups * c.flow_groups, sm[2] != 0, lds, &last);
+    colour_flow(c, w, p0, np, seat, groups, blk / c.flow_groups * c.flow_groups, lds, &last);
     if (!last) return;
   }
   colour_world<T>(c, w, p0, np, pool_bytes, lds, sm);

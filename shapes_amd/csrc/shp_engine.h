@@ -57,7 +57,8 @@ enum { FLOW_ORDERED_MIN_BODIES = 3072, FLOW_ORDERED_PAIRS = 128, FLOW_ORDERED_GR
 enum { FLOW_MIN_BODIES = 2048, FLOW_GROUP_BODIES = 64, FLOW_GROUP_MAX = 384,
        FLOW_MAX_GROUPS = 256, FLOW_DEGREE = 32, FLOW_CTL = 32, FLOW_LINE = 16 };
 enum { FC_SEATS = 0, FC_GROUPS = 1, FC_DONE = 2, FC_BAD = 3, FS_SEATS = 4, FS_GROUPS = 5,
-       FS_ABORT = 6, FS_ALONE = 7, FC_ROWS = 8, FC_SHARE = 9 };
+       FS_ABORT = 6, FS_ALONE = 7, FC_ROWS = 8, FC_SHARE = 9,
+       FC_FULL = 10 };
 // col_info: colours | serial tail << 16 | flow schedule << 17 (then sched_level
 // holds colours and places, and sched_order is written by the packing pass)
 enum { COL_TAIL = 1 << 16, COL_FLOW = 1 << 17 };

@@ -442,7 +442,7 @@ __device__ __forceinline__ void sat_pair(const Ctx& c, int p) {
     const int ib = sb ? 0 : atomicAdd(&c.adj_n[fb], 1);
     if (!sa && ia < FLOW_DEGREE) c.adj[(long)fa * FLOW_DEGREE + ia] = (uint32_t)p;
     if (!sb && ib < FLOW_DEGREE) c.adj[(long)fb * FLOW_DEGREE + ib] = (uint32_t)p;
-    if (max(ia, ib) >= FLOW_DEGREE) c.flow_ctl[w * FLOW_CTL + FC_BAD] = 1;
+    if (max(ia, ib) >= FLOW_DEGREE) c.flow_ctl[w * FLOW_CTL + FC_FULL] = 1;
   }
 }
 

@@ -720,7 +720,7 @@ __global__ __launch_bounds__(256) void k_solve_flow(Ctx c) {
   if (np == 0) return;
   // bodies of too many manifolds, too many pairs, or contacts beyond the
   // capacity: k_solve_ordered
-  if (peek(ctl + FC_BAD) != 0 || want > c.flow_groups || c.coff[p0 + np] > c.contact_cap) {
+  if (ctl[FC_FULL] != 0 || want > c.flow_groups || c.coff[p0 + np] > c.contact_cap) {
     if (blk == 0 && threadIdx.x == 0) ctl[FS_ALONE] = 1;
     return;
   }
